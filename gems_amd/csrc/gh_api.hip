@@ -1362,13 +1362,15 @@ struct StepRec {
 }  // namespace
 
 static int finish_mid_step(gh_ctx *c) {
-  // the stopped step's forces (the list re-sized if needed) and its stepb
-  GH_TRY(interact(c));
-  GH_TRY(check_status(c));
-  GH_TRY(c->integ == GH_INT_ERMAK ? gh_launch_ermak_b(c) : gh_launch_vv_b(c));
+  // the stopped step's forces (the list re-sized if needed) and its stepb,
+  // under that step's number (its displacement maximum, its random numbers)
   c->step += 1;
-  c->mid_step = false;
-  return 0;
+  int rc = interact(c);
+  if (rc == 0) rc = check_status(c);
+  if (rc == 0) rc = c->integ == GH_INT_ERMAK ? gh_launch_ermak_b(c) : gh_launch_vv_b(c);
+  if (rc == 0) c->mid_step = false;
+  else c->step -= 1;
+  return rc;
 }
 
 #ifndef GH_CHAIN_AHEAD

@@ -138,7 +138,11 @@ struct TileGeom {
 #define GH_LIST_PAD_QUADS 2
 
 struct GhStatus {                     // device-resident counters
-  unsigned long long maxdisp2_bits;   // max |dx|^2 since the last build
+  // max |dx|^2 since the last build, as step s finds it in [s & 1]: what moves
+  // the atoms into step s folds its workgroup maxima (and the maximum of step
+  // s - 1) there, and step s's own force pass, which may move them on to step
+  // s + 1 while later workgroups of it still test the rule, into the other
+  unsigned long long maxdisp2_bits[2];
   int rebuild;                        // rebuild at this step
   int overflow;                       // a row exceeded the capacity (sticky)
   int maxnn;                          // longest row at the last build
@@ -310,12 +314,8 @@ struct FuseVV {
   double *vel;
   const double *xold;
   double4 *pos_next;
-  unsigned long long *maxd2;  // GhStatus::maxdisp2_bits
   int ncap;
 };
-
-// Device address of the displacement maximum the integrators fold into.
-inline unsigned long long *gh_maxd2(gh_ctx *c) { return &c->status->maxdisp2_bits; }
 
 // launchers (gh_kernels.hip)
 int gh_launch_rebuild(gh_ctx *c, bool force);

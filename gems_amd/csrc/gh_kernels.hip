@@ -41,8 +41,8 @@ __global__ void k_fill_int(int *__restrict__ p, int v, int n) {
 // once while GhStatus::halt is set (raise_halt).
 // ---------------------------------------------------------------------------
 // Decision of the O(N^2) list mode (one thread).
-__global__ void k_decide(GhStatus *st, double skin) {
-  st->rebuild = !st->halt && rebuild_due(st, skin);
+__global__ void k_decide(GhStatus *st, double skin, long long step) {
+  st->rebuild = !st->halt && rebuild_due(st, skin, step);
   rebuild_book(st);
 }
 
@@ -509,14 +509,14 @@ struct WrapArgs {
 // copied out, which reproduces do_pbc_1 (Set_Properties.f90:444-470).
 // Workgroup maximum of |x - x_old|^2 folded into the device-wide maximum with
 // one atomicMax (no fence: the next kernel reads it).
-__device__ __forceinline__ void disp_reduce(double d2, unsigned long long *__restrict__ maxd2) {
+__device__ __forceinline__ void disp_reduce(double d2, GhStatus *st, long long step) {
   __shared__ double part[GH_BLOCK / 64];
   d2 = wave_max(d2);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = d2;
   __syncthreads();
   if (threadIdx.x == 0) {
     for (int w = 1; w < GH_BLOCK / 64; ++w) d2 = fmax(d2, part[w]);
-    atomicMax(maxd2, (unsigned long long)__double_as_longlong(d2));
+    fold_disp2(st, d2, step);
   }
 }
 
@@ -525,7 +525,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_vv_a(
     int n, int ncap, double dt, MassArgs ma,
     const int *__restrict__ type, double4 *__restrict__ pos, double *__restrict__ vel,
     double *__restrict__ acc, const double *__restrict__ frc, const double *__restrict__ xold,
-    GhStatus *st) {
+    GhStatus *st, long long step) {
   if (halted(st)) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double d2 = 0.0;
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_vv_a(
     p.z = x[2];
     pos[i] = p;
   }
-  disp_reduce(d2, &st->maxdisp2_bits);
+  disp_reduce(d2, st, step);
 }
 
 // velocity_verlet_b of one step fused with velocity_verlet_a of the next
@@ -559,7 +559,8 @@ __global__ __launch_bounds__(GH_BLOCK) void k_vv_a(
 __global__ __launch_bounds__(GH_BLOCK) void k_vv_ba(
     int n, int ncap, double dt, MassArgs ma,
     const int *__restrict__ type, double4 *__restrict__ pos, double *__restrict__ vel,
-    const double *__restrict__ frc, const double *__restrict__ xold, GhStatus *st) {
+    const double *__restrict__ frc, const double *__restrict__ xold, GhStatus *st,
+    long long step) {
   if (halted(st)) return;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double d2 = 0.0;
@@ -582,7 +583,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_vv_ba(
     p.z = x[2];
     pos[i] = p;
   }
-  disp_reduce(d2, &st->maxdisp2_bits);
+  disp_reduce(d2, st, step);
 }
 
 // velocity_verlet_b (Integration.F90:1171-1186).
@@ -631,6 +632,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_ermak_a(
     const double *__restrict__ vel, const double *__restrict__ acc,
     const double *__restrict__ xold, GhStatus *st) {
   if (halted(st)) return;
+  const long long step = k.step;
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   double d2 = 0.0;
   if (i < n) {
@@ -651,7 +653,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_ermak_a(
     p.z = x[2];
     pos[i] = p;
   }
-  disp_reduce(d2, &st->maxdisp2_bits);
+  disp_reduce(d2, st, step);
 }
 
 // ermak_b (Integration.F90:1013-1031); vel_v is re-derived from the same
@@ -811,8 +813,7 @@ __global__ void k_wrap(int n, WrapArgs wa, double4 *__restrict__ pos) {
 // the rebuild test.
 __global__ __launch_bounds__(GH_BLOCK) void k_set_positions(
     int n, int ncap, WrapArgs wa, const int *__restrict__ orig, const double *__restrict__ x,
-    double4 *__restrict__ pos, const double *__restrict__ xold,
-    unsigned long long *__restrict__ maxd2) {
+    double4 *__restrict__ pos, const double *__restrict__ xold, GhStatus *st, long long step) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
   double d2 = 0.0;
   if (s < n) {
@@ -831,7 +832,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_set_positions(
     p.z = v[2];
     pos[s] = p;
   }
-  disp_reduce(d2, maxd2);
+  disp_reduce(d2, st, step);
 }
 
 __global__ void k_wrap_rebuild(const GhStatus *st, int n, WrapArgs wa,
@@ -932,7 +933,7 @@ int gh_launch_rebuild(gh_ctx *c, bool force) {
   if (force) GH_TRY(gh_request_rebuild(c));
   const int n = c->n, nb = nblocks(n);
   if (c->list_mode == 1) return gh_launch_rebuild_cells(c);  // decides in its first kernels
-  { k_decide<<<1, 1, 0, s>>>(c->status, c->skin); ++c->launches; }
+  { k_decide<<<1, 1, 0, s>>>(c->status, c->skin, c->step); ++c->launches; }
   if (c->list_mode == 0 && c->boxed && (c->pbc[0] || c->pbc[1] || c->pbc[2]))
     { k_wrap_rebuild<<<nb, GH_BLOCK, 0, s>>>(c->status, n, make_wrap(c), c->pos); ++c->launches; }
   const GridArgs g = make_grid(c);
@@ -1048,7 +1049,8 @@ int gh_launch_forces(gh_ctx *c, hipEvent_t mid, bool fuse_vv) {
 int gh_launch_vv_a(gh_ctx *c) {
   { k_vv_a<<<nblocks(c->n), GH_BLOCK, 0, c->stream>>>(c->n, c->ncap, c->dt,
                                                     make_mass(c), c->type, c->pos, c->vel,
-                                                    c->acc, c->frc, c->xold, c->status); ++c->launches; }
+                                                    c->acc, c->frc, c->xold, c->status,
+                                                    c->step); ++c->launches; }
   GH_HIP(c, hipGetLastError());
   return 0;
 }
@@ -1056,7 +1058,8 @@ int gh_launch_vv_a(gh_ctx *c) {
 int gh_launch_vv_ba(gh_ctx *c) {
   { k_vv_ba<<<nblocks(c->n), GH_BLOCK, 0, c->stream>>>(c->n, c->ncap, c->dt,
                                                      make_mass(c), c->type, c->pos, c->vel,
-                                                     c->frc, c->xold, c->status); ++c->launches; }
+                                                     c->frc, c->xold, c->status,
+                                                     c->step); ++c->launches; }
   GH_HIP(c, hipGetLastError());
   return 0;
 }
@@ -1107,7 +1110,8 @@ int gh_launch_energies(gh_ctx *c, double *epot_ui, double *ekin_ui) {
 
 int gh_launch_set_positions(gh_ctx *c, const double *x_dev) {
   { k_set_positions<<<nblocks(c->n), GH_BLOCK, 0, c->stream>>>(
-      c->n, c->ncap, make_wrap(c), c->orig, x_dev, c->pos, c->xold, gh_maxd2(c)); ++c->launches; }
+      c->n, c->ncap, make_wrap(c), c->orig, x_dev, c->pos, c->xold, c->status,
+      c->step); ++c->launches; }
   GH_HIP(c, hipGetLastError());
   return 0;
 }
@@ -1163,7 +1167,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_static_init(unsigned char *scr, in
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   GhStatus *st = reinterpret_cast<GhStatus *>(scr);
   if (i == 0) {
-    st->maxdisp2_bits = 0ull;
+    st->maxdisp2_bits[0] = st->maxdisp2_bits[1] = 0ull;
     st->rebuild = 1;
     st->overflow = 0;
     st->maxnn = 0;

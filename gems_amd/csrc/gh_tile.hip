@@ -206,9 +206,11 @@ __device__ __forceinline__ double fused_vv(const FuseVV &f, int a, const double4
   return fused_vv(f, a, p, t, Fx, Fy, Fz, vv_load(f, a));
 }
 
-// Workgroup maximum of d2, stored at dst[b] (all threads call it).
-// Workgroup maximum of |x - x_old|^2 folded into the device-wide maximum.
-__device__ __forceinline__ void block_max_atomic(double d2, unsigned long long *maxd2) {
+// Workgroup maximum of |x - x_old|^2 of the positions a fused pass of `step`
+// has just written, folded into the maximum the next step tests: the pass's
+// own test (step_gate) reads the other one, so a workgroup that starts late
+// decides as the first one did.  All threads call it.
+__device__ __forceinline__ void block_max_atomic(double d2, GhStatus *st, long long step) {
   __shared__ double part[GH_TBMAX / 64];
   d2 = wave_max(d2);
   if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = d2;
@@ -216,7 +218,7 @@ __device__ __forceinline__ void block_max_atomic(double d2, unsigned long long *
   if (threadIdx.x == 0) {
     const int nw = (int)(blockDim.x >> 6);
     for (int w = 1; w < nw; ++w) d2 = fmax(d2, part[w]);
-    atomicMax(maxd2, (unsigned long long)__double_as_longlong(d2));
+    fold_disp2(st, d2, step + 1);
   }
 }
 
@@ -706,7 +708,7 @@ __global__ __launch_bounds__(GH_BINBLOCK) void k_cell_bin(GhStatus *st,
                                                         const ChainArgs *__restrict__ C,
                                                         double4 *pos, double skin,
                                                         long long step) {
-  const bool due = !st->halt && rebuild_due(st, skin);
+  const bool due = !st->halt && rebuild_due(st, skin, step);
   if (blockIdx.x == 0 && threadIdx.x == 0) st->rebuild = due ? 1 : 0;
   if (!due) return;
   const CellArgs &R = C->R;
@@ -1173,11 +1175,11 @@ struct StepArgs {
 };
 __device__ __forceinline__ bool step_gate(GhStatus *st, const StepArgs &sa) {
   const int h = halted(st);
-  const bool stop = h || rebuild_due(st, sa.skin);
+  const bool stop = h || rebuild_due(st, sa.skin, sa.step);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (stop && !h) raise_halt(st, GH_HALT_REBUILD, sa.step);
     step_publish(sa.prog, sa.step, h ? h : (stop ? GH_HALT_REBUILD : 0),
-                 h ? st->halt_step : sa.step, st->maxdisp2_bits);
+                 h ? st->halt_step : sa.step, st->maxdisp2_bits[sa.step & 1]);
   }
   return stop;
 }
@@ -1393,7 +1395,7 @@ __device__ __forceinline__ void tb_force_fx_body(
       epa[a] = (ei - sqrt(rho[a])) * ev_ui;
     }
   }
-  if (FUSED) block_max_atomic(dmax2, fv.maxd2);
+  if (FUSED) block_max_atomic(dmax2, st, step);
 }
 template <bool SINGLE, bool FUSED, int S, int G>
 __global__ __launch_bounds__(GH_TBMAX) void k_tb_force_fx(
@@ -1556,7 +1558,7 @@ __device__ __forceinline__ void tb_force64_body(
       epa[a] = (ei - sqrt(rho[a])) * ev_ui;
     }
   }
-  if (fv.on) block_max_atomic(dmax2, fv.maxd2);
+  if (fv.on) block_max_atomic(dmax2, st, step);
 }
 template <bool SINGLE, int G>
 __global__ __launch_bounds__(GH_TBMAX) void k_tb_force64_tiled(
@@ -1688,7 +1690,7 @@ __device__ __forceinline__ void lj_tiled_body(
       epa[a] = ei * 0.5 * ev_ui;
     }
   }
-  if (FUSED) block_max_atomic(dmax2, fv.maxd2);
+  if (FUSED) block_max_atomic(dmax2, st, step);
 }
 // One pass per step: gated (and publishing) as a first pass.
 template <bool MIXED, int POT, bool FUSED, int G>
@@ -1800,7 +1802,7 @@ __global__ __launch_bounds__(GH_TBMAX) void k_lj_fx(
       epa[a] = ei * 0.5 * ev_ui;
     }
   }
-  if (FUSED) block_max_atomic(dmax2, fv.maxd2);
+  if (FUSED) block_max_atomic(dmax2, st, sa.step);
 }
 
 }  // namespace
@@ -2039,7 +2041,6 @@ int gh_launch_forces_tiled(gh_ctx *c, hipEvent_t mid, bool fuse_vv) {
   fv.vel = c->vel;
   fv.xold = c->xold;
   fv.pos_next = c->pos_next;
-  fv.maxd2 = gh_maxd2(c);
   fv.ncap = c->ncap;
   const int grid = xgrid(c->tg.nbrick * c->tg.chunks);
   const int ld = c->ncap;

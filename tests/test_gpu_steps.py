@@ -162,3 +162,38 @@ def test_atom_outside_grid_reported_then_recovers():
     Fo, _, epo, _ = O.smatb_force(f["x"], f["types"], box, s, nn, lst)
     assert cm.force_err(F, Fo) <= 1e-10
     c.close()
+
+
+@pytest.mark.parametrize("prec", [hip.GH_FP64, hip.GH_MIXED], ids=["fp64", "mixed"])
+def test_fused_pass_of_many_workgroups_moves_every_atom(prec):
+    """A pair potential's fused pass moves its atoms while later workgroups of
+    the same launch (here ~2000, more than the chip holds at once) still test
+    the rebuild rule: they decide on the step's own displacement maximum.  A
+    hot liquid (a rebuild every few steps) stepped fused against the same
+    steps with an energy row each (separate update kernels): the two differ by
+    rounding alone, so 40 steps apart they agree far below 1e-9 sigma; a
+    workgroup that skips one step leaves its atoms off by v dt ~ 1e-2."""
+    a = (4.0 / 0.8442) ** (1.0 / 3.0)
+    x = cm.fcc(48, a) + np.random.default_rng(7).normal(0.0, 0.02, (4 * 48 ** 3, 3))
+    L = 48 * a
+    x = np.mod(x, L)
+    out = []
+    for each in (0, 1):
+        with hip.Context(0, prec) as c:
+            c.set_box([L] * 3, (1, 1, 1))
+            c.set_atoms(x)
+            c.set_masses([1.0])
+            c.set_lj(1.0, 1.0, 2.5)
+            c.set_skin(0.3)
+            c.set_tile((3, 2, 2))
+            c.prng_lcg(31)
+            c.set_gdist(1.5 / 8.617385e-05)
+            c.integrator_vv(0.005 * 0.01018047)
+            for _ in range(3):
+                c.run(40, each=each)
+            out.append(c.state()[:2] + (c.stats()["nupd"],))
+    print("rebuilds", out[0][2], out[1][2])
+    assert out[0][2] == out[1][2] >= 6
+    d = out[0][0] - out[1][0]
+    d -= L * np.round(d / L)
+    assert np.max(np.abs(d)) < (1e-9 if prec == hip.GH_FP64 else 1e-3)
