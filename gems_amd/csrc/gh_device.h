@@ -10,9 +10,9 @@
 namespace ghd {
 
 // Rebuild test of step `step` on the displacement maximum the integrators
-// fold into GhStatus::maxdisp2_bits (one atomicMax per workgroup).
+// fold into GhStatus::maxdisp2 (one atomicMax per workgroup).
 __device__ __forceinline__ bool rebuild_due(const GhStatus *st, double skin, long long step) {
-  const double d2 = __longlong_as_double((long long)st->maxdisp2_bits[step & 1]);
+  const double d2 = __longlong_as_double((long long)st->maxdisp2[step & 1].bits);
   return st->force_rebuild || 2.0 * sqrt(d2) > skin;
 }
 
@@ -26,16 +26,17 @@ __device__ __forceinline__ void rebuild_book(GhStatus *st) {
     st->nupd += 1;
     st->force_rebuild = 0;
     st->maxnn = 0;
-    st->maxdisp2_bits[0] = st->maxdisp2_bits[1] = 0ull;
+    st->maxdisp2[0].bits = st->maxdisp2[1].bits = 0ull;
   }
 }
 
 // Folds a workgroup's largest |x - x_old|^2 of the positions of step `step`
-// into that step's running maximum, which continues the one of step - 1.
+// into that step's running maximum; the grid's first workgroup carries the
+// maximum of step - 1 on.
 __device__ __forceinline__ void fold_disp2(GhStatus *st, double d2, long long step) {
-  const unsigned long long b = (unsigned long long)__double_as_longlong(d2);
-  const unsigned long long before = st->maxdisp2_bits[(step & 1) ^ 1];
-  atomicMax(&st->maxdisp2_bits[step & 1], b > before ? b : before);
+  unsigned long long b = (unsigned long long)__double_as_longlong(d2);
+  if (blockIdx.x == 0) b = max(b, st->maxdisp2[(step & 1) ^ 1].bits);
+  atomicMax(&st->maxdisp2[step & 1].bits, b);
 }
 
 // Stops the run at `step` (the first raiser wins and records the step):

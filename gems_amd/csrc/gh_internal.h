@@ -137,12 +137,18 @@ struct TileGeom {
 // list traversals prefetch two quads ahead without a bounds clamp.
 #define GH_LIST_PAD_QUADS 2
 
+struct alignas(128) GhLine {          // a word that owns its cache line
+  unsigned long long bits;
+};
+
 struct GhStatus {                     // device-resident counters
   // max |dx|^2 since the last build, as step s finds it in [s & 1]: what moves
   // the atoms into step s folds its workgroup maxima (and the maximum of step
   // s - 1) there, and step s's own force pass, which may move them on to step
   // s + 1 while later workgroups of it still test the rule, into the other
-  unsigned long long maxdisp2_bits[2];
+  // (on cache lines of their own: thousands of workgroups read the one while
+  // others update the other atomically, 70-100 us per 1M-atom pass on a shared line)
+  GhLine maxdisp2[2];
   int rebuild;                        // rebuild at this step
   int overflow;                       // a row exceeded the capacity (sticky)
   int maxnn;                          // longest row at the last build

@@ -34,7 +34,7 @@ __global__ void k_fill_int(int *__restrict__ p, int v, int n) {
 // rebuilds when the two largest displacements since the last build sum past
 // the skin.  Here the displacement is the true (minimum-image) one, and the
 // test uses 2*max, which bounds d1+d2 from above.  Integrators fold each
-// workgroup's max |x - x_old|^2 into GhStatus::maxdisp2_bits with one
+// workgroup's max |x - x_old|^2 into GhStatus::maxdisp2 with one
 // atomicMax (non-negative doubles order as their bit patterns); it runs over
 // the steps since the last build and the first kernel of a rebuild sequence
 // reads it (rebuild_due, rebuild_book).  State-changing kernels return at
@@ -1167,7 +1167,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_static_init(unsigned char *scr, in
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   GhStatus *st = reinterpret_cast<GhStatus *>(scr);
   if (i == 0) {
-    st->maxdisp2_bits[0] = st->maxdisp2_bits[1] = 0ull;
+    st->maxdisp2[0].bits = st->maxdisp2[1].bits = 0ull;
     st->rebuild = 1;
     st->overflow = 0;
     st->maxnn = 0;

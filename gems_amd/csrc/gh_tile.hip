@@ -1179,7 +1179,7 @@ __device__ __forceinline__ bool step_gate(GhStatus *st, const StepArgs &sa) {
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     if (stop && !h) raise_halt(st, GH_HALT_REBUILD, sa.step);
     step_publish(sa.prog, sa.step, h ? h : (stop ? GH_HALT_REBUILD : 0),
-                 h ? st->halt_step : sa.step, st->maxdisp2_bits[sa.step & 1]);
+                 h ? st->halt_step : sa.step, st->maxdisp2[sa.step & 1].bits);
   }
   return stop;
 }
