@@ -172,33 +172,42 @@ int gh_upload_tbf(gh_ctx *c, int k) {
   return 0;
 }
 
+void gh_tbdev_fill(const GhTbPair &t, double e0, TbDev &o) {
+  const double log2e = 1.4426950408889634;
+  Tb64 &d = o.d;
+  d.r0 = t.r0;
+  d.rci = t.rci;
+  d.rce = t.rce;
+  d.rce2 = t.rce * t.rce;
+  d.eps2 = t.xi * t.xi;
+  d.cq = -2.0 * t.q / t.r0 * log2e;
+  d.ca = t.A;
+  d.cp = -t.p / t.r0 * log2e;
+  d.fa = 2.0 * t.A * t.p / t.r0;
+  d.fb = t.xi * t.xi * t.q / t.r0;
+  d.b1 = t.b1;
+  d.b2 = t.b2;
+  d.b3 = t.b3;
+  d.b1x5 = 5.0 * t.b1;
+  d.b2x4 = 4.0 * t.b2;
+  d.b3x3 = 3.0 * t.b3;
+  d.r1 = t.r1;
+  d.r2 = t.r2;
+  d.r3 = t.r3;
+  d.r1m10 = -10.0 * t.r1;
+  d.r2m8 = -8.0 * t.r2;
+  d.r3m6 = -6.0 * t.r3;
+  gh_tbf_fill(t, 0, e0, o.f);
+}
+
 int gh_upload_tb(gh_ctx *c) {
   TbDev h[GH_MAXT * GH_MAXT];
   memset(h, 0, sizeof(h));
   c->tb_e0 = gh_tb_e0(c->tb);
   for (int a = 0; a < c->nt; ++a)
-    for (int b = 0; b < c->nt; ++b) {
-      const GhTbPair &t = c->tb[a * GH_MAXT + b];
-      TbDev &d = h[a * GH_MAXT + b];
-      d.ca = t.A;
-      d.eps2 = t.xi * t.xi;
-      d.p = t.p;
-      d.q = t.q;
-      d.r0 = t.r0;
-      d.one_r0 = 1.0 / t.r0;
-      d.rci = t.rci;
-      d.rce = t.rce;
-      d.rce2 = t.rce * t.rce;
-      d.b1 = t.b1;
-      d.b2 = t.b2;
-      d.b3 = t.b3;
-      d.r1 = t.r1;
-      d.r2 = t.r2;
-      d.r3 = t.r3;
-      d.p_r0 = t.p / t.r0;
-      d.q2_r0 = 2.0 * t.q / t.r0;
-      gh_tbf_fill(t, 0, c->tb_e0, d.f);
-    }
+    for (int b = 0; b < c->nt; ++b)
+      gh_tbdev_fill(c->tb[a * GH_MAXT + b], c->tb_e0, h[a * GH_MAXT + b]);
+  c->tb64_0 = h[0].d;
   GH_TRY(dalloc(c, &c->tbd, GH_MAXT * GH_MAXT));
   // ordered on the context's stream (a non-blocking stream does not wait for
   // null-stream copies); h lives until the stream has drained

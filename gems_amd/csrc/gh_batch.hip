@@ -255,8 +255,12 @@ __device__ void sys_forces(const BatchArgs &B, const Sys &S) {
           float band;
           if (tb_rho_fx(P.f, fma(vx, vx, fma(vy, vy, vz * vz)), band)) acc += (double)band;
         } else {
-          const double dr = sqrt(dist2_rn(vx, vy, vz));
-          if (dr <= P.rce) acc += tb_band64(P, dr);
+          const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+          if (rd <= P.d.rce2) {
+            double dr, ir;
+            sqrt_rsq64(rd, dr, ir);
+            acc += tb_band64(P.d, dr);
+          }
         }
       });
     }
@@ -323,14 +327,15 @@ __device__ void sys_forces(const BatchArgs &B, const Sys &S) {
             ei += (double)repul;
           }
         } else {
-          const double dr = sqrt(dist2_rn(vx, vy, vz));
-          if (dr <= P.rce) {
-            double factor, repul;
-            tb_pair64(P, dr, ebi + B.eband[j], factor, repul);
-            const double sf = factor / dr;
-            fxs -= sf * vx;
-            fys -= sf * vy;
-            fzs -= sf * vz;
+          const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+          if (rd <= P.d.rce2) {
+            double dr, ir, factor, repul;
+            sqrt_rsq64(rd, dr, ir);
+            tb_pair64(P.d, dr, ebi + B.eband[j], factor, repul);
+            const double sf = factor * ir;
+            fxs = fma(-sf, vx, fxs);
+            fys = fma(-sf, vy, fys);
+            fzs = fma(-sf, vz, fzs);
             ei += repul;
           }
         }

@@ -95,39 +95,102 @@ __device__ __forceinline__ double dist2_rn(double x, double y, double z) {
   return __dadd_rn(__dadd_rn(__dmul_rn(x, x), __dmul_rn(y, y)), __dmul_rn(z, z));
 }
 
-__device__ __forceinline__ void load_params(TbDev *sp, const TbDev *__restrict__ tbd, int nt) {
+// The parameter blocks of every type pair (FP64 forms, or both forms) to LDS.
+__device__ __forceinline__ void load_params(Tb64 *sp, const TbDev *__restrict__ tbd, int nt) {
   for (int k = threadIdx.x; k < GH_MAXT * GH_MAXT; k += blockDim.x) {
     int a = k / GH_MAXT, b = k % GH_MAXT;
-    if (a < nt && b < nt) sp[k] = tbd[k];
+    if (a < nt && b < nt) sp[k] = tbd[k].d;
+  }
+}
+__device__ __forceinline__ void load_params(TbF *sp, const TbDev *__restrict__ tbd, int nt) {
+  for (int k = threadIdx.x; k < GH_MAXT * GH_MAXT; k += blockDim.x) {
+    int a = k / GH_MAXT, b = k % GH_MAXT;
+    if (a < nt && b < nt) sp[k] = tbd[k].f;
   }
 }
 
 // ---------------------------------------------------------------------------
-// SMA-TB pair terms (TB.F90:405-423 density, 493-531 force), for r <= rce.
-// FP64 form: the reference's arithmetic.  FP32 form: see TbDev.
+// FP64 building blocks of the pair terms.  The IEEE square root, the division
+// and the library exponential cost about 15, 12 and 28 instructions each; a
+// pair needs one root, one or two exponentials and one to three divisions,
+// and these passes are bound by VALU issue.  With the forms below instead:
+// FP64 LJ pass (fused) 239 -> 136 us at 1,048,571 atoms, 17.7 -> 13.2 at
+// 4,000; the SMA-TB density and force passes 150 -> 110 and 210 -> 159 us at
+// 1,000,188 Au atoms; plj 117 -> 85 us at 256,000.  Forces differ from 64-bit
+// references by as much as before (1.5e-13 after 200 steps of Au 32k).
+//
+// r = sqrt(x) and y = 1/sqrt(x) from the hardware estimate y0 (relative error
+// e/2 < 2^-23, e = 1 - x y0^2): 1/sqrt(1 - e) = 1 + e/2 + 3e^2/8 + O(e^3), the
+// remainder below 2^-66.  r is the estimate x y0 plus a correction from its
+// exact residual (half an ulp), y is within one ulp.  x = 0 gives r = 0 and
+// y = inf (the clamp keeps x y0 finite), NaN gives NaN.
 // ---------------------------------------------------------------------------
-__device__ __forceinline__ double tb_band64(const TbDev &P, double dr) {
-  if (dr < P.rci) return P.eps2 * exp(-2.0 * P.q * (dr * P.one_r0 - 1.0));
+__device__ __forceinline__ void sqrt_rsq64(double x, double &r, double &y) {
+  const double y0 = fmin(__builtin_amdgcn_rsq(x), 1e308);
+  const double h = x * y0;
+  const double e = fma(-h, y0, 1.0);
+  const double c = fma(0.375, e, 0.5);
+  r = fma(fma(-h, h, x) * y0, c, h);
+  y = fma(y0 * e, c, y0);
+}
+// 1/x from the hardware estimate y0 (e = 1 - x y0, |e| < 2^-22): y0 (1 + e +
+// e^2), the remainder below 2^-66.  x = 0 gives a huge finite value (the
+// clamp), NaN gives NaN.
+__device__ __forceinline__ double rcp64(double x) {
+  const double y0 = fmin(__builtin_amdgcn_rcp(x), 1e100);
+  const double e = fma(-x, y0, 1.0);
+  return fma(y0 * e, 1.0 + e, y0);
+}
+// 2^t: t = n + f with |f| <= 1/2 (n from the rounding of t + 1.5 2^52, whose
+// low word is n), 2^f by interpolation at the Chebyshev points of degree 11
+// (remainder 3e-18), scaled by the exponent instruction (overflow and
+// underflow included).
+__device__ __forceinline__ double exp2_64(double t) {
+  const double m = t + 6755399441055744.0;
+  const int n = __double2loint(m);
+  const double f = t - (m - 6755399441055744.0);
+  double q = 4.4558179083360645e-10;
+  q = fma(q, f, 7.074194297288521e-09);
+  q = fma(q, f, 1.0178057087733941e-07);
+  q = fma(q, f, 1.3215432535912375e-06);
+  q = fma(q, f, 1.5252733841556773e-05);
+  q = fma(q, f, 0.00015403530463724353);
+  q = fma(q, f, 0.001333355814640647);
+  q = fma(q, f, 0.009618129107587256);
+  q = fma(q, f, 0.055504108664821625);
+  q = fma(q, f, 0.24022650695910158);
+  q = fma(q, f, 0.6931471805599453);
+  q = fma(q, f, 1.0);
+  return __builtin_amdgcn_ldexp(q, n);
+}
+
+// ---------------------------------------------------------------------------
+// SMA-TB pair terms (TB.F90:405-423 density, 493-531 force), for r <= rce.
+// FP64 form; the FP32 form: see TbF.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ double tb_band64(const Tb64 &P, double dr) {
+  if (dr < P.rci) return P.eps2 * exp2_64(P.cq * (dr - P.r0));
   const double d = dr - P.rce;
-  const double d2 = d * d, d3 = d2 * d, d4 = d3 * d, d5 = d4 * d;
-  const double b = P.b1 * d5 + P.b2 * d4 + P.b3 * d3;
+  const double b = d * d * d * fma(d, fma(d, P.b1, P.b2), P.b3);
   return b * b;
 }
 
 // factor = -dE/dr of the pair; repul = the pair's repulsion booked on atom i.
-__device__ __forceinline__ void tb_pair64(const TbDev &P, double dr, double ebs, double &factor,
+__device__ __forceinline__ void tb_pair64(const Tb64 &P, double dr, double ebs, double &factor,
                                           double &repul) {
   if (dr <= P.rci) {
-    const double t = dr * P.one_r0 - 1.0;
-    repul = P.ca * exp(-P.p * t);
-    factor = 2.0 * repul * P.p_r0 - P.eps2 * 0.5 * exp(-2.0 * P.q * t) * P.q2_r0 * ebs;
+    const double s = dr - P.r0;
+    const double ep = exp2_64(P.cp * s), eq = exp2_64(P.cq * s);
+    repul = P.ca * ep;
+    factor = fma(P.fa, ep, -(P.fb * ebs) * eq);
   } else {
     const double d = dr - P.rce;
-    const double d2 = d * d, d3 = d2 * d, d4 = d3 * d, d5 = d4 * d;
-    factor = (P.b1 * d5 + P.b2 * d4 + P.b3 * d3) *
-             (5.0 * P.b1 * d4 + 4.0 * P.b2 * d3 + 3.0 * P.b3 * d2) * ebs;
-    factor = factor - 2.0 * (5.0 * P.r1 * d4 + 4.0 * P.r2 * d3 + 3.0 * P.r3 * d2);
-    repul = P.r1 * d5 + P.r2 * d4 + P.r3 * d3;
+    const double d2 = d * d, d3 = d2 * d;
+    const double pp = d3 * fma(d, fma(d, P.b1, P.b2), P.b3);
+    const double dp = d2 * fma(d, fma(d, P.b1x5, P.b2x4), P.b3x3);
+    const double drm = d2 * fma(d, fma(d, P.r1m10, P.r2m8), P.r3m6);  // -2 dR/dd
+    factor = fma(pp * dp, ebs, drm);
+    repul = d3 * fma(d, fma(d, P.r1, P.r2), P.r3);
   }
 }
 
@@ -352,14 +415,15 @@ __device__ __forceinline__ bool tb_force_fx(const TbF &P, double r2, float dl, f
 // Tabulated Lennard-Jones pairs: energy p and f/r with f = -dp/dr, for r^2
 // within the pair's cut.  POT: GH_POT_PLJ (plj_interact, Pairs.F90:293-370),
 // GH_POT_SLJ (slj_interact, :403-493), GH_POT_WCA (wca_interact, :508-560).
-// FP64 follows the reference's arithmetic; FP32 uses the hardware
-// reciprocal square root.
+// FP64 takes 1/r^2 and r from the refined estimates above (sm1, which may
+// meet r = 0, keeps the IEEE root); FP32 uses the hardware reciprocal square
+// root.
 template <int POT>
 __device__ __forceinline__ void table_pair64(const PljDev &P, double r2, double &p,
                                              double &f_r) {
-  const double dr = sqrt(r2);
-  double f;
   if (POT == 6) {  // sm1: f here is minus the reference's attractive factor
+    const double dr = sqrt(r2);
+    double f;
     if (dr > P.rs) {
       const double w = P.rc - P.rs;
       const double a = M_PI * (dr - P.sa8) / w;
@@ -369,19 +433,30 @@ __device__ __forceinline__ void table_pair64(const PljDev &P, double r2, double 
       p = -P.e;
       f = 0.0;
     }
-  } else if (POT == 4 && !(dr < P.rs)) {
-    const double d = dr - P.rc, d2 = d * d, s4 = d2 * d2;  // (dr - rcut)**4
-    p = P.sa4 * s4 + P.sa8 * s4 * s4;
-    f = -(4.0 * P.sa4 * s4 + 8.0 * P.sa8 * s4 * s4) / (dr - P.rc);
-  } else {
-    const double t = P.s / dr;
-    const double t2 = t * t, t4 = t2 * t2, s6 = t4 * t2;  // (s/dr)**6
-    if (POT == 3) p = 4.0 * P.e * (s6 * s6 - s6) - P.prc - P.frc * (dr - P.rc);
-    else if (POT == 4) p = 4.0 * P.e * (s6 - 1.0) * s6;
-    else p = 4.0 * P.e * (s6 * s6 - s6) + P.e;
-    f = P.e * (48.0 * s6 - 24.0) * s6 / dr + (POT == 3 ? P.frc : 0.0);
+    f_r = f == 0.0 ? 0.0 : f / dr;
+    return;
   }
-  f_r = POT == 6 && f == 0.0 ? 0.0 : f / dr;
+  if (POT == 4) {
+    double dr, ir;
+    sqrt_rsq64(r2, dr, ir);
+    if (!(dr < P.rs)) {
+      const double d = dr - P.rc, d2 = d * d, s4 = d2 * d2;  // (dr - rcut)**4
+      p = s4 * fma(P.sa8, s4, P.sa4);
+      f_r = -(d2 * d) * fma(8.0 * P.sa8, s4, 4.0 * P.sa4) * ir;
+      return;
+    }
+  }
+  const double ir2 = rcp64(r2);
+  const double s2 = P.s * P.s * ir2, s6 = s2 * s2 * s2;  // (s/dr)**6
+  if (POT == 3) {
+    double dr, ir;
+    sqrt_rsq64(r2, dr, ir);
+    p = 4.0 * P.e * (s6 * s6 - s6) - P.prc - P.frc * (dr - P.rc);
+    f_r = fma(P.e * fma(48.0, s6, -24.0) * s6, ir2, P.frc * ir);
+  } else {
+    p = POT == 4 ? 4.0 * P.e * (s6 - 1.0) * s6 : 4.0 * P.e * (s6 * s6 - s6) + P.e;
+    f_r = P.e * fma(48.0, s6, -24.0) * s6 * ir2;
+  }
 }
 template <int POT>
 __device__ __forceinline__ void table_pair32(const PljDev &P, float r2f, float &p, float &f_r) {

@@ -76,13 +76,25 @@ struct TbF {
   float r1f, r2f, r3f, r1m10, r2m8, r3m6;          // tail repulsion and -10r1, -8r2, -6r3
 };
 
-// Kernel-side parameter block (one per type pair): the FP64 form (the
-// reference's arithmetic) and the FP32 form in Angstrom.
+// FP64 form of one type pair's SMA-TB terms.  The exponentials are powers of
+// two of a multiple of s = r - r0 (exact for r within a factor two of r0):
+// e^{-p(r/r0-1)} = 2^{cp s}, e^{-2q(r/r0-1)} = 2^{cq s}.
+struct Tb64 {
+  double r0, rci, rce, rce2;
+  double eps2, cq;                   // density eps2 2^{cq s}, eps2 = xi^2
+  double ca, cp;                     // repulsion ca 2^{cp s}
+  double fa, fb;                     // force fa 2^{cp s} - fb (eb_i + eb_j) 2^{cq s}
+  double b1, b2, b3, b1x5, b2x4, b3x3;       // tail density polynomial and 5b1, 4b2, 3b3
+  double r1, r2, r3, r1m10, r2m8, r3m6;      // tail repulsion and -10r1, -8r2, -6r3
+};
+
+// Kernel-side parameter block (one per type pair): both forms.
 struct TbDev {
-  double ca, eps2, p, q, r0, one_r0, rci, rce, rce2, b1, b2, b3, r1, r2, r3;
-  double p_r0, q2_r0;  // p/r0, 2q/r0
+  Tb64 d;
   TbF f;               // FP32 form, u = 1 A
 };
+// Fills both forms of pair t (FP32 in Angstrom) with the context constant e0.
+void gh_tbdev_fill(const GhTbPair &t, double e0, TbDev &o);
 // Fills the FP32 form of pair t in the unit 2^-k A with the context constant e0.
 void gh_tbf_fill(const GhTbPair &t, int k, double e0, TbF &o);
 // e0 of a parameter set: 1/sqrt(rho) of a type-0 atom with twelve neighbours at r0.
@@ -269,6 +281,7 @@ struct gh_ctx {
   TbDev *tbd = nullptr;                       // [MAXT*MAXT]
   TbF *tbf = nullptr;                         // [MAXT*MAXT]
   TbF tbf0;                                   // host copy of tbf[0] (one-type kernel argument)
+  Tb64 tb64_0;                                // the same of tbd[0].d
   int tbf_k = -1;                             // fixed-point unit exponent tbf was filled for
   double tb_e0 = 0.0;                         // eband reference of the FP32 forms
   PljDev *pljd = nullptr;                     // [MAXT*MAXT] shifted LJ per type pair

@@ -157,13 +157,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_rho64(
     double L0, double L1, double L2, double *__restrict__ rho, double *__restrict__ eband,
     float *__restrict__ eband32) {
   __shared__ ShiftLds sh;
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  __shared__ Tb64 sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
   load_shift(sh, L0, L1, L2);
-  if (SINGLE) {
-    if (threadIdx.x == 0) sp[0] = tbd[0];
-  } else {
-    load_params(sp, tbd, nt);
-  }
+  load_params(sp, tbd, SINGLE ? 1 : nt);
   __syncthreads();
   const int i = xcd_block() * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -179,19 +175,12 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_rho64(
     const double vx = (pj.x - pi.x) + sh.x[w];
     const double vy = (pj.y - pi.y) + sh.y[w];
     const double vz = (pj.z - pi.z) + sh.z[w];
-    const TbDev &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
-    const double dr = sqrt(dist2_rn(vx, vy, vz));
-    if (dr > P.rce) continue;
-    double banda;
-    if (dr < P.rci) {
-      banda = P.eps2 * exp(-2.0 * P.q * (dr * P.one_r0 - 1.0));
-    } else {
-      const double d = dr - P.rce;
-      const double d2 = d * d, d3 = d2 * d, d4 = d3 * d, d5 = d4 * d;
-      banda = P.b1 * d5 + P.b2 * d4 + P.b3 * d3;
-      banda = banda * banda;
-    }
-    acc += banda;
+    const Tb64 &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
+    const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+    if (rd > P.rce2) continue;
+    double dr, ir;
+    sqrt_rsq64(rd, dr, ir);
+    acc += tb_band64(P, dr);
   }
   rho[i] = acc;
   const double eb = 1.0 / sqrt(acc);
@@ -212,13 +201,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_force64(
     const double *__restrict__ eband, double ev_ui, double *__restrict__ frc,
     double *__restrict__ epa) {
   __shared__ ShiftLds sh;
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  __shared__ Tb64 sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
   load_shift(sh, L0, L1, L2);
-  if (SINGLE) {
-    if (threadIdx.x == 0) sp[0] = tbd[0];
-  } else {
-    load_params(sp, tbd, nt);
-  }
+  load_params(sp, tbd, SINGLE ? 1 : nt);
   __syncthreads();
   const int i = xcd_block() * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -235,27 +220,16 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_force64(
     const double vx = (pj.x - pi.x) + sh.x[w];
     const double vy = (pj.y - pi.y) + sh.y[w];
     const double vz = (pj.z - pi.z) + sh.z[w];
-    const TbDev &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
-    const double dr = sqrt(dist2_rn(vx, vy, vz));
-    if (dr > P.rce) continue;
-    double factor, repul;
-    if (dr <= P.rci) {
-      const double t = dr * P.one_r0 - 1.0;
-      repul = P.ca * exp(-P.p * t);
-      factor = 2.0 * repul * P.p_r0 -
-               P.eps2 * 0.5 * exp(-2.0 * P.q * t) * P.q2_r0 * (ebi + eband[j]);
-    } else {
-      const double d = dr - P.rce;
-      const double d2 = d * d, d3 = d2 * d, d4 = d3 * d, d5 = d4 * d;
-      factor = (P.b1 * d5 + P.b2 * d4 + P.b3 * d3) *
-               (5.0 * P.b1 * d4 + 4.0 * P.b2 * d3 + 3.0 * P.b3 * d2) * (ebi + eband[j]);
-      factor = factor - 2.0 * (5.0 * P.r1 * d4 + 4.0 * P.r2 * d3 + 3.0 * P.r3 * d2);
-      repul = P.r1 * d5 + P.r2 * d4 + P.r3 * d3;
-    }
-    const double s = factor / dr;
-    fx -= s * vx;
-    fy -= s * vy;
-    fz -= s * vz;
+    const Tb64 &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
+    const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+    if (rd > P.rce2) continue;
+    double dr, ir, factor, repul;
+    sqrt_rsq64(rd, dr, ir);
+    tb_pair64(P, dr, ebi + eband[j], factor, repul);
+    const double s = factor * ir;
+    fx = fma(-s, vx, fx);
+    fy = fma(-s, vy, fy);
+    fz = fma(-s, vz, fz);
     ei += repul;
   }
   frc[i] = fx * ev_ui;
@@ -277,13 +251,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_rho_mx(
     double L0, double L1, double L2, double *__restrict__ rho, double *__restrict__ eband,
     float *__restrict__ ebd32, double e0) {
   __shared__ ShiftLds sh;
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  __shared__ TbF sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
   load_shift(sh, L0, L1, L2);
-  if (SINGLE) {
-    if (threadIdx.x == 0) sp[0] = tbd[0];
-  } else {
-    load_params(sp, tbd, nt);
-  }
+  load_params(sp, tbd, SINGLE ? 1 : nt);
   __syncthreads();
   const int i = xcd_block() * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -299,9 +269,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_rho_mx(
     const double vx = (pj.x - pi.x) + sh.x[w];
     const double vy = (pj.y - pi.y) + sh.y[w];
     const double vz = (pj.z - pi.z) + sh.z[w];
-    const TbDev &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
+    const TbF &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
     float band;
-    if (tb_rho_fx(P.f, fma(vx, vx, fma(vy, vy, vz * vz)), band)) acc += (double)band;
+    if (tb_rho_fx(P, fma(vx, vx, fma(vy, vy, vz * vz)), band)) acc += (double)band;
   }
   rho[i] = acc;
   const double eb = 1.0 / sqrt(acc);
@@ -317,13 +287,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_force_mx(
     const float *__restrict__ ebd32, double ev_ui, double *__restrict__ frc,
     double *__restrict__ epa) {
   __shared__ ShiftLds sh;
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  __shared__ TbF sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
   load_shift(sh, L0, L1, L2);
-  if (SINGLE) {
-    if (threadIdx.x == 0) sp[0] = tbd[0];
-  } else {
-    load_params(sp, tbd, nt);
-  }
+  load_params(sp, tbd, SINGLE ? 1 : nt);
   __syncthreads();
   const int i = xcd_block() * blockDim.x + threadIdx.x;
   if (i >= n) return;
@@ -340,9 +306,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_tb_force_mx(
     const double vx = (pj.x - pi.x) + sh.x[w];
     const double vy = (pj.y - pi.y) + sh.y[w];
     const double vz = (pj.z - pi.z) + sh.z[w];
-    const TbDev &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
+    const TbF &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
     float sf, repul;
-    if (!tb_force_fx<true>(P.f, fma(vx, vx, fma(vy, vy, vz * vz)), di + ebd32[j], sf, repul))
+    if (!tb_force_fx<true>(P, fma(vx, vx, fma(vy, vy, vz * vz)), di + ebd32[j], sf, repul))
       continue;
     const double s = (double)sf;
     fx = fma(-s, vx, fx);
@@ -372,6 +338,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_lj64(
   if (i >= n) return;
   const double4 pi = pos[i];
   const int m = nn[i];
+  const double sig2 = sigma * sigma;
   double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
   for (int k = 0; k < m; ++k) {
     const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
@@ -383,16 +350,13 @@ __global__ __launch_bounds__(GH_BLOCK) void k_lj64(
     const double vz = (pj.z - pi.z) + sh.z[w];
     const double r2 = dist2_rn(vx, vy, vz);
     if (r2 > rc2) continue;
-    const double dr = sqrt(r2);
-    const double t = sigma / dr;
-    const double t2 = t * t, t4 = t2 * t2, s6 = t4 * t2;
-    const double p = 4.0 * eps * (s6 * s6 - s6);
-    const double f = eps * (48.0 * s6 - 24.0) * s6 / dr;
-    ei += p;
-    const double s = f / dr;
-    fx -= s * vx;
-    fy -= s * vy;
-    fz -= s * vz;
+    const double ir2 = rcp64(r2);
+    const double s2 = sig2 * ir2, s6 = s2 * s2 * s2;
+    ei += 4.0 * eps * (s6 * s6 - s6);
+    const double s = eps * fma(48.0, s6, -24.0) * s6 * ir2;
+    fx = fma(-s, vx, fx);
+    fy = fma(-s, vy, fy);
+    fz = fma(-s, vz, fz);
   }
   frc[i] = fx * ev_ui;
   frc[ncap + i] = fy * ev_ui;
@@ -1253,25 +1217,7 @@ extern "C" int gh_cluster_forces_static(int device, int precision, int n, int nt
       if (!(r0[k] > 0) || !(rci[k] > 0) || !(rce[k] > rci[k])) rc = GH_EINVAL;
       GhTbPair t{A[k], xi[k], p[k], q[k], r0[k], rci[k], rce[k], 0, 0, 0, 0, 0, 0};
       gh_tb_coeffs(t);
-      TbDev &d = tb.t[k];
-      d.ca = t.A;
-      d.eps2 = t.xi * t.xi;
-      d.p = t.p;
-      d.q = t.q;
-      d.r0 = t.r0;
-      d.one_r0 = 1.0 / t.r0;
-      d.rci = t.rci;
-      d.rce = t.rce;
-      d.rce2 = t.rce * t.rce;
-      d.b1 = t.b1;
-      d.b2 = t.b2;
-      d.b3 = t.b3;
-      d.r1 = t.r1;
-      d.r2 = t.r2;
-      d.r3 = t.r3;
-      d.p_r0 = t.p / t.r0;
-      d.q2_r0 = 2.0 * t.q / t.r0;
-      gh_tbf_fill(t, 0, e0, d.f);
+      gh_tbdev_fill(t, e0, tb.t[k]);
       rcut = std::max(rcut, t.rce);
     }
   if (rc == 0) {

@@ -1410,25 +1410,21 @@ __global__ __launch_bounds__(GH_TBMAX) void k_tb_force_fx(
 }
 
 // ---------------------------------------------------------------------------
-// SMA-TB, plain FP64 (the reference's arithmetic; LDS holds FP64 positions
-// with the image shift applied).
+// SMA-TB, plain FP64 (LDS holds FP64 positions with the image shift applied).
+// One type: the parameters come as a kernel argument (scalar registers).
 // ---------------------------------------------------------------------------
 template <bool SINGLE, int G>
 __global__ __launch_bounds__(GH_TBMAX) void k_tb_rho64_tiled(
     GhStatus *st, TileGeom t, const double4 *__restrict__ pos, const int *__restrict__ type,
     const int *__restrict__ cell_start, const int *__restrict__ nn,
     const unsigned short *__restrict__ list16, int ld, const TbDev *__restrict__ tbd, int nt,
-    double *__restrict__ rho, double *__restrict__ eband, float *__restrict__ eband32,
+    double *__restrict__ rho, double *__restrict__ eband, float *__restrict__ eband32, Tb64 p1,
     StepArgs sa) {
   if (step_gate(st, sa)) return;
   extern __shared__ double dyn[];
   __shared__ Halo H;
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
-  if (SINGLE) {
-    if (threadIdx.x == 0) sp[0] = tbd[0];
-  } else {
-    load_params(sp, tbd, nt);
-  }
+  __shared__ Tb64 sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  if (!SINGLE) load_params(sp, tbd, nt);
   int kc;  // this workgroup's share of the brick's atoms
   const int b = pass_brick(t, kc);
   if (b >= t.nbrick) return;
@@ -1461,9 +1457,13 @@ __global__ __launch_bounds__(GH_TBMAX) void k_tb_rho64_tiled(
     double acc = 0.0;
     auto slot = [&](int s) {
       const double vx = px[s] - pi.x, vy = py[s] - pi.y, vz = pz[s] - pi.z;
-      const TbDev &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + ty[s]];
-      const double dr = sqrt(dist2_rn(vx, vy, vz));
-      if (dr <= P.rce) acc += tb_band64(P, dr);
+      const Tb64 &P = SINGLE ? p1 : sp[ti * GH_MAXT + ty[s]];
+      const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+      if (rd <= P.rce2) {
+        double dr, ir;
+        sqrt_rsq64(rd, dr, ir);
+        acc += tb_band64(P, dr);
+      }
     };
     if (G == 1) for_each_slot(list16, ld, a, nn[a], slot);
     else for_each_slot_g<G>(list16, ld, a, nn[a], sub, slot);
@@ -1476,21 +1476,18 @@ __global__ __launch_bounds__(GH_TBMAX) void k_tb_rho64_tiled(
   }
 }
 
-template <bool SINGLE, int G>
+template <bool SINGLE, bool FUSED, int G>
 __device__ __forceinline__ void tb_force64_body(
     GhStatus *st, const TileGeom &t, const double4 *__restrict__ pos, const int *__restrict__ type,
     const int *__restrict__ cell_start, const int *__restrict__ nn,
     const unsigned short *__restrict__ list16, int ld, int ncap, const TbDev *__restrict__ tbd,
     int nt, const double *__restrict__ rho, const double *__restrict__ eband, double ev_ui,
-    double *__restrict__ frc, double *__restrict__ epa, const FuseVV &fv, long long step) {
+    double *__restrict__ frc, double *__restrict__ epa, const FuseVV &fv, const Tb64 &p1,
+    long long step) {
   extern __shared__ double dyn[];
   __shared__ Halo H;
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
-  if (SINGLE) {
-    if (threadIdx.x == 0) sp[0] = tbd[0];
-  } else {
-    load_params(sp, tbd, nt);
-  }
+  __shared__ Tb64 sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  if (!SINGLE) load_params(sp, tbd, nt);
   int kc;  // this workgroup's share of the brick's atoms
   const int b = pass_brick(t, kc);
   if (b >= t.nbrick) return;
@@ -1527,16 +1524,17 @@ __device__ __forceinline__ void tb_force64_body(
     double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
     auto slot = [&](int s) {
       const double vx = px[s] - pi.x, vy = py[s] - pi.y, vz = pz[s] - pi.z;
-      const TbDev &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + ty[s]];
-      const double dr = sqrt(dist2_rn(vx, vy, vz));
-      if (dr <= P.rce) {
-        double factor, repul;
+      const Tb64 &P = SINGLE ? p1 : sp[ti * GH_MAXT + ty[s]];
+      const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+      if (rd <= P.rce2) {
+        double dr, ir, factor, repul;
+        sqrt_rsq64(rd, dr, ir);
         tb_pair64(P, dr, ebi + eb[s], factor, repul);
-        const double sf = factor / dr;
-        fx -= sf * vx;
-        fy -= sf * vy;
-        fz -= sf * vz;
-        ei += repul;
+        const double sf = factor * ir;
+        fx = fma(-sf, vx, fx);
+        fy = fma(-sf, vy, fy);
+        fz = fma(-sf, vz, fz);
+        if (!FUSED) ei += repul;
       }
     };
     if (G == 1) for_each_slot(list16, ld, a, nn[a], slot);
@@ -1545,11 +1543,11 @@ __device__ __forceinline__ void tb_force64_body(
       fx = group_sum<G>(fx);
       fy = group_sum<G>(fy);
       fz = group_sum<G>(fz);
-      ei = group_sum<G>(ei);
+      if (!FUSED) ei = group_sum<G>(ei);
     }
     if (sub != 0) continue;
     const double Fx = fx * ev_ui, Fy = fy * ev_ui, Fz = fz * ev_ui;
-    if (fv.on) {
+    if (FUSED) {
       dmax2 = fmax(dmax2, fused_vv(fv, a, pi, ti, Fx, Fy, Fz));
     } else {
       frc[a] = Fx;
@@ -1558,18 +1556,18 @@ __device__ __forceinline__ void tb_force64_body(
       epa[a] = (ei - sqrt(rho[a])) * ev_ui;
     }
   }
-  if (fv.on) block_max_atomic(dmax2, st, step);
+  if (FUSED) block_max_atomic(dmax2, st, step);
 }
-template <bool SINGLE, int G>
+template <bool SINGLE, bool FUSED, int G>
 __global__ __launch_bounds__(GH_TBMAX) void k_tb_force64_tiled(
     GhStatus *st, TileGeom t, const double4 *__restrict__ pos, const int *__restrict__ type,
     const int *__restrict__ cell_start, const int *__restrict__ nn,
     const unsigned short *__restrict__ list16, int ld, int ncap, const TbDev *__restrict__ tbd,
     int nt, const double *__restrict__ rho, const double *__restrict__ eband, double ev_ui,
-    double *__restrict__ frc, double *__restrict__ epa, FuseVV fv, StepArgs sa) {
+    double *__restrict__ frc, double *__restrict__ epa, FuseVV fv, Tb64 p1, StepArgs sa) {
   if (!halted(st))
-    tb_force64_body<SINGLE, G>(st, t, pos, type, cell_start, nn, list16, ld, ncap, tbd, nt, rho,
-                            eband, ev_ui, frc, epa, fv, sa.step);
+    tb_force64_body<SINGLE, FUSED, G>(st, t, pos, type, cell_start, nn, list16, ld, ncap, tbd, nt,
+                                      rho, eband, ev_ui, frc, epa, fv, p1, sa.step);
 }
 
 // Lennard-Jones (lj_interact, Pairs.F90:207-279), tiled, FP64 LDS positions.
@@ -1613,6 +1611,7 @@ __device__ __forceinline__ void lj_tiled_body(
   }
   __syncthreads();
   const float epsf = (float)eps, sig2f = (float)(sigma * sigma);
+  const double sig2 = sigma * sigma, e4 = 4.0 * eps, e24 = 24.0 * eps, e48 = 48.0 * eps;
   double dmax2 = 0.0;
   const int sub = (int)(threadIdx.x & (G - 1));  // G lanes per atom (small systems)
   int ca0, ca1;
@@ -1658,15 +1657,15 @@ __device__ __forceinline__ void lj_tiled_body(
             table_pair64<POT>(P, r2, p, sf);
             if (!FUSED) ei += p;
           } else {
-            const double dr = sqrt(r2);
-            const double tt = sigma / dr;
-            const double t2 = tt * tt, t4 = t2 * t2, s6 = t4 * t2;
-            if (!FUSED) ei += 4.0 * eps * (s6 * s6 - s6);
-            sf = eps * (48.0 * s6 - 24.0) * s6 / dr / dr;
+            const double ir2 = rcp64(r2);
+            const double s2 = sig2 * ir2;
+            const double s6 = s2 * s2 * s2;
+            if (!FUSED) ei += e4 * (s6 * s6 - s6);
+            sf = fma(e48, s6, -e24) * s6 * ir2;
           }
-          fx -= sf * vx;
-          fy -= sf * vy;
-          fz -= sf * vz;
+          fx = fma(-sf, vx, fx);
+          fy = fma(-sf, vy, fy);
+          fz = fma(-sf, vz, fz);
         }
       }
     };
@@ -1826,9 +1825,12 @@ size_t gh_pair_slot_bytes(int pot, int precision) {
   return 25 + (gh_is_table_pot(pot) ? 1 : 0);
 }
 size_t gh_tile_static_bytes(int precision, int nt) {
-  const size_t params = nt > 1 ? (precision == GH_MIXED ? sizeof(TbF) : sizeof(TbDev)) *
+  // (an upper bound of both precisions' tables: the brick shapes chosen from
+  // it do not depend on which fields a form keeps)
+  const size_t params = nt > 1 ? (precision == GH_MIXED ? sizeof(TbF) : (size_t)240) *
                                      GH_MAXT * GH_MAXT
-                               : sizeof(TbDev);
+                               : (size_t)240;
+  static_assert(sizeof(Tb64) <= 240, "the LDS budget of the FP64 tables");
   return sizeof(Halo) + params;
 }
 
@@ -2123,11 +2125,16 @@ int gh_launch_forces_tiled(gh_ctx *c, hipEvent_t mid, bool fuse_vv) {
 #define RHO64(SG, GG)                                                                       \
   k_tb_rho64_tiled<SG, GG><<<grid, c->tg.tpb, lds1, s>>>(                                    \
       c->status, c->tg, c->pos, c->type, c->cell_start, c->nn, c->list16, ld, c->tbd, c->nt, \
-      rho1, c->eband, c->eband32, sa)
-#define FORCE64(SG, GG)                                                                     \
-  k_tb_force64_tiled<SG, GG><<<grid, c->tg.tpb, lds2, s>>>(                                  \
+      rho1, c->eband, c->eband32, c->tb64_0, sa)
+#define FORCE64F(SG, FU, GG)                                                                \
+  k_tb_force64_tiled<SG, FU, GG><<<grid, c->tg.tpb, lds2, s>>>(                              \
       c->status, c->tg, c->pos, c->type, c->cell_start, c->nn, c->list16, ld, c->ncap,       \
-      c->tbd, c->nt, c->rho, c->eband, ev_ui, c->frc, c->epa, fv, sa)
+      c->tbd, c->nt, c->rho, c->eband, ev_ui, c->frc, c->epa, fv, c->tb64_0, sa)
+#define FORCE64(SG, GG)                                                                     \
+  do {                                                                                      \
+    if (fuse_vv) FORCE64F(SG, true, GG);                                                    \
+    else FORCE64F(SG, false, GG);                                                           \
+  } while (0)
       const bool g4 = c->tg.lanes == 4;
       if (single) {
         if (g4) RHO64(true, 4);
@@ -2148,6 +2155,7 @@ int gh_launch_forces_tiled(gh_ctx *c, hipEvent_t mid, bool fuse_vv) {
       ++c->launches;
 #undef RHO64
 #undef FORCE64
+#undef FORCE64F
     }
   } else if (c->pot == GH_POT_LJ || gh_is_table_pot(c->pot)) {
     if (mid) GH_HIP(c, hipEventRecord(mid, s));
