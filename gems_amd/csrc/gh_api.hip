@@ -208,6 +208,7 @@ int gh_upload_tb(gh_ctx *c) {
     for (int b = 0; b < c->nt; ++b)
       gh_tbdev_fill(c->tb[a * GH_MAXT + b], c->tb_e0, h[a * GH_MAXT + b]);
   c->tb64_0 = h[0].d;
+  c->tbf_a0 = h[0].f;
   GH_TRY(dalloc(c, &c->tbd, GH_MAXT * GH_MAXT));
   // ordered on the context's stream (a non-blocking stream does not wait for
   // null-stream copies); h lives until the stream has drained
@@ -1215,7 +1216,10 @@ int gh_neighbors(gh_ctx *c, int *nn_out, int *idx, int cap) {
   std::vector<int> row;
   for (int s = 0; s < c->n; ++s) {
     row.clear();
-    for (int k = 0; k < nn[s]; ++k) row.push_back(orig[lst[(size_t)k * c->ncap + s] & 0x07FFFFFFu]);
+    for (int k = 0; k < nn[s]; ++k) {
+      const size_t at = c->list_mode == 1 ? (size_t)k * c->ncap + s : (size_t)s * c->cap + k;
+      row.push_back(orig[lst[at] & 0x07FFFFFFu]);
+    }
     std::sort(row.begin(), row.end());
     const int i = orig[s];
     const int m = std::min((int)row.size(), cap);

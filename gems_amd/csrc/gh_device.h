@@ -73,13 +73,34 @@ __device__ __forceinline__ int xcd_block() {
 }
 inline int xgrid(int nb) { return (nb + GH_NXCD - 1) / GH_NXCD * GH_NXCD; }
 
-__device__ __forceinline__ unsigned ld_stream(const unsigned *p) {
-  return __builtin_nontemporal_load(p);
-}
-
 __device__ __forceinline__ double wave_sum(double v) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
+}
+// Wavefront total of v in every lane: within each row of 16 lanes by DPP
+// (lane ^ 1, lane ^ 2, mirrored halves, mirrored row), the four row sums
+// through scalar registers.  No LDS round trips (the shuffle form waits for
+// six of them).
+template <int CTRL>
+__device__ __forceinline__ double dpp64(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double lane64(double v, int l) {
+  return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), l),
+                          __builtin_amdgcn_readlane(__double2loint(v), l));
+}
+__device__ __forceinline__ double row_total(double v) {
+  v += dpp64<0xB1>(v);   // quad_perm [1,0,3,2]
+  v += dpp64<0x4E>(v);   // quad_perm [2,3,0,1]
+  v += dpp64<0x141>(v);  // row_half_mirror
+  v += dpp64<0x140>(v);  // row_mirror
+  return v;
+}
+__device__ __forceinline__ double wave_total(double v) {
+  v = row_total(v);
+  return (lane64(v, 0) + lane64(v, 16)) + (lane64(v, 32) + lane64(v, 48));
 }
 __device__ __forceinline__ double wave_max(double v) {
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o, 64));
@@ -88,6 +109,12 @@ __device__ __forceinline__ double wave_max(double v) {
 __device__ __forceinline__ int wave_imax(int v) {
   for (int o = 32; o > 0; o >>= 1) v = max(v, __shfl_xor(v, o, 64));
   return v;
+}
+
+// Lanes of the wavefront below this one set in mask.
+__device__ __forceinline__ int lane_rank(unsigned long long mask) {
+  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
+                                        __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
 }
 
 // |vd|^2 rounded exactly as the reference's dot_product (no contraction).

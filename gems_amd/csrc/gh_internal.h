@@ -273,7 +273,7 @@ struct gh_ctx {
   int *cell_count = nullptr, *cell_start = nullptr;
   int *perm = nullptr;                        // [ncap]
   int *nn = nullptr;                          // [ncap]
-  int *list = nullptr;                        // [cap][ncap] ELL (O(N^2) mode)
+  int *list = nullptr;                        // [ncap][cap] rows (O(N^2) mode)
   unsigned short *list16 = nullptr;           // [cap][ncap] ELL of LDS slots (cell mode)
   void *chain_dev = nullptr;                  // rebuild-chain arguments (device copy)
   void *chain_pin = nullptr;                  // their pinned staging copy
@@ -282,6 +282,7 @@ struct gh_ctx {
   TbF *tbf = nullptr;                         // [MAXT*MAXT]
   TbF tbf0;                                   // host copy of tbf[0] (one-type kernel argument)
   Tb64 tb64_0;                                // the same of tbd[0].d
+  TbF tbf_a0;                                 // and of tbd[0].f (in Angstrom)
   int tbf_k = -1;                             // fixed-point unit exponent tbf was filled for
   double tb_e0 = 0.0;                         // eband reference of the FP32 forms
   PljDev *pljd = nullptr;                     // [MAXT*MAXT] shifted LJ per type pair

@@ -6,9 +6,8 @@
 //   epa, rho, eband        double[ncap]
 //   eband32                float[ncap] (mixed precision: 1/sqrt(rho) - e0)
 //   type, orig, cellof     int[ncap]
-//   list   uint32[cap][ld] ELL: row k of all atoms is contiguous, so a
-//          wavefront reading entry k of 64 consecutive atoms is coalesced.
-//          entry = j | (image code << 27); image code w = (wx+1)+3(wy+1)+9(wz+1)
+//   list   uint32[ncap][cap]: the row of an atom is contiguous (a wavefront
+//          reads one row).  entry = j | (image code << 27); image code w = (wx+1)+3(wy+1)+9(wz+1)
 //          with the neighbour's periodic image at x_j + wd*L_d.
 // Wavefronts are 64 lanes; per-atom kernels use 256-thread workgroups.
 #include <math.h>
@@ -16,6 +15,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <type_traits>
 
 #include "gh_device.h"
 
@@ -55,7 +55,28 @@ struct GridArgs {
 
 
 
-// O(N^2) build (verlet_self, Neighbour.F90:676-759): rd > rl^2 -> skip, so
+// ---------------------------------------------------------------------------
+// The O(N^2) list mode (free clusters, boxes of a few cells, masked pairs):
+// a wavefront per atom, in the list build and in every pair pass.  These
+// systems hold tens to a few thousand atoms: with one lane per atom a 201-atom
+// cluster runs on four wavefronts whose lanes walk ~200 candidates or ~50
+// neighbours one dependent load after another; with a wavefront per atom its
+// row (rows are contiguous: entry k of atom i at i * cap + k) is one load and
+// one round of pair terms.  201 Ag-Cu atoms, FP64: build 45 -> 5.1 us, density
+// 32 -> 4.2, forces 41 -> 4.5.
+// ---------------------------------------------------------------------------
+struct N2Build {
+  const double4 *pos;
+  int n, cap, ncap;
+  GridArgs g;
+  double rl2;
+  int *nn;
+  unsigned *list;
+  double *xold;
+  const int *orig, *mfeel, *mfelt;
+};
+
+// List build (verlet_self, Neighbour.F90:676-759): rd > rl^2 -> skip, so
 // equality is kept.  Minimum image by rounding as vdistance does; or, with
 // ghost images (box mic F), every first-shell image x_j + w L, w in {-1,0,1}
 // on each periodic axis, of every atom j including i itself (not w = 0), as
@@ -68,70 +89,107 @@ struct GridArgs {
 // Interaction.f90:69-77, 128-131) atom i lists j only when
 // mfeel[i] & mfelt[j] is nonzero; i then takes the whole pair force and half
 // the pair energy, j no reaction.
-__global__ __launch_bounds__(GH_BLOCK) void k_build_n2(
-    GhStatus *st, const double4 *__restrict__ pos, int n, GridArgs g, double rl2,
-    int cap, int ld, int count_only, int *__restrict__ nn, unsigned *__restrict__ list,
-    double *__restrict__ xold, int ncap, const int *__restrict__ orig,
-    const int *__restrict__ mfeel, const int *__restrict__ mfelt, long long step) {
-  if (!st->rebuild) return;
-  int s = blockIdx.x * blockDim.x + threadIdx.x;
-  int m = 0;
-  if (s < n) {
-    const double4 pi = pos[s];
-    // one-sided interactions: j enters i's row only if i feels what j is felt by
-    const int fi = mfeel ? mfeel[orig[s]] : 0;
-    const double ob0 = 1.0 / g.L[0], ob1 = 1.0 / g.L[1], ob2 = 1.0 / g.L[2];
-    for (int j = 0; j < n && g.ghost; ++j) {
-      if (mfeel && !(fi & mfelt[orig[j]])) continue;
-      const double4 pj = pos[j];
-      const double ux = pj.x - pi.x, uy = pj.y - pi.y, uz = pj.z - pi.z;
-      for (int w = 0; w < 27; ++w) {
-        const int wx = w % 3 - 1, wy = (w / 3) % 3 - 1, wz = w / 9 - 1;
-        if ((wx && !g.pbc[0]) || (wy && !g.pbc[1]) || (wz && !g.pbc[2])) continue;
-        if (j == s && w == 13) continue;
+// A wavefront builds the rows of R consecutive atoms from s0 (uniform): its
+// lanes take 64 consecutive candidates (of (j, image) pairs with ghost
+// images), the ballot of the test gives each kept one its place, so a row is
+// in candidate order.  Returns the longest row asked for (uniform).
+template <int R>
+__device__ __forceinline__ int n2_rows(const N2Build &B, int s0) {
+  const GridArgs &g = B.g;
+  const int lane = threadIdx.x & 63, n = B.n, cap = B.cap;
+  if (s0 >= n) return 0;
+  double4 pi[R];
+  int m[R], fi[R];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    const int s = min(s0 + r, n - 1);
+    pi[r] = B.pos[s];
+    m[r] = 0;
+    fi[r] = B.mfeel ? B.mfeel[B.orig[s]] : -1;
+  }
+  auto put = [&](int r, bool keep, unsigned e) {
+    const unsigned long long k = __ballot(keep);
+    const int d = m[r] + lane_rank(k);
+    if (keep && d < cap) B.list[(size_t)(s0 + r) * cap + d] = e;
+    m[r] += __popcll(k);
+  };
+  if (g.ghost) {
+    const long long nw = 27ll * n;
+    for (long long t0 = 0; t0 < nw; t0 += 64) {
+      const long long t = min(t0 + lane, nw - 1);
+      const int j = (int)(t / 27), w = (int)(t - 27ll * j);
+      const int wx = w % 3 - 1, wy = (w / 3) % 3 - 1, wz = w / 9 - 1;
+      const bool live = t0 + lane < nw && !((wx && !g.pbc[0]) || (wy && !g.pbc[1]) || (wz && !g.pbc[2]));
+      const int fj = B.mfelt ? B.mfelt[B.orig[j]] : -1;
+      const double4 pj = B.pos[j];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        const double ux = pj.x - pi[r].x, uy = pj.y - pi[r].y, uz = pj.z - pi[r].z;
         const double rd = dist2_rn(ux + wx * g.L[0], uy + wy * g.L[1], uz + wz * g.L[2]);
-        if (rd <= rl2) {
-          if (!count_only && m < cap) list[(size_t)m * ld + s] = (unsigned)j | ((unsigned)w << 27);
-          ++m;
-        }
+        put(r, live && s0 + r < n && (fi[r] & fj) && !(j == s0 + r && w == 13) && rd <= B.rl2,
+            (unsigned)j | ((unsigned)w << 27));
       }
     }
-    for (int j = 0; j < n && !g.ghost; ++j) {
-      if (j == s) continue;
-      if (mfeel && !(fi & mfelt[orig[j]])) continue;
-      const double4 pj = pos[j];
-      double vx = pj.x - pi.x, vy = pj.y - pi.y, vz = pj.z - pi.z;
-      int wx = 0, wy = 0, wz = 0;
-      if (g.pbc[0]) { wx = -(int)round(vx * ob0); vx = vx + wx * g.L[0]; }
-      if (g.pbc[1]) { wy = -(int)round(vy * ob1); vy = vy + wy * g.L[1]; }
-      if (g.pbc[2]) { wz = -(int)round(vz * ob2); vz = vz + wz * g.L[2]; }
-      const double rd = dist2_rn(vx, vy, vz);
-      if (rd <= rl2) {
-        if (!count_only && m < cap) {
-          const unsigned code = (unsigned)((wx + 1) + 3 * (wy + 1) + 9 * (wz + 1)) << 27;
-          list[(size_t)m * ld + s] = (unsigned)j | code;
+  } else {
+    const bool wrap = g.pbc[0] || g.pbc[1] || g.pbc[2];
+    const double ob0 = 1.0 / g.L[0], ob1 = 1.0 / g.L[1], ob2 = 1.0 / g.L[2];
+    for (int j0 = 0; j0 < n; j0 += 64) {
+      const int j = min(j0 + lane, n - 1);
+      const int fj = B.mfelt ? B.mfelt[B.orig[j]] : -1;
+      const double4 pj = B.pos[j];
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        double vx = pj.x - pi[r].x, vy = pj.y - pi[r].y, vz = pj.z - pi[r].z;
+        int wx = 0, wy = 0, wz = 0;
+        if (wrap) {
+          if (g.pbc[0]) { wx = -(int)round(vx * ob0); vx = vx + wx * g.L[0]; }
+          if (g.pbc[1]) { wy = -(int)round(vy * ob1); vy = vy + wy * g.L[1]; }
+          if (g.pbc[2]) { wz = -(int)round(vz * ob2); vz = vz + wz * g.L[2]; }
         }
-        ++m;
+        const double rd = dist2_rn(vx, vy, vz);
+        put(r, j0 + lane < n && j != s0 + r && s0 + r < n && (fi[r] & fj) && rd <= B.rl2,
+            (unsigned)j | ((unsigned)((wx + 1) + 3 * (wy + 1) + 9 * (wz + 1)) << 27));
       }
-    }
-    if (!count_only) {
-      nn[s] = min(m, cap);
-      xold[s] = pi.x;
-      xold[ncap + s] = pi.y;
-      xold[2 * ncap + s] = pi.z;
     }
   }
-  int wm = wave_imax(m);
-  if ((threadIdx.x & 63) == 0 && wm > 0) {
-    atomicMax(&st->maxnn, wm);
-    if (wm > cap) {
+  int most = 0;
+#pragma unroll
+  for (int r = 0; r < R; ++r)
+    if (s0 + r < n) {
+      most = max(most, m[r]);
+      if (lane == 0) B.nn[s0 + r] = min(m[r], cap);
+      if (lane < 3)
+        B.xold[lane * B.ncap + s0 + r] = lane == 0 ? pi[r].x : lane == 1 ? pi[r].y : pi[r].z;
+    }
+  return most;
+}
+
+// The wavefront's first atom: R per wavefront.
+template <int R>
+__device__ __forceinline__ int n2_first() {
+  const int w = (int)(blockIdx.x * (GH_BLOCK / 64) + (threadIdx.x >> 6));
+  return __builtin_amdgcn_readfirstlane(w) * R;
+}
+
+template <int R>
+__global__ __launch_bounds__(GH_BLOCK) void k_build_n2(GhStatus *st, N2Build B, long long step) {
+  if (!st->rebuild) return;
+  __shared__ int part[GH_BLOCK / 64];
+  const int m = n2_rows<R>(B, n2_first<R>());
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int wm = m;
+    for (int w = 1; w < GH_BLOCK / 64; ++w) wm = max(wm, part[w]);
+    if (wm > 0) atomicMax(&st->maxnn, wm);
+    if (wm > B.cap) {
       st->overflow = 1;
-      if (cap > 0) raise_halt(st, GH_HALT_OVERFLOW, step);  // cap 0: the sizing count
+      if (B.cap > 0) raise_halt(st, GH_HALT_OVERFLOW, step);  // cap 0: the sizing count
     }
   }
 }
 
-// image shift table in LDS: shift[w] = (wx*L0, wy*L1, wz*L2)
+// Image shift table in LDS: shift[w] = (wx*L0, wy*L1, wz*L2).
 struct ShiftLds {
   double x[27], y[27], z[27];
 };
@@ -144,314 +202,206 @@ __device__ __forceinline__ void load_shift(ShiftLds &sh, double L0, double L1, d
   }
 }
 
-// ---------------------------------------------------------------------------
-// SMA-TB pass 1 (smatb_preinteraction, TB.F90:367-455):
-//   rho_i = sum_j [ r < rci ? xi^2 exp(-2q(r/r0-1)) : (b1 x^5 + b2 x^4 + b3 x^3)^2 ]
-//   with x = r - rce and r > rce skipped; eband_i = 1/sqrt(rho_i).
-// FP64 form.
-// ---------------------------------------------------------------------------
-template <bool SINGLE>
-__global__ __launch_bounds__(GH_BLOCK) void k_tb_rho64(
-    const double4 *__restrict__ pos, const int *__restrict__ type, const int *__restrict__ nn,
-    const unsigned *__restrict__ list, int ld, int n, const TbDev *__restrict__ tbd, int nt,
-    double L0, double L1, double L2, double *__restrict__ rho, double *__restrict__ eband,
-    float *__restrict__ eband32) {
-  __shared__ ShiftLds sh;
-  __shared__ Tb64 sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
-  load_shift(sh, L0, L1, L2);
-  load_params(sp, tbd, SINGLE ? 1 : nt);
-  __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int ti = SINGLE ? 0 : type[i];
-  const int m = nn[i];
-  double acc = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const Tb64 &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
-    const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
-    if (rd > P.rce2) continue;
-    double dr, ir;
-    sqrt_rsq64(rd, dr, ir);
-    acc += tb_band64(P, dr);
+// A pair pass over one row: f(j, vx, vy, vz) for every listed pair, the
+// wavefront's lanes 64 entries at a time.
+struct N2Row {
+  const double4 *pos;
+  const unsigned *list;  // the atom's row
+  int m;
+};
+template <class F>
+__device__ __forceinline__ void n2_each(const N2Row &row, const double4 &pi, const ShiftLds &sh,
+                                        F &&f) {
+  for (int k = threadIdx.x & 63; k < row.m; k += 64) {
+    const unsigned e = row.list[k];
+    const int j = (int)(e & GH_JMASK), w = (int)(e >> 27);
+    const double4 pj = row.pos[j];
+    f(j, (pj.x - pi.x) + sh.x[w], (pj.y - pi.y) + sh.y[w], (pj.z - pi.z) + sh.z[w]);
   }
-  rho[i] = acc;
-  const double eb = 1.0 / sqrt(acc);
-  eband[i] = eb;
-  eband32[i] = (float)eb;
 }
 
-// SMA-TB pass 2 (smatb_interact, TB.F90:457-586), full list, newton off:
+// The parameter block of a pair: kernel argument (one type) or LDS table.
+// FP64 (Tb64) and mixed precision (TbF in Angstrom; the pair vector stays
+// FP64, the pair terms are FP32, sums FP64).
+template <bool MIXED>
+using TbForm = typename std::conditional<MIXED, TbF, Tb64>::type;
+template <bool MIXED>
+__device__ __forceinline__ const TbForm<MIXED> &tb_form(const TbDev &d) {
+  if constexpr (MIXED) return d.f;
+  else return d.d;
+}
+
+// SMA-TB pass 1 of one atom (smatb_preinteraction, TB.F90:367-455):
+//   rho_i = sum_j [ r < rci ? xi^2 exp(-2q(r/r0-1)) : (b1 x^5 + b2 x^4 + b3 x^3)^2 ]
+//   with x = r - rce and r > rce skipped.  The same value in every lane.
+template <bool MIXED, bool SINGLE>
+__device__ __forceinline__ double n2_rho(const N2Row &row, const double4 &pi, const ShiftLds &sh,
+                                         const int *__restrict__ type, int ti,
+                                         const TbForm<MIXED> *sp, const TbForm<MIXED> &p1) {
+  double acc = 0.0;
+  n2_each(row, pi, sh, [&](int j, double vx, double vy, double vz) {
+    const TbForm<MIXED> &P = SINGLE ? p1 : sp[ti * GH_MAXT + type[j]];
+    const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+    if constexpr (MIXED) {
+      float band;
+      if (tb_rho_fx(P, rd, band)) acc += (double)band;
+    } else {
+      if (rd > P.rce2) return;
+      double dr, ir;
+      sqrt_rsq64(rd, dr, ir);
+      acc += tb_band64(P, dr);
+    }
+  });
+  return wave_total(acc);
+}
+
+// SMA-TB pass 2 of one atom (smatb_interact, TB.F90:457-586), full list,
+// newton off:
 //   r <= rci: repul = A e^{-p(r/r0-1)};
 //             factor = 2 repul p/r0 - xi^2/2 e^{-2q(r/r0-1)} (2q/r0)(eb_i+eb_j)
 //   rci < r <= rce: factor = P P' (eb_i+eb_j) - 2 R';  repul = R
 //   F_i -= factor * vd / r  (vd = x_j - x_i), e_i = sum repul - sqrt(rho_i).
-template <bool SINGLE>
-__global__ __launch_bounds__(GH_BLOCK) void k_tb_force64(
-    const double4 *__restrict__ pos, const int *__restrict__ type, const int *__restrict__ nn,
-    const unsigned *__restrict__ list, int ld, int n, int ncap, const TbDev *__restrict__ tbd,
-    int nt, double L0, double L1, double L2, const double *__restrict__ rho,
-    const double *__restrict__ eband, double ev_ui, double *__restrict__ frc,
-    double *__restrict__ epa) {
-  __shared__ ShiftLds sh;
-  __shared__ Tb64 sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
-  load_shift(sh, L0, L1, L2);
-  load_params(sp, tbd, SINGLE ? 1 : nt);
-  __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int ti = SINGLE ? 0 : type[i];
-  const double ebi = eband[i];
-  const int m = nn[i];
-  double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const Tb64 &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
+// eb is 1/sqrt(rho) (FP64) or its FP32 offset from e0 (mixed); f = {Fx, Fy,
+// Fz, sum repul} in every lane.
+template <bool MIXED, bool SINGLE, class EB>
+__device__ __forceinline__ void n2_force(const N2Row &row, const double4 &pi, const ShiftLds &sh,
+                                         const int *__restrict__ type, int ti,
+                                         const TbForm<MIXED> *sp, const TbForm<MIXED> &p1,
+                                         const EB *eb, EB ebi, double (&f)[4]) {
+  f[0] = f[1] = f[2] = f[3] = 0.0;
+  n2_each(row, pi, sh, [&](int j, double vx, double vy, double vz) {
+    const TbForm<MIXED> &P = SINGLE ? p1 : sp[ti * GH_MAXT + type[j]];
     const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
-    if (rd > P.rce2) continue;
-    double dr, ir, factor, repul;
-    sqrt_rsq64(rd, dr, ir);
-    tb_pair64(P, dr, ebi + eband[j], factor, repul);
-    const double s = factor * ir;
-    fx = fma(-s, vx, fx);
-    fy = fma(-s, vy, fy);
-    fz = fma(-s, vz, fz);
-    ei += repul;
-  }
-  frc[i] = fx * ev_ui;
-  frc[ncap + i] = fy * ev_ui;
-  frc[2 * ncap + i] = fz * ev_ui;
-  epa[i] = (ei - sqrt(rho[i])) * ev_ui;
-}
-
-// ---------------------------------------------------------------------------
-// Mixed precision SMA-TB: positions and the pair vector stay FP64 (the
-// difference x_j - x_i is exact to FP64 rounding); the pair terms are the
-// FP32 forms of TbDev::f (Angstrom units; r^2 in FP64); rho, energies and
-// forces accumulate in FP64.  Pass 1 stores d = 1/sqrt(rho) - e0 in FP32.
-// ---------------------------------------------------------------------------
-template <bool SINGLE>
-__global__ __launch_bounds__(GH_BLOCK) void k_tb_rho_mx(
-    const double4 *__restrict__ pos, const int *__restrict__ type, const int *__restrict__ nn,
-    const unsigned *__restrict__ list, int ld, int n, const TbDev *__restrict__ tbd, int nt,
-    double L0, double L1, double L2, double *__restrict__ rho, double *__restrict__ eband,
-    float *__restrict__ ebd32, double e0) {
-  __shared__ ShiftLds sh;
-  __shared__ TbF sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
-  load_shift(sh, L0, L1, L2);
-  load_params(sp, tbd, SINGLE ? 1 : nt);
-  __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int ti = SINGLE ? 0 : type[i];
-  const int m = nn[i];
-  double acc = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const TbF &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
-    float band;
-    if (tb_rho_fx(P, fma(vx, vx, fma(vy, vy, vz * vz)), band)) acc += (double)band;
-  }
-  rho[i] = acc;
-  const double eb = 1.0 / sqrt(acc);
-  eband[i] = eb;
-  ebd32[i] = (float)(eb - e0);
-}
-
-template <bool SINGLE>
-__global__ __launch_bounds__(GH_BLOCK) void k_tb_force_mx(
-    const double4 *__restrict__ pos, const int *__restrict__ type, const int *__restrict__ nn,
-    const unsigned *__restrict__ list, int ld, int n, int ncap, const TbDev *__restrict__ tbd,
-    int nt, double L0, double L1, double L2, const double *__restrict__ rho,
-    const float *__restrict__ ebd32, double ev_ui, double *__restrict__ frc,
-    double *__restrict__ epa) {
-  __shared__ ShiftLds sh;
-  __shared__ TbF sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
-  load_shift(sh, L0, L1, L2);
-  load_params(sp, tbd, SINGLE ? 1 : nt);
-  __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int ti = SINGLE ? 0 : type[i];
-  const float di = ebd32[i];
-  const int m = nn[i];
-  double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const TbF &P = SINGLE ? sp[0] : sp[ti * GH_MAXT + type[j]];
-    float sf, repul;
-    if (!tb_force_fx<true>(P, fma(vx, vx, fma(vy, vy, vz * vz)), di + ebd32[j], sf, repul))
-      continue;
-    const double s = (double)sf;
-    fx = fma(-s, vx, fx);
-    fy = fma(-s, vy, fy);
-    fz = fma(-s, vz, fz);
-    ei += (double)repul;
-  }
-  frc[i] = fx * ev_ui;
-  frc[ncap + i] = fy * ev_ui;
-  frc[2 * ncap + i] = fz * ev_ui;
-  epa[i] = (ei - sqrt(rho[i])) * ev_ui;
-}
-
-// ---------------------------------------------------------------------------
-// Lennard-Jones (lj_interact, Pairs.F90:207-279), full list, newton off:
-//   r^2 > rc^2 skipped; p = 4e(s6^2 - s6); f = e(48 s6 - 24) s6 / r;
-//   e_i += p/2; F_i -= f vd / r.
-// ---------------------------------------------------------------------------
-__global__ __launch_bounds__(GH_BLOCK) void k_lj64(
-    const double4 *__restrict__ pos, const int *__restrict__ nn, const unsigned *__restrict__ list,
-    int ld, int n, int ncap, double eps, double sigma, double rc2, double L0, double L1,
-    double L2, double ev_ui, double *__restrict__ frc, double *__restrict__ epa) {
-  __shared__ ShiftLds sh;
-  load_shift(sh, L0, L1, L2);
-  __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int m = nn[i];
-  const double sig2 = sigma * sigma;
-  double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const double r2 = dist2_rn(vx, vy, vz);
-    if (r2 > rc2) continue;
-    const double ir2 = rcp64(r2);
-    const double s2 = sig2 * ir2, s6 = s2 * s2 * s2;
-    ei += 4.0 * eps * (s6 * s6 - s6);
-    const double s = eps * fma(48.0, s6, -24.0) * s6 * ir2;
-    fx = fma(-s, vx, fx);
-    fy = fma(-s, vy, fy);
-    fz = fma(-s, vz, fz);
-  }
-  frc[i] = fx * ev_ui;
-  frc[ncap + i] = fy * ev_ui;
-  frc[2 * ncap + i] = fz * ev_ui;
-  epa[i] = ei * 0.5 * ev_ui;
-}
-
-// Tabulated Lennard-Jones forms (plj_interact, Pairs.F90:293-370;
-// slj_interact, :403-493; wca_interact, :508-560) on the O(N^2)-mode list,
-// newton off, per type pair: e_i += p/2; F_i -= f vd / r.
-template <bool MIXED, int POT>
-__global__ __launch_bounds__(GH_BLOCK) void k_plj(
-    const double4 *__restrict__ pos, const int *__restrict__ type, const int *__restrict__ nn,
-    const unsigned *__restrict__ list, int ld, int n, int ncap, const PljDev *__restrict__ pljd,
-    double rc2, double L0, double L1, double L2, double ev_ui, double *__restrict__ frc,
-    double *__restrict__ epa) {
-  __shared__ ShiftLds sh;
-  __shared__ PljDev pp[GH_MAXT * GH_MAXT];
-  load_shift(sh, L0, L1, L2);
-  for (int k = threadIdx.x; k < GH_MAXT * GH_MAXT; k += blockDim.x) pp[k] = pljd[k];
-  __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int ti = type[i], m = nn[i];
-  double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const double r2 = MIXED ? fma(vx, vx, fma(vy, vy, vz * vz)) : dist2_rn(vx, vy, vz);
-    if (r2 > rc2) continue;
-    const PljDev &P = pp[ti * GH_MAXT + type[j]];
-    if (r2 > P.rc2) continue;  // this pair's cut
-    double p, sf;
-    if (MIXED) {
-      float pf, fr;
-      table_pair32<POT>(P, (float)r2, pf, fr);
-      p = (double)pf;
-      sf = (double)fr;
+    double s, rep;
+    if constexpr (MIXED) {
+      float sf, repul;
+      if (!tb_force_fx<true>(P, rd, ebi + eb[j], sf, repul)) return;
+      s = (double)sf;
+      rep = (double)repul;
     } else {
-      table_pair64<POT>(P, r2, p, sf);
+      if (rd > P.rce2) return;
+      double dr, ir, factor;
+      sqrt_rsq64(rd, dr, ir);
+      tb_pair64(P, dr, ebi + eb[j], factor, rep);
+      s = factor * ir;
     }
-    ei += p;
-    fx -= sf * vx;
-    fy -= sf * vy;
-    fz -= sf * vz;
-  }
-  frc[i] = fx * ev_ui;
-  frc[ncap + i] = fy * ev_ui;
-  frc[2 * ncap + i] = fz * ev_ui;
-  epa[i] = ei * 0.5 * ev_ui;
+    f[0] = fma(-s, vx, f[0]);
+    f[1] = fma(-s, vy, f[1]);
+    f[2] = fma(-s, vz, f[2]);
+    f[3] += rep;
+  });
+#pragma unroll
+  for (int d = 0; d < 4; ++d) f[d] = wave_total(f[d]);
 }
 
-__global__ __launch_bounds__(GH_BLOCK) void k_lj_mx(
-    const double4 *__restrict__ pos, const int *__restrict__ nn, const unsigned *__restrict__ list,
-    int ld, int n, int ncap, float eps, float sigma2, double rc2, double L0, double L1,
-    double L2, double ev_ui, double *__restrict__ frc, double *__restrict__ epa) {
+struct N2Pass {
+  const double4 *pos;
+  const int *type, *nn;
+  const unsigned *list;
+  int n, cap, ncap, nt;
+  double L[3];
+  const TbDev *tbd;
+  double *rho, *eband;
+  float *eband32;
+  double e0, ev_ui;
+  double *frc, *epa;
+};
+
+template <bool MIXED, bool SINGLE>
+__global__ __launch_bounds__(GH_BLOCK) void k_n2_rho(N2Pass A, TbForm<MIXED> p1) {
   __shared__ ShiftLds sh;
-  load_shift(sh, L0, L1, L2);
+  __shared__ TbForm<MIXED> sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  load_shift(sh, A.L[0], A.L[1], A.L[2]);
+  if (!SINGLE) load_params(sp, A.tbd, A.nt);
   __syncthreads();
-  const int i = xcd_block() * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const double4 pi = pos[i];
-  const int m = nn[i];
-  double fx = 0.0, fy = 0.0, fz = 0.0, ei = 0.0;
-  for (int k = 0; k < m; ++k) {
-    const unsigned e = ld_stream(&list[(size_t)k * ld + i]);
-    const int j = (int)(e & GH_JMASK);
-    const int w = (int)(e >> 27);
-    const double4 pj = pos[j];
-    const double vx = (pj.x - pi.x) + sh.x[w];
-    const double vy = (pj.y - pi.y) + sh.y[w];
-    const double vz = (pj.z - pi.z) + sh.z[w];
-    const double r2 = fma(vx, vx, fma(vy, vy, vz * vz));
-    if (r2 > rc2) continue;
-    const float ir2 = __builtin_amdgcn_rcpf((float)r2);
-    const float s2 = sigma2 * ir2;
-    const float s6 = s2 * s2 * s2;
-    const float p = 4.0f * eps * (s6 * s6 - s6);
-    const float fr2 = eps * fmaf(48.0f, s6, -24.0f) * s6 * ir2;  // f / r
-    ei += (double)p;
-    const double s = (double)fr2;
-    fx = fma(-s, vx, fx);
-    fy = fma(-s, vy, fy);
-    fz = fma(-s, vz, fz);
+  const int i = n2_first<1>();
+  if (i >= A.n) return;
+  const N2Row row{A.pos, A.list + (size_t)i * A.cap, A.nn[i]};
+  const double rho = n2_rho<MIXED, SINGLE>(row, A.pos[i], sh, A.type, SINGLE ? 0 : A.type[i], sp, p1);
+  if ((threadIdx.x & 63) == 0) {
+    A.rho[i] = rho;
+    const double eb = 1.0 / sqrt(rho);
+    A.eband[i] = eb;
+    A.eband32[i] = (float)(eb - A.e0);
   }
-  frc[i] = fx * ev_ui;
-  frc[ncap + i] = fy * ev_ui;
-  frc[2 * ncap + i] = fz * ev_ui;
-  epa[i] = ei * 0.5 * ev_ui;
+}
+
+template <bool MIXED, bool SINGLE>
+__global__ __launch_bounds__(GH_BLOCK) void k_n2_force(N2Pass A, TbForm<MIXED> p1) {
+  __shared__ ShiftLds sh;
+  __shared__ TbForm<MIXED> sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+  load_shift(sh, A.L[0], A.L[1], A.L[2]);
+  if (!SINGLE) load_params(sp, A.tbd, A.nt);
+  __syncthreads();
+  const int i = n2_first<1>();
+  if (i >= A.n) return;
+  const N2Row row{A.pos, A.list + (size_t)i * A.cap, A.nn[i]};
+  const double4 pi = A.pos[i];
+  const int ti = SINGLE ? 0 : A.type[i];
+  double f[4];
+  if constexpr (MIXED) n2_force<true, SINGLE>(row, pi, sh, A.type, ti, sp, p1, A.eband32, A.eband32[i], f);
+  else n2_force<false, SINGLE>(row, pi, sh, A.type, ti, sp, p1, A.eband, A.eband[i], f);
+  const int lane = threadIdx.x & 63;
+  if (lane < 3) A.frc[lane * A.ncap + i] = (lane == 0 ? f[0] : lane == 1 ? f[1] : f[2]) * A.ev_ui;
+  else if (lane == 3) A.epa[i] = (f[3] - sqrt(A.rho[i])) * A.ev_ui;
+}
+
+// Pair potentials, full list, newton off: e_i += p/2; F_i -= f vd / r.
+// POT: GH_POT_LJ (lj_interact, Pairs.F90:207-279: r^2 > rc^2 skipped; p =
+// 4e(s6^2 - s6); f = e(48 s6 - 24) s6 / r) or a tabulated form per type pair
+// (plj_interact, Pairs.F90:293-370; slj_interact, :403-493; wca_interact,
+// :508-560; sm1_interact, :916-990).
+template <bool MIXED, int POT>
+__global__ __launch_bounds__(GH_BLOCK) void k_n2_pair(N2Pass A, const PljDev *__restrict__ pljd,
+                                                      double eps, double sig2, double rc2) {
+  constexpr bool TAB = POT != GH_POT_LJ;
+  __shared__ ShiftLds sh;
+  __shared__ PljDev pp[TAB ? GH_MAXT * GH_MAXT : 1];
+  load_shift(sh, A.L[0], A.L[1], A.L[2]);
+  if (TAB)
+    for (int k = threadIdx.x; k < GH_MAXT * GH_MAXT; k += blockDim.x) pp[k] = pljd[k];
+  __syncthreads();
+  const int i = n2_first<1>();
+  if (i >= A.n) return;
+  const N2Row row{A.pos, A.list + (size_t)i * A.cap, A.nn[i]};
+  const int ti = TAB ? A.type[i] : 0;
+  double f[4] = {0.0, 0.0, 0.0, 0.0};
+  n2_each(row, A.pos[i], sh, [&](int j, double vx, double vy, double vz) {
+    const double r2 = MIXED ? fma(vx, vx, fma(vy, vy, vz * vz)) : dist2_rn(vx, vy, vz);
+    if (r2 > rc2) return;
+    double p, s;
+    if constexpr (TAB) {
+      const PljDev &P = pp[ti * GH_MAXT + A.type[j]];
+      if (r2 > P.rc2) return;  // this pair's cut
+      if constexpr (MIXED) {
+        float pf, fr;
+        table_pair32<POT>(P, (float)r2, pf, fr);
+        p = (double)pf;
+        s = (double)fr;
+      } else {
+        table_pair64<POT>(P, r2, p, s);
+      }
+    } else if constexpr (MIXED) {
+      const float ef = (float)eps, ir2 = __builtin_amdgcn_rcpf((float)r2);
+      const float s2 = (float)sig2 * ir2, s6 = s2 * s2 * s2;
+      p = (double)(4.0f * ef * (s6 * s6 - s6));
+      s = (double)(ef * fmaf(48.0f, s6, -24.0f) * s6 * ir2);  // f / r
+    } else {
+      const double ir2 = rcp64(r2);
+      const double s2 = sig2 * ir2, s6 = s2 * s2 * s2;
+      p = 4.0 * eps * (s6 * s6 - s6);
+      s = eps * fma(48.0, s6, -24.0) * s6 * ir2;
+    }
+    f[0] = fma(-s, vx, f[0]);
+    f[1] = fma(-s, vy, f[1]);
+    f[2] = fma(-s, vz, f[2]);
+    f[3] += p;
+  });
+#pragma unroll
+  for (int d = 0; d < 4; ++d) f[d] = wave_total(f[d]);
+  const int lane = threadIdx.x & 63;
+  if (lane < 3) A.frc[lane * A.ncap + i] = (lane == 0 ? f[0] : lane == 1 ? f[1] : f[2]) * A.ev_ui;
+  else if (lane == 3) A.epa[i] = f[3] * 0.5 * A.ev_ui;
 }
 
 // ---------------------------------------------------------------------------
@@ -835,6 +785,24 @@ GridArgs make_grid(const gh_ctx *c) {
   return g;
 }
 
+inline int n2_blocks(int n, int rows) {
+  const int per = GH_BLOCK / 64 * rows;
+  return (n + per - 1) / per;
+}
+
+N2Build make_n2_build(const gh_ctx *c) {
+  const double rl = c->rcut + c->skin;
+  return N2Build{c->pos, c->n, c->cap, c->ncap, make_grid(c), rl * rl, c->nn,
+                 reinterpret_cast<unsigned *>(c->list), c->xold, c->orig,
+                 c->masked ? c->mfeel : nullptr, c->masked ? c->mfelt : nullptr};
+}
+
+N2Pass make_n2_pass(const gh_ctx *c) {
+  return N2Pass{c->pos, c->type, c->nn, reinterpret_cast<const unsigned *>(c->list),
+                c->n, c->cap, c->ncap, c->nt, {c->L[0], c->L[1], c->L[2]}, c->tbd,
+                c->rho, c->eband, c->eband32, c->tb_e0, ghc::ev_ui(), c->frc, c->epa};
+}
+
 MassArgs make_mass(const gh_ctx *c) {
   MassArgs m;
   for (int t = 0; t < GH_MAXT; ++t) {
@@ -900,14 +868,14 @@ int gh_launch_rebuild(gh_ctx *c, bool force) {
   { k_decide<<<1, 1, 0, s>>>(c->status, c->skin, c->step); ++c->launches; }
   if (c->list_mode == 0 && c->boxed && (c->pbc[0] || c->pbc[1] || c->pbc[2]))
     { k_wrap_rebuild<<<nb, GH_BLOCK, 0, s>>>(c->status, n, make_wrap(c), c->pos); ++c->launches; }
-  const GridArgs g = make_grid(c);
-  const double rl = c->rcut + c->skin;
-  const double rl2 = rl * rl;
-  const int ld = c->ncap;
-  { k_build_n2<<<nb, GH_BLOCK, 0, s>>>(c->status, c->pos, n, g, rl2, c->cap, ld, 0, c->nn,
-                                     (unsigned *)c->list, c->xold, c->ncap, c->orig,
-                                     c->masked ? c->mfeel : nullptr,
-                                     c->masked ? c->mfelt : nullptr, c->step); ++c->launches; }
+  const N2Build B = make_n2_build(c);
+  // rows per wavefront: one where the atoms do not fill the chip's wavefront
+  // slots anyway, several where every wavefront reads all positions (32 n^2
+  // bytes through the caches: 130 MB at 2,048 atoms, 33 MB with four rows)
+  if (n <= 1024) k_build_n2<1><<<n2_blocks(n, 1), GH_BLOCK, 0, s>>>(c->status, B, c->step);
+  else if (n <= 8192) k_build_n2<4><<<n2_blocks(n, 4), GH_BLOCK, 0, s>>>(c->status, B, c->step);
+  else k_build_n2<8><<<n2_blocks(n, 8), GH_BLOCK, 0, s>>>(c->status, B, c->step);
+  ++c->launches;
   GH_HIP(c, hipGetLastError());
   return 0;
 }
@@ -921,88 +889,42 @@ int gh_launch_forces(gh_ctx *c, hipEvent_t mid, bool fuse_vv) {
   if (c->list_mode == 1) return gh_launch_forces_tiled(c, mid, fuse_vv);
   if (fuse_vv) return gh_fail(c, GH_ESTATE, "fused integration needs the tiled path");
   hipStream_t s = c->stream;
-  const int n = c->n, nb = nblocks(n);
-  const int ld = c->ncap;
-  const double ev_ui = ghc::ev_ui();
-  const double L0 = c->L[0], L1 = c->L[1], L2 = c->L[2];
-  const unsigned *list = (const unsigned *)c->list;
-  const bool single = c->nt == 1;
-  const bool mixed = c->precision == GH_MIXED;
+  const int nb = n2_blocks(c->n, 1);
+  const bool single = c->nt == 1, mixed = c->precision == GH_MIXED;
+  const N2Pass A = make_n2_pass(c);
   if (c->pot == GH_POT_SMATB) {
-    if (mixed) {
-      if (single)
-        { k_tb_rho_mx<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n, c->tbd,
-                                                  c->nt, L0, L1, L2, c->rho, c->eband,
-                                                  c->eband32, c->tb_e0); ++c->launches; }
-      else
-        { k_tb_rho_mx<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n, c->tbd,
-                                                   c->nt, L0, L1, L2, c->rho, c->eband,
-                                                   c->eband32, c->tb_e0); ++c->launches; }
-    } else {
-      if (single)
-        { k_tb_rho64<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n, c->tbd,
-                                                 c->nt, L0, L1, L2, c->rho, c->eband,
-                                                 c->eband32); ++c->launches; }
-      else
-        { k_tb_rho64<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n, c->tbd,
-                                                  c->nt, L0, L1, L2, c->rho, c->eband,
-                                                  c->eband32); ++c->launches; }
-    }
-    if (mid) GH_HIP(c, hipEventRecord(mid, s));
-    if (mixed) {
-      if (single)
-        { k_tb_force_mx<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n,
-                                                    c->ncap, c->tbd, c->nt, L0, L1, L2, c->rho,
-                                                    c->eband32, ev_ui, c->frc, c->epa); ++c->launches; }
-      else
-        { k_tb_force_mx<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n,
-                                                     c->ncap, c->tbd, c->nt, L0, L1, L2,
-                                                     c->rho, c->eband32, ev_ui, c->frc,
-                                                     c->epa); ++c->launches; }
-    } else {
-      if (single)
-        { k_tb_force64<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n,
-                                                   c->ncap, c->tbd, c->nt, L0, L1, L2, c->rho,
-                                                   c->eband, ev_ui, c->frc, c->epa); ++c->launches; }
-      else
-        { k_tb_force64<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n,
-                                                    c->ncap, c->tbd, c->nt, L0, L1, L2, c->rho,
-                                                    c->eband, ev_ui, c->frc, c->epa); ++c->launches; }
-    }
-  } else if (c->pot == GH_POT_LJ) {
-    if (mid) GH_HIP(c, hipEventRecord(mid, s));
-    const double rc2 = c->lj_rc * c->lj_rc;
-    if (mixed)
-      { k_lj_mx<<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->nn, list, ld, n, c->ncap, (float)c->lj_eps,
-                                      (float)(c->lj_sigma * c->lj_sigma), rc2, L0, L1, L2,
-                                      ev_ui, c->frc, c->epa); ++c->launches; }
-    else
-      { k_lj64<<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->nn, list, ld, n, c->ncap, c->lj_eps,
-                                     c->lj_sigma, rc2, L0, L1, L2, ev_ui, c->frc, c->epa); ++c->launches; }
-  } else if (gh_is_table_pot(c->pot)) {
-    if (mid) GH_HIP(c, hipEventRecord(mid, s));
-    const double rc2 = c->lj_rc * c->lj_rc;
-#define PLJ_LAUNCH(MX, PT)                                                                  \
+#define N2_TB(KERNEL)                                                                       \
   do {                                                                                      \
-    k_plj<MX, PT><<<xgrid(nb), GH_BLOCK, 0, s>>>(c->pos, c->type, c->nn, list, ld, n,        \
-                                                 c->ncap, c->pljd, rc2, L0, L1, L2, ev_ui,  \
-                                                 c->frc, c->epa);                           \
+    if (mixed) {                                                                            \
+      if (single) KERNEL<true, true><<<nb, GH_BLOCK, 0, s>>>(A, c->tbf_a0);                  \
+      else KERNEL<true, false><<<nb, GH_BLOCK, 0, s>>>(A, c->tbf_a0);                        \
+    } else {                                                                                \
+      if (single) KERNEL<false, true><<<nb, GH_BLOCK, 0, s>>>(A, c->tb64_0);                 \
+      else KERNEL<false, false><<<nb, GH_BLOCK, 0, s>>>(A, c->tb64_0);                       \
+    }                                                                                       \
     ++c->launches;                                                                          \
   } while (0)
-#define PLJ_POTS(MX)                                                                        \
-  switch (c->pot) {                                                                         \
-    case GH_POT_SLJ: PLJ_LAUNCH(MX, GH_POT_SLJ); break;                                     \
-    case GH_POT_WCA: PLJ_LAUNCH(MX, GH_POT_WCA); break;                                     \
-    case GH_POT_SM1: PLJ_LAUNCH(MX, GH_POT_SM1); break;                                     \
-    default: PLJ_LAUNCH(MX, GH_POT_PLJ);                                                    \
-  }
-    if (mixed) {
-      PLJ_POTS(true)
-    } else {
-      PLJ_POTS(false)
+    N2_TB(k_n2_rho);
+    if (mid) GH_HIP(c, hipEventRecord(mid, s));
+    N2_TB(k_n2_force);
+#undef N2_TB
+  } else if (c->pot == GH_POT_LJ || gh_is_table_pot(c->pot)) {
+    if (mid) GH_HIP(c, hipEventRecord(mid, s));
+    const double rc2 = c->lj_rc * c->lj_rc, sig2 = c->lj_sigma * c->lj_sigma;
+#define N2_PAIR(PT)                                                                         \
+  do {                                                                                      \
+    if (mixed) k_n2_pair<true, PT><<<nb, GH_BLOCK, 0, s>>>(A, c->pljd, c->lj_eps, sig2, rc2); \
+    else k_n2_pair<false, PT><<<nb, GH_BLOCK, 0, s>>>(A, c->pljd, c->lj_eps, sig2, rc2);      \
+    ++c->launches;                                                                          \
+  } while (0)
+    switch (c->pot) {
+      case GH_POT_SLJ: N2_PAIR(GH_POT_SLJ); break;
+      case GH_POT_WCA: N2_PAIR(GH_POT_WCA); break;
+      case GH_POT_SM1: N2_PAIR(GH_POT_SM1); break;
+      case GH_POT_PLJ: N2_PAIR(GH_POT_PLJ); break;
+      default: N2_PAIR(GH_POT_LJ);
     }
-#undef PLJ_POTS
-#undef PLJ_LAUNCH
+#undef N2_PAIR
   } else {
     return gh_fail(c, GH_ESTATE, "no potential set");
   }
@@ -1232,48 +1154,45 @@ extern "C" int gh_cluster_forces_static(int device, int precision, int n, int nt
     float *eb32 = reinterpret_cast<float *>(scr + kSOffEb32);
     double *frc = reinterpret_cast<double *>(scr + kSOffFrc);
     const TbDev *tbd = reinterpret_cast<const TbDev *>(scr + kSOffTb);
-    const int nb = nblocks(n), ld = GH_STATIC_MAXN;
+    const int nb = nblocks(n), nw = n2_blocks(n, 1);
     const double L = 1e6, rl = rcut + skin;
-    GridArgs g;
-    memset(&g, 0, sizeof(g));
+    N2Build B;
+    memset(&B, 0, sizeof(B));
     for (int d = 0; d < 3; ++d) {
-      g.nc[d] = g.gn[d] = 1;
-      g.L[d] = L;
-      g.one_cell[d] = 1.0 / L;
+      B.g.nc[d] = B.g.gn[d] = 1;
+      B.g.L[d] = L;
+      B.g.one_cell[d] = 1.0 / L;
     }
-    g.ncell = 1;
-    const double ev_ui = ghc::ev_ui();
+    B.g.ncell = 1;
+    B.pos = pos;
+    B.n = n;
+    B.cap = GH_STATIC_CAP;
+    B.ncap = GH_STATIC_MAXN;
+    B.rl2 = rl * rl;
+    B.nn = nn;
+    B.list = list;
+    B.xold = xold;
+    const N2Pass P{pos, type, nn, list, n, GH_STATIC_CAP, GH_STATIC_MAXN, nt, {L, L, L}, tbd,
+                   rho, eband, eb32, e0, ghc::ev_ui(), frc, e_atom};
     const bool single = nt == 1;
     k_static_init<<<std::max(nb, 1), GH_BLOCK, 0, s>>>(scr, n, nt, x, tb);
-    k_build_n2<<<nb, GH_BLOCK, 0, s>>>(st, pos, n, g, rl * rl, GH_STATIC_CAP, ld, 0, nn, list,
-                                        xold, ld, nullptr, nullptr, nullptr, 0);
+    if (n <= 1024) k_build_n2<1><<<nw, GH_BLOCK, 0, s>>>(st, B, 0);
+    else k_build_n2<4><<<n2_blocks(n, 4), GH_BLOCK, 0, s>>>(st, B, 0);
     if (precision == GH_MIXED) {
       if (single) {
-        k_tb_rho_mx<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, tbd, nt, L, L,
-                                                         L, rho, eband, eb32, e0);
-        k_tb_force_mx<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, ld, tbd,
-                                                           nt, L, L, L, rho, eb32, ev_ui, frc,
-                                                           e_atom);
+        k_n2_rho<true, true><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].f);
+        k_n2_force<true, true><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].f);
       } else {
-        k_tb_rho_mx<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, tbd, nt, L,
-                                                          L, L, rho, eband, eb32, e0);
-        k_tb_force_mx<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, ld, tbd,
-                                                            nt, L, L, L, rho, eb32, ev_ui, frc,
-                                                            e_atom);
+        k_n2_rho<true, false><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].f);
+        k_n2_force<true, false><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].f);
       }
     } else {
       if (single) {
-        k_tb_rho64<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, tbd, nt, L, L,
-                                                        L, rho, eband, eb32);
-        k_tb_force64<true><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, ld, tbd, nt,
-                                                          L, L, L, rho, eband, ev_ui, frc,
-                                                          e_atom);
+        k_n2_rho<false, true><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].d);
+        k_n2_force<false, true><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].d);
       } else {
-        k_tb_rho64<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, tbd, nt, L,
-                                                         L, L, rho, eband, eb32);
-        k_tb_force64<false><<<xgrid(nb), GH_BLOCK, 0, s>>>(pos, type, nn, list, ld, n, ld, tbd,
-                                                           nt, L, L, L, rho, eband, ev_ui, frc,
-                                                           e_atom);
+        k_n2_rho<false, false><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].d);
+        k_n2_force<false, false><<<nw, GH_BLOCK, 0, s>>>(P, tb.t[0].d);
       }
     }
     k_static_out<<<nb, GH_BLOCK, 0, s>>>(scr, n, F);

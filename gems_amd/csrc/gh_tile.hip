@@ -222,12 +222,6 @@ __device__ __forceinline__ void block_max_atomic(double d2, GhStatus *st, long l
   }
 }
 
-// Lanes of the wavefront below this one set in mask.
-__device__ __forceinline__ int lane_rank(unsigned long long mask) {
-  return (int)__builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32),
-                                        __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
-}
-
 __device__ __forceinline__ size_t qidx(int k, int a, int ld) {
   return (((size_t)(k >> 2) * ld + a) << 2) + (k & 3);
 }
