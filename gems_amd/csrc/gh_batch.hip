@@ -1,26 +1,41 @@
-// Batched free clusters: many independent unboxed systems advanced in one
-// launch, one workgroup per system, largest system first.
+// Batched free clusters: many independent unboxed systems on one device.
 //
 // GEMS has no batching (one system per process, replica exchange over MPI
 // ranks, src/ReplicaExchange.f90:27-151); per system the work is the same hot
 // path: the O(N^2) verlet_self list (Neighbour.F90:676-759, rd <= rl^2 kept),
 // the two SMA-TB passes (TB.F90:367-586) and the Ermak update
 // (Integration.F90:963-1031).  A system's atoms are contiguous; all state is
-// FP64 in HBM (SoA with stride ld), neighbour lists are ELL rows of 16-bit
-// indices local to the system.  Within a workgroup the steps of a system are
-// separated by workgroup barriers only, so nsteps need one launch.
+// FP64 in HBM (SoA with stride ld).
+//
+// Forces and Langevin dynamics run over the atoms of all systems at once, 16
+// or 8 lanes per atom, two launches per step (density; forces with the update to
+// the next step): a step then costs the chip's throughput, not the time one
+// compute unit needs for the largest cluster (a workgroup per system took 170
+// us per step for 2,000 atoms while the compute units of the smaller systems
+// idled; 128 Ag-Cu clusters of 38..2000 atoms, mixed: 206 -> 68 us per step;
+// 16 clusters of 38..600 96 -> 18).  FIRE, whose every iteration needs sums over each system, keeps a
+// workgroup per system (largest first) and all iterations in one launch.
+//
+// Neighbour rows: cap 16-bit indices local to the system, contiguous per
+// atom; the pairs inside the inner bound at build time fill a row from its
+// front, the others from its back, so the 16 lanes of an atom take one branch
+// of the pair function per round.
 #include <math.h>
 #include <stdint.h>
 
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 #include <vector>
 
 #include "gh_device.h"
 
-#define GH_BBLOCK 512  // largest workgroup of the batch kernels for the ordinary systems
+#define GH_FBS 256  // workgroup of the FIRE kernel
 #define GH_BIGSYS 1024  // systems above this many atoms get 1024-thread workgroups
 
+namespace {
+struct FireState;
+}
 struct gh_batch {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -41,20 +56,23 @@ struct gh_batch {
   std::vector<double> T_h, epot_h;
   // device
   int *off = nullptr, *order = nullptr, *type = nullptr, *nn = nullptr, *flags = nullptr;
-  double4 *pos = nullptr;
+  int *sysof = nullptr, *a0of = nullptr;   // each atom's system and that system's first atom
+  GhLine *dmax = nullptr;                  // [2][nsys] largest |x - x_old|^2, by step parity
+  double4 *pos = nullptr, *pos_next = nullptr;  // x, y, z, type
+  double4 *pk = nullptr;  // what the force pass reads of a neighbour (density pass)
   double *vel = nullptr, *acc = nullptr, *frc = nullptr, *e = nullptr, *rho = nullptr,
-         *eband = nullptr, *xold = nullptr, *T = nullptr, *out = nullptr, *scale = nullptr;
-  float *eband32 = nullptr;
-  float *gn = nullptr;  // [6][ld] this step's normals (stepa -> stepb)
+         *xold = nullptr, *T = nullptr, *out = nullptr, *scale = nullptr;
+  FireState *fst = nullptr;         // [nsys] between the FIRE launches
   unsigned short *list = nullptr;
   TbDev *tbd = nullptr;
   TbF *tbf = nullptr;
+  TbDev tbd0;           // host copies of tbd[0] and tbf[0] (one-type kernel arguments)
+  TbF tbf0;
   double tb_e0 = 0.0;
   int nst = 0;   // LDS staging slots per workgroup (largest system + sentinel)
-  int nmax = 0;  // atoms of the largest system
-  // systems above GH_BIGSYS atoms (the first nbig of the largest-first order)
-  // run on a second stream beside the rest; nmax_rest = the largest of the rest
-  int nbig = 0, nmax_rest = 0;
+  // FIRE: systems above GH_BIGSYS atoms (the first nbig of the largest-first
+  // order) run on a second stream beside the rest
+  int nbig = 0;
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
@@ -63,24 +81,23 @@ namespace {
 using namespace ghd;
 
 struct BatchArgs {
-  const int *off, *order, *type;
-  int first;  // this launch's workgroup b works on system order[first + b]
-  double4 *pos;
-  double *vel, *acc, *frc, *e, *rho, *eband, *xold;
-  float *eband32;
-  float *gn;
-  int *nn;
+  const int *off, *order, *type, *sysof, *a0of;
+  int first;  // FIRE: this launch's workgroup b works on system order[first + b]
+  int nsys, ntot;
+  double4 *pos, *pos_next, *pk;
+  double *vel, *acc, *frc, *e, *rho, *xold;
+  int *nn;    // row lengths: pairs at the front | pairs at the back << 16
   unsigned short *list;
   int cap, ld;
   const TbDev *tbd;
   const TbF *tbf;
   int nt;
   double om[GH_MAXT], osm[GH_MAXT];
-  double rl2;
-  float near2f, lo2f, hi2f;  // build: inner-branch bound, FP32 prefilter band
-  int nst;                   // LDS staging slots (largest system + sentinel); 0 = none
+  double rl2, near2;  // build: list cut, inner-branch bound
+  int nst;            // LDS staging slots (largest system + sentinel); 0 = none
   double ev_ui;
   const double *T;
+  GhLine *dmax;
   double *out;  // per system: [0] epot ui, [1] ekin ui, [2] rebuilds, [3] fmax eV/A,
                 // [4] iterations, [5] converged
   int *flags;   // [0] list overflow, [1] longest row asked for past the capacity
@@ -115,261 +132,451 @@ __device__ __forceinline__ void bsum(BlockRed<BS> &R, double (&v)[NV]) {
   __syncthreads();
 }
 
-template <int BS>
-__device__ __forceinline__ double bmax(BlockRed<BS> &R, double v) {
-  v = wave_max(v);
+// Block-wide sums of the first NV values of v and the maximum of m, returned
+// to every thread; two barriers, the second before the next use of R.
+template <int BS, int NV>
+__device__ __forceinline__ void bred(BlockRed<BS> &R, double (&v)[3], double &m) {
+#pragma unroll
+  for (int k = 0; k < NV; ++k) v[k] = wave_total(v[k]);
+  m = wave_top(m);
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) R.v[threadIdx.x >> 6][k] = v[k];
+    R.v[threadIdx.x >> 6][3] = m;
+  }
   __syncthreads();
-  if ((threadIdx.x & 63) == 0) R.v[threadIdx.x >> 6][0] = v;
-  __syncthreads();
-  double m = R.v[0][0];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) v[k] = 0.0;
 #pragma unroll 4
-  for (int w = 1; w < BS / 64; ++w) m = fmax(m, R.v[w][0]);
+  for (int w = 0; w < BS / 64; ++w) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k) v[k] += R.v[w][k];
+    m = fmax(m, R.v[w][3]);
+  }
   __syncthreads();
-  return m;
 }
 
-// Per-workgroup state of one system: its atom range, the LDS staging of its
-// positions (fixed point around its first atom) and the parameter tables.
-struct Sys {
-  int a0, n;
-  bool staged;          // positions are in q (all within 64 A of the origin, 2^24 steps per A)
-  int4 *q;              // [n + 1]: positions, payload; q[n] = sentinel
-  unsigned char *ty;    // [n + 1] types
-  const TbDev *sp;      // FP64 parameters
-  const TbF *sf;        // FP32 parameters
+// Lane groups of G = 16 or 4: the group's bits of a wave mask, and sums over
+// a group in every lane of it.
+template <int G>
+__device__ __forceinline__ unsigned group_bits(unsigned long long m) {
+  return (unsigned)(m >> (threadIdx.x & 63 & ~(G - 1))) & ((1u << G) - 1);
+}
+template <int G>
+__device__ __forceinline__ double group_total(double v) {
+  v += dpp64<0xB1>(v);  // quad_perm [1,0,3,2]
+  v += dpp64<0x4E>(v);  // quad_perm [2,3,0,1]
+  if (G >= 8) v += dpp64<0x141>(v);   // row_half_mirror
+  if (G == 16) v += dpp64<0x140>(v);  // row_mirror
+  return v;
+}
+
+// The row of atom k of a system (verlet_self, Neighbour.F90:676-759: all
+// pairs with rd <= rl^2, itself excluded; rd rounded as the reference's
+// dot_product) by 16 lanes, 64 candidates per round; inner pairs fill it from
+// the front, the others from the back.  `on` is the same in the 16 lanes;
+// every lane of the wavefront calls it.
+__device__ __forceinline__ void batch_row(const BatchArgs &B, bool on, int a0, int n, int k) {
+  const int sub = threadIdx.x & 15, i = a0 + k, cap = B.cap;
+  const unsigned below = (1u << sub) - 1;
+  const double4 pi = B.pos[i];
+  unsigned short *row = B.list + (size_t)i * cap;
+  int m0 = 0, m1 = 0;
+  for (int j0 = 0; __any(on && j0 < n); j0 += 64) {
+    double4 p[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) p[u] = B.pos[a0 + min(j0 + 16 * u + sub, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = j0 + 16 * u + sub;
+      const double rd = dist2_rn(p[u].x - pi.x, p[u].y - pi.y, p[u].z - pi.z);
+      const bool keep = on && j < n && j != k && rd <= B.rl2, near = rd < B.near2;
+      const unsigned b0 = group_bits<16>(__ballot(keep && near));
+      const unsigned b1 = group_bits<16>(__ballot(keep && !near));
+      const int d = near ? m0 + __popc(b0 & below) : cap - 1 - (m1 + __popc(b1 & below));
+      if (keep && d >= 0 && d < cap) row[d] = (unsigned short)j;
+      m0 += __popc(b0);
+      m1 += __popc(b1);
+    }
+  }
+  if (!on) return;
+  if (sub == 0) {
+    if (m0 + m1 > cap) {
+      B.flags[0] = 1;
+      atomicMax(&B.flags[1], m0 + m1);
+    }
+    const int f = min(m0, cap);
+    B.nn[i] = f | (min(m1, cap - f) << 16);
+  }
+  if (sub < 3) B.xold[sub * B.ld + i] = sub == 0 ? pi.x : sub == 1 ? pi.y : pi.z;
+}
+
+// The row of atom i: its ends and, for 16 and 8 lanes, the first 16 pairs of
+// the front and the first 48 of the back, which are nearly always all of them.
+// These loads need nothing but the atom's number, so they are in flight
+// together with the atom's own data.
+template <int G>
+struct RowHead {
+  static constexpr int NF = 16 / G, NB = 48 / G;  // entries of a lane
+  const unsigned short *row;
+  int m0, m1, s[G >= 8 ? NF + NB : 1];
+};
+template <int G>
+__device__ __forceinline__ RowHead<G> row_head(const BatchArgs &B, int i, bool on) {
+  RowHead<G> r;
+  r.row = B.list + (size_t)i * B.cap;
+  const int w = on ? B.nn[i] : 0;
+  r.m0 = w & 0xFFFF;
+  r.m1 = w >> 16;
+  if constexpr (G >= 8) {
+    const int sub = threadIdx.x & (G - 1);
+#pragma unroll
+    for (int u = 0; u < r.NF; ++u) r.s[u] = r.row[min(sub + G * u, B.cap - 1)];
+#pragma unroll
+    for (int u = 0; u < r.NB; ++u) r.s[r.NF + u] = r.row[max(B.cap - 1 - (sub + G * u), 0)];
+  }
+  return r;
+}
+// Runs f(u) for every pair of a row after load(u, s), s the neighbour's index
+// in the system, four payloads in flight.  16 and 8 lanes: lane sub takes
+// entries sub, sub + G, ... of the front, then of the back.  4 lanes: lane sub
+// takes the quads sub, sub + 4, ... (one 8-byte load each, the next one in
+// flight while one is used).
+template <int G, class LOAD, class F>
+__device__ __forceinline__ void batch_each(const BatchArgs &B, const RowHead<G> &r, LOAD &&load,
+                                           F &&f) {
+  const int sub = threadIdx.x & (G - 1);
+  if constexpr (G >= 8) {
+#pragma unroll
+    for (int c = 0; c < r.NF + r.NB; c += 4) {
+      bool on[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const int e = c + u;
+        on[u] = e < r.NF ? sub + G * e < r.m0 : sub + G * (e - r.NF) < r.m1;
+        if (on[u]) load(u, r.s[e]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (on[u]) f(u);
+    }
+    auto run = [&](int k0, int m, const unsigned short *first, int dir) {
+      for (; k0 < m; k0 += 4 * G) {
+        int s[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[u] = first[dir * min(k0 + u * G, m - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) load(u, s[u]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          if (k0 + u * G < m) f(u);
+      }
+    };
+    run(sub + 16, r.m0, r.row, 1);
+    run(sub + 48, r.m1, r.row + (B.cap - 1), -1);
+  } else {
+    static_assert(G == 4, "16, 8 or 4 lanes per atom");
+    // virtual quads: the front's, padded to whole rounds of the four lanes,
+    // then the back's
+    const unsigned long long *qf = reinterpret_cast<const unsigned long long *>(r.row);
+    const int nf = ((r.m0 + 15) >> 4) << 2, nq = nf + ((r.m1 + 3) >> 2), last = (B.cap >> 2) - 1;
+    auto quad = [&](int v) { return v < nf ? qf[min(v, last)] : qf[max(last - (v - nf), 0)]; };
+    unsigned long long w = nq > 0 ? quad(sub) : 0ull;
+    for (int v = sub; v < nq; v += 4) {
+      const unsigned long long nw = quad(min(v + 4, nq));
+      const bool front = v < nf;
+      const int k0 = 4 * (front ? v : v - nf), m = front ? r.m0 : r.m1;
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        load(u, k0 + u < m ? GH_QSLOT(w, front ? u : 3 - u) : 0);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (k0 + u < m) f(u);
+      w = nw;
+    }
+  }
+}
+
+// One SMA-TB form of the passes.  FP64: Tb64.  Mixed: the FP32 forms on
+// positions quantised to 2^-GH_BFXK A about the system's first atom (QUANT:
+// pair vectors are then exact differences of integers below 2^53, held in
+// FP64) with TbF in that unit, or on FP64 positions with TbF in Angstrom
+// (systems whose staging does not fit LDS in the FIRE kernel; one rule for
+// all kernels, so a system's forces do not depend on the kernel).
+template <bool MIXED>
+using BForm = typename std::conditional<MIXED, TbF, Tb64>::type;
+
+template <bool QUANT>
+__device__ __forceinline__ double bq(double p, double o) {
+  return QUANT ? rint((p - o) * GH_BFXS) : p;
+}
+
+template <bool MIXED, bool SINGLE>
+struct BTable {
+  BForm<MIXED> t[SINGLE ? 1 : GH_MAXT * GH_MAXT];
+};
+template <bool MIXED, bool QUANT, bool SINGLE>
+__device__ __forceinline__ void load_table(BTable<MIXED, SINGLE> &T, const BatchArgs &B) {
+  if (SINGLE) return;
+  for (int k = threadIdx.x; k < GH_MAXT * GH_MAXT; k += blockDim.x)
+    if (k / GH_MAXT < B.nt && k % GH_MAXT < B.nt) {
+      if constexpr (!MIXED) T.t[k] = B.tbd[k].d;
+      else if constexpr (QUANT) T.t[k] = B.tbf[k];
+      else T.t[k] = B.tbd[k].f;
+    }
+  __syncthreads();
+}
+
+// What the force pass reads of an atom: its position (quantised, QUANT), and
+// 1/sqrt(rho) (FP64) or its FP32 offset and the type (mixed) in w.
+template <bool MIXED>
+__device__ __forceinline__ double pk_w(double eb, double e0, int t) {
+  if (!MIXED) return eb;
+  return __hiloint2double(t, __float_as_int((float)(eb - e0)));
+}
+
+// Density of atom i (smatb_preinteraction, TB.F90:367-455) by G lanes, stored
+// with its pack.  Positions from global memory (a system's are cached).
+template <bool MIXED, bool QUANT, bool SINGLE, int G>
+__device__ __forceinline__ void batch_rho(const BatchArgs &B, const BTable<MIXED, SINGLE> &T,
+                                          const BForm<MIXED> &p1, int a0, int i, bool on,
+                                          const RowHead<G> &row) {
+  const double4 o = QUANT ? B.pos[a0] : make_double4(0, 0, 0, 0);
+  const double4 pi = B.pos[i];
+  const double xi = bq<QUANT>(pi.x, o.x), yi = bq<QUANT>(pi.y, o.y), zi = bq<QUANT>(pi.z, o.z);
+  const int ti = SINGLE ? 0 : (int)pi.w;
+  double acc = 0.0;
+  double4 p[4];
+  batch_each<G>(
+      B, row, [&](int u, int s) { p[u] = B.pos[a0 + s]; },
+      [&](int u) {
+        const double vx = bq<QUANT>(p[u].x, o.x) - xi, vy = bq<QUANT>(p[u].y, o.y) - yi,
+                     vz = bq<QUANT>(p[u].z, o.z) - zi;
+        const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+        const BForm<MIXED> &P = SINGLE ? p1 : T.t[ti * GH_MAXT + (int)p[u].w];
+        if constexpr (MIXED) {
+          float band;
+          if (tb_rho_fx(P, rd, band)) acc += (double)band;
+        } else if (rd <= P.rce2) {
+          double dr, ir;
+          sqrt_rsq64(rd, dr, ir);
+          acc += tb_band64(P, dr);
+        }
+      });
+  acc = group_total<G>(acc);
+  if (on && (threadIdx.x & (G - 1)) == 0) {
+    B.rho[i] = acc;
+    B.pk[i] = make_double4(xi, yi, zi, pk_w<MIXED>(1.0 / sqrt(acc), B.e0, ti));
+  }
+}
+
+// Forces and repulsion of atom i (smatb_interact, TB.F90:457-586) by G lanes:
+// f = {Fx, Fy, Fz, sum of repulsions} (eV units) in each.
+template <bool MIXED, bool SINGLE, int G>
+__device__ __forceinline__ void batch_force(const BatchArgs &B, const BTable<MIXED, SINGLE> &T,
+                                            const BForm<MIXED> &p1, int a0, int i,
+                                            const RowHead<G> &row, double (&f)[4]) {
+  const double4 pi = B.pk[i];
+  const int ti = SINGLE ? 0 : MIXED ? __double2hiint(pi.w) : B.type[i];
+  f[0] = f[1] = f[2] = f[3] = 0.0;
+  double4 p[4];
+  int t[4];
+  batch_each<G>(
+      B, row,
+      [&](int u, int s) {
+        p[u] = B.pk[a0 + s];
+        if (!MIXED && !SINGLE) t[u] = B.type[a0 + s];
+      },
+      [&](int u) {
+        const double vx = p[u].x - pi.x, vy = p[u].y - pi.y, vz = p[u].z - pi.z;
+        const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
+        const int tj = SINGLE ? 0 : MIXED ? __double2hiint(p[u].w) : t[u];
+        const BForm<MIXED> &P = SINGLE ? p1 : T.t[ti * GH_MAXT + tj];
+        double s, rep;
+        if constexpr (MIXED) {
+          float sf, repul;
+          if (!tb_force_fx<true>(P, rd,
+                                 __int_as_float(__double2loint(pi.w)) +
+                                     __int_as_float(__double2loint(p[u].w)),
+                                 sf, repul))
+            return;
+          s = (double)sf;  // factor / r per unit of the pair vector
+          rep = (double)repul;
+        } else {
+          if (!(rd <= P.rce2)) return;
+          double dr, ir, factor;
+          sqrt_rsq64(rd, dr, ir);
+          tb_pair64(P, dr, pi.w + p[u].w, factor, rep);
+          s = factor * ir;
+        }
+        f[0] = fma(-s, vx, f[0]);
+        f[1] = fma(-s, vy, f[1]);
+        f[2] = fma(-s, vz, f[2]);
+        f[3] += rep;
+      });
+#pragma unroll
+  for (int d = 0; d < 4; ++d) f[d] = group_total<G>(f[d]);
+}
+
+// ---------------------------------------------------------------------------
+// Forces and Langevin steps over all systems: 16 lanes per atom.  What bounds
+// a step is the vector issue of the pair terms and, for small batches, the
+// two launches.
+// ---------------------------------------------------------------------------
+#define GH_BWG 256
+// Step `par` (parity): builds the rows of the systems whose atoms have moved
+// past the skin (`always`: of every system), then the densities.
+template <bool MIXED, bool QUANT, bool SINGLE, int G>
+__global__ __launch_bounds__(GH_BWG) void k_batch_rho(BatchArgs B, BForm<MIXED> p1, double skin,
+                                                      int par, int always) {
+  __shared__ BTable<MIXED, SINGLE> T;
+  load_table<MIXED, QUANT, SINGLE>(T, B);
+  const int i0 = (int)(blockIdx.x * GH_BWG + threadIdx.x) / G;
+  const bool live = i0 < B.ntot;
+  const int i = min(i0, B.ntot - 1), sub = threadIdx.x & (G - 1);
+  const int s = B.sysof[i], a0 = B.a0of[i];
+  RowHead<G> row = row_head<G>(B, i, live);
+  const double d2 = __longlong_as_double((long long)B.dmax[par * B.nsys + s].bits);
+  const bool due = live && (always || 2.0 * sqrt(d2) > skin);
+  if (live && i == a0 && sub == 0) {
+    // the next step's maximum starts from nothing (its writer is the force pass)
+    B.dmax[(par ^ 1) * B.nsys + s].bits = 0ull;
+    if (due && !always) B.out[s * OUTW + 2] += 1.0;
+  }
+  if (__any(due)) {
+    // 16 lanes build the rows of their 16 / G atoms one after the other
+#pragma unroll
+    for (int h = 0; h < 16 / G; ++h) {
+      const int src = (int)(threadIdx.x & 63 & ~15) + h * G;
+      const int ih = __shfl(i, src, 64), sh = __shfl(s, src, 64);
+      const bool on = __shfl((int)due, src, 64) != 0;
+      const int b0 = B.off[sh];
+      batch_row(B, on, b0, B.off[sh + 1] - b0, ih - b0);
+    }
+    __threadfence_block();  // the wavefront reads the rows its own lanes wrote
+    row = row_head<G>(B, i, live);
+  }
+  batch_rho<MIXED, QUANT, SINGLE, G>(B, T, p1, a0, i, live, row);
+}
+
+struct ErmakC {
+  double c0, c1, c2, sdr, sdv, crv1, crv2, dt, kB_ui;
 };
 
-// Stages positions (and types) of the system; `staged` is uniform.
-__device__ void sys_stage(const BatchArgs &B, Sys &S, int *flag, bool multi) {
-  if (B.nst == 0) {
-    S.staged = false;
+// Lane sub (0..2) of a 16-lane group: normals 2 sub and 2 sub + 1 of atom
+// `id` at `step` (philox_normals, one axis of it).
+__device__ __forceinline__ void axis_normals(unsigned long long seed, long long step, int id,
+                                             int axis, float &ga, float &gb) {
+  const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
+  const unsigned s0 = (unsigned)step, s1 = (unsigned)((unsigned long long)step >> 32);
+  const uint4 c = philox(make_uint4((unsigned)id, axis == 2 ? 1u : 0u, s0, s1), key);
+  philox_pair(axis == 1 ? c.z : c.x, axis == 1 ? c.w : c.y, ga, gb);
+}
+
+// The workgroup's displacements folded into their systems' maxima: one atomic
+// where its atoms share a system, one per atom otherwise.  Each maximum has a
+// cache line of its own (128 of them on eight lines, one atomic per
+// wavefront: 66 us per step more at 82,000 atoms).  d2: the same in a group's
+// lanes; all threads call it.
+template <int G>
+__device__ __forceinline__ void fold_sys_disp2(const BatchArgs &B, double d2, int s, bool live,
+                                               int par) {
+  __shared__ double part[GH_BWG / 64];
+  __shared__ int same[2];
+  if (threadIdx.x == 0) same[0] = s;
+  if (threadIdx.x == GH_BWG - 1) same[1] = s;
+  d2 = live ? d2 : 0.0;
+  const double w = wave_max(d2);
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = w;
+  __syncthreads();
+  GhLine *dst = B.dmax + (size_t)par * B.nsys;
+  if (same[0] == same[1]) {  // systems are contiguous
+    if (threadIdx.x == 0) {
+      double m = part[0];
+      for (int k = 1; k < GH_BWG / 64; ++k) m = fmax(m, part[k]);
+      atomicMax(&dst[s].bits, (unsigned long long)__double_as_longlong(m));
+    }
+  } else if (live && (threadIdx.x & (G - 1)) == 0) {
+    atomicMax(&dst[s].bits, (unsigned long long)__double_as_longlong(d2));
+  }
+}
+
+// ermak_a of the first step (Integration.F90:963-1011) for every atom, its
+// 16 lanes as in k_batch_force; positions move in place.
+__global__ __launch_bounds__(GH_BWG) void k_batch_ermak_a(BatchArgs B, ErmakC k,
+                                                          unsigned long long seed, long long step) {
+  const int i0 = (int)(blockIdx.x * GH_BWG + threadIdx.x) >> 4;
+  const bool live = i0 < B.ntot;
+  const int i = min(i0, B.ntot - 1), sub = threadIdx.x & 15, s = B.sysof[i];
+  double d2 = 0.0;
+  if (live && sub < 3) {
+    float ga, gb;
+    axis_normals(seed, step, i, sub, ga, gb);
+    const double f_lan = sqrt(k.kB_ui * B.T[s]) * B.osm[B.type[i]];
+    double *x = reinterpret_cast<double *>(B.pos + i) + sub;
+    const double v = *x + k.c1 * B.vel[sub * B.ld + i] + k.c2 * k.dt * B.acc[sub * B.ld + i] +
+                     f_lan * k.sdr * (double)ga;
+    *x = v;
+    const double dd = v - B.xold[sub * B.ld + i];
+    d2 = dd * dd;
+  }
+  fold_sys_disp2<16>(B, group_total<16>(d2), s, live, (int)(step & 1));
+}
+
+// Forces; MODE 0: stored with the per-atom energies (batch_compute); 1: then
+// ermak_b of `step` (Integration.F90:1013-1031) and ermak_a of the next, the
+// new positions to pos_next; 2: the run's last step, ermak_b and energies.
+// Lanes 0..2 of an atom's group hold its axes, lanes 4..6 draw the next
+// step's normals beside them.
+template <bool MIXED, bool QUANT, bool SINGLE, int G, int MODE>
+__global__ __launch_bounds__(GH_BWG) void k_batch_force(BatchArgs B, BForm<MIXED> p1, ErmakC k,
+                                                        unsigned long long seed, long long step) {
+  __shared__ BTable<MIXED, SINGLE> T;
+  load_table<MIXED, QUANT, SINGLE>(T, B);
+  const int i0 = (int)(blockIdx.x * GH_BWG + threadIdx.x) / G;
+  const bool live = i0 < B.ntot;
+  const int i = min(i0, B.ntot - 1), sub = threadIdx.x & (G - 1);
+  const int s = B.sysof[i], a0 = B.a0of[i];
+  const RowHead<G> row = row_head<G>(B, i, live);
+  const int ax = min(sub & 3, 2);
+  double v = 0.0, a = 0.0, xo = 0.0, x = 0.0;
+  if (MODE != 0) {  // issued before the pair loop
+    v = B.vel[ax * B.ld + i];
+    a = B.acc[ax * B.ld + i];
+    if (MODE == 1) {
+      xo = B.xold[ax * B.ld + i];
+      x = reinterpret_cast<const double *>(B.pos + i)[ax];
+    }
+  }
+  double f[4];
+  batch_force<MIXED, SINGLE, G>(B, T, p1, a0, i, row, f);
+  if (MODE != 1 && live && sub == 3) B.e[i] = (f[3] - sqrt(B.rho[i])) * B.ev_ui;
+  const double F = (ax == 0 ? f[0] : ax == 1 ? f[1] : f[2]) * B.ev_ui;
+  if (MODE == 0) {
+    if (live && sub < 3) B.frc[sub * B.ld + i] = F;
     return;
   }
-  const double4 o = B.pos[S.a0];
-  if (threadIdx.x == 0) *flag = 0;
-  __syncthreads();
-  for (int k = threadIdx.x; k < S.n; k += blockDim.x) {
-    const double4 p = B.pos[S.a0 + k];
-    const double dx = (p.x - o.x) * GH_BFXS, dy = (p.y - o.y) * GH_BFXS,
-                 dz = (p.z - o.z) * GH_BFXS;
-    if (fabs(dx) >= GH_FXLIM || fabs(dy) >= GH_FXLIM || fabs(dz) >= GH_FXLIM) *flag = 1;
-    const int t = B.type[S.a0 + k];
-    S.q[k] = make_int4(__double2int_rn(dx), __double2int_rn(dy), __double2int_rn(dz), t);
-    if (multi) S.ty[k] = (unsigned char)t;
+  float ga, gb;
+  axis_normals(seed, step + (sub >= 4 ? 1 : 0), i, ax, ga, gb);
+  const float ga_next = __shfl_down(ga, 4, 64);
+  const int t = B.type[i];
+  const double f_lan = sqrt(k.kB_ui * B.T[s]) * B.osm[t], om = B.om[t];
+  const double vel_v = f_lan * k.sdv * (k.crv1 * (double)ga + k.crv2 * (double)gb);
+  v = k.c0 * v + (k.c1 - k.c2) * a + k.c2 * F * om + vel_v;
+  a = F * om;
+  double d2 = 0.0;
+  if (MODE == 1) {
+    x = x + k.c1 * v + k.c2 * k.dt * a + f_lan * k.sdr * (double)ga_next;
+    d2 = x - xo;
+    d2 = live && sub < 3 ? d2 * d2 : 0.0;
   }
-  if (threadIdx.x == 0) {
-    S.q[S.n] = make_int4(GH_FXFAR, GH_FXFAR, GH_FXFAR, 0);
-    if (multi) S.ty[S.n] = 0;
+  if (live && sub < 3) {
+    B.vel[sub * B.ld + i] = v;
+    B.acc[sub * B.ld + i] = a;
+    if (MODE == 1) reinterpret_cast<double *>(B.pos_next + i)[sub] = x;
   }
-  __syncthreads();
-  S.staged = *flag == 0;
-  __syncthreads();
+  if (MODE == 1) fold_sys_disp2<G>(B, group_total<G>(d2), s, live, (int)((step + 1) & 1));
 }
-
-// verlet_self list of one system (Neighbour.F90:676-759: all pairs with
-// rd <= rl^2, i excluded; rd rounded as the reference's dot_product).  Rows
-// hold system-local indices, the pairs with r^2 < near2 first; the sentinel
-// index is n.  Staged: an FP32 prefilter on the exact fixed-point differences
-// decides all pairs but those within the band [lo2f, hi2f] around rl^2, which
-// the FP64 rd decides.  Ends with a barrier.
-__device__ void sys_build(const BatchArgs &B, const Sys &S) {
-  const int a0 = S.a0, n = S.n;
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const int i = a0 + k;
-    const double4 pi = B.pos[i];
-    RowWriter row{reinterpret_cast<unsigned long long *>(B.list), B.ld, i, B.cap, 0, 0ull};
-    if (S.staged) {
-      const int4 qi = S.q[k];
-      for (int sweep = 0; sweep < 2; ++sweep)
-        for (int j = 0; j < n; ++j) {
-          if (j == k) continue;
-          const int4 qj = S.q[j];
-          const float ux = (float)(qj.x - qi.x), uy = (float)(qj.y - qi.y),
-                      uz = (float)(qj.z - qi.z);
-          const float r2f = fmaf(ux, ux, fmaf(uy, uy, uz * uz)) * (float)(1.0 / (GH_BFXS * GH_BFXS));
-          if (r2f > B.hi2f || ((r2f < B.near2f) != (sweep == 0))) continue;
-          if (r2f >= B.lo2f) {
-            const double4 pj = B.pos[a0 + j];
-            if (dist2_rn(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z) > B.rl2) continue;
-          }
-          row.put(j);
-        }
-    } else {
-      for (int j = 0; j < n; ++j) {
-        if (j == k) continue;
-        const double4 pj = B.pos[a0 + j];
-        if (dist2_rn(pj.x - pi.x, pj.y - pi.y, pj.z - pi.z) <= B.rl2) row.put(j);
-      }
-    }
-    row.finish(n);
-    if (row.m > B.cap) {
-      B.flags[0] = 1;
-      atomicMax(&B.flags[1], row.m);
-    }
-    B.nn[i] = min(row.m, B.cap);
-    B.xold[i] = pi.x;
-    B.xold[B.ld + i] = pi.y;
-    B.xold[2 * B.ld + i] = pi.z;
-  }
-  __syncthreads();
-}
-
-// Both SMA-TB passes of one system (TB.F90:367-586); ends with a barrier.
-// MIXED and staged: LDS fixed-point pair vectors and the FP32 pair forms;
-// otherwise FP64 positions from global memory (L1/L2 resident per system).
-template <bool MIXED, bool SINGLE>
-__device__ void sys_forces(const BatchArgs &B, const Sys &S) {
-  const int a0 = S.a0, n = S.n;
-  const bool fx = MIXED && S.staged;
-  // pass 1: density
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const int i = a0 + k;
-    const int ti = SINGLE ? 0 : B.type[i];
-    double acc = 0.0;
-    if (fx) {
-      const int4 qi = S.q[k];
-      auto pair = [&](const int4 &q) {
-        const double dx = fxd(q.x, qi.x), dy = fxd(q.y, qi.y), dz = fxd(q.z, qi.z);
-        float band;
-        if (tb_rho_fx(SINGLE ? S.sf[0] : S.sf[ti * GH_MAXT + q.w],
-                      fma(dx, dx, fma(dy, dy, dz * dz)), band))
-          acc += (double)band;
-      };
-      for_each_quad(B.list, B.ld, i, B.nn[i], [&](unsigned long long w) {
-        const int4 q0 = S.q[GH_QSLOT(w, 0)], q1 = S.q[GH_QSLOT(w, 1)], q2 = S.q[GH_QSLOT(w, 2)],
-                   q3 = S.q[GH_QSLOT(w, 3)];
-        pair(q0);
-        pair(q1);
-        pair(q2);
-        pair(q3);
-      });
-    } else {
-      const double4 pi = B.pos[i];
-      for_each_slot(B.list, B.ld, i, B.nn[i], [&](int s) {
-        if (s >= n) return;  // sentinel
-        const int j = a0 + s;
-        const double4 pj = B.pos[j];
-        const TbDev &P = SINGLE ? S.sp[0] : S.sp[ti * GH_MAXT + B.type[j]];
-        const double vx = pj.x - pi.x, vy = pj.y - pi.y, vz = pj.z - pi.z;
-        if (MIXED) {
-          float band;
-          if (tb_rho_fx(P.f, fma(vx, vx, fma(vy, vy, vz * vz)), band)) acc += (double)band;
-        } else {
-          const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
-          if (rd <= P.d.rce2) {
-            double dr, ir;
-            sqrt_rsq64(rd, dr, ir);
-            acc += tb_band64(P.d, dr);
-          }
-        }
-      });
-    }
-    B.rho[i] = acc;
-    const double eb = 1.0 / sqrt(acc);
-    B.eband[i] = eb;
-    B.eband32[i] = (float)(eb - B.e0);  // the FP32 forms take 1/sqrt(rho) - e0
-  }
-  __syncthreads();
-  if (fx) {
-    for (int k = threadIdx.x; k < n; k += blockDim.x) S.q[k].w = __float_as_int(B.eband32[a0 + k]);
-    if (threadIdx.x == 0) S.q[n].w = 0;
-    __syncthreads();
-  }
-  // pass 2: forces and per-atom energies
-  for (int k = threadIdx.x; k < n; k += blockDim.x) {
-    const int i = a0 + k;
-    const int ti = SINGLE ? 0 : B.type[i];
-    double fxs = 0.0, fys = 0.0, fzs = 0.0, ei = 0.0, scale = B.ev_ui;
-    if (fx) {
-      const int4 qi = S.q[k];
-      const float di = __int_as_float(qi.w);
-      auto pair = [&](const int4 &q, int s) {
-        const double dx = fxd(q.x, qi.x), dy = fxd(q.y, qi.y), dz = fxd(q.z, qi.z);
-        float sf, repul;
-        if (tb_force_fx<true>(SINGLE ? S.sf[0] : S.sf[ti * GH_MAXT + S.ty[s]],
-                              fma(dx, dx, fma(dy, dy, dz * dz)), di + __int_as_float(q.w), sf,
-                              repul)) {
-          const double sfd = (double)sf;
-          fxs = fma(-sfd, dx, fxs);
-          fys = fma(-sfd, dy, fys);
-          fzs = fma(-sfd, dz, fzs);
-          ei += (double)repul;
-        }
-      };
-      for_each_quad(B.list, B.ld, i, B.nn[i], [&](unsigned long long w) {
-        const int s0 = GH_QSLOT(w, 0), s1 = GH_QSLOT(w, 1), s2 = GH_QSLOT(w, 2),
-                  s3 = GH_QSLOT(w, 3);
-        const int4 q0 = S.q[s0], q1 = S.q[s1], q2 = S.q[s2], q3 = S.q[s3];
-        pair(q0, s0);
-        pair(q1, s1);
-        pair(q2, s2);
-        pair(q3, s3);
-      });
-      scale = B.ev_ui;  // tb_force_fx returns factor / r per step: forces come out in ui/A
-    } else {
-      const double4 pi = B.pos[i];
-      const double ebi = B.eband[i];
-      const float di = B.eband32[i];
-      for_each_slot(B.list, B.ld, i, B.nn[i], [&](int s) {
-        if (s >= n) return;  // sentinel
-        const int j = a0 + s;
-        const double4 pj = B.pos[j];
-        const TbDev &P = SINGLE ? S.sp[0] : S.sp[ti * GH_MAXT + B.type[j]];
-        const double vx = pj.x - pi.x, vy = pj.y - pi.y, vz = pj.z - pi.z;
-        if (MIXED) {
-          float sf32, repul;
-          if (tb_force_fx<true>(P.f, fma(vx, vx, fma(vy, vy, vz * vz)), di + B.eband32[j],
-                                sf32, repul)) {
-            const double sf = (double)sf32;
-            fxs = fma(-sf, vx, fxs);
-            fys = fma(-sf, vy, fys);
-            fzs = fma(-sf, vz, fzs);
-            ei += (double)repul;
-          }
-        } else {
-          const double rd = fma(vx, vx, fma(vy, vy, vz * vz));
-          if (rd <= P.d.rce2) {
-            double dr, ir, factor, repul;
-            sqrt_rsq64(rd, dr, ir);
-            tb_pair64(P.d, dr, ebi + B.eband[j], factor, repul);
-            const double sf = factor * ir;
-            fxs = fma(-sf, vx, fxs);
-            fys = fma(-sf, vy, fys);
-            fzs = fma(-sf, vz, fzs);
-            ei += repul;
-          }
-        }
-      });
-    }
-    B.frc[i] = fxs * scale;
-    B.frc[B.ld + i] = fys * scale;
-    B.frc[2 * B.ld + i] = fzs * scale;
-    B.e[i] = (ei - sqrt(B.rho[i])) * B.ev_ui;
-  }
-  __syncthreads();
-}
-
-// Shared tables and the system of this workgroup.
-#define SYS_SETUP(SINGLE)                                                                  \
-  extern __shared__ int4 dyn_q[];                                                          \
-  __shared__ TbDev sp[SINGLE ? 1 : GH_MAXT * GH_MAXT];                                     \
-  __shared__ TbF sf[SINGLE ? 1 : GH_MAXT * GH_MAXT];                                       \
-  __shared__ BlockRed<BS> R;                                                               \
-  __shared__ int sflag;                                                                    \
-  for (int k_ = threadIdx.x; k_ < (SINGLE ? 1 : GH_MAXT * GH_MAXT); k_ += blockDim.x) {    \
-    sp[k_] = B.tbd[k_];                                                                    \
-    sf[k_] = B.tbf[k_];                                                                    \
-  }                                                                                        \
-  const int s = B.order[B.first + blockIdx.x];                                             \
-  Sys S;                                                                                   \
-  S.a0 = B.off[s];                                                                         \
-  S.n = B.off[s + 1] - S.a0;                                                               \
-  S.q = dyn_q;                                                                             \
-  S.ty = reinterpret_cast<unsigned char *>(dyn_q + B.nst);                                 \
-  S.sp = sp;                                                                               \
-  S.sf = sf;                                                                               \
-  S.staged = false;                                                                        \
-  __syncthreads();
 
 // epot (ui) and ekin about the centre of mass (ui) of one system.
 template <int BS>
@@ -396,236 +603,332 @@ __device__ void sys_energies(const BatchArgs &B, BlockRed<BS> &R, int a0, int a1
   epot = s[0];
   ekin = 0.5 * k[0];
 }
-
-template <bool MIXED, bool SINGLE, int BS>
-__global__ __launch_bounds__(BS) void k_batch_compute(BatchArgs B) {
-  SYS_SETUP(SINGLE)
-  sys_stage(B, S, &sflag, !SINGLE);
-  sys_build(B, S);
-  sys_forces<MIXED, SINGLE>(B, S);
+// The energies of every system, a workgroup each.
+__global__ __launch_bounds__(GH_BWG) void k_batch_energies(BatchArgs B) {
+  __shared__ BlockRed<GH_BWG> R;
+  const int s = blockIdx.x;
   double ep, ek;
-  sys_energies(B, R, S.a0, S.a0 + S.n, ep, ek);
+  sys_energies(B, R, B.off[s], B.off[s + 1], ep, ek);
   if (threadIdx.x == 0) {
     B.out[s * OUTW + 0] = ep;
     B.out[s * OUTW + 1] = ek;
   }
 }
 
-struct ErmakC {
-  double c0, c1, c2, sdr, sdv, crv1, crv2, dt, kB_ui;
-};
-
-// nsteps Ermak steps of every system (ermak_a / ermak_b with the Philox
-// stream keyed by (seed, step, atom)); lists rebuilt per system when
-// 2 max|x - x_old| exceeds the skin.
-template <bool MIXED, bool SINGLE, int BS>
-__global__ __launch_bounds__(BS) void k_batch_langevin(BatchArgs B, int nsteps,
-                                                              long long step0, ErmakC k,
-                                                              unsigned long long seed,
-                                                              double skin) {
-  // The step constants live in LDS and are read where they are used: held in
-  // scalar registers for the whole kernel they were spilled, and the ROCm 7.2
-  // compiler has mis-allocated such spills here (a later kernel-argument load
-  // overwrote the registers before they were saved).
-  __shared__ ErmakC kc;
-  __shared__ unsigned long long kseed;
-  __shared__ double kskin;
-  if (threadIdx.x == 0) {
-    kc = k;
-    kseed = seed;
-    kskin = skin;
-  }
-  SYS_SETUP(SINGLE)
-  const int a0 = S.a0, a1 = S.a0 + S.n;
-  const double skt = sqrt(kc.kB_ui * B.T[s]);
-  int nreb = 0;
-  for (int st = 0; st < nsteps; ++st) {
-    const long long step = step0 + st;
-    double d2 = 0.0;
-    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
-      double g[6];
-      philox_normals(kseed, step, i, g);
-#pragma unroll
-      for (int q = 0; q < 6; ++q) B.gn[q * B.ld + i] = (float)g[q];  // exact: FP32 normals
-      const double f_lan = skt * B.osm[B.type[i]];
-      double4 p = B.pos[i];
-      double x[3] = {p.x, p.y, p.z};
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double pos_v = f_lan * kc.sdr * g[2 * d];
-        x[d] = x[d] + kc.c1 * B.vel[d * B.ld + i] + kc.c2 * kc.dt * B.acc[d * B.ld + i] + pos_v;
-        const double dd = x[d] - B.xold[d * B.ld + i];
-        d2 += dd * dd;
-      }
-      p.x = x[0];
-      p.y = x[1];
-      p.z = x[2];
-      B.pos[i] = p;
-    }
-    const double dmax2 = bmax(R, d2);
-    if (MIXED) sys_stage(B, S, &sflag, !SINGLE);
-    if (2.0 * sqrt(dmax2) > kskin) {
-      if (!MIXED) sys_stage(B, S, &sflag, !SINGLE);
-      sys_build(B, S);
-      ++nreb;
-    }
-    sys_forces<MIXED, SINGLE>(B, S);
-    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
-      double g[6];
-#pragma unroll
-      for (int q = 0; q < 6; ++q) g[q] = (double)B.gn[q * B.ld + i];  // this step's stepa draw
-      const int t = B.type[i];
-      const double f_lan = skt * B.osm[t];
-      const double om = B.om[t];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double vel_v = f_lan * kc.sdv * (kc.crv1 * g[2 * d] + kc.crv2 * g[2 * d + 1]);
-        const double f = B.frc[d * B.ld + i];
-        B.vel[d * B.ld + i] = kc.c0 * B.vel[d * B.ld + i] + (kc.c1 - kc.c2) * B.acc[d * B.ld + i] +
-                              kc.c2 * f * om + vel_v;
-        B.acc[d * B.ld + i] = f * om;
-      }
-    }
-    __syncthreads();
-  }
-  double ep, ek;
-  sys_energies(B, R, a0, a1, ep, ek);
-  if (threadIdx.x == 0) {
-    B.out[s * OUTW + 0] = ep;
-    B.out[s * OUTW + 1] = ek;
-    B.out[s * OUTW + 2] += nreb;
-  }
-}
-
+// ---------------------------------------------------------------------------
+// FIRE (Bitzek et al. 2006), a workgroup per system and all its iterations in
+// one launch: velocity-Verlet MD step, then P = F.v; v <- (1-a) v + a |v|
+// F/|F|; P > 0 for more than N_min steps grows dt (x1.1, capped at dt_max) and
+// shrinks a (x0.99); P <= 0 halves dt, zeroes v and resets a.  Mixed
+// precision: a first launch runs every system with the FP32 pair terms until
+// max|F| < fswitch, a second goes on in FP64; convergence is max|F| < ftol in
+// FP64.  (Both in one kernel held 146 registers, three wavefronts per SIMD;
+// the mixed one fits the 128 of four.)
+//
+// An iteration is a chain of passes over the system's atoms with barriers
+// between them, so what counts is how few trips to memory it makes and how
+// many systems a compute unit holds: four lanes per atom in the passes; one
+// loop over the atoms does the mixing of the last iteration, the first half
+// kick and the drift and stages the new positions (every thread forms the
+// new position of the first atom, the staging's origin, itself); the force
+// pass does the second half kick and the sums.  1024 Au clusters of 13..309
+// atoms, mixed: 54 us per iteration with one lane per atom and a loop per
+// operation, 44 now.
+// ---------------------------------------------------------------------------
 struct FireC {
-  double dt_max, alpha0, fswitch, ftol, ui_ev;
-  int max_iter, mixed;
+  double dt_max, alpha0, fstop, ui_ev;  // fstop: fswitch (mixed) or ftol, eV/A
+  int max_iter, resume;
+};
+struct FireState {  // between the launches, per system
+  double dt, alpha, fmax;
+  int npos, it, done, conv;
 };
 
-template <bool SINGLE>
-__device__ __forceinline__ void fire_forces(const BatchArgs &B, Sys &S, int *flag, bool mixed) {
-  if (mixed) {
-    sys_stage(B, S, flag, !SINGLE);
-    sys_forces<true, SINGLE>(B, S);
-  } else {
-    sys_forces<false, SINGLE>(B, S);
+// The rows of the system's atoms; ends with a barrier.
+__device__ void sys_build(const BatchArgs &B, int a0, int n) {
+  const int per = (int)blockDim.x >> 4, g = (int)threadIdx.x >> 4;
+  for (int k0 = 0; k0 < n; k0 += per) batch_row(B, k0 + g < n, a0, n, min(k0 + g, n - 1));
+  __syncthreads();
+}
+
+#define GH_FG 4  // lanes per atom
+// LDS staging of a mixed system: positions in steps of 2^-GH_BFXK A about its
+// first atom with eband32 as the fourth word, and types; `far`: an atom lies
+// 64 A or more away, the passes then quantise positions from global memory.
+struct Stage {
+  int4 *q;
+  unsigned char *ty;
+  int *far;
+};
+__device__ __forceinline__ void stage_atom(const Stage &S, int k, const double (&x)[3],
+                                           const double (&o)[3]) {
+  const double dx = (x[0] - o[0]) * GH_BFXS, dy = (x[1] - o[1]) * GH_BFXS,
+               dz = (x[2] - o[2]) * GH_BFXS;
+  if (!(fabs(dx) < GH_FXLIM && fabs(dy) < GH_FXLIM && fabs(dz) < GH_FXLIM)) *S.far = 1;
+  S.q[k] = make_int4(__double2int_rn(dx), __double2int_rn(dy), __double2int_rn(dz), 0);
+}
+
+template <bool MIXED, bool QUANT, bool SINGLE>
+__device__ __forceinline__ void fire_rho(const BatchArgs &B, const Stage &S,
+                                         const BTable<MIXED, SINGLE> &T, const BForm<MIXED> &p1,
+                                         int a0, int n) {
+  const int sub = threadIdx.x & (GH_FG - 1), g = (int)threadIdx.x / GH_FG;
+  const int per = (int)blockDim.x / GH_FG;
+  const bool lds = QUANT && !*S.far;
+  for (int k0 = 0; k0 < n; k0 += per) {
+    const bool on = k0 + g < n;
+    const int k = min(k0 + g, n - 1), i = a0 + k;
+    const RowHead<GH_FG> row = row_head<GH_FG>(B, i, on);
+    if (!lds) {
+      batch_rho<MIXED, QUANT, SINGLE, GH_FG>(B, T, p1, a0, i, on, row);
+    } else if constexpr (QUANT) {
+      const int4 qi = S.q[k];
+      const int ti = SINGLE ? 0 : S.ty[k];
+      double acc = 0.0;
+      int4 q[4];
+      int t[4];
+      batch_each<GH_FG>(
+          B, row,
+          [&](int u, int s) {
+            q[u] = S.q[s];
+            t[u] = SINGLE ? 0 : S.ty[s];
+          },
+          [&](int u) {
+            const double dx = fxd(q[u].x, qi.x), dy = fxd(q[u].y, qi.y), dz = fxd(q[u].z, qi.z);
+            float band;
+            if (tb_rho_fx(SINGLE ? p1 : T.t[ti * GH_MAXT + t[u]],
+                          fma(dx, dx, fma(dy, dy, dz * dz)), band))
+              acc += (double)band;
+          });
+      acc = group_total<GH_FG>(acc);
+      if (on && sub == 0) {
+        B.rho[i] = acc;
+        S.q[k].w = __float_as_int((float)(1.0 / sqrt(acc) - B.e0));
+      }
+    }
+  }
+  __syncthreads();
+}
+
+// Forces and energies; hdt > 0: then the second half kick (v += hdt F / m)
+// and the sums pv = {F.v, |v|^2, |F|^2} of the thread's atoms.  fm2: the
+// largest |F|^2 of its atoms.
+template <bool MIXED, bool QUANT, bool SINGLE>
+__device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
+                                           const BTable<MIXED, SINGLE> &T, const BForm<MIXED> &p1,
+                                           int a0, int n, double hdt, double (&pv)[3],
+                                           double &fm2) {
+  const int sub = threadIdx.x & (GH_FG - 1), g = (int)threadIdx.x / GH_FG;
+  const int per = (int)blockDim.x / GH_FG;
+  const bool lds = QUANT && !*S.far;
+  for (int k0 = 0; k0 < n; k0 += per) {
+    const bool on = k0 + g < n;
+    const int k = min(k0 + g, n - 1), i = a0 + k;
+    const RowHead<GH_FG> row = row_head<GH_FG>(B, i, on);
+    const int ax = min(sub, 2);
+    const double v0 = hdt > 0.0 ? B.vel[ax * B.ld + i] : 0.0;
+    double f[4] = {0.0, 0.0, 0.0, 0.0};
+    if (!lds) {
+      batch_force<MIXED, SINGLE, GH_FG>(B, T, p1, a0, i, row, f);
+    } else if constexpr (QUANT) {
+      const int4 qi = S.q[k];
+      const int ti = SINGLE ? 0 : S.ty[k];
+      const float di = __int_as_float(qi.w);
+      int4 q[4];
+      int t[4];
+      batch_each<GH_FG>(
+          B, row,
+          [&](int u, int s) {
+            q[u] = S.q[s];
+            t[u] = SINGLE ? 0 : S.ty[s];
+          },
+          [&](int u) {
+            const double dx = fxd(q[u].x, qi.x), dy = fxd(q[u].y, qi.y), dz = fxd(q[u].z, qi.z);
+            float sf, repul;
+            if (tb_force_fx<true>(SINGLE ? p1 : T.t[ti * GH_MAXT + t[u]],
+                                  fma(dx, dx, fma(dy, dy, dz * dz)),
+                                  di + __int_as_float(q[u].w), sf, repul)) {
+              const double sfd = (double)sf;
+              f[0] = fma(-sfd, dx, f[0]);
+              f[1] = fma(-sfd, dy, f[1]);
+              f[2] = fma(-sfd, dz, f[2]);
+              f[3] += (double)repul;
+            }
+          });
+#pragma unroll
+      for (int d = 0; d < 4; ++d) f[d] = group_total<GH_FG>(f[d]);
+    }
+    const double F = (ax == 0 ? f[0] : ax == 1 ? f[1] : f[2]) * B.ev_ui;
+    if (on && sub < 3) {
+      B.frc[sub * B.ld + i] = F;
+      if (hdt > 0.0) {
+        const double v = v0 + hdt * F * B.om[SINGLE ? 0 : B.type[i]];
+        B.vel[sub * B.ld + i] = v;
+        pv[0] += F * v;
+        pv[1] += v * v;
+        pv[2] += F * F;
+      }
+    } else if (on) {
+      B.e[i] = (f[3] - sqrt(B.rho[i])) * B.ev_ui;
+    }
+    if (on && sub == 0) {
+      const double Fy = f[1] * B.ev_ui, Fz = f[2] * B.ev_ui;
+      fm2 = fmax(fm2, F * F + Fy * Fy + Fz * Fz);
+    }
   }
 }
 
-template <int BS>
-__device__ double sys_fmax(const BatchArgs &B, BlockRed<BS> &R, int a0, int a1) {
-  double m = 0.0;
-  for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
-    const double fx = B.frc[i], fy = B.frc[B.ld + i], fz = B.frc[2 * B.ld + i];
-    m = fmax(m, fx * fx + fy * fy + fz * fz);
-  }
-  return sqrt(bmax(R, m));
-}
-
-// FIRE (Bitzek et al. 2006) per system: velocity-Verlet MD step, then
-// P = F.v; v <- (1-a) v + a |v| F/|F|; P > 0 for more than N_min steps grows
-// dt (x1.1, capped at dt_max) and shrinks a (x0.99); P <= 0 halves dt, zeroes
-// v and resets a.  Mixed precision switches to FP64 pair terms once
-// max|F| < fswitch; convergence is max|F| < ftol in FP64.
-template <bool SINGLE, int BS>
-__global__ __launch_bounds__(BS) void k_batch_fire(BatchArgs B, FireC fc_arg, double skin_arg) {
-  // constants in LDS, read where used (see k_batch_langevin)
+template <bool MIXED, bool QUANT, bool SINGLE, int BS>
+__global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg, double skin_arg,
+                                                   FireState *fst, BForm<MIXED> p_arg) {
+  // The constants live in LDS and are read where they are used: held in
+  // scalar registers for a whole kernel of this kind they were spilled, and
+  // the ROCm 7.2 compiler has mis-allocated such spills (a later
+  // kernel-argument load overwrote the registers before they were saved).
   __shared__ FireC fc;
   __shared__ double skin;
+  __shared__ BForm<MIXED> p1;
+  extern __shared__ int4 dyn_q[];
+  __shared__ BTable<MIXED, SINGLE> T;
+  __shared__ BlockRed<BS> R;
+  __shared__ int sfar;
+  const int s = B.order[B.first + blockIdx.x];
+  FireState st = fst[s];
+  if (fc_arg.resume && st.done) return;
   if (threadIdx.x == 0) {
     fc = fc_arg;
     skin = skin_arg;
+    p1 = p_arg;
+    sfar = 0;
   }
-  SYS_SETUP(SINGLE)
-  const int a0 = S.a0, a1 = S.a0 + S.n;
-  bool mixed = fc.mixed != 0;
-  for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x)
-    for (int d = 0; d < 3; ++d) B.vel[d * B.ld + i] = 0.0;
-  sys_stage(B, S, &sflag, !SINGLE);
-  sys_build(B, S);
-  fire_forces<SINGLE>(B, S, &sflag, mixed);
-  double dt = fc.dt_max * 0.1, alpha = fc.alpha0;
-  int npos = 0, it = 0, conv = 0;
-  double fmax = 0.0;
-  for (it = 0; it < fc.max_iter; ++it) {
-    fmax = sys_fmax(B, R, a0, a1) * fc.ui_ev;  // eV/A
-    if (mixed && fmax < fc.fswitch) {
-      mixed = false;
-      fire_forces<SINGLE>(B, S, &sflag, mixed);
-      fmax = sys_fmax(B, R, a0, a1) * fc.ui_ev;
+  load_table<MIXED, QUANT, SINGLE>(T, B);
+  const int a0 = B.off[s], a1 = B.off[s + 1], n = a1 - a0;
+  Stage S{dyn_q, reinterpret_cast<unsigned char *>(dyn_q + B.nst), &sfar};
+  __syncthreads();
+  if (!fc.resume) {
+    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x)
+      for (int d = 0; d < 3; ++d) B.vel[d * B.ld + i] = 0.0;
+    st.dt = fc.dt_max * 0.1;
+    st.alpha = fc.alpha0;
+    st.npos = st.it = st.done = st.conv = 0;
+    sys_build(B, a0, n);
+  }
+  if (QUANT) {
+    const double4 o4 = B.pos[a0];
+    const double o[3] = {o4.x, o4.y, o4.z};
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+      const double4 p = B.pos[a0 + k];
+      const double x[3] = {p.x, p.y, p.z};
+      stage_atom(S, k, x, o);
+      if (!SINGLE) S.ty[k] = (unsigned char)B.type[a0 + k];
     }
-    if (!mixed && fmax < fc.ftol) {
-      conv = 1;
+    __syncthreads();
+  }
+  double pv[3] = {0.0, 0.0, 0.0}, fm2 = 0.0;
+  fire_rho<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n);
+  fire_force<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+  // the mixing of the last iteration, still to be applied to v: v <- cm v + mixv F
+  double cm = 1.0, mixv = 0.0;
+  bool pend = false;
+  bred<BS, 0>(R, pv, fm2);
+  double dt = st.dt, alpha = st.alpha, fnow = sqrt(fm2) * fc.ui_ev;  // eV/A
+  int it = st.it, npos = st.npos;
+  bool stop = false;
+  for (; it < fc.max_iter; ++it) {
+    st.fmax = fnow;
+    if (fnow < fc.fstop) {
+      stop = true;
       break;
     }
-    // velocity Verlet step
-    double d2 = 0.0;
-    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
-      const double om = B.om[B.type[i]];
-      double4 p = B.pos[i];
-      double x[3] = {p.x, p.y, p.z};
+    // mixing, first half kick, drift; the origin of the staging first
+    double o[3] = {0.0, 0.0, 0.0}, d2 = 0.0;
+    auto move = [&](int i, double (&x)[3], bool store) {
+      const double4 p = B.pos[i];
+      const double om = B.om[SINGLE ? 0 : (int)p.w];
+      x[0] = p.x;
+      x[1] = p.y;
+      x[2] = p.z;
+      double e2 = 0.0;
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        const double v = B.vel[d * B.ld + i] + 0.5 * dt * B.frc[d * B.ld + i] * om;
-        B.vel[d * B.ld + i] = v;
+        const double F = B.frc[d * B.ld + i];
+        double v = B.vel[d * B.ld + i];
+        if (pend) v = cm * v + mixv * F;
+        v = v + 0.5 * dt * F * om;
         x[d] += dt * v;
-        const double dd = x[d] - B.xold[d * B.ld + i];
-        d2 += dd * dd;
+        if (store) {
+          B.vel[d * B.ld + i] = v;
+          const double dd = x[d] - B.xold[d * B.ld + i];
+          e2 += dd * dd;
+        }
       }
-      p.x = x[0];
-      p.y = x[1];
-      p.z = x[2];
-      B.pos[i] = p;
+      if (store) B.pos[i] = make_double4(x[0], x[1], x[2], p.w);
+      return e2;
+    };
+    if (QUANT) {
+      move(a0, o, false);
+      if (threadIdx.x == 0) sfar = 0;
+      __syncthreads();  // every thread has read atom a0 before it moves
     }
-    const double dmax2 = bmax(R, d2);
-    if (2.0 * sqrt(dmax2) > skin) {
-      sys_stage(B, S, &sflag, !SINGLE);
-      sys_build(B, S);
+    for (int k = threadIdx.x; k < n; k += blockDim.x) {
+      double x[3];
+      d2 = fmax(d2, move(a0 + k, x, true));
+      if (QUANT) stage_atom(S, k, x, o);
     }
-    fire_forces<SINGLE>(B, S, &sflag, mixed);
-    double pv[3] = {0.0, 0.0, 0.0};  // F.v, |v|^2, |F|^2
-    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
-      const double om = B.om[B.type[i]];
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double f = B.frc[d * B.ld + i];
-        const double v = B.vel[d * B.ld + i] + 0.5 * dt * f * om;
-        B.vel[d * B.ld + i] = v;
-        pv[0] += f * v;
-        pv[1] += v * v;
-        pv[2] += f * f;
-      }
-    }
-    bsum<BS, 3>(R, pv);
-    const double mixv = pv[2] > 0.0 ? alpha * sqrt(pv[1]) / sqrt(pv[2]) : 0.0;
-    const bool up = pv[0] > 0.0;
-    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x)
-#pragma unroll
-      for (int d = 0; d < 3; ++d) {
-        const double v = B.vel[d * B.ld + i];
-        B.vel[d * B.ld + i] = up ? (1.0 - alpha) * v + mixv * B.frc[d * B.ld + i] : 0.0;
-      }
-    if (up) {
+    double none[3] = {0.0, 0.0, 0.0};
+    bred<BS, 0>(R, none, d2);
+    if (2.0 * sqrt(d2) > skin) sys_build(B, a0, n);
+    pv[0] = pv[1] = pv[2] = fm2 = 0.0;
+    fire_rho<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n);
+    fire_force<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
+    bred<BS, 3>(R, pv, fm2);
+    fnow = sqrt(fm2) * fc.ui_ev;
+    pend = true;
+    if (pv[0] > 0.0) {
+      cm = 1.0 - alpha;
+      mixv = pv[2] > 0.0 ? alpha * sqrt(pv[1]) / sqrt(pv[2]) : 0.0;
       ++npos;
       if (npos > 5) {
         dt = fmin(dt * 1.1, fc.dt_max);
         alpha *= 0.99;
       }
     } else {
+      cm = mixv = 0.0;
       npos = 0;
       dt *= 0.5;
       alpha = fc.alpha0;
     }
-    __syncthreads();
   }
-  double ep, ek;
-  sys_energies(B, R, a0, a1, ep, ek);
+  if (pend)
+    for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x)
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double v = B.vel[d * B.ld + i];
+        B.vel[d * B.ld + i] = cm == 0.0 && mixv == 0.0 ? 0.0 : cm * v + mixv * B.frc[d * B.ld + i];
+      }
+  const bool done = !MIXED || !stop;  // a mixed system below fswitch goes on in FP64
+  double ep = 0.0, ek = 0.0;
+  if (done) sys_energies(B, R, a0, a1, ep, ek);
   if (threadIdx.x == 0) {
-    B.out[s * OUTW + 0] = ep;
-    B.out[s * OUTW + 3] = fmax;
-    B.out[s * OUTW + 4] = it;
-    B.out[s * OUTW + 5] = conv;
+    st.dt = dt;
+    st.alpha = alpha;
+    st.npos = npos;
+    st.it = it;
+    st.done = done;
+    st.conv = !MIXED && stop;
+    fst[s] = st;
+    if (done) {
+      B.out[s * OUTW + 0] = ep;
+      B.out[s * OUTW + 3] = st.fmax;
+      B.out[s * OUTW + 4] = it;
+      B.out[s * OUTW + 5] = st.conv;
+    }
   }
+}
+
+__global__ void k_batch_zero(GhLine *p, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) p[i].bits = 0ull;
 }
 
 __global__ void k_batch_scale(int nsys, const int *__restrict__ off,
@@ -675,16 +978,19 @@ static BatchArgs bargs(const gh_batch *b) {
   A.order = b->order;
   A.first = 0;
   A.type = b->type;
+  A.sysof = b->sysof;
+  A.a0of = b->a0of;
+  A.nsys = b->nsys;
+  A.ntot = b->ntot;
   A.pos = b->pos;
+  A.pos_next = b->pos_next;
+  A.pk = b->pk;
   A.vel = b->vel;
   A.acc = b->acc;
   A.frc = b->frc;
   A.e = b->e;
   A.rho = b->rho;
-  A.eband = b->eband;
   A.xold = b->xold;
-  A.eband32 = b->eband32;
-  A.gn = b->gn;
   A.nn = b->nn;
   A.list = b->list;
   A.cap = b->cap;
@@ -694,21 +1000,17 @@ static BatchArgs bargs(const gh_batch *b) {
   A.e0 = b->tb_e0;
   A.nt = b->nt;
   A.nst = b->nst;
+  A.dmax = b->dmax;
   for (int t = 0; t < GH_MAXT; ++t) {
     A.om[t] = 1.0 / b->mass_t[t];
     A.osm[t] = sqrt(A.om[t]);
   }
   const double rl = b->rcut + b->skin;
   A.rl2 = rl * rl;
-  // FP32 prefilter of the build: its error on r^2 stays below 1e-4 A^2 for
-  // staged clusters (< 64 A); the band is thirty times that
-  const double margin = std::max(3e-3, 1e-4 * A.rl2);
-  A.lo2f = (float)(A.rl2 - margin);
-  A.hi2f = (float)(A.rl2 + margin);
   double rci = 1e300;
   for (int i = 0; i < b->nt; ++i)
     for (int j = 0; j < b->nt; ++j) rci = std::min(rci, b->tb[i * GH_MAXT + j].rci);
-  A.near2f = (float)(rci * rci);
+  A.near2 = rci * rci;
   A.ev_ui = ghc::ev_ui();
   A.T = b->T;
   A.out = b->out;
@@ -764,37 +1066,46 @@ static int batch_ready(gh_batch *b) {
     int est = (int)(4.18879 * rl * rl * rl * dens) + 16;
     b->cap = std::max(8, std::min(nmax, std::max(est, b->cap_req)));
     b->cap = (b->cap + 7) / 8 * 8;
-    BT(balloc(b, &b->list, (size_t)(b->cap + 4 * GH_LIST_PAD_QUADS) * b->ld));
+    BT(balloc(b, &b->list, (size_t)b->cap * b->ld));
     // LDS staging of the largest system (int4 + type byte per atom, and the
-    // sentinel) beside the static tables; larger systems use global memory
-    const size_t stat = (b->nt > 1 ? GH_MAXT * GH_MAXT : 1) * (sizeof(TbDev) + sizeof(TbF)) +
-                        sizeof(double) * 8 * (GH_BBLOCK / 64) + 64;
+    // sentinel) beside tables of 344 B per type pair, within 64 KB; larger
+    // systems use global memory.  The rule also says which FP32 form a mixed
+    // batch computes (quantised positions where it holds), so it does not
+    // follow the size of the tables' structures.
+    const size_t stat = (b->nt > 1 ? GH_MAXT * GH_MAXT : 1) * 344 +
+                        sizeof(double) * 8 * 8 + 64;
     const size_t need = 17 * (size_t)(nmax + 1);
-    b->nmax = nmax;
     b->nst = stat + need <= 65536 ? nmax + 1 : 0;
   }
   return 0;
 }
 
-static size_t batch_lds(const gh_batch *b) { return 17 * (size_t)b->nst; }
-
-// One batch kernel over all systems.  The systems above GH_BIGSYS atoms bound
-// the run (one workgroup each, largest first), so they get 1024-thread
-// workgroups (four wavefronts per SIMD) on a second stream while the rest
-// run on the batch stream; `big(first, count, stream)` and `rest(first,
-// count, nmax, stream)` launch the two parts.  Variants whose 1024-thread
-// form would spill registers pass big_ok = false and keep 512 threads.
-template <class BIG, class REST>
-static int split_launch(gh_batch *b, bool big_ok, BIG &&big, REST &&rest) {
-  const int nbig = big_ok ? b->nbig : 0;
+// The FIRE kernel over all systems.  Multi-type systems above GH_BIGSYS atoms
+// bound a run (one workgroup each, largest first), so they get 1024-thread
+// workgroups on a second stream beside the rest (one-type variants would
+// need more than the registers of a 1024-thread workgroup).  256 threads
+// otherwise: four systems then share a compute unit and hide each other's
+// barriers (1024 Au clusters, mixed, a quench of 100 iterations: 128 threads
+// 9.9 ms, 256 6.7, 512 7.2; registers for five wavefronts per SIMD instead
+// of four spill: 9.0).
+template <bool MIXED, bool QUANT>
+static int launch_fire(gh_batch *b, const BatchArgs &A, const FireC &fc, const BForm<MIXED> &p) {
+  const size_t lds = QUANT ? 17 * (size_t)b->nst : 0;
+  const int nbig = b->nt > 1 ? b->nbig : 0;
+  BatchArgs A1 = A;
   if (nbig > 0) {
     BH(b, hipEventRecord(b->ev_fork, b->stream));
     BH(b, hipStreamWaitEvent(b->stream2, b->ev_fork, 0));
-    big(0, nbig, b->stream2);
+    k_batch_fire<MIXED, QUANT, false, 1024><<<nbig, 1024, lds, b->stream2>>>(A1, fc, b->skin, b->fst, p);
     BH(b, hipGetLastError());
   }
   if (b->nsys > nbig) {
-    rest(nbig, b->nsys - nbig, nbig > 0 ? b->nmax_rest : b->nmax, b->stream);
+    A1.first = nbig;
+    const int count = b->nsys - nbig;
+    if (b->nt == 1)
+      k_batch_fire<MIXED, QUANT, true, GH_FBS><<<count, GH_FBS, lds, b->stream>>>(A1, fc, b->skin, b->fst, p);
+    else
+      k_batch_fire<MIXED, QUANT, false, GH_FBS><<<count, GH_FBS, lds, b->stream>>>(A1, fc, b->skin, b->fst, p);
     BH(b, hipGetLastError());
   }
   if (nbig > 0) {
@@ -803,6 +1114,48 @@ static int split_launch(gh_batch *b, bool big_ok, BIG &&big, REST &&rest) {
   }
   return 0;
 }
+
+static int batch_blocks(const gh_batch *b, int lanes) {
+  const int per = GH_BWG / lanes;
+  return (b->ntot + per - 1) / per;
+}
+// Lanes per atom of the passes: 16, or 8 where 16 would fill the chip's
+// wavefront slots many times over and the fixed work per wavefront (sums,
+// random numbers, update) counts more than the wavefronts in flight.
+// Langevin step, mixed, 16 against 8 lanes: 2,600 atoms 18 and 23 us, 80,000
+// 72 and 81, 320,000 200 and 186 (FP64 230 and 206).
+static bool batch_g8(const gh_batch *b) { return b->ntot >= 200000; }
+
+// Launches kernel<MIXED, QUANT, SINGLE, lanes, ...> for the batch's form
+// (mixed batches on quantised positions where their systems would fit the LDS
+// staging).
+#define BATCH_FORM(KERNEL, MX, QU, ARGS, ...)                                                \
+  do {                                                                                       \
+    const bool one = b->nt == 1;                                                             \
+    if (batch_g8(b)) {                                                                       \
+      const int gr = batch_blocks(b, 8);                                                     \
+      if (one) KERNEL<MX, QU, true, 8 __VA_ARGS__><<<gr, GH_BWG, 0, b->stream>>> ARGS;        \
+      else KERNEL<MX, QU, false, 8 __VA_ARGS__><<<gr, GH_BWG, 0, b->stream>>> ARGS;           \
+    } else {                                                                                 \
+      const int gr = batch_blocks(b, 16);                                                    \
+      if (one) KERNEL<MX, QU, true, 16 __VA_ARGS__><<<gr, GH_BWG, 0, b->stream>>> ARGS;       \
+      else KERNEL<MX, QU, false, 16 __VA_ARGS__><<<gr, GH_BWG, 0, b->stream>>> ARGS;          \
+    }                                                                                        \
+  } while (0)
+
+static void launch_rho(gh_batch *b, const BatchArgs &A, int par, int always) {
+  if (b->precision != GH_MIXED) BATCH_FORM(k_batch_rho, false, false, (A, b->tbd0.d, b->skin, par, always));
+  else if (b->nst > 0) BATCH_FORM(k_batch_rho, true, true, (A, b->tbf0, b->skin, par, always));
+  else BATCH_FORM(k_batch_rho, true, false, (A, b->tbd0.f, b->skin, par, always));
+}
+template <int MODE>
+static void launch_force(gh_batch *b, const BatchArgs &A, const ErmakC &k, uint64_t seed,
+                         long long step) {
+  if (b->precision != GH_MIXED) BATCH_FORM(k_batch_force, false, false, (A, b->tbd0.d, k, seed, step), , MODE);
+  else if (b->nst > 0) BATCH_FORM(k_batch_force, true, true, (A, b->tbf0, k, seed, step), , MODE);
+  else BATCH_FORM(k_batch_force, true, false, (A, b->tbd0.f, k, seed, step), , MODE);
+}
+#undef BATCH_FORM
 
 extern "C" {
 
@@ -836,8 +1189,8 @@ void gh_batch_destroy(gh_batch *b) {
   if (b->stream) (void)hipStreamSynchronize(b->stream);
   if (b->stream2) (void)hipStreamSynchronize(b->stream2);
   void *p[] = {b->off, b->order, b->type, b->nn, b->flags, b->pos, b->vel, b->acc, b->frc,
-               b->e, b->rho, b->eband, b->xold, b->T, b->out, b->scale, b->eband32, b->list,
-               b->tbd, b->tbf, b->gn};
+               b->e, b->rho, b->xold, b->T, b->out, b->scale, b->list,
+               b->tbd, b->tbf, b->sysof, b->a0of, b->dmax, b->pos_next, b->pk, b->fst};
   for (void *q : p)
     if (q) (void)hipFree(q);
   if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -879,7 +1232,6 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
   b->nbig = 0;
   while (b->nbig < nsys && off[b->order_h[b->nbig] + 1] - off[b->order_h[b->nbig]] > GH_BIGSYS)
     ++b->nbig;
-  b->nmax_rest = b->nbig < nsys ? off[b->order_h[b->nbig] + 1] - off[b->order_h[b->nbig]] : 0;
   b->T_h.assign(nsys, 0.0);
   BT(balloc(b, &b->off, nsys + 1));
   BT(balloc(b, &b->order, nsys));
@@ -891,13 +1243,16 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
   BT(balloc(b, &b->frc, 3 * (size_t)ld));
   BT(balloc(b, &b->e, ld));
   BT(balloc(b, &b->rho, ld));
-  BT(balloc(b, &b->eband, ld));
-  BT(balloc(b, &b->eband32, ld));
-  BT(balloc(b, &b->gn, 6 * (size_t)ld));
+  BT(balloc(b, &b->pos_next, ld));
+  BT(balloc(b, &b->pk, ld));
+  BT(balloc(b, &b->sysof, ld));
+  BT(balloc(b, &b->a0of, ld));
+  BT(balloc(b, &b->dmax, 2 * (size_t)nsys));
   BT(balloc(b, &b->xold, 3 * (size_t)ld));
   BT(balloc(b, &b->T, nsys));
   BT(balloc(b, &b->out, (size_t)nsys * OUTW));
   BT(balloc(b, &b->scale, nsys));
+  BT(balloc(b, &b->fst, nsys));
   b->cap = 0;
   b->cap_req = 0;
   if (b->list) {
@@ -907,16 +1262,24 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
   std::vector<double4> hp(ld, make_double4(0, 0, 0, 0));
   std::vector<int> ht(ld, 0);
   for (int i = 0; i < b->ntot; ++i) {
-    hp[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], 0.0);
     ht[i] = type ? type[i] : 0;
+    hp[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], (double)ht[i]);
     if (ht[i] < 0 || ht[i] >= GH_MAXT) return bfail(b, GH_EINVAL, "type out of range");
+  }
+  std::vector<int> hs(ld, nsys - 1), ha(ld, off[nsys - 1]);
+  for (int k = 0; k < nsys; ++k) {
+    std::fill(hs.begin() + off[k], hs.begin() + off[k + 1], k);
+    std::fill(ha.begin() + off[k], ha.begin() + off[k + 1], off[k]);
   }
   // every upload and clear is ordered on the batch stream (a non-blocking
   // stream does not wait for work on the null stream)
   hipStream_t st = b->stream;
   BH(b, hipMemcpyAsync(b->pos, hp.data(), sizeof(double4) * ld, hipMemcpyHostToDevice, st));
+  BH(b, hipMemcpyAsync(b->pos_next, hp.data(), sizeof(double4) * ld, hipMemcpyHostToDevice, st));
   BH(b, hipMemcpyAsync(b->type, ht.data(), sizeof(int) * ld, hipMemcpyHostToDevice, st));
   BH(b, hipMemcpyAsync(b->off, off, sizeof(int) * (nsys + 1), hipMemcpyHostToDevice, st));
+  BH(b, hipMemcpyAsync(b->sysof, hs.data(), sizeof(int) * ld, hipMemcpyHostToDevice, st));
+  BH(b, hipMemcpyAsync(b->a0of, ha.data(), sizeof(int) * ld, hipMemcpyHostToDevice, st));
   BH(b, hipMemcpyAsync(b->order, b->order_h.data(), sizeof(int) * nsys, hipMemcpyHostToDevice,
                        st));
   BH(b, hipMemsetAsync(b->vel, 0, sizeof(double) * 3 * ld, st));
@@ -947,6 +1310,9 @@ int gh_batch_set_smatb(gh_batch *b, int nt, const double *A, const double *xi, c
   b->tbf = tmp.tbf;
   tmp.tbf = nullptr;
   b->tb_e0 = tmp.tb_e0;
+  b->tbd0.d = tmp.tb64_0;
+  b->tbd0.f = tmp.tbf_a0;
+  b->tbf0 = tmp.tbf0;
   b->nt = nt;
   b->rcut = tmp.rcut;
   b->have_pot = true;
@@ -998,30 +1364,10 @@ int gh_batch_compute(gh_batch *b, double *F, double *epot) {
   BH(b, hipSetDevice(b->device));
   BT(batch_ready(b));
   const BatchArgs A = bargs(b);
-  const bool mixed = b->precision == GH_MIXED, single = b->nt == 1;
-  const size_t lds = batch_lds(b);
-#define LAUNCH(MX, SG)                                                                     \
-  BT(split_launch(                                                                         \
-      b, true,                                                                             \
-      [&](int first, int count, hipStream_t st) {                                          \
-        BatchArgs A1 = A;                                                                  \
-        A1.first = first;                                                                  \
-        k_batch_compute<MX, SG, 1024><<<count, 1024, lds, st>>>(A1);                       \
-      },                                                                                   \
-      [&](int first, int count, int nmax, hipStream_t st) {                                \
-        BatchArgs A1 = A;                                                                  \
-        A1.first = first;                                                                  \
-        if (nmax > 512)                                                                    \
-          k_batch_compute<MX, SG, 512><<<count, 512, lds, st>>>(A1);                       \
-        else                                                                               \
-          k_batch_compute<MX, SG, 256><<<count, 256, lds, st>>>(A1);                       \
-      }))
-  if (mixed) {
-    if (single) LAUNCH(true, true); else LAUNCH(true, false);
-  } else {
-    if (single) LAUNCH(false, true); else LAUNCH(false, false);
-  }
-#undef LAUNCH
+  launch_rho(b, A, 0, 1);
+  launch_force<0>(b, A, ErmakC{}, 0, 0);
+  k_batch_energies<<<b->nsys, GH_BWG, 0, b->stream>>>(A);
+  BH(b, hipGetLastError());
   BT(check_flags(b));
   b->lists_valid = true;
   b->forces_valid = true;
@@ -1047,7 +1393,8 @@ int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t
                       double *epot, double *ekin) {
   if (!b || nsteps < 0 || !(dt > 0) || !(gamma > 0))
     return bfail(b, GH_EINVAL, "langevin needs nsteps >= 0, dt > 0, gamma > 0");
-  if (!b->forces_valid) BT(gh_batch_compute(b, nullptr, nullptr));
+  // (cap 0: the skin changed since the rows were sized)
+  if (!b->forces_valid || b->cap == 0) BT(gh_batch_compute(b, nullptr, nullptr));
   ErmakC k;
   k.c0 = exp(-dt * gamma);
   k.c1 = (1.0 - k.c0) / gamma;
@@ -1058,38 +1405,25 @@ int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t
   k.crv2 = sqrt(1.0 - (k.crv1 * k.crv1));
   k.dt = dt;
   k.kB_ui = ghc::kB_ui();
-  const BatchArgs A = bargs(b);
-  const bool mixed = b->precision == GH_MIXED, single = b->nt == 1;
-  const size_t lds = batch_lds(b);
-  const long long step0 = b->step + 1;
-  // one-type variants need more than the 128 VGPRs of a 1024-thread workgroup
-#define LAUNCH(MX, SG)                                                                     \
-  BT(split_launch(                                                                         \
-      b, !SG,                                                                              \
-      [&](int first, int count, hipStream_t st) {                                          \
-        if constexpr (!SG) {                                                               \
-          BatchArgs A1 = A;                                                                \
-          A1.first = first;                                                                \
-          k_batch_langevin<MX, SG, 1024><<<count, 1024, lds, st>>>(A1, nsteps, step0, k,   \
-                                                                   seed, b->skin);         \
-        }                                                                                  \
-      },                                                                                   \
-      [&](int first, int count, int nmax, hipStream_t st) {                                \
-        BatchArgs A1 = A;                                                                  \
-        A1.first = first;                                                                  \
-        if (nmax > 512)                                                                    \
-          k_batch_langevin<MX, SG, 512><<<count, 512, lds, st>>>(A1, nsteps, step0, k,     \
-                                                                 seed, b->skin);           \
-        else                                                                               \
-          k_batch_langevin<MX, SG, 256><<<count, 256, lds, st>>>(A1, nsteps, step0, k,     \
-                                                                 seed, b->skin);           \
-      }))
-  if (mixed) {
-    if (single) LAUNCH(true, true); else LAUNCH(true, false);
-  } else {
-    if (single) LAUNCH(false, true); else LAUNCH(false, false);
+  if (nsteps > 0) {
+    const long long step0 = b->step + 1;
+    BatchArgs A = bargs(b);
+    k_batch_zero<<<(2 * b->nsys + GH_BWG - 1) / GH_BWG, GH_BWG, 0, b->stream>>>(b->dmax, 2 * b->nsys);
+    k_batch_ermak_a<<<batch_blocks(b, 16), GH_BWG, 0, b->stream>>>(A, k, seed, step0);
+    for (int st = 0; st < nsteps; ++st) {
+      const long long step = step0 + st;
+      launch_rho(b, A, (int)(step & 1), 0);
+      if (st + 1 < nsteps) {
+        launch_force<1>(b, A, k, seed, step);
+        std::swap(b->pos, b->pos_next);
+        std::swap(A.pos, A.pos_next);
+      } else {
+        launch_force<2>(b, A, k, seed, step);
+      }
+    }
   }
-#undef LAUNCH
+  k_batch_energies<<<b->nsys, GH_BWG, 0, b->stream>>>(bargs(b));
+  BH(b, hipGetLastError());
   b->step += nsteps;
   BT(check_flags(b));
   std::vector<double> o;
@@ -1154,40 +1488,21 @@ int gh_batch_fire(gh_batch *b, int max_iter, double dt_max, double alpha0, doubl
   if (!b || max_iter < 0 || !(dt_max > 0)) return bfail(b, GH_EINVAL, "gh_batch_fire");
   BH(b, hipSetDevice(b->device));
   BT(batch_ready(b));
+  const BatchArgs A = bargs(b);
   FireC fc;
   fc.dt_max = dt_max;
   fc.alpha0 = alpha0;
-  fc.fswitch = fswitch;
-  fc.ftol = ftol;
   fc.ui_ev = ghc::ui_ev();
   fc.max_iter = max_iter;
-  fc.mixed = b->precision == GH_MIXED;
-  const BatchArgs A = bargs(b);
-  const size_t lds = batch_lds(b);
-#define LAUNCH(SG)                                                                         \
-  BT(split_launch(                                                                         \
-      b, !SG,                                                                              \
-      [&](int first, int count, hipStream_t st) {                                          \
-        if constexpr (!SG) {                                                               \
-          BatchArgs A1 = A;                                                                \
-          A1.first = first;                                                                \
-          k_batch_fire<SG, 1024><<<count, 1024, lds, st>>>(A1, fc, b->skin);               \
-        }                                                                                  \
-      },                                                                                   \
-      [&](int first, int count, int nmax, hipStream_t st) {                                \
-        BatchArgs A1 = A;                                                                  \
-        A1.first = first;                                                                  \
-        if (nmax > 512)                                                                    \
-          k_batch_fire<SG, 512><<<count, 512, lds, st>>>(A1, fc, b->skin);                 \
-        else                                                                               \
-          k_batch_fire<SG, 256><<<count, 256, lds, st>>>(A1, fc, b->skin);                 \
-      }))
-  if (b->nt == 1) {
-    LAUNCH(true);
-  } else {
-    LAUNCH(false);
+  fc.resume = 0;
+  if (b->precision == GH_MIXED) {
+    fc.fstop = fswitch;
+    if (b->nst > 0) BT((launch_fire<true, true>(b, A, fc, b->tbf0)));
+    else BT((launch_fire<true, false>(b, A, fc, b->tbd0.f)));
+    fc.resume = 1;
   }
-#undef LAUNCH
+  fc.fstop = ftol;
+  BT((launch_fire<false, false>(b, A, fc, b->tbd0.d)));
   BT(check_flags(b));
   b->lists_valid = true;
   b->forces_valid = false;  // the last forces may be FP64 while precision is mixed

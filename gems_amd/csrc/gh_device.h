@@ -98,6 +98,14 @@ __device__ __forceinline__ double row_total(double v) {
   v += dpp64<0x140>(v);  // row_mirror
   return v;
 }
+// Wavefront maximum (v >= 0) in every lane, the same way.
+__device__ __forceinline__ double wave_top(double v) {
+  v = fmax(v, dpp64<0xB1>(v));
+  v = fmax(v, dpp64<0x4E>(v));
+  v = fmax(v, dpp64<0x141>(v));
+  v = fmax(v, dpp64<0x140>(v));
+  return fmax(fmax(lane64(v, 0), lane64(v, 16)), fmax(lane64(v, 32), lane64(v, 48)));
+}
 __device__ __forceinline__ double wave_total(double v) {
   v = row_total(v);
   return (lane64(v, 0) + lane64(v, 16)) + (lane64(v, 32) + lane64(v, 48));
@@ -528,6 +536,15 @@ __device__ __forceinline__ uint4 philox(uint4 c, uint2 k) {
   return c;
 }
 
+// One Box-Muller pair of standard normals from two words of the stream.
+__device__ __forceinline__ void philox_pair(unsigned w0, unsigned w1, float &ga, float &gb) {
+  const float u1 = ((float)(w0 >> 8) + 0.5f) * 5.9604644775390625e-08f;  // (0,1)
+  const float a = (float)(w1 >> 8) * 3.7450702829239286e-07f;            // 2 pi u
+  const float r = __builtin_sqrtf(-2.0f * __logf(u1));
+  ga = r * __cosf(a);
+  gb = r * __sinf(a);
+}
+
 // Six standard normals for atom `id` at step `step`: two Philox4x32-10 draws
 // (counter (id, b, step), key = seed) give 24-bit uniforms, turned into three
 // Box-Muller pairs in FP32 with the fast hardware log and sin/cos (the noise
@@ -541,11 +558,10 @@ __device__ __forceinline__ void philox_normals(unsigned long long seed, long lon
   const unsigned w[6] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y};
 #pragma unroll
   for (int b = 0; b < 3; ++b) {
-    const float u1 = ((float)(w[2 * b] >> 8) + 0.5f) * 5.9604644775390625e-08f;  // (0,1)
-    const float a = (float)(w[2 * b + 1] >> 8) * 3.7450702829239286e-07f;        // 2 pi u
-    const float r = __builtin_sqrtf(-2.0f * __logf(u1));
-    g[2 * b] = (double)(r * __cosf(a));
-    g[2 * b + 1] = (double)(r * __sinf(a));
+    float ga, gb;
+    philox_pair(w[2 * b], w[2 * b + 1], ga, gb);
+    g[2 * b] = (double)ga;
+    g[2 * b + 1] = (double)gb;
   }
 }
 
