@@ -511,9 +511,7 @@ static int report_halt(gh_ctx *c, GhStatus &h) {
   }
 }
 
-static int check_status(gh_ctx *c) {
-  GhStatus h;
-  GH_TRY(read_status(c, &h));
+static int judge_status(gh_ctx *c, GhStatus &h) {
   if (h.halt) return report_halt(c, h);
   if (h.overflow) {
     c->ready = false;
@@ -535,6 +533,12 @@ static int check_status(gh_ctx *c) {
     return gh_fail(c, GH_ERANGE, "an atom left the cell grid of a non-periodic box axis");
   }
   return 0;
+}
+
+static int check_status(gh_ctx *c) {
+  GhStatus h;
+  GH_TRY(read_status(c, &h));
+  return judge_status(c, h);
 }
 
 // ---------------------------------------------------------------------------
@@ -578,6 +582,64 @@ static hipEvent_t ev_at(gh_ctx *c, int k) {
 static int rec(gh_ctx *c, int k) {
   if (!c->timing) return 0;
   GH_HIP(c, hipEventRecord(ev_at(c, k), c->stream));
+  return 0;
+}
+
+// ---------------------------------------------------------------------------
+// State between the caller's arrays (caller's order, pageable) and the sorted
+// device arrays.  The device reorders; fetching the permutation and every
+// array and reordering in host loops took most of a call.  Up to
+// GH_DIRECT_BYTES the kernels read and write pinned buffers in place (no copy
+// command, one synchronisation); larger transfers go through a device buffer
+// and the runtime's staged copies (17 GB/s out, 28 in), which overlap their
+// host copy with the bus.  The line lies at 2 MiB: pinned buffers up to 16 MiB
+// would make repeated calls of 108,000 atoms 10 % faster and cost the first
+// one 4 ms for their allocation.  set_positions + compute, before and now: 561
+// atoms (free) 123 -> 41 us, 8,788 246 -> 104, 32,000 263 -> 150, 108,000 629
+// -> 425, 442,331 2,750 -> 1,500; the state of 1M atoms in and out 22 -> 10 ms.
+// ---------------------------------------------------------------------------
+#define GH_DIRECT_BYTES (size_t)(2 << 20)
+static int need_pinned(gh_ctx *c, double **p, size_t *have, size_t len) {
+  if (*have >= len) return 0;
+  if (*p) GH_HIP(c, hipHostFree(*p));
+  *p = nullptr;
+  *have = 0;
+  GH_HIP(c, hipHostMalloc((void **)p, sizeof(double) * len, hipHostMallocDefault));
+  *have = len;
+  return 0;
+}
+static int need_dbuf(gh_ctx *c, size_t len) {
+  if (c->dbuf_len >= len) return 0;
+  c->dbuf_len = 0;
+  GH_TRY(dalloc(c, &c->dbuf, len));
+  c->dbuf_len = len;
+  return 0;
+}
+static int release_buffers(gh_ctx *c) {  // sized for the atom count: given back when it changes
+  GH_HIP(c, hipStreamSynchronize(c->stream));
+  if (c->hin) GH_HIP(c, hipHostFree(c->hin));
+  if (c->hout) GH_HIP(c, hipHostFree(c->hout));
+  c->hin = c->hout = nullptr;
+  c->hin_len = c->hout_len = c->dbuf_len = 0;
+  c->hin_busy = false;
+  return dalloc(c, &c->dbuf, 0);
+}
+// `len` doubles of the caller's for the next kernel on the stream; the
+// caller's memory may change once this returns.
+static int stage_in(gh_ctx *c, const double *in, size_t len, const double **src) {
+  if (len * sizeof(double) <= GH_DIRECT_BYTES) {
+    if (c->hin_busy) GH_HIP(c, hipStreamSynchronize(c->stream));
+    c->hin_busy = false;
+    GH_TRY(need_pinned(c, &c->hin, &c->hin_len, len));
+    memcpy(c->hin, in, sizeof(double) * len);
+    c->hin_busy = true;
+    *src = c->hin;
+    return 0;
+  }
+  GH_TRY(need_dbuf(c, len));
+  GH_HIP(c, hipMemcpyAsync(c->dbuf, in, sizeof(double) * len, hipMemcpyHostToDevice, c->stream));
+  GH_HIP(c, hipStreamSynchronize(c->stream));
+  *src = c->dbuf;
   return 0;
 }
 
@@ -660,7 +722,10 @@ int gh_create(gh_ctx **out, int device, int precision) {
   if (hipSetDevice(device) != hipSuccess ||
       hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
       hipMalloc((void **)&c->status, sizeof(GhStatus)) != hipSuccess ||
-      hipHostMalloc((void **)&c->red_h, sizeof(double) * 16, hipHostMallocDefault) != hipSuccess ||
+      hipHostMalloc((void **)&c->rep_h, sizeof(GhReport), hipHostMallocDefault) != hipSuccess ||
+      hipMalloc((void **)&c->red, sizeof(double) * (2 * 5 * 256 + 8)) != hipSuccess ||
+      hipMalloc((void **)&c->red_tick, sizeof(unsigned)) != hipSuccess ||
+      hipMemsetAsync(c->red_tick, 0, sizeof(unsigned), c->stream) != hipSuccess ||
       hipHostMalloc((void **)&c->prog_h, sizeof(GhProgress), hipHostMallocCoherent) !=
           hipSuccess ||
       hipHostGetDevicePointer((void **)&c->prog_d, c->prog_h, 0) != hipSuccess) {
@@ -689,12 +754,15 @@ void gh_destroy(gh_ctx *c) {
                  c->rho, c->eband, c->eband32, c->type, c->type_t, c->orig, c->orig_t,
                  c->xold, c->posv, c->velv, c->gauss, c->cellof, c->cellid, c->cell_count,
                  c->cell_start, c->perm, c->nn, c->list, c->tbd, c->tbf, c->status,
-                 c->red, c->list16, c->xin, c->chain_dev, c->pljd, c->mfeel, c->mfelt};
+                 c->red, c->red_tick, c->list16, c->dbuf, c->inv, c->chain_dev, c->pljd, c->mfeel,
+                 c->mfelt};
   for (void *p : dev)
     if (p) (void)hipFree(p);
   if (c->chain_pin) (void)hipHostFree(c->chain_pin);
   if (c->gauss_h) (void)hipHostFree(c->gauss_h);
-  if (c->red_h) (void)hipHostFree(c->red_h);
+  if (c->rep_h) (void)hipHostFree(c->rep_h);
+  if (c->hin) (void)hipHostFree(c->hin);
+  if (c->hout) (void)hipHostFree(c->hout);
   if (c->prog_h) (void)hipHostFree(c->prog_h);
   for (hipEvent_t e : c->evpool) (void)hipEventDestroy(e);
   if (c->stream) (void)hipStreamDestroy(c->stream);
@@ -922,15 +990,11 @@ int gh_set_atoms(gh_ctx *c, int n, const double *x, const int *type) {
     GH_TRY(dalloc(c, &c->cellid, ncap));
     GH_TRY(dalloc(c, &c->perm, ncap));
     GH_TRY(dalloc(c, &c->nn, ncap));
-    c->nred = std::min(1024, std::max(1, (ncap + 255) / 256));
-    GH_TRY(dalloc(c, &c->red, (size_t)c->nred * 10 + 16));
+    GH_TRY(dalloc(c, &c->inv, ncap));
+    GH_TRY(release_buffers(c));
     if (c->gauss) {
       GH_HIP(c, hipFree(c->gauss));
       c->gauss = nullptr;
-    }
-    if (c->xin) {
-      GH_HIP(c, hipFree(c->xin));
-      c->xin = nullptr;
     }
     if (c->gauss_h) {
       GH_HIP(c, hipHostFree(c->gauss_h));
@@ -975,6 +1039,7 @@ int gh_set_atoms(gh_ctx *c, int n, const double *x, const int *type) {
   GH_HIP(c, hipMemcpyAsync(c->pos, hp.data(), sizeof(double4) * ncap, hipMemcpyHostToDevice, st));
   GH_HIP(c, hipMemcpyAsync(c->type, ht.data(), sizeof(int) * ncap, hipMemcpyHostToDevice, st));
   GH_HIP(c, hipMemcpyAsync(c->orig, ho.data(), sizeof(int) * ncap, hipMemcpyHostToDevice, st));
+  GH_HIP(c, hipMemcpyAsync(c->inv, ho.data(), sizeof(int) * ncap, hipMemcpyHostToDevice, st));
   GH_HIP(c, hipMemsetAsync(c->vel, 0, sizeof(double) * 3 * ncap, st));
   GH_HIP(c, hipMemsetAsync(c->acc, 0, sizeof(double) * 3 * ncap, st));
   GH_HIP(c, hipMemsetAsync(c->frc, 0, sizeof(double) * 3 * ncap, st));
@@ -1006,22 +1071,49 @@ static int fetch_orig(gh_ctx *c, std::vector<int> &orig) {
   return 0;
 }
 
-static int fetch_soa3(gh_ctx *c, const double *d, const std::vector<int> &orig, double *out) {
-  std::vector<double> h(3 * (size_t)c->ncap);
-  GH_HIP(c, hipMemcpyAsync(h.data(), d, sizeof(double) * 3 * c->ncap, hipMemcpyDeviceToHost,
-                           c->stream));
-  GH_HIP(c, hipStreamSynchronize(c->stream));
-  for (int s = 0; s < c->n; ++s)
-    for (int k = 0; k < 3; ++k) out[3 * (size_t)orig[s] + k] = h[(size_t)k * c->ncap + s];
-  return 0;
+// One vector set (3n, caller's order) into a sorted device array; null: zeros.
+// The caller's memory may change once this returns.
+static int put3(gh_ctx *c, double *dst, const double *in) {
+  if (!in) {
+    GH_HIP(c, hipMemsetAsync(dst, 0, sizeof(double) * 3 * (size_t)c->ncap, c->stream));
+    return 0;
+  }
+  const double *src;
+  GH_TRY(stage_in(c, in, 3 * (size_t)c->n, &src));
+  return gh_launch_put3(c, dst, src);
 }
 
-static int put_soa3(gh_ctx *c, double *d, const std::vector<int> &orig, const double *in) {
-  std::vector<double> h(3 * (size_t)c->ncap, 0.0);
-  for (int s = 0; s < c->n; ++s)
-    for (int k = 0; k < 3; ++k) h[(size_t)k * c->ncap + s] = in ? in[3 * (size_t)orig[s] + k] : 0.0;
-  GH_HIP(c, hipMemcpyAsync(d, h.data(), sizeof(double) * 3 * c->ncap, hipMemcpyHostToDevice,
-                           c->stream));
+// The state (any pointer may be null) in the caller's order; with `status`
+// the status is judged first and nothing is written on an error.
+// Synchronises the stream.
+static int get_state(gh_ctx *c, double *x, double *v, double *F, double *e, bool status) {
+  double *out[4] = {x, v, F, e}, *at[4] = {nullptr, nullptr, nullptr, nullptr};
+  const size_t n = (size_t)c->n, len[4] = {3 * n, 3 * n, 3 * n, n};
+  size_t total = 0;
+  for (int k = 0; k < 4; ++k) total += out[k] ? len[k] : 0;
+  const bool direct = total * sizeof(double) <= GH_DIRECT_BYTES;
+  if (total) GH_TRY(direct ? need_pinned(c, &c->hout, &c->hout_len, total) : need_dbuf(c, total));
+  double *p = direct ? c->hout : c->dbuf;
+  for (int k = 0; k < 4; ++k)
+    if (out[k]) {
+      at[k] = p;
+      p += len[k];
+    }
+  GH_TRY(gh_launch_get(c, at[0], at[1], at[2], at[3], status));
+  if (direct || status) {
+    GH_HIP(c, hipStreamSynchronize(c->stream));
+    c->hin_busy = false;
+    if (status) GH_TRY(judge_status(c, c->rep_h->st));
+  }
+  if (direct) {
+    for (int k = 0; k < 4; ++k)
+      if (out[k]) memcpy(out[k], at[k], sizeof(double) * len[k]);
+    return 0;
+  }
+  for (int k = 0; k < 4; ++k)
+    if (out[k])
+      GH_HIP(c, hipMemcpyAsync(out[k], at[k], sizeof(double) * len[k], hipMemcpyDeviceToHost,
+                               c->stream));
   GH_HIP(c, hipStreamSynchronize(c->stream));
   return 0;
 }
@@ -1030,24 +1122,19 @@ int gh_set_positions(gh_ctx *c, const double *x) {
   if (!c || !x) return gh_fail(c, GH_EINVAL, "gh_set_positions: bad arguments");
   if (!c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms: call gh_set_atoms first");
   GH_HIP(c, hipSetDevice(c->device));
-  if (!c->xin) GH_TRY(dalloc(c, &c->xin, 3 * (size_t)c->ncap));
-  GH_HIP(c, hipMemcpyAsync(c->xin, x, sizeof(double) * 3 * (size_t)c->n, hipMemcpyHostToDevice,
-                           c->stream));
-  return gh_launch_set_positions(c, c->xin);
+  const double *src;
+  GH_TRY(stage_in(c, x, 3 * (size_t)c->n, &src));
+  return gh_launch_set_positions(c, src);
 }
 
 int gh_set_velocities(gh_ctx *c, const double *v) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
-  std::vector<int> orig;
-  GH_TRY(fetch_orig(c, orig));
-  return put_soa3(c, c->vel, orig, v);
+  return put3(c, c->vel, v);
 }
 
 int gh_set_accelerations(gh_ctx *c, const double *a) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
-  std::vector<int> orig;
-  GH_TRY(fetch_orig(c, orig));
-  return put_soa3(c, c->acc, orig, a);
+  return put3(c, c->acc, a);
 }
 
 int gh_set_smatb(gh_ctx *c, int nt, const double *A, const double *xi, const double *p,
@@ -1168,23 +1255,9 @@ int gh_compute(gh_ctx *c, double *F, double *e_atom, double *e_tot) {
   if (!c) return GH_EINVAL;
   GH_HIP(c, hipSetDevice(c->device));
   GH_TRY(interact(c));
-  GH_TRY(check_status(c));
-  std::vector<int> orig;
-  GH_TRY(fetch_orig(c, orig));
-  if (F) GH_TRY(fetch_soa3(c, c->frc, orig, F));
-  if (e_atom || e_tot) {
-    std::vector<double> h(c->n);
-    GH_HIP(c, hipMemcpyAsync(h.data(), c->epa, sizeof(double) * c->n, hipMemcpyDeviceToHost,
-                             c->stream));
-    GH_HIP(c, hipStreamSynchronize(c->stream));
-    if (e_atom)
-      for (int s = 0; s < c->n; ++s) e_atom[orig[s]] = h[s];
-    if (e_tot) {
-      double ep, ek;
-      GH_TRY(gh_launch_energies(c, &ep, &ek));
-      *e_tot = ep;
-    }
-  }
+  if (e_tot) GH_TRY(gh_launch_epot(c));
+  GH_TRY(get_state(c, nullptr, nullptr, F, e_atom, true));
+  if (e_tot) *e_tot = c->rep_h->epot;
   return 0;
 }
 
@@ -1258,10 +1331,8 @@ int gh_set_lcg_state(gh_ctx *c, const int state[3]) {
 int gh_set_gdist(gh_ctx *c, double T) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
   const int n = c->n;
-  std::vector<int> orig;
-  GH_TRY(fetch_orig(c, orig));
   std::vector<double> v(3 * (size_t)n);
-  GH_TRY(fetch_soa3(c, c->vel, orig, v.data()));
+  GH_TRY(get_state(c, nullptr, v.data(), nullptr, nullptr, false));
   std::vector<double> m(n);
   for (int i = 0; i < n; ++i) m[i] = c->mass_t[c->type_h[i]];
   auto cmv = [&](double cm[3]) {
@@ -1304,7 +1375,7 @@ int gh_set_gdist(gh_ctx *c, double T) {
   cmv(cm);
   for (int i = 0; i < n; ++i)
     for (int d = 0; d < 3; ++d) v[3 * (size_t)i + d] = v[3 * (size_t)i + d] + (-cm[d]);
-  return put_soa3(c, c->vel, orig, v.data());
+  return put3(c, c->vel, v.data());
 }
 
 int gh_integrator_vv(gh_ctx *c, double dt) {
@@ -1548,9 +1619,8 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
       }
       if (each > 0 && ns % each == 0) {
         double ep, ek;
-        GH_TRY(gh_launch_energies(c, &ep, &ek));  // synchronises the stream
         GhStatus h;
-        GH_TRY(read_status(c, &h));
+        GH_TRY(gh_launch_energies(c, &ep, &ek, &h));  // synchronises the stream
         if (h.halt) {
           GH_TRY(resume(h));
           continue;
@@ -1682,35 +1752,7 @@ int gh_lbfgs(gh_ctx *c, int m, double eps, int max_iter, int *iters, double *epo
 
 int gh_get_state(gh_ctx *c, double *x, double *v, double *F, double *e) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
-  std::vector<int> orig;
-  GH_TRY(fetch_orig(c, orig));
-  if (x) {
-    std::vector<double4> h(c->n);
-    GH_HIP(c, hipMemcpyAsync(h.data(), c->pos, sizeof(double4) * c->n, hipMemcpyDeviceToHost,
-                             c->stream));
-    GH_HIP(c, hipStreamSynchronize(c->stream));
-    for (int s = 0; s < c->n; ++s) {
-      double v[3] = {h[s].x, h[s].y, h[s].z};
-      // positions run continuously between rebuilds (at most half a skin
-      // outside the box); report them wrapped as do_pbc_1 does
-      for (int d = 0; d < 3; ++d)
-        if (c->boxed && c->pbc[d]) {
-          if (v[d] >= c->L[d]) v[d] -= c->L[d];
-          else if (v[d] < 0.0) v[d] += c->L[d];
-        }
-      for (int d = 0; d < 3; ++d) x[3 * (size_t)orig[s] + d] = v[d];
-    }
-  }
-  if (v) GH_TRY(fetch_soa3(c, c->vel, orig, v));
-  if (F) GH_TRY(fetch_soa3(c, c->frc, orig, F));
-  if (e) {
-    std::vector<double> h(c->n);
-    GH_HIP(c, hipMemcpyAsync(h.data(), c->epa, sizeof(double) * c->n, hipMemcpyDeviceToHost,
-                             c->stream));
-    GH_HIP(c, hipStreamSynchronize(c->stream));
-    for (int s = 0; s < c->n; ++s) e[orig[s]] = h[s];
-  }
-  return 0;
+  return get_state(c, x, v, F, e, false);
 }
 
 int gh_get_stats(gh_ctx *c, gh_stats *s) {

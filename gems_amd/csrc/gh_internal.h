@@ -194,6 +194,13 @@ struct GhProgress {
   int pad;
 };
 
+// Energies and status written into pinned host memory by the last kernel of a
+// call, read after one synchronisation.
+struct GhReport {
+  double epot, ekin2;  // ui; ekin2 = sum m |v - v_cm|^2
+  GhStatus st;
+};
+
 struct gh_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -262,9 +269,17 @@ struct gh_ctx {
   float *eband32 = nullptr;                   // [ncap]
   int *type = nullptr, *type_t = nullptr;     // [ncap]
   int *orig = nullptr, *orig_t = nullptr;     // caller index of sorted atom
+  int *inv = nullptr;                         // sorted index of a caller's atom
   double *xold = nullptr;                     // [3][ncap] positions at build
   double *posv = nullptr;                     // Ermak random displacement [3][ncap]
-  double *xin = nullptr;                      // gh_set_positions upload [3n] (caller order)
+  // transfers of state in the caller's order: pinned host memory that kernels
+  // read and write in place (small systems), a device buffer for copies from
+  // and to the caller's arrays (large ones)
+  double *hin = nullptr, *hout = nullptr;
+  size_t hin_len = 0, hout_len = 0;
+  bool hin_busy = false;                      // a kernel may still read hin
+  double *dbuf = nullptr;
+  size_t dbuf_len = 0;
   double *velv = nullptr;                     // Ermak random velocity [3][ncap]
   double *gauss = nullptr;                    // host-stream gaussians [6][ncap] (caller order)
   double *gauss_h = nullptr;                  // pinned host staging
@@ -293,8 +308,8 @@ struct gh_ctx {
   GhProgress *prog_h = nullptr;               // pinned: the latest step's outcome
   GhProgress *prog_d = nullptr;               // its device address
   double *red = nullptr;                      // reduction scratch
-  int nred = 0;
-  double *red_h = nullptr;                    // pinned result
+  unsigned *red_tick = nullptr;               // its tickets
+  GhReport *rep_h = nullptr;                  // pinned: energies and status of the last report
   int cell_alloc = 0;
 
   // timing: a pool of events, 8 per step, read back when the pool fills
@@ -340,6 +355,9 @@ struct FuseVV {
 // launchers (gh_kernels.hip)
 int gh_launch_rebuild(gh_ctx *c, bool force);
 int gh_launch_set_positions(gh_ctx *c, const double *x_dev);
+int gh_launch_put3(gh_ctx *c, double *dst, const double *in);
+int gh_launch_get(gh_ctx *c, double *x, double *v, double *F, double *e, bool status);
+int gh_launch_epot(gh_ctx *c);
 int gh_launch_forces(gh_ctx *c, hipEvent_t mid, bool fuse_vv = false);
 bool gh_can_fuse_vv(const gh_ctx *c);
 int gh_launch_vv_a(gh_ctx *c);
@@ -347,7 +365,7 @@ int gh_launch_vv_b(gh_ctx *c);
 int gh_launch_vv_ba(gh_ctx *c);
 int gh_launch_ermak_a(gh_ctx *c);
 int gh_launch_ermak_b(gh_ctx *c);
-int gh_launch_energies(gh_ctx *c, double *epot_ui, double *ekin_ui);
+int gh_launch_energies(gh_ctx *c, double *epot_ui, double *ekin_ui, GhStatus *st = nullptr);
 int gh_launch_rebuild_cells(gh_ctx *c);
 int gh_launch_forces_tiled(gh_ctx *c, hipEvent_t mid, bool fuse_vv);
 int gh_fill_int(gh_ctx *c, int *p, int v, int n);

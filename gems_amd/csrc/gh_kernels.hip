@@ -644,11 +644,63 @@ __device__ __forceinline__ void block_sum_dd(double (&s)[NV], double (&c)[NV]) {
   }
 }
 
+// True in every thread of the grid's last workgroup to arrive, whose reads then
+// see the others' writes; the ticket is left at zero.  (256 workgroups at
+// most: each arrival is a fence.)
+__device__ __forceinline__ bool last_block(unsigned *ticket) {
+  __shared__ bool last;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    __threadfence();
+    last = atomicAdd(ticket, 1u) == gridDim.x - 1;
+  }
+  __syncthreads();
+  if (!last) return false;
+  __threadfence();
+  if (threadIdx.x == 0) *ticket = 0u;
+  return true;
+}
+
+// The workgroups' compensated sums of NV values to their grid total, formed by
+// the last workgroup; true there, the totals in v of thread 0.  (A launch of
+// its own for the totals cost 4-6 us per energy row.)
+template <int NV>
+__device__ __forceinline__ bool grid_sum_dd(double (&v)[NV], double (&e)[NV], double *part,
+                                            unsigned *ticket) {
+  block_sum_dd<NV>(v, e);
+  if (threadIdx.x == 0)
+    for (int k = 0; k < NV; ++k) {
+      part[(blockIdx.x * NV + k) * 2] = v[k];
+      part[(blockIdx.x * NV + k) * 2 + 1] = e[k];
+    }
+  if (!last_block(ticket)) return false;
+  for (int k = 0; k < NV; ++k) v[k] = e[k] = 0.0;
+  for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x)
+    for (int k = 0; k < NV; ++k) {
+      dd_add(v[k], e[k], part[(b * NV + k) * 2]);
+      e[k] += part[(b * NV + k) * 2 + 1];
+    }
+  block_sum_dd<NV>(v, e);
+  for (int k = 0; k < NV; ++k) v[k] += e[k];
+  return true;
+}
+
+// Potential energy alone (gh_compute).
+__global__ __launch_bounds__(GH_BLOCK) void k_red_epot(int n, const double *__restrict__ epa,
+                                                       double *part, unsigned *ticket,
+                                                       GhReport *rep) {
+  double v[1] = {0.0}, e[1] = {0.0};
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
+    dd_add(v[0], e[0], epa[i]);
+  if (grid_sum_dd<1>(v, e, part, ticket) && threadIdx.x == 0) rep->epot = v[0];
+}
+
 __global__ __launch_bounds__(GH_BLOCK) void k_red_a(int n, int ncap, MassArgs ma,
                                                     const int *__restrict__ type,
                                                     const double *__restrict__ epa,
-                                                    const double *__restrict__ vel,
-                                                    double *__restrict__ part) {
+                                                    const double *__restrict__ vel, double *part,
+                                                    unsigned *ticket, double *sums,
+                                                    GhReport *rep) {
   double v[5] = {0, 0, 0, 0, 0}, e[5] = {0, 0, 0, 0, 0};
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     const double m = 1.0 / ma.om[type[i]];
@@ -658,35 +710,18 @@ __global__ __launch_bounds__(GH_BLOCK) void k_red_a(int n, int ncap, MassArgs ma
     dd_add(v[3], e[3], m * vel[ncap + i]);
     dd_add(v[4], e[4], m * vel[2 * ncap + i]);
   }
-  block_sum_dd<5>(v, e);
-  if (threadIdx.x == 0)
-    for (int k = 0; k < 5; ++k) {
-      part[(blockIdx.x * 5 + k) * 2] = v[k];
-      part[(blockIdx.x * 5 + k) * 2 + 1] = e[k];
-    }
-}
-
-// One workgroup: out[k] = the compensated total of the nblk (sum, error)
-// partials of value k (nv <= 5).
-__global__ __launch_bounds__(GH_BLOCK) void k_red_final(int nblk, int nv,
-                                                        const double *__restrict__ part,
-                                                        double *__restrict__ out) {
-  double v[5] = {0, 0, 0, 0, 0}, e[5] = {0, 0, 0, 0, 0};
-  for (int b = threadIdx.x; b < nblk; b += blockDim.x)
-    for (int k = 0; k < nv; ++k) {
-      dd_add(v[k], e[k], part[(b * nv + k) * 2]);
-      e[k] += part[(b * nv + k) * 2 + 1];
-    }
-  block_sum_dd<5>(v, e);
-  if (threadIdx.x == 0)
-    for (int k = 0; k < nv; ++k) out[k] = v[k] + e[k];
+  if (grid_sum_dd<5>(v, e, part, ticket) && threadIdx.x == 0) {
+    rep->epot = v[0];
+    for (int k = 0; k < 5; ++k) sums[k] = v[k];
+  }
 }
 
 __global__ __launch_bounds__(GH_BLOCK) void k_red_b(int n, int ncap, MassArgs ma,
                                                     const int *__restrict__ type,
                                                     const double *__restrict__ vel,
-                                                    const double *__restrict__ sums,
-                                                    double *__restrict__ part) {
+                                                    const double *__restrict__ sums, double *part,
+                                                    unsigned *ticket, const GhStatus *st,
+                                                    GhReport *rep) {
   const double M = sums[1];
   const double cx = sums[2] / M, cy = sums[3] / M, cz = sums[4] / M;
   double v[1] = {0}, e[1] = {0};
@@ -695,10 +730,9 @@ __global__ __launch_bounds__(GH_BLOCK) void k_red_b(int n, int ncap, MassArgs ma
     const double wx = vel[i] - cx, wy = vel[ncap + i] - cy, wz = vel[2 * ncap + i] - cz;
     dd_add(v[0], e[0], (wx * wx + wy * wy + wz * wz) * m);
   }
-  block_sum_dd<1>(v, e);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = v[0];
-    part[2 * blockIdx.x + 1] = e[0];
+  if (grid_sum_dd<1>(v, e, part, ticket) && threadIdx.x == 0) {
+    rep->ekin2 = v[0];
+    rep->st = *st;
   }
 }
 
@@ -721,19 +755,57 @@ __global__ void k_wrap(int n, WrapArgs wa, double4 *__restrict__ pos) {
   pos[i] = p;
 }
 
+// State in the caller's order (AoS), one thread per value so that the writes
+// are consecutive: they may go to pinned host memory directly.  Any output may
+// be null.  Positions are reported wrapped as do_pbc_1 does (they run
+// continuously between rebuilds, at most half a skin outside the box).
+__global__ __launch_bounds__(GH_BLOCK) void k_get(int n, int ncap, WrapArgs wa,
+                                                  const int *__restrict__ inv,
+                                                  const double4 *__restrict__ pos,
+                                                  const double *__restrict__ vel,
+                                                  const double *__restrict__ frc,
+                                                  const double *__restrict__ epa, double *x,
+                                                  double *v, double *F, double *e,
+                                                  const GhStatus *st, GhReport *rep) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0 && rep) rep->st = *st;
+  if (k >= 3 * n) return;
+  const int i = k / 3, d = k - 3 * i, s = inv[i];
+  if (x) {
+    double p = reinterpret_cast<const double *>(pos + s)[d];
+    if (wa.pbc[d]) {
+      if (p >= wa.L[d]) p -= wa.L[d];
+      else if (p < 0.0) p += wa.L[d];
+    }
+    x[k] = p;
+  }
+  if (v) v[k] = vel[d * ncap + s];
+  if (F) F[k] = frc[d * ncap + s];
+  if (e && k < n) e[k] = epa[inv[k]];
+}
+// Vectors of the caller's atoms (3n, AoS) into a sorted array [3][ncap].
+__global__ __launch_bounds__(GH_BLOCK) void k_put3(int n, int ncap, const int *__restrict__ inv,
+                                                   const double *__restrict__ in,
+                                                   double *__restrict__ dst) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k >= 3 * n) return;
+  const int i = k / 3, d = k - 3 * i;
+  dst[d * ncap + inv[i]] = in[k];
+}
+
 // New positions from the host, in caller order (x: 3n, AoS): each atom's
 // coordinate moves to the periodic image nearest its current one (a host-side
 // wrap is no displacement), and its displacement since the last build joins
 // the rebuild test.
 __global__ __launch_bounds__(GH_BLOCK) void k_set_positions(
-    int n, int ncap, WrapArgs wa, const int *__restrict__ orig, const double *__restrict__ x,
+    int n, int ncap, WrapArgs wa, const int *__restrict__ inv, const double *__restrict__ x,
     double4 *__restrict__ pos, const double *__restrict__ xold, GhStatus *st, long long step) {
-  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  const int o = blockIdx.x * blockDim.x + threadIdx.x;
   double d2 = 0.0;
-  if (s < n) {
-    const int o = orig[s];
-    double4 p = pos[s];
+  if (o < n) {  // in the caller's order: x may be in host memory
     double v[3] = {x[3 * (size_t)o], x[3 * (size_t)o + 1], x[3 * (size_t)o + 2]};
+    const int s = inv[o];
+    double4 p = pos[s];
     const double old[3] = {p.x, p.y, p.z};
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -974,29 +1046,52 @@ int gh_launch_ermak_b(gh_ctx *c) {
   return 0;
 }
 
-// epot and ekin (ui) of the current state; host-synchronous.
-int gh_launch_energies(gh_ctx *c, double *epot_ui, double *ekin_ui) {
-  hipStream_t s = c->stream;
-  const int nblk = std::min(c->nred, std::max(1, nblocks(c->n)));
-  const MassArgs ma = make_mass(c);
-  double *part = c->red;                 // [nblk*5] (sum, error) pairs
-  double *sums = c->red + 10 * c->nred;  // [5]
-  double *kin = sums + 8;                // [1]
-  { k_red_a<<<nblk, GH_BLOCK, 0, s>>>(c->n, c->ncap, ma, c->type, c->epa, c->vel, part); ++c->launches; }
-  { k_red_final<<<1, GH_BLOCK, 0, s>>>(nblk, 5, part, sums); ++c->launches; }
-  { k_red_b<<<nblk, GH_BLOCK, 0, s>>>(c->n, c->ncap, ma, c->type, c->vel, sums, part); ++c->launches; }
-  { k_red_final<<<1, GH_BLOCK, 0, s>>>(nblk, 1, part, kin); ++c->launches; }
+// Reduction grids: 256 workgroups at most (last_block).
+static int red_blocks(int n) { return std::min(256, std::max(1, nblocks(n))); }
+
+// epot of the current forces into the report; asynchronous.
+int gh_launch_epot(gh_ctx *c) {
+  { k_red_epot<<<red_blocks(c->n), GH_BLOCK, 0, c->stream>>>(c->n, c->epa, c->red, c->red_tick,
+                                                             c->rep_h); ++c->launches; }
   GH_HIP(c, hipGetLastError());
-  GH_HIP(c, hipMemcpyAsync(c->red_h, sums, sizeof(double) * 9, hipMemcpyDeviceToHost, s));
+  return 0;
+}
+
+// epot and ekin (ui) of the current state, and the status; host-synchronous.
+int gh_launch_energies(gh_ctx *c, double *epot_ui, double *ekin_ui, GhStatus *st) {
+  hipStream_t s = c->stream;
+  const int nblk = red_blocks(c->n);
+  const MassArgs ma = make_mass(c);
+  double *part = c->red, *sums = c->red + 2 * 5 * 256;
+  { k_red_a<<<nblk, GH_BLOCK, 0, s>>>(c->n, c->ncap, ma, c->type, c->epa, c->vel, part, c->red_tick,
+                                      sums, c->rep_h); ++c->launches; }
+  { k_red_b<<<nblk, GH_BLOCK, 0, s>>>(c->n, c->ncap, ma, c->type, c->vel, sums, part, c->red_tick,
+                                      c->status, c->rep_h); ++c->launches; }
+  GH_HIP(c, hipGetLastError());
   GH_HIP(c, hipStreamSynchronize(s));
-  *epot_ui = c->red_h[0];
-  *ekin_ui = c->red_h[8] * 0.5;
+  *epot_ui = c->rep_h->epot;
+  *ekin_ui = c->rep_h->ekin2 * 0.5;
+  if (st) *st = c->rep_h->st;
+  return 0;
+}
+
+int gh_launch_get(gh_ctx *c, double *x, double *v, double *F, double *e, bool status) {
+  { k_get<<<nblocks(3 * c->n), GH_BLOCK, 0, c->stream>>>(
+      c->n, c->ncap, make_wrap(c), c->inv, c->pos, c->vel, c->frc, c->epa, x, v, F, e, c->status,
+      status ? c->rep_h : nullptr); ++c->launches; }
+  GH_HIP(c, hipGetLastError());
+  return 0;
+}
+
+int gh_launch_put3(gh_ctx *c, double *dst, const double *in) {
+  { k_put3<<<nblocks(3 * c->n), GH_BLOCK, 0, c->stream>>>(c->n, c->ncap, c->inv, in, dst); ++c->launches; }
+  GH_HIP(c, hipGetLastError());
   return 0;
 }
 
 int gh_launch_set_positions(gh_ctx *c, const double *x_dev) {
   { k_set_positions<<<nblocks(c->n), GH_BLOCK, 0, c->stream>>>(
-      c->n, c->ncap, make_wrap(c), c->orig, x_dev, c->pos, c->xold, c->status,
+      c->n, c->ncap, make_wrap(c), c->inv, x_dev, c->pos, c->xold, c->status,
       c->step); ++c->launches; }
   GH_HIP(c, hipGetLastError());
   return 0;

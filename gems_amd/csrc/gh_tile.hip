@@ -471,7 +471,7 @@ struct CellArgs {
   int n, ncap, nkey;
   double4 *pos, *pos_t;
   double *vel, *vel_t, *acc, *acc_t;
-  int *type, *type_t, *orig, *orig_t;
+  int *type, *type_t, *orig, *orig_t, *inv;
   int *cellid, *cellof, *count, *start, *perm;
 };
 
@@ -678,6 +678,7 @@ __device__ void cell_rank_gather(const CellArgs &R, double4 *__restrict__ pos, i
     }
     R.type[d] = R.type_t[v];
     R.orig[d] = key;
+    R.inv[key] = d;
     R.cellof[d] = c;
   }
 }
@@ -1953,6 +1954,7 @@ int gh_launch_rebuild_cells(gh_ctx *c) {
   R.type_t = c->type_t;
   R.orig = c->orig;
   R.orig_t = c->orig_t;
+  R.inv = c->inv;
   R.cellid = c->cellid;
   R.cellof = c->cellof;
   R.count = c->cell_count;
