@@ -387,6 +387,7 @@ static int ensure_ready(gh_ctx *c) {
     return gh_fail(c, GH_EINVAL, "one-sided interactions are served for pair potentials only");
   if (c->ready) return 0;
   setup_grid(c);
+  c->rows = c->list_mode == 1 && gh_rows_path(c);
   if (c->boxed) GH_TRY(gh_launch_wrap(c));
   GhStatus h;
   GH_TRY(read_status(c, &h));
@@ -400,7 +401,7 @@ static int ensure_ready(gh_ctx *c) {
       GH_TRY(gh_fill_int(c, c->cell_count, 0, c->tg.nkey));
       c->tg.slot_cap = 65535;  // count pass: any halo (the build reads L2 past its LDS)
       c->cap = 0;
-      GH_TRY(gh_launch_rebuild(c, true));
+      GH_TRY(gh_launch_rebuild(c, true, false));
       int max_halo = 0, max_brick = 0;
       GH_TRY(gh_tile_occupancy(c, &max_halo, &max_brick));
       GH_TRY(read_status(c, &h));
@@ -430,7 +431,7 @@ static int ensure_ready(gh_ctx *c) {
     }
   } else {
     c->cap = 0;
-    GH_TRY(gh_launch_rebuild(c, true));
+    GH_TRY(gh_launch_rebuild(c, true, false));
     GH_TRY(read_status(c, &h));
     maxnn = h.maxnn;
   }
@@ -439,7 +440,9 @@ static int ensure_ready(gh_ctx *c) {
   cap = roundup(std::max(cap, 8), 8);
   if ((size_t)cap * c->ncap > (size_t)1 << 31)
     return gh_fail(c, GH_EINVAL, "neighbour list too large");
-  if (c->list_mode == 1) {
+  // (the rows path orders a row in LDS, 16 rows per workgroup)
+  if (cap > 512) c->rows = false;
+  if (c->list_mode == 1 && !c->rows) {
     if (c->list) {
       GH_HIP(c, hipFree(c->list));
       c->list = nullptr;
@@ -459,7 +462,7 @@ static int ensure_ready(gh_ctx *c) {
   h.halt_step = 0;
   h.nupd = nupd0;
   GH_TRY(write_status(c, &h));
-  GH_TRY(gh_launch_rebuild(c, true));
+  GH_TRY(gh_launch_rebuild(c, true, false));
   GH_TRY(read_status(c, &h));
   if (h.overflow || h.tile_overflow) {
     const bool rows = h.overflow != 0;
@@ -782,6 +785,8 @@ int gh_set_tile(gh_ctx *c, const int *bd) {
   return 0;
 }
 
+static int interact(gh_ctx *c);
+
 int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
   if (!c || reps <= 0) return GH_EINVAL;
   GH_HIP(c, hipSetDevice(c->device));
@@ -789,6 +794,24 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
   if (c->list_mode != 1) {
     if (bd_out) bd_out[0] = bd_out[1] = bd_out[2] = 0;
     if (us_out) *us_out = 0.0;
+    return 0;
+  }
+  if (c->rows) {
+    // rows of atom numbers: the bricks only order the atoms, nothing to choose
+    hipEvent_t e[2];
+    for (hipEvent_t &ev : e) GH_HIP(c, hipEventCreate(&ev));
+    GH_TRY(interact(c));
+    GH_HIP(c, hipEventRecord(e[0], c->stream));
+    for (int r = 0; r < reps; ++r) GH_TRY(gh_launch_forces(c, nullptr));
+    GH_HIP(c, hipEventRecord(e[1], c->stream));
+    GH_HIP(c, hipEventSynchronize(e[1]));
+    float ms = 0.f;
+    GH_HIP(c, hipEventElapsedTime(&ms, e[0], e[1]));
+    for (hipEvent_t ev : e) (void)hipEventDestroy(ev);
+    GH_TRY(check_status(c));
+    if (bd_out)
+      for (int d = 0; d < 3; ++d) bd_out[d] = c->tg.bd[d];
+    if (us_out) *us_out = 1e3 * ms / reps;
     return 0;
   }
   GhStatus h0;
@@ -838,7 +861,7 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
         if (rate > 0.0) {
           GH_TRY(gh_request_rebuild(c));
           GH_HIP(c, hipEventRecord(e0, c->stream));
-          GH_TRY(gh_launch_rebuild(c, false));
+          GH_TRY(gh_launch_rebuild(c, false, false));
           GH_HIP(c, hipEventRecord(e1, c->stream));
           GH_HIP(c, hipEventSynchronize(e1));
           float ms = 0.f;
@@ -1241,10 +1264,10 @@ int gh_set_skin(gh_ctx *c, double skin) {
 static int interact(gh_ctx *c) {
   GH_TRY(ensure_ready(c));
   if (c->pos_dirty) {
-    GH_TRY(gh_launch_rebuild(c, true));
+    GH_TRY(gh_launch_rebuild(c, true, true));
     c->pos_dirty = false;
   } else {
-    GH_TRY(gh_launch_rebuild(c, false));
+    GH_TRY(gh_launch_rebuild(c, false, true));
   }
   GH_TRY(gh_launch_forces(c, nullptr));
   c->first_force = false;
@@ -1268,7 +1291,8 @@ int gh_neighbors(gh_ctx *c, int *nn_out, int *idx, int cap) {
   GH_TRY(fetch_orig(c, orig));
   std::vector<int> nn(c->n);
   std::vector<unsigned> lst((size_t)c->cap * c->ncap);
-  if (c->list_mode == 1) {
+  const bool tiled = c->list_mode == 1 && !c->rows;
+  if (tiled) {
     int *tmp = nullptr;
     GH_HIP(c, hipMalloc((void **)&tmp, sizeof(int) * (size_t)c->cap * c->ncap));
     int rc2 = gh_tiled_to_global(c, tmp);
@@ -1290,7 +1314,7 @@ int gh_neighbors(gh_ctx *c, int *nn_out, int *idx, int cap) {
   for (int s = 0; s < c->n; ++s) {
     row.clear();
     for (int k = 0; k < nn[s]; ++k) {
-      const size_t at = c->list_mode == 1 ? (size_t)k * c->ncap + s : (size_t)s * c->cap + k;
+      const size_t at = tiled ? (size_t)k * c->ncap + s : (size_t)s * c->cap + k;
       row.push_back(orig[lst[at] & 0x07FFFFFFu]);
     }
     std::sort(row.begin(), row.end());
@@ -1424,10 +1448,9 @@ static int lcg_step_normals(gh_ctx *c) {
 // [epot, ekin, sum] in eV every `each` steps.
 //
 // Each step enqueues stepa (unless the previous step's force pass applied
-// it), the rebuild chain, the force passes and stepb.  On the tiled velocity
-// Verlet path the rebuild chain is enqueued only where the host expects a
-// rebuild: every step the first force pass tests the device's rebuild rule
-// itself, and if a rebuild is due without its chain it stops the run at that
+// it), the rebuild chain, the force passes and stepb.  In cell mode the
+// rebuild chain is enqueued only where the host expects a rebuild: every step
+// the first force pass tests the device's rebuild rule itself, and if a rebuild is due without its chain it stops the run at that
 // step (GhStatus::halt; every state-changing kernel then returns at once, so
 // the state stays the one the step started from).  The last pass of each
 // step publishes the step and any stop into pinned host memory; the host
@@ -1492,10 +1515,10 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
     GH_TRY(interact(c));
     GH_TRY(check_status(c));
   }
-  // the chain only where expected: tiled velocity Verlet without per-step events
-  const bool lazy = !ermak && !c->timing && gh_can_fuse_vv(c);
-  // the tiled passes publish each step: the host then stays within kLead steps
-  const bool publishes = c->list_mode == 1;
+  // the chain only where expected: cell mode without per-step events (a stopped
+  // step is enqueued again, which would draw the host's random stream twice)
+  const bool lazy = !lcg && !c->timing && c->list_mode == 1;
+  const bool fusable = gh_can_fuse(c);
   const int kLead = 3;
   const int kRing = 64;
   std::vector<StepRec> ring(kRing);
@@ -1503,10 +1526,9 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
   volatile GhProgress *pg = c->prog_h;
   pg->halt = 0;
   pg->step = c->step;
-  // velocity Verlet: stepb of step n and stepa of step n+1 run as one kernel
-  // unless the state after stepb is observed (energy output, end of the run).
-  // In the tiled path the force pass itself applies stepb of step n and stepa
-  // of step n+1 (fused); elsewhere one kernel does both (k_vv_ba).
+  // The force pass itself applies stepb of step n and stepa of step n+1 (fused)
+  // unless the state after stepb is observed (energy output, end of the run);
+  // Ermak with the Philox stream on tiles: one kernel does both (k_ermak_ba).
   bool pending_b = false, stepa_done = false, chain = false;
   // The host enqueues the rebuild chain where it expects the device's rule to
   // fire: from the published displacement maximum (the running maximum since
@@ -1539,13 +1561,10 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
     GH_TRY(read_status(c, &h));
     const long long k = h.halt_step - s0;
     if (k < 1 || k > ns) return gh_fail(c, GH_ESTATE, "stop outside the run");
-    if (k >= ns - kRing + 1) {
-      const StepRec &r = ring[k % kRing];
-      c->pos = r.pos;
-      c->pos_next = r.pos_next;
-    } else if (publishes) {
-      return gh_fail(c, GH_ESTATE, "stop older than the step record");
-    }  // else no step swaps the positions buffers
+    if (k < ns - kRing + 1) return gh_fail(c, GH_ESTATE, "stop older than the step record");
+    const StepRec &r = ring[k % kRing];
+    c->pos = r.pos;
+    c->pos_next = r.pos_next;
     c->step = h.halt_step - 1;
     iout = each > 0 ? (int)((k - 1) / each) : 0;
     if (h.halt != GH_HALT_REBUILD) {
@@ -1566,23 +1585,21 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
   };
   for (;;) {
     while (ns <= nsteps) {
-      if (publishes) {
-        // at most kLead steps beyond the last one published
-        const long long need = s0 + ns - 1 - kLead;
-        for (int spin = 0; pg->step < need && !pg->halt; ++spin) {
-          std::this_thread::yield();
-          if ((spin & 1023) == 1023) {  // an idle stream has published every step it ran
-            const hipError_t q = hipStreamQuery(c->stream);
-            if (q == hipSuccess && pg->step < need && !pg->halt)
-              return gh_fail(c, GH_ESTATE, "a step was not published");
-            if (q != hipSuccess && q != hipErrorNotReady) GH_HIP(c, q);
-          }
+      // at most kLead steps beyond the last one published
+      const long long need = s0 + ns - 1 - kLead;
+      for (int spin = 0; pg->step < need && !pg->halt; ++spin) {
+        std::this_thread::yield();
+        if ((spin & 1023) == 1023) {  // an idle stream has published every step it ran
+          const hipError_t q = hipStreamQuery(c->stream);
+          if (q == hipSuccess && pg->step < need && !pg->halt)
+            return gh_fail(c, GH_ESTATE, "a step was not published");
+          if (q != hipSuccess && q != hipErrorNotReady) GH_HIP(c, q);
         }
-        if (pg->halt) {
-          GhStatus h;
-          GH_TRY(resume(h));
-          continue;
-        }
+      }
+      if (pg->halt) {
+        GhStatus h;
+        GH_TRY(resume(h));
+        continue;
       }
       if (lazy && !chain) {
         while (!unseen.empty() && unseen.front() <= pg->step) unseen.pop_front();
@@ -1592,26 +1609,28 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
       ring[ns % kRing] = StepRec{c->pos, c->pos_next};
       if (lcg) GH_TRY(lcg_step_normals(c));
       GH_TRY(rec(c, 0));
-      if (pending_b) GH_TRY(gh_launch_vv_ba(c));
+      if (pending_b) GH_TRY(gh_launch_ermak_ba(c));
       else if (!stepa_done) GH_TRY(ermak ? gh_launch_ermak_a(c) : gh_launch_vv_a(c));
       pending_b = stepa_done = false;
       GH_TRY(rec(c, 1));
       if (!lazy || chain) {
-        GH_TRY(gh_launch_rebuild(c, false));
+        GH_TRY(gh_launch_rebuild(c, false, true));
         if (lazy) unseen.push_back(c->step);
       }
       chain = false;
       GH_TRY(rec(c, 2));
       const bool observed = ns == nsteps || (each > 0 && ns % each == 0);
-      const bool fuse = !ermak && !observed && gh_can_fuse_vv(c);
+      const bool fuse = !observed && fusable;
       GH_TRY(gh_launch_forces(c, ev_at(c, 3), fuse));
       if (fuse) {
         std::swap(c->pos, c->pos_next);
         stepa_done = true;
       }
       GH_TRY(rec(c, 4));
-      if (ermak || observed) GH_TRY(ermak ? gh_launch_ermak_b(c) : gh_launch_vv_b(c));
-      else if (!fuse) pending_b = true;
+      if (!fuse) {
+        if (observed || lcg) GH_TRY(ermak ? gh_launch_ermak_b(c) : gh_launch_vv_b(c));
+        else pending_b = true;  // Ermak on tiles: with the next step's stepa
+      }
       GH_TRY(rec(c, 5));
       if (c->timing) {
         c->evused += 1;

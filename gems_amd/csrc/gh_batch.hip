@@ -463,16 +463,6 @@ struct ErmakC {
   double c0, c1, c2, sdr, sdv, crv1, crv2, dt, kB_ui;
 };
 
-// Lane sub (0..2) of a 16-lane group: normals 2 sub and 2 sub + 1 of atom
-// `id` at `step` (philox_normals, one axis of it).
-__device__ __forceinline__ void axis_normals(unsigned long long seed, long long step, int id,
-                                             int axis, float &ga, float &gb) {
-  const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
-  const unsigned s0 = (unsigned)step, s1 = (unsigned)((unsigned long long)step >> 32);
-  const uint4 c = philox(make_uint4((unsigned)id, axis == 2 ? 1u : 0u, s0, s1), key);
-  philox_pair(axis == 1 ? c.z : c.x, axis == 1 ? c.w : c.y, ga, gb);
-}
-
 // The workgroup's displacements folded into their systems' maxima: one atomic
 // where its atoms share a system, one per atom otherwise.  Each maximum has a
 // cache line of its own (128 of them on eight lines, one atomic per

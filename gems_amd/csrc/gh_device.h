@@ -9,10 +9,23 @@
 
 namespace ghd {
 
+// |x - x_old|^2 of the positions of step `step`, running maximum (bits of a
+// non-negative double, in its order).
+__device__ __forceinline__ unsigned long long disp2_max(const GhStatus *st, long long step) {
+  unsigned long long b = 0ull;
+#pragma unroll
+  for (int k = 0; k < GH_DISP_SLOTS; ++k) b = max(b, st->maxdisp2[step & 1][k].bits);
+  return b;
+}
+__device__ __forceinline__ void disp2_clear(GhStatus *st, long long step) {
+#pragma unroll
+  for (int k = 0; k < GH_DISP_SLOTS; ++k) st->maxdisp2[step & 1][k].bits = 0ull;
+}
+
 // Rebuild test of step `step` on the displacement maximum the integrators
 // fold into GhStatus::maxdisp2 (one atomicMax per workgroup).
 __device__ __forceinline__ bool rebuild_due(const GhStatus *st, double skin, long long step) {
-  const double d2 = __longlong_as_double((long long)st->maxdisp2[step & 1].bits);
+  const double d2 = __longlong_as_double((long long)disp2_max(st, step));
   return st->force_rebuild || 2.0 * sqrt(d2) > skin;
 }
 
@@ -26,17 +39,27 @@ __device__ __forceinline__ void rebuild_book(GhStatus *st) {
     st->nupd += 1;
     st->force_rebuild = 0;
     st->maxnn = 0;
-    st->maxdisp2[0].bits = st->maxdisp2[1].bits = 0ull;
+    disp2_clear(st, 0);
+    disp2_clear(st, 1);
   }
 }
 
 // Folds a workgroup's largest |x - x_old|^2 of the positions of step `step`
-// into that step's running maximum; the grid's first workgroup carries the
-// maximum of step - 1 on.
+// into that step's running maximum.  The grid's first workgroup carries the
+// maximum of step - 1 on, so the others need their atomic only above it (few
+// workgroups hold a new extreme: one atomic each on one line took 17 us of a
+// 30 us pass of 2,000 workgroups); on the step after a build, where all
+// do, they share the lines of the slots.  STABLE: no thread of the running
+// kernel restarts the maximum of step - 1.
+template <bool STABLE = true>
 __device__ __forceinline__ void fold_disp2(GhStatus *st, double d2, long long step) {
   unsigned long long b = (unsigned long long)__double_as_longlong(d2);
-  if (blockIdx.x == 0) b = max(b, st->maxdisp2[(step & 1) ^ 1].bits);
-  atomicMax(&st->maxdisp2[step & 1].bits, b);
+  if (STABLE || blockIdx.x == 0) {
+    const unsigned long long prev = disp2_max(st, step - 1);
+    if (blockIdx.x == 0) b = max(b, prev);
+    else if (b <= prev) return;
+  }
+  atomicMax(&st->maxdisp2[step & 1][blockIdx.x % GH_DISP_SLOTS].bits, b);
 }
 
 // Stops the run at `step` (the first raiser wins and records the step):
@@ -61,6 +84,27 @@ __device__ __forceinline__ void step_publish(GhProgress *prog, long long step, i
   __hip_atomic_store(&prog->halt, halt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&prog->halt_step, halt_step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
   __hip_atomic_store(&prog->step, step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Per-step arguments of the force passes.  The first pass of a step runs
+// only if the run is not halted and the step's rebuild is not due (when the
+// host has not enqueued the rebuild chain for the step, a due rebuild stops
+// the run there; the host re-runs the step with the chain); its workgroup 0
+// publishes the step (step_publish).
+struct StepArgs {
+  long long step;
+  double skin;
+  GhProgress *prog;  // null: nothing published
+};
+__device__ __forceinline__ bool step_gate(GhStatus *st, const StepArgs &sa) {
+  const int h = halted(st);
+  const bool stop = h || rebuild_due(st, sa.skin, sa.step);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (stop && !h) raise_halt(st, GH_HALT_REBUILD, sa.step);
+    step_publish(sa.prog, sa.step, h ? h : (stop ? GH_HALT_REBUILD : 0),
+                 h ? st->halt_step : sa.step, disp2_max(st, sa.step));
+  }
+  return stop;
 }
 
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.
@@ -360,7 +404,7 @@ __device__ __forceinline__ void for_each_slot_g(const unsigned short *__restrict
                                                 int a, int m, int sub, F &&f) {
   for_each_quad_g<G>(list16, ld, a, m, sub, [&](unsigned long long w) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) f(GH_QSLOT(w, u));
+    for (int u = 0; u < 4; ++u) f(u, GH_QSLOT(w, u));
   });
 }
 // Sum over the G lanes of an atom group (aligned groups of G lanes of one
@@ -370,6 +414,24 @@ __device__ __forceinline__ double group_sum(double v) {
 #pragma unroll
   for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
+}
+
+// FP64 sums of a tiled pass: with four lanes per atom, lane `sub` holds one
+// accumulator per entry of its quads, so accumulator (sub, u) has summed the
+// row's entries 4 sub + u, + 16, ..., in order; they meet in the order in which
+// the 16 lanes of the rows path do (neighbouring pairs, pairs of pairs, ...).
+// One lane: its one accumulator.
+template <int G>
+__device__ __forceinline__ double sums_total(const double (&v)[G]) {
+  if constexpr (G == 1) {
+    return v[0];
+  } else {
+    static_assert(G == 4, "four lanes, four entries per quad");
+    double t = (v[0] + v[1]) + (v[2] + v[3]);
+    t += __shfl_xor(t, 1, 64);
+    t += __shfl_xor(t, 2, 64);
+    return t;
+  }
 }
 
 // SMA-TB FP32 pair forms (the TbF terms; r2 in the TbF unit, FP64).  r is
@@ -563,6 +625,16 @@ __device__ __forceinline__ void philox_normals(unsigned long long seed, long lon
     g[2 * b] = (double)ga;
     g[2 * b + 1] = (double)gb;
   }
+}
+
+// Normals 2 axis and 2 axis + 1 of atom `id` at `step`: one axis of
+// philox_normals.
+__device__ __forceinline__ void axis_normals(unsigned long long seed, long long step, int id,
+                                             int axis, float &ga, float &gb) {
+  const uint2 key = make_uint2((unsigned)seed, (unsigned)(seed >> 32));
+  const unsigned s0 = (unsigned)step, s1 = (unsigned)((unsigned long long)step >> 32);
+  const uint4 c = philox(make_uint4((unsigned)id, axis == 2 ? 1u : 0u, s0, s1), key);
+  philox_pair(axis == 1 ? c.z : c.x, axis == 1 ? c.w : c.y, ga, gb);
 }
 
 }  // namespace ghd

@@ -149,6 +149,7 @@ struct TileGeom {
 // list traversals prefetch two quads ahead without a bounds clamp.
 #define GH_LIST_PAD_QUADS 2
 
+#define GH_DISP_SLOTS 8
 struct alignas(128) GhLine {          // a word that owns its cache line
   unsigned long long bits;
 };
@@ -158,13 +159,14 @@ struct GhStatus {                     // device-resident counters
   // the atoms into step s folds its workgroup maxima (and the maximum of step
   // s - 1) there, and step s's own force pass, which may move them on to step
   // s + 1 while later workgroups of it still test the rule, into the other
-  // (on cache lines of their own: thousands of workgroups read the one while
+  // (on cache lines of their own, a workgroup's by its number: thousands of them read the one while
   // others update the other atomically, 70-100 us per 1M-atom pass on a shared line)
-  GhLine maxdisp2[2];
+  GhLine maxdisp2[2][GH_DISP_SLOTS];
   int rebuild;                        // rebuild at this step
   int overflow;                       // a row exceeded the capacity (sticky)
   int maxnn;                          // longest row at the last build
   int outside;                        // an atom left a non-periodic grid
+  unsigned long long maxnn_tag;       // rows built inside a pass: (nupd + 1) << 32 | longest row
   long long nupd;                     // rebuilds so far
   int force_rebuild;                  // host request
   int tile_overflow;                  // a brick's halo exceeded slot_cap (sticky)
@@ -242,6 +244,7 @@ struct gh_ctx {
 
   // neighbour grid
   int list_mode = 1;          // 0 = O(N^2), 1 = cells
+  bool rows = false;          // cells, but rows of atom numbers (gh_rows_path) instead of tiles
   int nc[3] = {1, 1, 1};      // cells per dim (interior)
   int gofs[3] = {0, 0, 0};    // 1 for a non-periodic dim (one guard cell)
   int gn[3] = {1, 1, 1};      // cells per dim including guard cells
@@ -288,7 +291,7 @@ struct gh_ctx {
   int *cell_count = nullptr, *cell_start = nullptr;
   int *perm = nullptr;                        // [ncap]
   int *nn = nullptr;                          // [ncap]
-  int *list = nullptr;                        // [ncap][cap] rows (O(N^2) mode)
+  unsigned *list = nullptr;                   // [ncap][cap] rows (O(N^2) mode, rows path)
   unsigned short *list16 = nullptr;           // [cap][ncap] ELL of LDS slots (cell mode)
   void *chain_dev = nullptr;                  // rebuild-chain arguments (device copy)
   void *chain_pin = nullptr;                  // their pinned staging copy
@@ -343,7 +346,6 @@ int gh_fail(gh_ctx *c, int code, const std::string &msg);
 // Velocity Verlet fused into the force pass (stepb of this step, stepa of the
 // next) for the atoms whose forces the pass has just summed.
 struct FuseVV {
-  int on;
   double dt, acel_dv, acel_dx;
   double om[GH_MAXT];
   double *vel;
@@ -352,17 +354,38 @@ struct FuseVV {
   int ncap;
 };
 
+// Ermak coefficients (set_ermak, Integration.F90:936-952) of one step.
+struct ErmakArgs {
+  double c0, c1, c2, sdr, sdv, crv1, crv2, skt, dt;
+  int philox;
+  unsigned long long seed;
+  long long step;
+};
+// ermak_b of this step and ermak_a of the next, fused into the force pass
+// (Philox stream).
+struct FuseErmak {
+  ErmakArgs k;
+  double om[GH_MAXT], osm[GH_MAXT];
+  double *vel, *acc;
+  const double *xold;
+  const int *orig;
+  double4 *pos_next;
+  int ncap;
+};
+
 // launchers (gh_kernels.hip)
-int gh_launch_rebuild(gh_ctx *c, bool force);
+int gh_launch_rebuild(gh_ctx *c, bool force, bool forces_follow);
 int gh_launch_set_positions(gh_ctx *c, const double *x_dev);
 int gh_launch_put3(gh_ctx *c, double *dst, const double *in);
 int gh_launch_get(gh_ctx *c, double *x, double *v, double *F, double *e, bool status);
 int gh_launch_epot(gh_ctx *c);
-int gh_launch_forces(gh_ctx *c, hipEvent_t mid, bool fuse_vv = false);
-bool gh_can_fuse_vv(const gh_ctx *c);
+int gh_launch_forces(gh_ctx *c, hipEvent_t mid, bool fuse = false);
+bool gh_can_fuse(const gh_ctx *c);  // the force pass can apply the update to the next step
+bool gh_rows_path(const gh_ctx *c);
+FuseVV gh_fuse_vv(const gh_ctx *c);
 int gh_launch_vv_a(gh_ctx *c);
 int gh_launch_vv_b(gh_ctx *c);
-int gh_launch_vv_ba(gh_ctx *c);
+int gh_launch_ermak_ba(gh_ctx *c);
 int gh_launch_ermak_a(gh_ctx *c);
 int gh_launch_ermak_b(gh_ctx *c);
 int gh_launch_energies(gh_ctx *c, double *epot_ui, double *ekin_ui, GhStatus *st = nullptr);
