@@ -243,13 +243,27 @@ static int max_slots(const gh_ctx *c) {
   return (int)std::min<size_t>((GH_LDS_BYTES - stat) / per - 1, 65534);  // - the sentinel
 }
 
-// Threads per workgroup of the force passes, two candidates: one per atom of
-// the fullest brick at sizing (plus 1/16 for the atoms' motion), so that no
-// brick's atom loop runs a second round (spare wavefronts of emptier bricks
-// end at once); or one per atom of the mean brick (fewer wave slots held,
-// a few bricks run a short second round).  Rounded up to whole wavefronts,
-// at least one thread per halo cell (halo_setup), at most 1024.  The
-// autotuner times both; the fullest-brick rule is the default.
+// Threads per workgroup of the force passes, in whole wavefronts, at least one
+// per halo cell (halo_setup), at most 1024.  Candidates:
+//  0  mixed SMA-TB, one lane per atom, more than two bricks per CU: the brick
+//     an atom is typically in (the atom-weighted mean: empty and cut bricks
+//     don't count), in multiples of four wavefronts.  A workgroup's wavefronts
+//     spread over the CU's four SIMDs, and the odd one of a workgroup meets
+//     the same SIMD as the next one's: of nine wavefronts with the force
+//     pass's registers (six to a SIMD) two workgroups fit, of eight three.
+//     Fuller bricks run a short second round.  1M Au, 4 x 3 x 3 cells (464
+//     atoms a brick, 530 at most), density + fused forces: 576 threads 80 + 115
+//     us, 512 70 + 90, 768 82 + 104; 3 x 3 x 2 (243): 320 threads 80 + 113, 256
+//     75 + 109; 4 x 3 x 2 (309): 384 threads 82 + 118, 512 85 + 109, 256 84 +
+//     117; 4 x 4 x 4 (787; one workgroup fits either way): 896 threads 4 %
+//     faster than 1,024.
+//     Otherwise as 1: the other passes' registers leave eight wavefronts to a
+//     SIMD and the second round costs more than it frees (FP64 LJ, 1M atoms, 320
+//     threads 147 us, 256 153; two workgroups to a CU: all fit anyway).
+//  1  one per atom of the fullest brick at sizing (plus 1/16 for the atoms'
+//     motion): no brick's atom loop runs a second round.
+//  2  one per atom of the mean brick.
+// The autotuner times all; 0 is the default.
 #ifndef GH_STAGE_ROUNDS
 #define GH_STAGE_ROUNDS 3
 #endif
@@ -273,9 +287,13 @@ static void set_force_pass_threads(gh_ctx *c) {
   const int mb = (c->max_brick + t.chunks - 1) / t.chunks;
   const long long units = (long long)t.nbrick * t.chunks;
   const int stage = t.chunks > 1 ? (t.slot_cap + GH_STAGE_ROUNDS - 1) / GH_STAGE_ROUNDS : 0;
-  t.tpb_max = force_pass_threads(t, std::max(stage, t.lanes * (mb + mb / 16 + 1)));
-  t.tpb_avg = force_pass_threads(t, std::max(stage, t.lanes * (int)((c->n + units - 1) / units)));
-  t.tpb = c->tpb_mean ? t.tpb_avg : t.tpb_max;
+  t.tpb_c[1] = force_pass_threads(t, std::max(stage, t.lanes * (mb + mb / 16 + 1)));
+  t.tpb_c[2] = force_pass_threads(t, std::max(stage, t.lanes * (int)((c->n + units - 1) / units)));
+  const int typ = force_pass_threads(t, std::max(stage, (c->typ_brick + t.chunks - 1) / t.chunks));
+  const bool four = t.lanes == 1 && typ <= 768 && units > 512 && c->pot == GH_POT_SMATB &&
+                    c->precision == GH_MIXED;
+  t.tpb_c[0] = four ? (typ + 255) / 256 * 256 : t.tpb_c[1];
+  t.tpb = t.tpb_c[c->tpb_pick];
 }
 
 // Brick edges (cells) for the tiled passes: the largest brick whose expected
@@ -403,7 +421,7 @@ static int ensure_ready(gh_ctx *c) {
       c->cap = 0;
       GH_TRY(gh_launch_rebuild(c, true, false));
       int max_halo = 0, max_brick = 0;
-      GH_TRY(gh_tile_occupancy(c, &max_halo, &max_brick));
+      GH_TRY(gh_tile_occupancy(c, &max_halo, &max_brick, &c->typ_brick));
       GH_TRY(read_status(c, &h));
       int slot_cap = max_halo + std::max(32, max_halo / 8);
       slot_cap = roundup(slot_cap, 32);
@@ -779,7 +797,7 @@ int gh_set_tile(gh_ctx *c, const int *bd) {
   for (int d = 0; d < 3; ++d)
     if (bd && (bd[d] < 0 || bd[d] > 4)) return gh_fail(c, GH_EINVAL, "brick edges must be 0..4");
   for (int d = 0; d < 3; ++d) c->bd_req[d] = bd ? bd[d] : 0;
-  c->tpb_mean = 0;
+  c->tpb_pick = 0;
   c->chunks_req = c->chunks_env;
   c->ready = false;
   return 0;
@@ -840,7 +858,7 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
   hipEvent_t e0, e1;
   GH_HIP(c, hipEventCreate(&e0));
   GH_HIP(c, hipEventCreate(&e1));
-  int best[3] = {0, 0, 0}, best_mean = 0, best_chunks = 1;
+  int best[3] = {0, 0, 0}, best_pick = 0, best_chunks = 1;
   double best_us = 1e30, best_score = 1e30;
   for (int bz = 1; bz <= 4; ++bz)
     for (int by = bz; by <= 4; ++by)
@@ -878,9 +896,9 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
           if (k > 1 && !c->chunks_env && c->tg.nbrick * k > 512) continue;
           c->chunks_req = k;
           set_force_pass_threads(c);
-          const int cand[2] = {c->tg.tpb_max, c->tg.tpb_avg};
-          for (int m = 0; m < 2; ++m) {
-            if (m == 1 && cand[1] == cand[0]) break;
+          const int *cand = c->tg.tpb_c;
+          for (int m = 0; m < 3; ++m) {
+            if (m > 0 && (cand[m] == cand[0] || cand[m] == cand[m - 1])) continue;
             c->tg.tpb = cand[m];
             GH_TRY(gh_launch_forces(c, nullptr));
             GH_HIP(c, hipEventRecord(e0, c->stream));
@@ -894,7 +912,7 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
             if (us + rate * chain_us < best_score) {
               best_score = us + rate * chain_us;
               best_us = us;
-              best_mean = m;
+              best_pick = m;
               best_chunks = k;
               for (int d = 0; d < 3; ++d) best[d] = b[d];
             }
@@ -904,7 +922,7 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   for (int d = 0; d < 3; ++d) c->bd_req[d] = best[d];
-  c->tpb_mean = best_mean;
+  c->tpb_pick = best_pick;
   c->chunks_req = best_chunks;
   c->ready = false;
   c->err.clear();

@@ -133,7 +133,7 @@ struct TileGeom {
   int nkey;       // nbrick * cpb
   int slot_cap;   // LDS slots per workgroup (halo atoms)
   int tpb;        // threads per workgroup of the force passes (a multiple of 64)
-  int tpb_max, tpb_avg;  // its two candidates: the fullest brick, the mean brick
+  int tpb_c[3];          // its candidates (set_force_pass_threads)
   int lanes = 1;  // lanes per atom in the force passes: 4 below 131072 atoms (fixed by n)
   int chunks = 1; // workgroups per brick in the force passes (each a share of its atoms)
   int fxk;        // fixed-point steps per Angstrom: 2^fxk (mixed SMA-TB)
@@ -172,6 +172,7 @@ struct GhStatus {                     // device-resident counters
   int tile_overflow;                  // a brick's halo exceeded slot_cap (sticky)
   int max_halo;                       // largest halo (atoms) at the last build
   int max_brick;                      // largest brick (atoms) at the last build
+  unsigned long long brick_sq;        // sum of the squares of the bricks' atom counts there
   int ticket;                         // binning workgroups done (last one scans)
   int halt;                           // GH_HALT_*: every state-changing kernel returns
   long long halt_step;                // step at which halt was raised
@@ -252,10 +253,11 @@ struct gh_ctx {
   int ncell = 1;
   TileGeom tg;                // brick grouping (cell mode)
   int bd_req[3] = {0, 0, 0};  // requested brick edge (0 = automatic)
-  int tpb_mean = 0;           // 1: force-pass workgroups sized to the mean brick (autotuned)
+  int tpb_pick = 0;           // which of TileGeom::tpb_c (autotuned)
   int chunks_req = 0;         // force-pass workgroups per brick (autotuned; 0 = 1)
   int chunks_env = 0;         // GEMS_HIP_CHUNKS: forced workgroups per brick (0 = free)
   int max_brick = 0;          // atoms of the fullest brick at the last sizing
+  int typ_brick = 0;          // of the brick that an atom finds itself in, mean over atoms
   int list_rows = 0;          // GEMS_HIP_LIST_BUILD: 1 = rows (one thread per atom), 2 = coop, 0 auto
   int list_build = 0;         // kernel of the last enqueued build: 1 per-thread, 2 cooperative
   int cap = 0;                // list row capacity
@@ -393,7 +395,7 @@ int gh_launch_rebuild_cells(gh_ctx *c);
 int gh_launch_forces_tiled(gh_ctx *c, hipEvent_t mid, bool fuse_vv);
 int gh_fill_int(gh_ctx *c, int *p, int v, int n);
 int gh_launch_wrap(gh_ctx *c);
-int gh_tile_occupancy(gh_ctx *c, int *max_halo, int *max_brick);
+int gh_tile_occupancy(gh_ctx *c, int *max_halo, int *max_brick, int *typ_brick);
 int gh_request_rebuild(gh_ctx *c);  // the next rebuild chain rebuilds whatever the displacement
 int gh_tiled_to_global(gh_ctx *c, int *dst);
 int gh_upload_tb(gh_ctx *c);

@@ -1239,7 +1239,9 @@ __global__ __launch_bounds__(GH_TBLOCK) void k_tile_occupancy(TileGeom t,
   if (!halo_setup(t, b, cell_start, H, st, false)) return;
   if (threadIdx.x == 0) {
     atomicMax(&st->max_halo, H.total);
-    atomicMax(&st->max_brick, H.a1 - H.a0);
+    const unsigned long long na = (unsigned long long)(H.a1 - H.a0);
+    atomicMax(&st->max_brick, (int)na);
+    atomicAdd(&st->brick_sq, na * na);
   }
 }
 
@@ -2110,12 +2112,13 @@ int gh_launch_rebuild_cells(gh_ctx *c) {
   return 0;
 }
 
-int gh_tile_occupancy(gh_ctx *c, int *max_halo, int *max_brick) {
+int gh_tile_occupancy(gh_ctx *c, int *max_halo, int *max_brick, int *typ_brick) {
   GhStatus h;
   GH_HIP(c, hipMemcpyAsync(&h, c->status, sizeof(h), hipMemcpyDeviceToHost, c->stream));
   GH_HIP(c, hipStreamSynchronize(c->stream));
   h.max_halo = 0;
   h.max_brick = 0;
+  h.brick_sq = 0ull;
   GH_HIP(c, hipMemcpyAsync(c->status, &h, sizeof(h), hipMemcpyHostToDevice, c->stream));
   { k_tile_occupancy<<<c->tg.nbrick, GH_TBLOCK, 0, c->stream>>>(c->tg, c->cell_start, c->status); ++c->launches; }
   GH_HIP(c, hipGetLastError());
@@ -2123,6 +2126,7 @@ int gh_tile_occupancy(gh_ctx *c, int *max_halo, int *max_brick) {
   GH_HIP(c, hipStreamSynchronize(c->stream));
   *max_halo = h.max_halo;
   *max_brick = h.max_brick;
+  *typ_brick = (int)(h.brick_sq / (unsigned long long)c->n);
   return 0;
 }
 
