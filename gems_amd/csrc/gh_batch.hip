@@ -372,7 +372,7 @@ __device__ __forceinline__ void batch_rho(const BatchArgs &B, const BTable<MIXED
 
 // Forces and repulsion of atom i (smatb_interact, TB.F90:457-586) by G lanes:
 // f = {Fx, Fy, Fz, sum of repulsions} (eV units) in each.
-template <bool MIXED, bool SINGLE, int G>
+template <bool MIXED, bool SINGLE, int G, bool ENERGY = true>
 __device__ __forceinline__ void batch_force(const BatchArgs &B, const BTable<MIXED, SINGLE> &T,
                                             const BForm<MIXED> &p1, int a0, int i,
                                             const RowHead<G> &row, double (&f)[4]) {
@@ -395,13 +395,13 @@ __device__ __forceinline__ void batch_force(const BatchArgs &B, const BTable<MIX
         double s, rep;
         if constexpr (MIXED) {
           float sf, repul;
-          if (!tb_force_fx<true>(P, rd,
-                                 __int_as_float(__double2loint(pi.w)) +
-                                     __int_as_float(__double2loint(p[u].w)),
-                                 sf, repul))
+          if (!tb_force_fx<ENERGY>(P, rd,
+                                   __int_as_float(__double2loint(pi.w)) +
+                                       __int_as_float(__double2loint(p[u].w)),
+                                   sf, repul))
             return;
           s = (double)sf;  // factor / r per unit of the pair vector
-          rep = (double)repul;
+          if (ENERGY) rep = (double)repul;
         } else {
           if (!(rd <= P.rce2)) return;
           double dr, ir, factor;
@@ -412,10 +412,10 @@ __device__ __forceinline__ void batch_force(const BatchArgs &B, const BTable<MIX
         f[0] = fma(-s, vx, f[0]);
         f[1] = fma(-s, vy, f[1]);
         f[2] = fma(-s, vz, f[2]);
-        f[3] += rep;
+        if (ENERGY) f[3] += rep;
       });
 #pragma unroll
-  for (int d = 0; d < 4; ++d) f[d] = group_total<G>(f[d]);
+  for (int d = 0; d < (ENERGY ? 4 : 3); ++d) f[d] = group_total<G>(f[d]);
 }
 
 // ---------------------------------------------------------------------------
@@ -700,10 +700,13 @@ __device__ __forceinline__ void fire_rho(const BatchArgs &B, const Stage &S,
   __syncthreads();
 }
 
-// Forces and energies; hdt > 0: then the second half kick (v += hdt F / m)
-// and the sums pv = {F.v, |v|^2, |F|^2} of the thread's atoms.  fm2: the
-// largest |F|^2 of its atoms.
-template <bool MIXED, bool QUANT, bool SINGLE>
+// WHAT 0: forces; 1: the per-atom energies of the last ones; 2: both.  A
+// quench reads energies at its end only, so the iterations of a mixed one don't
+// sum them (6.9 -> 6.5 ms with the order above; in FP64, where the repulsion is
+// part of the force anyway, a pass of its own for them costs registers: 12.1 ms
+// against 13.9).  hdt > 0: then the second half kick (v += hdt F / m) and the sums pv = {F.v, |v|^2, |F|^2} of
+// the thread's atoms.  fm2: the largest |F|^2 of its atoms.
+template <bool MIXED, bool QUANT, bool SINGLE, int WHAT>
 __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
                                            const BTable<MIXED, SINGLE> &T, const BForm<MIXED> &p1,
                                            int a0, int n, double hdt, double (&pv)[3],
@@ -716,10 +719,10 @@ __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
     const int k = min(k0 + g, n - 1), i = a0 + k;
     const RowHead<GH_FG> row = row_head<GH_FG>(B, i, on);
     const int ax = min(sub, 2);
-    const double v0 = hdt > 0.0 ? B.vel[ax * B.ld + i] : 0.0;
+    const double v0 = WHAT != 1 && hdt > 0.0 ? B.vel[ax * B.ld + i] : 0.0;
     double f[4] = {0.0, 0.0, 0.0, 0.0};
     if (!lds) {
-      batch_force<MIXED, SINGLE, GH_FG>(B, T, p1, a0, i, row, f);
+      batch_force<MIXED, SINGLE, GH_FG, (WHAT > 0)>(B, T, p1, a0, i, row, f);
     } else if constexpr (QUANT) {
       const int4 qi = S.q[k];
       const int ti = SINGLE ? 0 : S.ty[k];
@@ -735,19 +738,21 @@ __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
           [&](int u) {
             const double dx = fxd(q[u].x, qi.x), dy = fxd(q[u].y, qi.y), dz = fxd(q[u].z, qi.z);
             float sf, repul;
-            if (tb_force_fx<true>(SINGLE ? p1 : T.t[ti * GH_MAXT + t[u]],
-                                  fma(dx, dx, fma(dy, dy, dz * dz)),
-                                  di + __int_as_float(q[u].w), sf, repul)) {
+            if (tb_force_fx<(WHAT > 0)>(SINGLE ? p1 : T.t[ti * GH_MAXT + t[u]],
+                                        fma(dx, dx, fma(dy, dy, dz * dz)),
+                                        di + __int_as_float(q[u].w), sf, repul)) {
               const double sfd = (double)sf;
               f[0] = fma(-sfd, dx, f[0]);
               f[1] = fma(-sfd, dy, f[1]);
               f[2] = fma(-sfd, dz, f[2]);
-              f[3] += (double)repul;
+              if (WHAT > 0) f[3] += (double)repul;
             }
           });
 #pragma unroll
-      for (int d = 0; d < 4; ++d) f[d] = group_total<GH_FG>(f[d]);
+      for (int d = WHAT == 1 ? 3 : 0; d < (WHAT > 0 ? 4 : 3); ++d) f[d] = group_total<GH_FG>(f[d]);
     }
+    if (WHAT > 0 && on && sub == 3) B.e[i] = (f[3] - sqrt(B.rho[i])) * B.ev_ui;
+    if (WHAT == 1) continue;
     const double F = (ax == 0 ? f[0] : ax == 1 ? f[1] : f[2]) * B.ev_ui;
     if (on && sub < 3) {
       B.frc[sub * B.ld + i] = F;
@@ -758,8 +763,6 @@ __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
         pv[1] += v * v;
         pv[2] += F * F;
       }
-    } else if (on) {
-      B.e[i] = (f[3] - sqrt(B.rho[i])) * B.ev_ui;
     }
     if (on && sub == 0) {
       const double Fy = f[1] * B.ev_ui, Fz = f[2] * B.ev_ui;
@@ -782,7 +785,11 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   __shared__ BTable<MIXED, SINGLE> T;
   __shared__ BlockRed<BS> R;
   __shared__ int sfar;
-  const int s = B.order[B.first + blockIdx.x];
+  // Systems come largest first and 256 workgroups fill one slot on each CU:
+  // every other 256 run in reverse, so that a CU's systems add up alike (1024
+  // Au clusters of 13 to 309 atoms, a quench of 100 iterations: 6.75 -> 6.58 ms).
+  const int wr = (int)blockIdx.x & ~255, ww = min(256, (int)gridDim.x - wr);
+  const int s = B.order[B.first + ((wr >> 8) & 1 ? 2 * wr + ww - 1 - (int)blockIdx.x : (int)blockIdx.x)];
   FireState st = fst[s];
   if (fc_arg.resume && st.done) return;
   if (threadIdx.x == 0) {
@@ -814,9 +821,10 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
     }
     __syncthreads();
   }
+  constexpr int kForce = MIXED ? 0 : 2;
   double pv[3] = {0.0, 0.0, 0.0}, fm2 = 0.0;
   fire_rho<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n);
-  fire_force<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+  fire_force<MIXED, QUANT, SINGLE, kForce>(B, S, T, p1, a0, n, 0.0, pv, fm2);
   // the mixing of the last iteration, still to be applied to v: v <- cm v + mixv F
   double cm = 1.0, mixv = 0.0;
   bool pend = false;
@@ -870,7 +878,7 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
     if (2.0 * sqrt(d2) > skin) sys_build(B, a0, n);
     pv[0] = pv[1] = pv[2] = fm2 = 0.0;
     fire_rho<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n);
-    fire_force<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
+    fire_force<MIXED, QUANT, SINGLE, kForce>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
     bred<BS, 3>(R, pv, fm2);
     fnow = sqrt(fm2) * fc.ui_ev;
     pend = true;
@@ -898,7 +906,13 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
       }
   const bool done = !MIXED || !stop;  // a mixed system below fswitch goes on in FP64
   double ep = 0.0, ek = 0.0;
-  if (done) sys_energies(B, R, a0, a1, ep, ek);
+  if (done) {
+    if (MIXED) {
+      fire_force<MIXED, QUANT, SINGLE, 1>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+      __syncthreads();
+    }
+    sys_energies(B, R, a0, a1, ep, ek);
+  }
   if (threadIdx.x == 0) {
     st.dt = dt;
     st.alpha = alpha;
