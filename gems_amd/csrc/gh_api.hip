@@ -279,11 +279,20 @@ static int force_pass_threads(const TileGeom &t, int atoms) {
 // With t.chunks workgroups per brick, each takes a contiguous share of the
 // brick's atoms and stages the whole halo: it gets at least a third as many
 // threads as halo slots, so that the staging takes at most three rounds of
-// loads (the atom loop's spare threads return at once).
+// loads (the atom loop's spare threads return at once).  Unless a shape, the
+// autotuner or the environment says otherwise, the small systems' bricks are
+// split as long as every workgroup has a CU to itself: a second round of
+// workgroups costs as much as the first.  200 velocity Verlet steps, mixed, one
+// workgroup per brick and with 2, 3, 4 (ms): Au 4,000 atoms (8 bricks) 8.4, 6.2,
+// 5.7, 5.3; 32,000 (80) 9.9, 7.0, 6.5, 8.6; 55,296 (96) 9.5, 7.4, 10.7, 9.9; 70,304
+// (150) 10.9, 11.0, 11.3, 13.0; Ag-Cu 32,000 (64) 11.0, 8.7, 7.6, 7.3; LJ 32,000
+// (96) 7.9, 7.0, 8.8, 8.5.
 static void set_force_pass_threads(gh_ctx *c) {
   TileGeom &t = c->tg;
   t.lanes = c->n < 131072 ? 4 : 1;
   t.chunks = std::max(1, c->chunks_req);
+  if (c->chunks_req == 0 && t.lanes == 4 && !c->rows)
+    t.chunks = std::min(4, std::max(1, 256 / t.nbrick));
   const int mb = (c->max_brick + t.chunks - 1) / t.chunks;
   const long long units = (long long)t.nbrick * t.chunks;
   const int stage = t.chunks > 1 ? (t.slot_cap + GH_STAGE_ROUNDS - 1) / GH_STAGE_ROUNDS : 0;
@@ -798,7 +807,8 @@ int gh_set_tile(gh_ctx *c, const int *bd) {
     if (bd && (bd[d] < 0 || bd[d] > 4)) return gh_fail(c, GH_EINVAL, "brick edges must be 0..4");
   for (int d = 0; d < 3; ++d) c->bd_req[d] = bd ? bd[d] : 0;
   c->tpb_pick = 0;
-  c->chunks_req = c->chunks_env;
+  const bool shape = c->bd_req[0] || c->bd_req[1] || c->bd_req[2];
+  c->chunks_req = c->chunks_env ? c->chunks_env : shape ? 1 : 0;
   c->ready = false;
   return 0;
 }

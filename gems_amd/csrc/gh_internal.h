@@ -254,7 +254,7 @@ struct gh_ctx {
   TileGeom tg;                // brick grouping (cell mode)
   int bd_req[3] = {0, 0, 0};  // requested brick edge (0 = automatic)
   int tpb_pick = 0;           // which of TileGeom::tpb_c (autotuned)
-  int chunks_req = 0;         // force-pass workgroups per brick (autotuned; 0 = 1)
+  int chunks_req = 0;         // force-pass workgroups per brick (0: by the bricks' number)
   int chunks_env = 0;         // GEMS_HIP_CHUNKS: forced workgroups per brick (0 = free)
   int max_brick = 0;          // atoms of the fullest brick at the last sizing
   int typ_brick = 0;          // of the brick that an atom finds itself in, mean over atoms

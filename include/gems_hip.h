@@ -250,9 +250,11 @@ typedef struct {
   int64_t steps;
   int64_t launches;  /* kernels the context has enqueued (no counterpart) */
   int32_t list_build; /* kernel of the last enqueued list build: 0 none, 1 one
-                         thread per atom, 2 cooperative (no counterpart) */
+                         thread per atom, 2 cooperative, 3 rows of atom numbers
+                         (no counterpart) */
   int32_t chunks;     /* workgroups per brick of the force passes, each taking
-                         a share of its atoms (cell mode; no counterpart) */
+                         a share of its atoms (cell mode by tiles; no
+                         counterpart) */
 } gh_stats;
 int gh_get_stats(gh_ctx *ctx, gh_stats *s);
 
