@@ -1114,28 +1114,28 @@ __global__ __launch_bounds__(GH_CBLOCK) void k_build_coop(GhStatus *st,
 }
 
 // ---------------------------------------------------------------------------
-// Rows of atom numbers (gh_rows_path): 16 lanes per
-// atom, candidates straight from global memory (a cell's atoms are contiguous
+// Rows of atom numbers (gh_rows_path): 16 or 32 lanes per atom, candidates straight from global memory (a cell's atoms are contiguous
 // and its 27 cells cached), cell by cell in the order of the tiled builds
 // (dz, dy, dx; within a cell as sorted), exact test and class; the kept ones
 // pass through an LDS row and leave it by class.  The rows are the tiled
 // builds', entry for entry, as (atom | image code << 27).  LJ 4,000 atoms
-// 12.7 us a build, 55,296 36 us (k_build_coop 44); Au 119,164 40 (24).
+// 9.9 us a build, 55,296 36 us (k_build_coop 44); Au 119,164 40 (24).
 // ---------------------------------------------------------------------------
-#define GH_RGROUPS (GH_TBLOCK / 16)
 static_assert(131072 < (1 << 25), "an entry's class sits in bits 25-26 while the row is ordered");
+template <int G>
 __global__ __launch_bounds__(GH_TBLOCK) void k_build_rows(GhStatus *st,
                                                           const ChainArgs *__restrict__ C,
                                                           const double4 *__restrict__ pos,
                                                           long long step) {
   if (!st->rebuild) return;
   extern __shared__ unsigned rowmem[];
-  __shared__ int cstart[GH_RGROUPS][27], ccount[GH_RGROUPS][27];  // count | image code << 24
+  constexpr int U = 32 / G;  // candidates of a lane in 32
+  __shared__ int cstart[GH_TBLOCK / G][27], ccount[GH_TBLOCK / G][27];  // count | image code << 24
   const CellArgs &R = C->R;
   const BuildArgs &A = C->A;
   const TileGeom &t = R.t;
-  const int g = threadIdx.x >> 4, sub = threadIdx.x & 15, cap = A.cap;
-  const int a0 = (int)(xcd_block() * GH_TBLOCK + threadIdx.x) >> 4;
+  const int g = threadIdx.x / G, sub = threadIdx.x & (G - 1), cap = A.cap;
+  const int a0 = (int)(xcd_block() * GH_TBLOCK + threadIdx.x) / G;
   const bool live = a0 < R.n;
   const int a = min(a0, R.n - 1);
   unsigned *buf = rowmem + g * cap;
@@ -1144,7 +1144,7 @@ __global__ __launch_bounds__(GH_TBLOCK) void k_build_rows(GhStatus *st,
     const int bx = b % t.nbr[0], by = (b / t.nbr[0]) % t.nbr[1], bz = b / (t.nbr[0] * t.nbr[1]);
     const int cc[3] = {bx * t.bd[0] + lc % t.bd[0], by * t.bd[1] + (lc / t.bd[0]) % t.bd[1],
                        bz * t.bd[2] + lc / (t.bd[0] * t.bd[1])};
-    for (int q = sub; q < 27; q += 16) {
+    for (int q = sub; q < 27; q += G) {
       int c3[3] = {cc[0] + q % 3 - 1, cc[1] + (q / 3) % 3 - 1, cc[2] + q / 9 - 1};
       int w[3] = {1, 1, 1};
       bool ok = true;
@@ -1174,35 +1174,48 @@ __global__ __launch_bounds__(GH_TBLOCK) void k_build_rows(GhStatus *st,
   }
   __builtin_amdgcn_wave_barrier();
   const unsigned below = (1u << sub) - 1;
-  const int shl = threadIdx.x & 48;  // the group's bits in a wave mask
-  auto bits = [&](bool v) { return (unsigned)(__ballot(v) >> shl) & 0xFFFFu; };
+  const int shl = threadIdx.x & (64 - G);  // the group's bits in a wave mask
+  auto bits = [&](bool v) { return (unsigned)(__ballot(v) >> shl) & (0xFFFFFFFFu >> (32 - G)); };
   const double4 pa = pos[a];
   int m = 0;
-  for (int q = 0; q < 27; ++q) {
-    const int s0 = cstart[g][q], cw = ccount[g][q], cnt = cw & 0xFFFFFF, code = cw >> 24;
-    const double sx = (double)(code % 3 - 1) * t.L[0], sy = (double)((code / 3) % 3 - 1) * t.L[1],
-                 sz = (double)(code / 9 - 1) * t.L[2];
-    for (int j0 = 0; __any(live && j0 < cnt); j0 += 32) {
-      double4 p[2];
+  // The first 32 candidates of three cells are in flight together: 27 cells one
+  // after another were 27 round trips (LJ 4,000 atoms 13.2 -> 11.5 us, 16 lanes).
+  for (int q0 = 0; q0 < 27; q0 += 3) {
+    int s0[3], cw[3];
+    double4 p[3][U];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) p[u] = pos[min(s0 + j0 + 16 * u + sub, R.n - 1)];
+    for (int c = 0; c < 3; ++c) {
+      s0[c] = cstart[g][q0 + c];
+      cw[c] = ccount[g][q0 + c];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int o = j0 + 16 * u + sub, j = s0 + o;
-        const double rd = dist2_rn((p[u].x - pa.x) + sx, (p[u].y - pa.y) + sy, (p[u].z - pa.z) + sz);
+      for (int u = 0; u < U; ++u) p[c][u] = pos[min(s0[c] + G * u + sub, R.n - 1)];
+    }
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int cnt = cw[c] & 0xFFFFFF, code = cw[c] >> 24;
+      const double sx = (double)(code % 3 - 1) * t.L[0],
+                   sy = (double)((code / 3) % 3 - 1) * t.L[1], sz = (double)(code / 9 - 1) * t.L[2];
+      auto take = [&](int o, const double4 &pj) {
+        const int j = s0[c] + o;
+        const double rd = dist2_rn((pj.x - pa.x) + sx, (pj.y - pa.y) + sy, (pj.z - pa.z) + sz);
         const bool keep = live && o < cnt && j != a && rd < A.rl2;
         const unsigned b = bits(keep);
         const int d = m + __popc(b & below);
         if (keep && d < cap)
           buf[d] = (unsigned)j | ((unsigned)row_class(rd, A) << 25) | ((unsigned)code << 27);
         m += __popc(b);
-      }
+      };
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (__any(live && G * u < cnt)) take(G * u + sub, p[c][u]);
+      for (int j0 = 32; __any(live && j0 < cnt); j0 += G)
+        take(j0 + sub, pos[min(s0[c] + j0 + sub, R.n - 1)]);
     }
   }
   __builtin_amdgcn_wave_barrier();
   const int mw = min(m, cap);
   int n0 = 0, n1 = 0, n2 = 0;
-  for (int k = sub; __any(k < mw); k += 16) {
+  for (int k = sub; __any(k < mw); k += G) {
     const int c = k < mw ? (int)(buf[k] >> 25) & 3 : 4;
     n0 += __popc(bits(c == 0));
     n1 += __popc(bits(c == 1));
@@ -1210,7 +1223,7 @@ __global__ __launch_bounds__(GH_TBLOCK) void k_build_rows(GhStatus *st,
   }
   int d0 = 0, d1 = n0, d2 = n0 + n1, d3 = n0 + n1 + n2;
   unsigned *row = A.list32 + (size_t)a * cap;
-  for (int k = sub; __any(k < mw); k += 16) {
+  for (int k = sub; __any(k < mw); k += G) {
     const unsigned e = k < mw ? buf[k] : 0u;
     const int c = k < mw ? (int)(e >> 25) & 3 : 4;
     const unsigned b0 = bits(c == 0), b1 = bits(c == 1), b2 = bits(c == 2), b3 = bits(c == 3);
@@ -2090,9 +2103,13 @@ int gh_launch_rebuild_cells(gh_ctx *c) {
   { k_cell_rank_gather<<<ga, GH_TBLOCK, 0, s>>>(c->status, C, c->pos); ++c->launches; }
   c->list_build = c->rows ? 3 : coop ? 2 : 1;
   if (c->rows) {
-    const int grid = xgrid((c->n + GH_RGROUPS - 1) / GH_RGROUPS);
-    k_build_rows<<<grid, GH_TBLOCK, sizeof(unsigned) * GH_RGROUPS * (size_t)c->cap, s>>>(
-        c->status, C, c->pos, c->step);
+    // (32 where 16 leave a SIMD two wavefronts or fewer, whose steps then wait on
+    // one another: LJ 4,000 atoms 9.9 against 11.5 us; 16,384 16.7 against 14.8)
+    const int lanes = c->n <= 8192 ? 32 : 16, per = GH_TBLOCK / lanes;
+    const int grid = xgrid((c->n + per - 1) / per);
+    const size_t rows = sizeof(unsigned) * per * (size_t)c->cap;
+    if (lanes == 32) k_build_rows<32><<<grid, GH_TBLOCK, rows, s>>>(c->status, C, c->pos, c->step);
+    else k_build_rows<16><<<grid, GH_TBLOCK, rows, s>>>(c->status, C, c->pos, c->step);
   } else if (coop) {
     // 4 to 16 wavefronts: about 24 atoms each of a workgroup's mean share
     // where the workgroups fill the CUs, about two where they do not (each
