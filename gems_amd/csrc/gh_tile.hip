@@ -947,7 +947,12 @@ __device__ __forceinline__ int halo_cell(const TileGeom &t, const Halo &H, int X
   return (lx + 1) + H.hd0 * ((ly + 1) + H.hd1 * (lz + 1));
 }
 
-__global__ __launch_bounds__(GH_CBLOCK) void k_build_coop(GhStatus *st,
+// Two workgroups of 16 wavefronts share a CU (LDS and, held to 64, the
+// registers): four wavefronts of each on every SIMD.  1M LJ liquid, us a build:
+// 9 or 10 wavefronts, which put three on one SIMD and two on others, 873 and
+// 970, 16 at 63 registers (seven to a SIMD: one workgroup fits) 948, 12 667, 16
+// of eight to a SIMD 630.
+__global__ __launch_bounds__(GH_CBLOCK) __attribute__((amdgpu_waves_per_eu(8))) void k_build_coop(GhStatus *st,
                                                           const ChainArgs *__restrict__ C,
                                                           const double4 *__restrict__ pos,
                                                           long long step) {
@@ -2123,15 +2128,13 @@ static BuildArgs build_args(const gh_ctx *c, int cap, size_t *lds_out) {
 // Sets the cooperative build's arguments; false where it does not apply: the
 // sizing count (cap 0, any halo), slot numbers beyond the 14 bits a tagged
 // row entry leaves, or LDS too small for one cell's candidate lists beside
-// the staged halo.  Automatic choice: the per-thread build with its rows in
-// LDS where bricks fill the chip (1024 and more: 1M-atom SMA-TB, 526 us
-// against 563 us per rebuild), the cooperative build elsewhere (few bricks,
-// or rows too long for LDS: the 1M-atom LJ liquid 824 us against 1241 us,
-// 4000 atoms 37 us against 235 us).
+// the staged halo.  The per-thread build is left for those (us a rebuild,
+// per thread and cooperative: 1M-atom SMA-TB, mixed, 558 and 428, 500,000 atoms
+// FP64 386 and 280, 442,000 Ag-Cu 393 and 246, the 1M-atom LJ liquid 1271 and 630,
+// 4,000 atoms 235 and 37).
 static bool coop_args(const gh_ctx *c, BuildArgs &A, size_t *lds_out) {
   const int slot_cap = c->tg.slot_cap;
   if (c->list_rows == 1 || A.cap <= 0 || slot_cap >= 16000) return false;
-  if (c->list_rows == 0 && A.lds_rows && c->tg.nbrick >= 1024) return false;
   const int nsl = (slot_cap + 4) / 4 * 4;  // + the far slot that pads the lists
   const int rstride = (A.cap + 1) / 2 * 2;
   const size_t fixed = (size_t)nsl * 17 + (size_t)(GH_CBLOCK / 64) * rstride * 2;
@@ -2213,14 +2216,14 @@ int gh_launch_rebuild_cells(gh_ctx *c) {
     if (lanes == 32) k_build_rows<32><<<grid, GH_TBLOCK, rows, s>>>(c->status, C, c->pos, c->step);
     else k_build_rows<16><<<grid, GH_TBLOCK, rows, s>>>(c->status, C, c->pos, c->step);
   } else if (coop) {
-    // 4 to 16 wavefronts: about 24 atoms each of a workgroup's mean share
-    // where the workgroups fill the CUs, about two where they do not (each
-    // CU then holds one workgroup, whose rows wait on their latencies)
+    // 16 wavefronts where the workgroups fill the CUs; about two atoms each,
+    // and 4 to 16, where they do not (each CU then holds one workgroup, whose
+    // rows wait on their latencies)
     const long long units = (long long)c->tg.nbrick * h.A.chunks;
     const long long share = (long long)c->n / units + 1;
-    const int apw = units < 256 ? 2 : 24;
-    const int waves = (int)std::min<long long>(GH_CBLOCK / 64,
-                                               std::max<long long>(4, (share + apw - 1) / apw));
+    const int waves = units >= 256 ? GH_CBLOCK / 64
+                                   : (int)std::min<long long>(GH_CBLOCK / 64,
+                                                              std::max<long long>(4, (share + 1) / 2));
     const int grid = xgrid(c->tg.nbrick * h.A.chunks);
     k_build_coop<<<grid, 64 * waves, lds_coop, s>>>(c->status, C, c->pos, c->step);
   } else {
