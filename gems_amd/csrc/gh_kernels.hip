@@ -1186,17 +1186,20 @@ int gh_launch_rebuild(gh_ctx *c, bool force, bool forces_follow) {
   return 0;
 }
 
-// Cell mode by rows of atom numbers instead of tiles: FP64, the atom counts
-// at which the tiled passes take four lanes per atom (the same bits either
-// way).  200 velocity Verlet steps, tiled -> rows, ms: Au 2,048 atoms 6.7 ->
-// 3.0, 32,000 7.7 -> 5.5, 119,164 17.8 -> 14.0; above, with one lane per atom,
+// Cell mode by rows of atom numbers instead of tiles: FP64, whatever the shape
+// asked for.  200 velocity Verlet steps, tiled -> rows, ms: Au 2,048 atoms
+// 6.7 -> 3.0, 32,000 7.7 -> 5.5, 119,164 17.8 -> 14.0 (the same bits either
+// way, tiles taking four lanes per atom there); above, with one lane per atom,
 // tiles win for one type (Au 256,000 21.3 against 28.2; a row entry is four
-// bytes and its neighbour's 32 come from the L2).  Pair potentials have one pass
-// and less to save: LJ 2,048 4.6 -> 3.4, 32,000 7.2 -> 5.9, 55,296 8.3 ->
-// 8.2, 119,164 12.6 against 14.2.  The environment's choice of a tiled list
-// build or of workgroups per brick keeps the tiles.
+// bytes and its neighbour's 32 come from the L2).  With several types a pair's
+// parameters come from LDS, which the tiles' positions and lists already load:
+// 40 steps Ag-Cu 143,748 9.5 -> 7.4, 256,000 14.9 -> 11.4; 442,368 21.6 and, at
+// the best shape, 18.6 against 18.7; 1M 39.3 against 42.7.  Pair potentials
+// have one pass and less to save: LJ 2,048 4.6 -> 3.4, 32,000 7.2 -> 5.9, 55,296
+// 8.3 -> 8.2, 119,164 12.6 against 14.2.  The environment's choice of a tiled
+// list build or of workgroups per brick keeps the tiles.
 bool gh_rows_path(const gh_ctx *c) {
-  const int most = c->pot == GH_POT_SMATB ? 131072 : 65536;
+  const int most = c->pot != GH_POT_SMATB ? 65536 : c->nt == 1 ? 131072 : 393216;
   return c->precision == GH_FP64 && c->n < most && c->list_rows == 0 && c->chunks_env == 0;
 }
 

@@ -1223,7 +1223,7 @@ __global__ __launch_bounds__(GH_CBLOCK) __attribute__((amdgpu_waves_per_eu(8))) 
 // builds', entry for entry, as (atom | image code << 27).  LJ 4,000 atoms
 // 9.9 us a build, 55,296 36 us (k_build_coop 44); Au 119,164 40 (24).
 // ---------------------------------------------------------------------------
-static_assert(131072 < (1 << 25), "an entry's class sits in bits 25-26 while the row is ordered");
+static_assert(393216 < (1 << 25), "an entry's class sits in bits 25-26 while the row is ordered");
 template <int G>
 __global__ __launch_bounds__(GH_TBLOCK) void k_build_rows(GhStatus *st,
                                                           const ChainArgs *__restrict__ C,

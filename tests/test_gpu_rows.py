@@ -112,6 +112,24 @@ def test_rows_match_tiles(pot, n, cut, pbc, gap, steps):
         assert np.array_equal(a, b)
 
 
+@pytest.mark.parametrize("n,cut", [((32, 32, 32), 0), ((46, 46, 47), 4592), ((46, 46, 47), 4593)])
+def test_rows_match_tiles_two_types_large(n, cut):
+    # several types keep the rows where the tiles take one lane per atom: the
+    # same pairs summed in another order, ~60 terms of up to a few rms(F) at 2^-53
+    x, t, L = _box("agcu", n, cut)
+    res = []
+    for tiled in (False, True):
+        with _ctx(tiled) as c:
+            c.set_box(L, (1, 1, 1))
+            c.set_atoms(x, t)
+            _pot(c, "agcu")
+            res.append(c.compute())
+            assert (c.stats()["list_build"] == 3) == (not tiled and len(x) < 393216)
+    (F, e, et), (F2, e2, et2) = res
+    assert np.max(np.abs(F - F2)) <= 1e-13 * 60 * np.sqrt(np.mean(F2 ** 2))
+    assert np.max(np.abs(e - e2)) <= 1e-13 * np.max(np.abs(e2)) and abs(et - et2) <= 1e-13 * abs(et2)
+
+
 @pytest.mark.parametrize("pot,n,kind,prec", [
     ("au", (5, 5, 4), "free", "fp64"), ("agcu", (5, 5, 4), "free", "fp64"),
     ("au", (7, 7, 6), "free", "fp64"), ("au", (5, 5, 4), "free", "mixed"),
