@@ -1084,34 +1084,48 @@ static int batch_ready(gh_batch *b) {
   return 0;
 }
 
-// The FIRE kernel over all systems.  Multi-type systems above GH_BIGSYS atoms
-// bound a run (one workgroup each, largest first), so they get 1024-thread
-// workgroups on a second stream beside the rest (one-type variants would
-// need more than the registers of a 1024-thread workgroup).  256 threads
-// otherwise: four systems then share a compute unit and hide each other's
-// barriers (1024 Au clusters, mixed, a quench of 100 iterations: 128 threads
-// 9.9 ms, 256 6.7, 512 7.2; registers for five wavefronts per SIMD instead
-// of four spill: 9.0).
+// The FIRE kernel over all systems, a workgroup each.  Threads: 256 where four
+// systems share a compute unit and hide each other's barriers (1024 Au clusters,
+// mixed, a quench of 100 iterations: 128 threads 9.9 ms, 256 6.7, 512 7.2;
+// registers for five wavefronts per SIMD instead of four spill: 9.0); fewer
+// systems leave units idle, and a system's rounds of atoms, one memory round
+// trip after another, bound its iteration: 512 up to 768 systems, 1024 up to 256,
+// no more than the largest system has lanes for.  80 iterations, clusters to 309
+// atoms, 256 / 512 / 1024 threads, ms, mixed (FP64): 200 systems 3.4 / 2.4 / 2.2
+// (5.3 / 4.2 / 4.2), 500 4.4 / 3.2 / 4.0 (7.0 / 5.6 / 7.3), 700 5.0 / 4.2 / 5.4
+// (8.2 / 7.4 / 9.4).  Beside them multi-type systems above GH_BIGSYS atoms,
+// which bound a run (largest first), get 1024 threads on a second stream.
 template <bool MIXED, bool QUANT>
 static int launch_fire(gh_batch *b, const BatchArgs &A, const FireC &fc, const BForm<MIXED> &p) {
   const size_t lds = QUANT ? 17 * (size_t)b->nst : 0;
-  const int nbig = b->nt > 1 ? b->nbig : 0;
+  const int big = b->order_h[0], nmax = b->off_h[big + 1] - b->off_h[big];
+  int bs = b->nsys <= 256 ? 1024 : b->nsys <= 768 ? 512 : GH_FBS;
+  while (bs > GH_FBS && bs / 2 >= GH_FG * nmax) bs /= 2;
+  const int nbig = b->nt > 1 && bs < 1024 ? b->nbig : 0;
   BatchArgs A1 = A;
+#define LAUNCH_FIRE(SG, BS, COUNT, STREAM) \
+  k_batch_fire<MIXED, QUANT, SG, BS><<<COUNT, BS, lds, STREAM>>>(A1, fc, b->skin, b->fst, p)
   if (nbig > 0) {
     BH(b, hipEventRecord(b->ev_fork, b->stream));
     BH(b, hipStreamWaitEvent(b->stream2, b->ev_fork, 0));
-    k_batch_fire<MIXED, QUANT, false, 1024><<<nbig, 1024, lds, b->stream2>>>(A1, fc, b->skin, b->fst, p);
+    LAUNCH_FIRE(false, 1024, nbig, b->stream2);
     BH(b, hipGetLastError());
   }
   if (b->nsys > nbig) {
     A1.first = nbig;
     const int count = b->nsys - nbig;
-    if (b->nt == 1)
-      k_batch_fire<MIXED, QUANT, true, GH_FBS><<<count, GH_FBS, lds, b->stream>>>(A1, fc, b->skin, b->fst, p);
-    else
-      k_batch_fire<MIXED, QUANT, false, GH_FBS><<<count, GH_FBS, lds, b->stream>>>(A1, fc, b->skin, b->fst, p);
+    if (b->nt == 1) {
+      if (bs == 1024) LAUNCH_FIRE(true, 1024, count, b->stream);
+      else if (bs == 512) LAUNCH_FIRE(true, 512, count, b->stream);
+      else LAUNCH_FIRE(true, GH_FBS, count, b->stream);
+    } else {
+      if (bs == 1024) LAUNCH_FIRE(false, 1024, count, b->stream);
+      else if (bs == 512) LAUNCH_FIRE(false, 512, count, b->stream);
+      else LAUNCH_FIRE(false, GH_FBS, count, b->stream);
+    }
     BH(b, hipGetLastError());
   }
+#undef LAUNCH_FIRE
   if (nbig > 0) {
     BH(b, hipEventRecord(b->ev_join, b->stream2));
     BH(b, hipStreamWaitEvent(b->stream, b->ev_join, 0));
