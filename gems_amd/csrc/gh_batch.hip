@@ -930,6 +930,84 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   }
 }
 
+// Langevin steps of mixed systems staged in LDS, a workgroup per system (largest
+// first) and all steps in one launch: no random gathers from the L2, which bound
+// the passes over all atoms, but the largest system takes its own time on one
+// CU (2,000 atoms 150 us a step).  Chosen by batch_staged.  The first step's
+// ermak_a has run.
+template <bool SINGLE, int BS>
+__global__ __launch_bounds__(BS, 4) void k_batch_langevin(BatchArgs B, ErmakC k_arg, double skin,
+                                                          TbF p_arg, unsigned long long seed,
+                                                          long long step0, int nsteps) {
+  __shared__ ErmakC k;
+  __shared__ TbF p1;
+  extern __shared__ int4 dyn_q[];
+  __shared__ BTable<true, SINGLE> T;
+  __shared__ BlockRed<BS> R;
+  __shared__ int sfar;
+  const int s = B.order[blockIdx.x], a0 = B.off[s], n = B.off[s + 1] - a0;
+  if (threadIdx.x == 0) {
+    k = k_arg;
+    p1 = p_arg;
+  }
+  load_table<true, true, SINGLE>(T, B);
+  Stage S{dyn_q, reinterpret_cast<unsigned char *>(dyn_q + B.nst), &sfar};
+  const double skt = sqrt(k_arg.kB_ui * B.T[s]);
+  const int sub = threadIdx.x & (GH_FG - 1), g = (int)threadIdx.x / GH_FG;
+  for (int st = 0; st < nsteps; ++st) {
+    if (threadIdx.x == 0) sfar = 0;
+    __syncthreads();
+    const double4 o4 = B.pos[a0];
+    const double o[3] = {o4.x, o4.y, o4.z};
+    double d2 = 0.0, none[3] = {0.0, 0.0, 0.0};
+    for (int q = threadIdx.x; q < n; q += BS) {
+      const double4 p = B.pos[a0 + q];
+      const double x[3] = {p.x, p.y, p.z};
+      double e2 = 0.0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double dd = x[d] - B.xold[d * B.ld + a0 + q];
+        e2 += dd * dd;
+      }
+      d2 = fmax(d2, e2);
+      stage_atom(S, q, x, o);
+      if (!SINGLE) S.ty[q] = (unsigned char)(int)p.w;
+    }
+    bred<BS, 0>(R, none, d2);
+    if (2.0 * sqrt(d2) > skin) {
+      sys_build(B, a0, n);
+      if (threadIdx.x == 0) B.out[s * OUTW + 2] += 1.0;
+    }
+    fire_rho<true, true, SINGLE>(B, S, T, p1, a0, n);
+    const bool last = st + 1 == nsteps;
+    double fm2 = 0.0;
+    if (last) fire_force<true, true, SINGLE, 2>(B, S, T, p1, a0, n, 0.0, none, fm2);
+    else fire_force<true, true, SINGLE, 0>(B, S, T, p1, a0, n, 0.0, none, fm2);
+    // ermak_b, and ermak_a of the next step: the lane that stored an axis'
+    // force moves it (the passes read positions from LDS)
+    const long long step = step0 + st;
+    for (int k0 = 0; k0 < n; k0 += BS / GH_FG) {
+      if (sub == 3 || k0 + g >= n) continue;
+      const int i = a0 + k0 + g, t = SINGLE ? 0 : B.type[i];
+      float ga, gb, gn, un;
+      axis_normals(seed, step, i, sub, ga, gb);
+      const double F = B.frc[sub * B.ld + i], om = B.om[t], f_lan = skt * B.osm[t];
+      const double vel_v = f_lan * k.sdv * (k.crv1 * (double)ga + k.crv2 * (double)gb);
+      const double v = k.c0 * B.vel[sub * B.ld + i] + (k.c1 - k.c2) * B.acc[sub * B.ld + i] +
+                       k.c2 * F * om + vel_v;
+      const double a = F * om;
+      B.vel[sub * B.ld + i] = v;
+      B.acc[sub * B.ld + i] = a;
+      if (!last) {
+        axis_normals(seed, step + 1, i, sub, gn, un);
+        double *x = reinterpret_cast<double *>(B.pos + i) + sub;
+        *x = *x + k.c1 * v + k.c2 * k.dt * a + f_lan * k.sdr * (double)gn;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 __global__ void k_batch_zero(GhLine *p, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) p[i].bits = 0ull;
@@ -1407,6 +1485,19 @@ int gh_batch_compute(gh_batch *b, double *F, double *epot) {
   return 0;
 }
 
+// Mixed Langevin steps by a workgroup per system (k_batch_langevin) or over all
+// atoms: the former takes the largest system's time, the latter the sum's, so by
+// their ratio.  50 steps and an exchange, Ag-Cu clusters from 38 atoms, over all atoms and
+// per system, ms: 512 systems to 150 atoms 2.0 and 1.8, to 600 4.5 and 3.6, to 1000
+// 6.3 and 5.9, to 2000 10.1 and 13.3 (0.50 of the largest system per CU);
+// 256 to 150 1.28 and 1.00, to 600 2.5 and 3.1 (0.34); in long runs 304 to 500
+// (0.48) 43 and 33 us a step, 512 of 642 atoms on average, 2000 at most (0.64), 183
+// and 170.
+static bool batch_staged(const gh_batch *b) {
+  const int big = b->order_h[0], nmax = b->off_h[big + 1] - b->off_h[big];
+  return b->precision == GH_MIXED && b->nst > 0 && b->ntot >= (nmax <= 512 ? 115ll : 144ll) * nmax;
+}
+
 int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t seed,
                       double *epot, double *ekin) {
   if (!b || nsteps < 0 || !(dt > 0) || !(gamma > 0))
@@ -1428,7 +1519,12 @@ int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t
     BatchArgs A = bargs(b);
     k_batch_zero<<<(2 * b->nsys + GH_BWG - 1) / GH_BWG, GH_BWG, 0, b->stream>>>(b->dmax, 2 * b->nsys);
     k_batch_ermak_a<<<batch_blocks(b, 16), GH_BWG, 0, b->stream>>>(A, k, seed, step0);
-    for (int st = 0; st < nsteps; ++st) {
+    if (batch_staged(b)) {
+      const size_t lds = 17 * (size_t)b->nst;
+      if (b->nt == 1) k_batch_langevin<true, 1024><<<b->nsys, 1024, lds, b->stream>>>(A, k, b->skin, b->tbf0, seed, step0, nsteps);
+      else k_batch_langevin<false, 1024><<<b->nsys, 1024, lds, b->stream>>>(A, k, b->skin, b->tbf0, seed, step0, nsteps);
+    }
+    for (int st = 0; st < nsteps && !batch_staged(b); ++st) {
       const long long step = step0 + st;
       launch_rho(b, A, (int)(step & 1), 0);
       if (st + 1 < nsteps) {

@@ -23,7 +23,7 @@ __device__ __forceinline__ void disp2_clear(GhStatus *st, long long step) {
 }
 
 // Rebuild test of step `step` on the displacement maximum the integrators
-// fold into GhStatus::maxdisp2 (one atomicMax per workgroup).
+// fold into GhStatus::maxdisp2.
 __device__ __forceinline__ bool rebuild_due(const GhStatus *st, double skin, long long step) {
   const double d2 = __longlong_as_double((long long)disp2_max(st, step));
   return st->force_rebuild || 2.0 * sqrt(d2) > skin;

@@ -133,7 +133,7 @@ struct TileGeom {
   int nkey;       // nbrick * cpb
   int slot_cap;   // LDS slots per workgroup (halo atoms)
   int tpb;        // threads per workgroup of the force passes (a multiple of 64)
-  int tpb_c[3];          // its candidates (set_force_pass_threads)
+  int tpb_c[3];   // its candidates (set_force_pass_threads)
   int lanes = 1;  // lanes per atom in the force passes: 4 below 131072 atoms (fixed by n)
   int chunks = 1; // workgroups per brick in the force passes (each a share of its atoms)
   int fxk;        // fixed-point steps per Angstrom: 2^fxk (mixed SMA-TB)

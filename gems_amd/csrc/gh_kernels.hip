@@ -34,7 +34,7 @@ __global__ void k_fill_int(int *__restrict__ p, int v, int n) {
 // rebuilds when the two largest displacements since the last build sum past
 // the skin.  Here the displacement is the true (minimum-image) one, and the
 // test uses 2*max, which bounds d1+d2 from above.  Integrators fold each
-// workgroup's max |x - x_old|^2 into GhStatus::maxdisp2 with one
+// workgroup's max |x - x_old|^2 into GhStatus::maxdisp2 with at most one
 // atomicMax (non-negative doubles order as their bit patterns); it runs over
 // the steps since the last build and the first kernel of a rebuild sequence
 // reads it (rebuild_due, rebuild_book).  State-changing kernels return at
@@ -1143,7 +1143,7 @@ ErmakArgs make_ermak(const gh_ctx *c) {
 // launchers
 // ---------------------------------------------------------------------------
 // Neighbour rebuild.  force: request a rebuild regardless of displacement.
-// Every kernel of the rebuild reads the device flag set by k_decide, so the
+// Every kernel of the rebuild tests the rule or reads the flag its first one set, so the
 // sequence can be enqueued every step without a host round trip.
 using namespace ghd;
 

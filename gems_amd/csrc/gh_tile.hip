@@ -164,7 +164,7 @@ __device__ __forceinline__ int halo_of_slot(const Halo &H, int s) {
 
 // stepb of this step and stepa of the next for atom a (velocity_verlet_b,
 // Integration.F90:1171-1186, then velocity_verlet_a, :1150-1169): the same
-// operations in the same order as k_vv_ba, on the force just summed.
+// operations in the same order as k_vv_b and k_vv_a, on the force just summed.
 // New positions go to pos_next (other workgroups still stage pos); returns
 // |x_new - x_old|^2 for the skin test.
 // The update's loads of atom a (velocity, build position), issued together
