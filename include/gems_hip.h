@@ -157,16 +157,19 @@ int gh_set_skin(gh_ctx *ctx, double skin);
 /* Cell-tile shape of the tiled passes.  The reference fixes only the cell
  * grid (intergroup_setcells, Neighbour.F90:587-664); the device groups cells
  * into bricks of bd[0] x bd[1] x bd[2] cells (1..4 each, 0 = automatic), one
- * workgroup per brick (or per share of a brick's atoms where gh_autotune
- * chose several; setting the shape resets that to one).  No counterpart in
- * the reference. */
+ * workgroup per brick, or several, each with a share of its atoms (small
+ * mixed boxes, or where gh_autotune chose several; a shape other than 0 resets
+ * that to one).  FP64 boxes below 131,072 atoms (several types 393,216; pair
+ * potentials 65,536) take rows of atom numbers instead of tiles: bricks then only order the
+ * atoms.  No counterpart in the reference. */
 int gh_set_tile(gh_ctx *ctx, const int bd[3]);
 /* Autotuner: times `reps` force evaluations for each brick shape whose halo
  * fits the LDS budget and keeps the fastest; where the bricks are too few to
  * fill the chip it also tries two and four workgroups per brick, each
  * staging the brick's halo and taking a share of its atoms (results do not
  * depend on it; GEMS_HIP_CHUNKS=1|2|3|4 at context creation fixes the
- * count).  With velocities and a time step
+ * count).  Where rows of atom numbers are in use there is nothing to choose: the
+ * current shape and its time are returned.  With velocities and a time step
  * set, each shape's time is that of a force evaluation plus its rebuild
  * chain times the expected rebuilds per step (2 v_max dt / skin, at most 1).
  * Writes the chosen shape and its time per force evaluation (us); bd_out =
@@ -270,8 +273,9 @@ int gh_get_timing(gh_ctx *ctx, double ms[4], int64_t count[4]);
  * Batched free clusters.  GEMS runs one system per process
  * (src/Program_Types.F90:89-102) and replica exchange as one replica per MPI
  * rank (src/ReplicaExchange.f90:27-151); a batch holds many independent
- * unboxed systems on one device and advances all of them in one launch, one
- * workgroup per system (largest first).  Neighbour lists are the O(N^2)
+ * unboxed systems on one device and advances all of them together (Langevin:
+ * two launches per step over all atoms; FIRE: one launch, a workgroup per
+ * system, largest first).  Neighbour lists are the O(N^2)
  * verlet_self lists of each system (Neighbour.F90:676-759); forces are the
  * SMA-TB passes of TB.F90:367-586; Langevin is ermak_a/ermak_b
  * (Integration.F90:963-1031) with the Philox stream.
@@ -296,7 +300,7 @@ int gh_batch_set_temperatures(gh_batch *b, const double *T);
 /* Forces (ui/A, 3 per atom) and per-system potential energies (eV) of the
  * current positions: one interact() per system.  Either pointer may be NULL. */
 int gh_batch_compute(gh_batch *b, double *F, double *epot);
-/* nsteps Ermak steps (dt ps, gamma 1/ps) of every system in one launch.
+/* nsteps Ermak steps (dt ps, gamma 1/ps) of every system.
  * epot, ekin (eV, per system, after the last step; ekin about the CM) may be
  * NULL. */
 int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t seed,
