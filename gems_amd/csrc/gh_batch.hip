@@ -832,6 +832,7 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   double dt = st.dt, alpha = st.alpha, fnow = sqrt(fm2) * fc.ui_ev;  // eV/A
   int it = st.it, npos = st.npos;
   bool stop = false;
+  st.fmax = fnow;  // (no iterations: of the starting positions)
   for (; it < fc.max_iter; ++it) {
     st.fmax = fnow;
     if (fnow < fc.fstop) {

@@ -1,0 +1,44 @@
+"""FIRE without iterations reports the forces it starts from: max|F| of compute()
+in the same precision (FP64: the same pair terms summed in another order,
+1e-12; mixed: FP32 pair terms, 1e-5 of rms as test_gpu_batch.py, doubled).
+"""
+import numpy as np
+import pytest
+
+from gems_amd import clusters as CL
+from tests import common as cm
+
+pytestmark = pytest.mark.gpu
+hip = pytest.importorskip("gems_amd.hip")
+
+
+def _au(n, seed):
+    x = CL.fcc_sphere(n, 4.078, np.array([0.3, 0.1, -0.2]))
+    return x + np.random.default_rng(seed).normal(0.0, 0.1, x.shape)
+
+
+def _smatb(b):
+    b.set_smatb(1, *cm.matrices(cm.au_params(), 1))
+    b.set_masses([cm.MASS_AU])
+
+
+@pytest.mark.parametrize("prec,tol", [(hip.GH_FP64, 1e-12), (hip.GH_MIXED, 2e-5)],
+                         ids=["fp64", "mixed"])
+def test_fire_without_iterations_reports_its_forces(prec, tol):
+    sizes = [13, 55, 147]
+    off = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    x = np.concatenate([_au(n, n) for n in sizes])
+    with hip.Batch(0, prec) as b:
+        b.set_systems(off, x)
+        _smatb(b)
+        for earlier in (False, True):  # a new batch, and one that holds a quench's figures
+            if earlier:
+                b.fire(max_iter=7)
+            F, ep = b.compute()
+            r = b.fire(max_iter=0)
+            f = np.sqrt((F ** 2).sum(1)) * cm.UI_EV
+            for s in range(len(sizes)):
+                want = f[off[s]:off[s + 1]].max()
+                assert abs(r["fmax"][s] - want) <= tol * want
+            assert np.all(r["iters"] == 0) and np.all(r["converged"] == 0)
+            assert np.allclose(r["epot"], ep, rtol=max(tol, 1e-12), atol=0)
