@@ -1180,11 +1180,13 @@ int gh_set_positions(gh_ctx *c, const double *x) {
 
 int gh_set_velocities(gh_ctx *c, const double *v) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
+  GH_HIP(c, hipSetDevice(c->device));
   return put3(c, c->vel, v);
 }
 
 int gh_set_accelerations(gh_ctx *c, const double *a) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
+  GH_HIP(c, hipSetDevice(c->device));
   return put3(c, c->acc, a);
 }
 
@@ -1209,6 +1211,7 @@ int gh_set_smatb(gh_ctx *c, int nt, const double *A, const double *xi, const dou
       gh_tb_coeffs(t);
       rmax = std::max(rmax, rce[k]);
     }
+  GH_HIP(c, hipSetDevice(c->device));
   c->nt = nt;
   c->pot = GH_POT_SMATB;
   c->rcut = rmax;
@@ -1314,6 +1317,7 @@ int gh_compute(gh_ctx *c, double *F, double *e_atom, double *e_tot) {
 
 int gh_neighbors(gh_ctx *c, int *nn_out, int *idx, int cap) {
   if (!c || !nn_out || !idx || cap <= 0) return gh_fail(c, GH_EINVAL, "gh_neighbors: bad arguments");
+  GH_HIP(c, hipSetDevice(c->device));
   if (!c->ready) GH_TRY(interact(c));
   std::vector<int> orig;
   GH_TRY(fetch_orig(c, orig));
@@ -1382,6 +1386,7 @@ int gh_set_lcg_state(gh_ctx *c, const int state[3]) {
 // set_gdist + set_scal_vel + CM removal (Set_Properties.f90:301-377).
 int gh_set_gdist(gh_ctx *c, double T) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
+  GH_HIP(c, hipSetDevice(c->device));
   const int n = c->n;
   std::vector<double> v(3 * (size_t)n);
   GH_TRY(get_state(c, nullptr, v.data(), nullptr, nullptr, false));
@@ -1694,6 +1699,7 @@ int gh_run(gh_ctx *c, int nsteps, int each, double *energy) {
 
 int gh_energies(gh_ctx *c, double *epot, double *ekin) {
   if (!c) return GH_EINVAL;
+  GH_HIP(c, hipSetDevice(c->device));
   if (c->first_force) GH_TRY(interact(c));
   double ep, ek;
   GH_TRY(gh_launch_energies(c, &ep, &ek));
@@ -1799,6 +1805,7 @@ int gh_lbfgs(gh_ctx *c, int m, double eps, int max_iter, int *iters, double *epo
 
 int gh_get_state(gh_ctx *c, double *x, double *v, double *F, double *e) {
   if (!c || !c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms");
+  GH_HIP(c, hipSetDevice(c->device));
   return get_state(c, x, v, F, e, false);
 }
 

@@ -1503,6 +1503,7 @@ int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t
                       double *epot, double *ekin) {
   if (!b || nsteps < 0 || !(dt > 0) || !(gamma > 0))
     return bfail(b, GH_EINVAL, "langevin needs nsteps >= 0, dt > 0, gamma > 0");
+  BH(b, hipSetDevice(b->device));
   // (cap 0: the skin changed since the rows were sized)
   if (!b->forces_valid || b->cap == 0) BT(gh_batch_compute(b, nullptr, nullptr));
   ErmakC k;
@@ -1566,6 +1567,7 @@ int gh_batch_exchange(gh_batch *b, int nladder, int R, int *sys, int parity, uin
                       int *naccept) {
   if (!b || nladder <= 0 || R < 2 || !sys) return bfail(b, GH_EINVAL, "gh_batch_exchange");
   if ((int)b->epot_h.size() != b->nsys) return bfail(b, GH_ESTATE, "no energies yet");
+  BH(b, hipSetDevice(b->device));
   const double kB = ghc::kB_ui(), ev_ui = ghc::ev_ui();
   std::vector<double> scale(b->nsys, 1.0);
   uint64_t st = seed;
