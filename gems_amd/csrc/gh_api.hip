@@ -1169,13 +1169,18 @@ static int get_state(gh_ctx *c, double *x, double *v, double *F, double *e, bool
   return 0;
 }
 
+// The step whose positions the atoms are at: a run stopped inside a step has
+// moved them to it.  Their displacement since the build is kept under that
+// number's parity.
+static long long atoms_step(const gh_ctx *c) { return c->step + (c->mid_step ? 1 : 0); }
+
 int gh_set_positions(gh_ctx *c, const double *x) {
   if (!c || !x) return gh_fail(c, GH_EINVAL, "gh_set_positions: bad arguments");
   if (!c->have_atoms) return gh_fail(c, GH_ESTATE, "no atoms: call gh_set_atoms first");
   GH_HIP(c, hipSetDevice(c->device));
   const double *src;
   GH_TRY(stage_in(c, x, 3 * (size_t)c->n, &src));
-  return gh_launch_set_positions(c, src);
+  return gh_launch_set_positions(c, src, atoms_step(c));
 }
 
 int gh_set_velocities(gh_ctx *c, const double *v) {
@@ -1292,7 +1297,7 @@ int gh_set_skin(gh_ctx *c, double skin) {
   return 0;
 }
 
-static int interact(gh_ctx *c) {
+static int evaluate(gh_ctx *c) {
   GH_TRY(ensure_ready(c));
   if (c->pos_dirty) {
     GH_TRY(gh_launch_rebuild(c, true, true));
@@ -1303,6 +1308,14 @@ static int interact(gh_ctx *c) {
   GH_TRY(gh_launch_forces(c, nullptr));
   c->first_force = false;
   return 0;
+}
+
+static int interact(gh_ctx *c) {
+  const long long step = c->step;
+  c->step = atoms_step(c);
+  const int rc = evaluate(c);
+  c->step = step;
+  return rc;
 }
 
 int gh_compute(gh_ctx *c, double *F, double *e_atom, double *e_tot) {
@@ -1504,10 +1517,10 @@ struct StepRec {
 static int finish_mid_step(gh_ctx *c) {
   // the stopped step's forces (the list re-sized if needed) and its stepb,
   // under that step's number (its displacement maximum, its random numbers)
+  GH_TRY(interact(c));
+  GH_TRY(check_status(c));
   c->step += 1;
-  int rc = interact(c);
-  if (rc == 0) rc = check_status(c);
-  if (rc == 0) rc = c->integ == GH_INT_ERMAK ? gh_launch_ermak_b(c) : gh_launch_vv_b(c);
+  const int rc = c->integ == GH_INT_ERMAK ? gh_launch_ermak_b(c) : gh_launch_vv_b(c);
   if (rc == 0) c->mid_step = false;
   else c->step -= 1;
   return rc;

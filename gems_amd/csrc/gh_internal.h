@@ -377,7 +377,7 @@ struct FuseErmak {
 
 // launchers (gh_kernels.hip)
 int gh_launch_rebuild(gh_ctx *c, bool force, bool forces_follow);
-int gh_launch_set_positions(gh_ctx *c, const double *x_dev);
+int gh_launch_set_positions(gh_ctx *c, const double *x_dev, long long step);
 int gh_launch_put3(gh_ctx *c, double *dst, const double *in);
 int gh_launch_get(gh_ctx *c, double *x, double *v, double *F, double *e, bool status);
 int gh_launch_epot(gh_ctx *c);

@@ -1396,10 +1396,10 @@ int gh_launch_put3(gh_ctx *c, double *dst, const double *in) {
   return 0;
 }
 
-int gh_launch_set_positions(gh_ctx *c, const double *x_dev) {
+int gh_launch_set_positions(gh_ctx *c, const double *x_dev, long long step) {
   { k_set_positions<<<nblocks(c->n), GH_BLOCK, 0, c->stream>>>(
       c->n, c->ncap, make_wrap(c), c->inv, x_dev, c->pos, c->xold, c->status,
-      c->step); ++c->launches; }
+      step); ++c->launches; }
   GH_HIP(c, hipGetLastError());
   return 0;
 }
