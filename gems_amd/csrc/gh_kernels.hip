@@ -241,6 +241,8 @@ __device__ __forceinline__ void load_shift(ShiftLds &sh, double L0, double L1, d
 // A pair pass over one row, G lanes per atom: f(j, pj, vx, vy, vz) for every
 // listed pair, 64 entries a round; the first round's entries are loaded
 // before the row's length is known.
+// (The passes skip pairs beyond the cut, so that a distance that is not a
+// number reaches the sums.)
 template <int G>
 struct Row {
   static constexpr int U = 64 / G;  // entries of a lane in a round
@@ -710,7 +712,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_row_rho(RowArgs A, N2Build B, TbFo
     if constexpr (MIXED) {
       float band;
       if (tb_rho_fx(P, rd, band)) acc += (double)band;
-    } else if (rd <= P.rce2) {
+    } else if (!(rd > P.rce2)) {
       double dr, ir;
       sqrt_rsq64(rd, dr, ir);
       acc = __dadd_rn(acc, tb_band64(P, dr));
@@ -851,7 +853,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_row_force(RowArgs A, TbForm<MIXED>
       rep = (double)repul;
     } else {
       const TbForm<MIXED> &P = SINGLE ? p1 : sp[ti * GH_MAXT + A.type[j]];
-      if (!(rd <= P.rce2)) return;
+      if (rd > P.rce2) return;
       double dr, ir, factor;
       sqrt_rsq64(rd, dr, ir);
       tb_pair64(P, dr, pi.w + pj.w, factor, rep);
@@ -901,7 +903,7 @@ __global__ __launch_bounds__(GH_BLOCK) void k_row_pair(RowArgs A, const PljDev *
   double f[4] = {0.0, 0.0, 0.0, 0.0};
   row_each<G>(row, A.pos, pi, sh, [&](int j, const double4 &, double vx, double vy, double vz) {
     const double r2 = MIXED ? fma(vx, vx, fma(vy, vy, vz * vz)) : dist2_rn(vx, vy, vz);
-    if (!(r2 <= rc2)) return;
+    if (r2 > rc2) return;
     double p, s;
     if constexpr (TAB) {
       const PljDev &P = pp[ti * GH_MAXT + A.type[j]];
