@@ -64,7 +64,8 @@ __device__ __forceinline__ void n2_book(GhStatus *st, long long step) {  // one 
   st->rebuild = 0;
   st->nupd += 1;
   st->force_rebuild = 0;
-  st->maxnn = (int)(unsigned)st->maxnn_tag;
+  // (a build whose rows are all empty has left the tag of an earlier one)
+  st->maxnn = (st->maxnn_tag >> 32) == (unsigned long long)st->nupd ? (int)(unsigned)st->maxnn_tag : 0;
   disp2_clear(st, step);
 }
 __global__ void k_n2_book(GhStatus *st, long long step) { n2_book(st, step); }
