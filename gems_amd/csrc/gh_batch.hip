@@ -55,7 +55,8 @@ struct gh_batch {
   std::vector<int> off_h, order_h;
   std::vector<double> T_h, epot_h;
   // device
-  int *off = nullptr, *order = nullptr, *type = nullptr, *nn = nullptr, *flags = nullptr;
+  int *off = nullptr, *order = nullptr, *type = nullptr, *flags = nullptr;
+  unsigned *nn = nullptr;
   int *sysof = nullptr, *a0of = nullptr;   // each atom's system and that system's first atom
   GhLine *dmax = nullptr;                  // [2][nsys] largest |x - x_old|^2, by step parity
   double4 *pos = nullptr, *pos_next = nullptr;  // x, y, z, type
@@ -86,7 +87,7 @@ struct BatchArgs {
   int nsys, ntot;
   double4 *pos, *pos_next, *pk;
   double *vel, *acc, *frc, *e, *rho, *xold;
-  int *nn;    // row lengths: pairs at the front | pairs at the back << 16
+  unsigned *nn;  // row lengths: pairs at the front | pairs at the back << 16
   unsigned short *list;
   int cap, ld;
   const TbDev *tbd;
@@ -206,7 +207,7 @@ __device__ __forceinline__ void batch_row(const BatchArgs &B, bool on, int a0, i
       atomicMax(&B.flags[1], m0 + m1);
     }
     const int f = min(m0, cap);
-    B.nn[i] = f | (min(m1, cap - f) << 16);
+    B.nn[i] = (unsigned)f | ((unsigned)min(m1, cap - f) << 16);
   }
   if (sub < 3) B.xold[sub * B.ld + i] = sub == 0 ? pi.x : sub == 1 ? pi.y : pi.z;
 }
@@ -225,9 +226,9 @@ template <int G>
 __device__ __forceinline__ RowHead<G> row_head(const BatchArgs &B, int i, bool on) {
   RowHead<G> r;
   r.row = B.list + (size_t)i * B.cap;
-  const int w = on ? B.nn[i] : 0;
-  r.m0 = w & 0xFFFF;
-  r.m1 = w >> 16;
+  const unsigned w = on ? B.nn[i] : 0u;
+  r.m0 = (int)(w & 0xFFFFu);
+  r.m1 = (int)(w >> 16);
   if constexpr (G >= 8) {
     const int sub = threadIdx.x & (G - 1);
 #pragma unroll

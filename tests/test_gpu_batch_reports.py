@@ -1,4 +1,7 @@
-"""FIRE without iterations reports the forces it starts from: max|F| of compute()
+"""What a batch reports where there is nothing to iterate, little to pair and
+much to list.
+
+FIRE without iterations reports the forces it starts from: max|F| of compute()
 in the same precision (FP64: the same pair terms summed in another order,
 1e-12; mixed: FP32 pair terms, 1e-5 of rms as test_gpu_batch.py, doubled).
 """
@@ -42,3 +45,20 @@ def test_fire_without_iterations_reports_its_forces(prec, tol):
                 assert abs(r["fmax"][s] - want) <= tol * want
             assert np.all(r["iters"] == 0) and np.all(r["converged"] == 0)
             assert np.allclose(r["epot"], ep, rtol=max(tol, 1e-12), atol=0)
+
+
+def test_rows_longer_than_32767_pairs():
+    # a skin that lists every pair of 36,000 atoms (the pairs outside the inner
+    # bound number more than 15 bits); the same pairs are within the cut as with
+    # the usual skin: ~45 terms of a few rms(F) at 2^-53 each in another order
+    x = _au(36000, 5)
+    res = []
+    for skin in (1.0, 150.0):
+        with hip.Batch(0, hip.GH_FP64) as b:
+            b.set_skin(skin)
+            b.set_systems(np.array([0, len(x)], np.int32), x)
+            _smatb(b)
+            res.append(b.compute())
+    (F0, e0), (F1, e1) = res
+    assert cm.force_err(F1, F0) <= 1e-12
+    assert abs(e1[0] - e0[0]) <= 1e-12 * abs(e0[0])
