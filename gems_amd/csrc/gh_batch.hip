@@ -43,6 +43,7 @@ struct gh_batch {
   std::string err;
   int nsys = 0, ntot = 0, ld = 0;
   int nt = 1;
+  int types = 1;  // one past the largest type of an atom
   double mass_t[GH_MAXT] = {1, 1, 1, 1, 1, 1, 1, 1};
   GhTbPair tb[GH_MAXT * GH_MAXT];
   bool have_pot = false;
@@ -1082,7 +1083,7 @@ static BatchArgs bargs(const gh_batch *b) {
   A.tbd = b->tbd;
   A.tbf = b->tbf;
   A.e0 = b->tb_e0;
-  A.nt = b->nt;
+  A.nt = std::max(b->nt, b->types);  // (entries past the potential's are zero: no interaction)
   A.nst = b->nst;
   A.dmax = b->dmax;
   for (int t = 0; t < GH_MAXT; ++t) {
@@ -1364,6 +1365,7 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
     hp[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], (double)ht[i]);
     if (ht[i] < 0 || ht[i] >= GH_MAXT) return bfail(b, GH_EINVAL, "type out of range");
   }
+  b->types = 1 + *std::max_element(ht.begin(), ht.end());
   std::vector<int> hs(ld, nsys - 1), ha(ld, off[nsys - 1]);
   for (int k = 0; k < nsys; ++k) {
     std::fill(hs.begin() + off[k], hs.begin() + off[k + 1], k);

@@ -62,3 +62,36 @@ def test_rows_longer_than_32767_pairs():
     (F0, e0), (F1, e1) = res
     assert cm.force_err(F1, F0) <= 1e-12
     assert abs(e1[0] - e0[0]) <= 1e-12 * abs(e0[0])
+
+
+@pytest.mark.parametrize("prec", [hip.GH_FP64, hip.GH_MIXED], ids=["fp64", "mixed"])
+def test_types_without_parameters_do_not_interact(prec):
+    # an atom whose type the potential has no parameters for: no force on it and
+    # none from it, whatever the tables in LDS held before
+    rng = np.random.default_rng(2)
+    off, x, t = np.array([0, 38, 93], np.int32), np.concatenate([_au(38, 1), _au(55, 2)]), \
+        (rng.random(93) < 0.5).astype(np.int32)
+    t[[5, 60]] = 3
+    keep = t != 3
+    many = np.arange(400, dtype=np.int32)
+    with hip.Batch(0, prec) as b:  # every entry of the tables filled, on every CU
+        b.set_systems(np.concatenate([many, [400]]) * 55, np.tile(_au(55, 2), (400, 1)),
+                      np.tile(np.arange(55, dtype=np.int32) % 8, 400))
+        b.set_smatb(8, *[m[0, 0] for m in CL.agcu_params()])
+        b.set_masses([100.0] * 8)
+        b.fire(max_iter=1)
+        b.compute()
+    res = []
+    for sel in (np.ones(93, bool), keep):
+        with hip.Batch(0, prec) as b:
+            b.set_systems(np.array([0, sel[:38].sum(), sel.sum()], np.int32), x[sel], t[sel])
+            b.set_smatb(2, *CL.agcu_params())
+            b.set_masses([CL.MASS_AG, CL.MASS_CU])
+            F, ep = b.compute()
+            r = b.fire(max_iter=0)
+            res.append((F, ep, r["epot"]))
+    (F, ep, er), (Fk, epk, erk) = res
+    tol = 1e-12 if prec == hip.GH_FP64 else 2e-5
+    assert np.all(F[~keep] == 0.0)
+    assert cm.force_err(F[keep], Fk) <= tol
+    assert np.allclose(ep, epk, rtol=tol, atol=0) and np.allclose(er, erk, rtol=tol, atol=0)
