@@ -1015,6 +1015,35 @@ int gh_set_atoms(gh_ctx *c, int n, const double *x, const int *type) {
   if (n > (int)GH_JMASK_HOST) return gh_fail(c, GH_EINVAL, "too many atoms (max 134217727)");
   GH_HIP(c, hipSetDevice(c->device));
   const int ncap = roundup(n, 256);
+  // (a refused call leaves the context's atoms as they are)
+  std::vector<double4> hp(ncap);
+  std::vector<int> types(n, 0);
+  std::vector<int> ho(ncap), ht(ncap, 0);
+  for (int i = 0; i < ncap; ++i) {
+    if (i < n) {
+      double v[3];
+      for (int d = 0; d < 3; ++d) {
+        v[d] = x[3 * i + d];
+        // do_pbc_1 (Set_Properties.f90:444-470): periodic axes start wrapped
+        if (c->boxed && c->pbc[d]) {
+          if (v[d] >= c->L[d]) v[d] -= c->L[d];
+          else if (v[d] < 0.0) v[d] += c->L[d];
+          if (v[d] < 0.0 || v[d] >= c->L[d])
+            return gh_fail(c, GH_EINVAL, "atom more than one box length outside a periodic box");
+        }
+      }
+      hp[i] = make_double4(v[0], v[1], v[2], 0.0);
+      int t = type ? type[i] : 0;
+      if (t < 0 || t >= GH_MAXT) return gh_fail(c, GH_EINVAL, "atom type out of range 0..7");
+      ht[i] = t;
+      types[i] = t;
+    } else {
+      hp[i] = make_double4(0, 0, 0, 0);
+    }
+    ho[i] = i;
+  }
+  c->type_h.swap(types);
+  c->n = n;
   c->masked = false;  // new atoms: masks, if any, are set again after this call
   if (ncap != c->ncap) {
     c->ncap = ncap;
@@ -1056,33 +1085,6 @@ int gh_set_atoms(gh_ctx *c, int n, const double *x, const int *type) {
       c->list = nullptr;
     }
     c->cap = 0;
-  }
-  c->n = n;
-  std::vector<double4> hp(ncap);
-  c->type_h.assign(n, 0);
-  std::vector<int> ho(ncap), ht(ncap, 0);
-  for (int i = 0; i < ncap; ++i) {
-    if (i < n) {
-      double v[3];
-      for (int d = 0; d < 3; ++d) {
-        v[d] = x[3 * i + d];
-        // do_pbc_1 (Set_Properties.f90:444-470): periodic axes start wrapped
-        if (c->boxed && c->pbc[d]) {
-          if (v[d] >= c->L[d]) v[d] -= c->L[d];
-          else if (v[d] < 0.0) v[d] += c->L[d];
-          if (v[d] < 0.0 || v[d] >= c->L[d])
-            return gh_fail(c, GH_EINVAL, "atom more than one box length outside a periodic box");
-        }
-      }
-      hp[i] = make_double4(v[0], v[1], v[2], 0.0);
-      int t = type ? type[i] : 0;
-      if (t < 0 || t >= GH_MAXT) return gh_fail(c, GH_EINVAL, "atom type out of range 0..7");
-      ht[i] = t;
-      c->type_h[i] = t;
-    } else {
-      hp[i] = make_double4(0, 0, 0, 0);
-    }
-    ho[i] = i;
   }
   // uploads and clears ordered on the context's stream, then drained (the host
   // vectors die on return)

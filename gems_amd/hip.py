@@ -192,9 +192,9 @@ class Context:
 
     def set_atoms(self, x, types=None):
         x = np.ascontiguousarray(x, np.float64)
-        self.n = x.shape[0]
         t = None if types is None else np.ascontiguousarray(types, np.int32)
-        self._ck(self.L.gh_set_atoms(self.h, self.n, _p(x), _p(t, _ip)))
+        self._ck(self.L.gh_set_atoms(self.h, x.shape[0], _p(x), _p(t, _ip)))
+        self.n = x.shape[0]
 
     def set_masses(self, masses):
         m = np.ascontiguousarray(np.atleast_1d(masses), np.float64)

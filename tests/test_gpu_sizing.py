@@ -24,3 +24,28 @@ def test_longest_row_of_atoms_without_neighbours(pot):
             nn, _ = c.neighbors(cap=256)
             assert c.stats()["maxnn"] == nn.max()
             assert (nn.max() == 0) == (len(y) < 3)
+
+
+@pytest.mark.parametrize("n", [100, 2000])
+@pytest.mark.parametrize("why", ["type", "position"])
+def test_refused_atoms_leave_the_context_as_it_was(n, why):
+    rng = np.random.default_rng(n)
+    x = np.mod(cm.fcc(6, 4.078) + rng.normal(0.0, 0.05, (864, 3)), 6 * 4.078)
+    v = rng.normal(0.0, 1.0, x.shape)
+    with hip.Context(0, hip.GH_FP64) as c:
+        c.set_box([6 * 4.078] * 3, (1, 1, 1))
+        c.set_atoms(x)
+        c.set_masses([cm.MASS_AU])
+        c.set_smatb(1, *cm.matrices(cm.au_params(), 1))
+        c.set_velocities(v)
+        F, e, et = c.compute()
+        y, t = rng.uniform(0.0, 20.0, (n, 3)), np.zeros(n, np.int32)
+        if why == "type":
+            t[n - 1] = 8
+        else:
+            y[n - 1, 2] = 100.0
+        with pytest.raises(hip.GhError):
+            c.set_atoms(y, t)
+        for a, b in zip(c.state(), (x, v, F, e)):
+            assert np.array_equal(a, b)
+        assert c.compute()[2] == et
