@@ -1317,6 +1317,9 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
     const int n = off[s + 1] - off[s];
     if (n < 1 || n > 65535) return bfail(b, GH_EINVAL, "systems need 1..65535 atoms");
   }
+  // (a refused call leaves the batch's systems as they are)
+  for (int i = 0; type && i < off[nsys]; ++i)
+    if (type[i] < 0 || type[i] >= GH_MAXT) return bfail(b, GH_EINVAL, "type out of range");
   BH(b, hipSetDevice(b->device));
   b->nsys = nsys;
   b->ntot = off[nsys];
@@ -1363,7 +1366,6 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
   for (int i = 0; i < b->ntot; ++i) {
     ht[i] = type ? type[i] : 0;
     hp[i] = make_double4(x[3 * i], x[3 * i + 1], x[3 * i + 2], (double)ht[i]);
-    if (ht[i] < 0 || ht[i] >= GH_MAXT) return bfail(b, GH_EINVAL, "type out of range");
   }
   b->types = 1 + *std::max_element(ht.begin(), ht.end());
   std::vector<int> hs(ld, nsys - 1), ha(ld, off[nsys - 1]);

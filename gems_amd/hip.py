@@ -386,12 +386,12 @@ class Batch:
     def set_systems(self, off, x, types=None):
         off = np.ascontiguousarray(off, np.int32)
         x = np.ascontiguousarray(x, np.float64)
+        t = None if types is None else np.ascontiguousarray(types, np.int32)
+        self._ck(self.L.gh_batch_set_systems(self.h, len(off) - 1, _p(off, _ip), _p(x),
+                                             _p(t, _ip)))
         self.nsys = len(off) - 1
         self.ntot = int(off[-1])
         self.off = off
-        t = None if types is None else np.ascontiguousarray(types, np.int32)
-        self._ck(self.L.gh_batch_set_systems(self.h, self.nsys, _p(off, _ip), _p(x),
-                                             _p(t, _ip)))
 
     def set_smatb(self, nt, A, xi, p, q, r0, rci, rce):
         arrs = [np.ascontiguousarray(np.broadcast_to(np.asarray(a, np.float64), (nt, nt)))

@@ -95,3 +95,27 @@ def test_types_without_parameters_do_not_interact(prec):
     assert np.all(F[~keep] == 0.0)
     assert cm.force_err(F[keep], Fk) <= tol
     assert np.allclose(ep, epk, rtol=tol, atol=0) and np.allclose(er, erk, rtol=tol, atol=0)
+
+
+@pytest.mark.parametrize("sizes", [[5], [40, 30, 20, 300]])
+@pytest.mark.parametrize("why", ["type", "size", "first"])
+def test_refused_systems_leave_the_batch_as_it_was(sizes, why):
+    off = np.array([0, 13, 68], np.int32)
+    x = np.concatenate([_au(13, 1), _au(55, 2)])
+    new = np.concatenate([[0], np.cumsum(sizes)]).astype(np.int32)
+    t = np.zeros(new[-1], np.int32)
+    if why == "type":
+        t[-1] = 8
+    elif why == "size":
+        new = np.concatenate([new, new[-1:]])  # a system without atoms
+    else:
+        new[0] = 1
+    with hip.Batch(0, hip.GH_FP64) as b:
+        b.set_systems(off, x)
+        _smatb(b)
+        F, ep = b.compute()
+        with pytest.raises(hip.GhError):
+            b.set_systems(new, np.zeros((len(t), 3)), t)
+        assert np.array_equal(b.state()[0], x)
+        F2, ep2 = b.compute()
+        assert np.array_equal(F, F2) and np.array_equal(ep, ep2)
