@@ -1103,6 +1103,7 @@ int gh_set_atoms(gh_ctx *c, int n, const double *x, const int *type) {
   c->ready = false;
   c->pos_dirty = true;
   c->first_force = true;
+  c->mid_step = false;  // (a stopped step was of the atoms before)
   return 0;
 }
 

@@ -67,3 +67,25 @@ def test_corrected_positions_after_a_stop(prec, tol, after, then):
     with _ctx(prec, y2, L) as c:
         F0 = c.compute()[0]
     assert cm.force_err(F, F0) <= tol
+
+
+def test_new_atoms_after_a_stop_start_a_step_of_their_own():
+    x = cm.fcc(8, A) + np.random.default_rng(4).normal(0.0, 0.05, (2048, 3))
+    L = np.array([8 * A] * 3)
+    x = np.clip(x, 0.0, L - 1e-9)
+    v = np.random.default_rng(5).normal(0.0, 1.0, x.shape)
+    rows = []
+    for stop in (True, False):
+        with _ctx(hip.GH_FP64, x, L) as c:
+            c.integrator_vv(0.002)
+            if stop:
+                w = v.copy()
+                w[int(np.argmax(x[:, 2])), 2] = 5000.0
+                c.set_velocities(w)
+                with pytest.raises(hip.GhError):
+                    c.run(3)
+                c.set_atoms(x)
+            c.set_velocities(v)
+            rows.append((c.run(4, 1),) + c.state()[:2])
+    for a, b in zip(*rows):
+        assert np.array_equal(a, b)
