@@ -868,7 +868,8 @@ int gh_autotune(gh_ctx *c, int reps, int *bd_out, double *us_out) {
   hipEvent_t e0, e1;
   GH_HIP(c, hipEventCreate(&e0));
   GH_HIP(c, hipEventCreate(&e1));
-  int best[3] = {0, 0, 0}, best_pick = 0, best_chunks = 1;
+  // (kept where no shape could be timed: the automatic choices)
+  int best[3] = {0, 0, 0}, best_pick = 0, best_chunks = c->chunks_env;
   double best_us = 1e30, best_score = 1e30;
   for (int bz = 1; bz <= 4; ++bz)
     for (int by = bz; by <= 4; ++by)

@@ -49,3 +49,21 @@ def test_refused_atoms_leave_the_context_as_it_was(n, why):
         for a, b in zip(c.state(), (x, v, F, e)):
             assert np.array_equal(a, b)
         assert c.compute()[2] == et
+
+
+def test_autotune_without_candidates_keeps_the_automatic_choice():
+    # cells so full that no brick of four of them fits the LDS: nothing to time
+    a = (4.0 / 0.8442) ** (1.0 / 3.0)
+    x = cm.fcc(11, a)
+    with hip.Context(0, hip.GH_MIXED) as c:
+        c.set_box([11 * a] * 3, (1, 1, 1))
+        c.set_atoms(x)
+        c.set_masses([1.0])
+        c.set_lj(1.0, 1.0, 4.2)
+        c.set_skin(0.4)
+        F, _, _ = c.compute()
+        before = c.stats()
+        assert before["list_mode"] == 1 and before["chunks"] > 1
+        c.autotune(reps=1)
+        assert c.stats()["chunks"] == before["chunks"]
+        assert cm.force_err(c.compute()[0], F) <= 1e-5
