@@ -62,6 +62,12 @@ __device__ __forceinline__ void fold_disp2(GhStatus *st, double d2, long long st
   atomicMax(&st->maxdisp2[step & 1][blockIdx.x % GH_DISP_SLOTS].bits, b);
 }
 
+// The carry of fold_disp2 by a first workgroup that leaves without atoms.
+__device__ __forceinline__ void carry_disp2(GhStatus *st, long long step) {
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    atomicMax(&st->maxdisp2[step & 1][0].bits, disp2_max(st, step - 1));
+}
+
 // Stops the run at `step` (the first raiser wins and records the step):
 // every kernel that changes the atoms' state returns at once while
 // st->halt is set, so the state stays the one the step started from.

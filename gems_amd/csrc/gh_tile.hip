@@ -1526,7 +1526,10 @@ __device__ __forceinline__ void tb_force_fx_body(
   int kc;  // this workgroup's share of the brick's atoms
   const int b = pass_brick(t, kc);
   if (b >= t.nbrick) return;
-  if (!halo_setup(t, b, cell_start, H, st, true, step)) return;
+  if (!halo_setup(t, b, cell_start, H, st, true, step)) {
+    if (FUSED) carry_disp2(st, step + 1);
+    return;
+  }
   const int ns = t.slot_cap + 1;  // slots + the sentinel
   unsigned char *scell = reinterpret_cast<unsigned char *>(q4 + (S > 0 ? S : ns));
   unsigned char *ty = scell + (S > 0 ? S : ns);
@@ -1699,7 +1702,10 @@ __device__ __forceinline__ void tb_force64_body(
   int kc;  // this workgroup's share of the brick's atoms
   const int b = pass_brick(t, kc);
   if (b >= t.nbrick) return;
-  if (!halo_setup(t, b, cell_start, H, st, true, step)) return;
+  if (!halo_setup(t, b, cell_start, H, st, true, step)) {
+    if (FUSED) carry_disp2(st, step + 1);
+    return;
+  }
   const int cap = t.slot_cap + 1;  // slots + the sentinel
   double *px = dyn, *py = dyn + cap, *pz = dyn + 2 * cap, *eb = dyn + 3 * cap;
   int *ty = reinterpret_cast<int *>(dyn + 4 * cap);
@@ -1794,7 +1800,10 @@ __device__ __forceinline__ void lj_tiled_body(
   int kc;  // this workgroup's share of the brick's atoms
   const int b = pass_brick(t, kc);
   if (b >= t.nbrick) return;
-  if (!halo_setup(t, b, cell_start, H, st, true, step)) return;
+  if (!halo_setup(t, b, cell_start, H, st, true, step)) {
+    if (FUSED) carry_disp2(st, step + 1);
+    return;
+  }
   const int cap = t.slot_cap + 1;  // slots + the sentinel
   double *px = dyn, *py = dyn + cap, *pz = dyn + 2 * cap;
   unsigned char *scell = reinterpret_cast<unsigned char *>(dyn + 3 * cap);
@@ -1941,7 +1950,10 @@ __global__ __launch_bounds__(GH_TBMAX) void k_lj_fx(
   int kc;  // this workgroup's share of the brick's atoms
   const int b = pass_brick(t, kc);
   if (b >= t.nbrick) return;
-  if (!halo_setup(t, b, cell_start, H, st, true, sa.step)) return;
+  if (!halo_setup(t, b, cell_start, H, st, true, sa.step)) {
+    if (FUSED) carry_disp2(st, sa.step + 1);
+    return;
+  }
   const int ns = t.slot_cap + 1;  // slots + the sentinel
   unsigned char *scell = reinterpret_cast<unsigned char *>(lq4 + ns);
   slot_map(H, scell);
