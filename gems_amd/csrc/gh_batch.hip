@@ -96,6 +96,9 @@ struct BatchArgs {
   int nt;
   double om[GH_MAXT], osm[GH_MAXT];
   double rl2, near2;  // build: list cut, inner-branch bound
+  // the same in steps of 2^-GH_BFXK A, squared: surely outside the cut above
+  // hi2q, surely inside below lo2q; within band2q of near2q neither side is sure
+  float hi2q, lo2q, near2q, band2q;
   int nst;            // LDS staging slots (largest system + sentinel); 0 = none
   double ev_ui;
   const double *T;
@@ -158,19 +161,35 @@ __device__ __forceinline__ void bred(BlockRed<BS> &R, double (&v)[3], double &m)
   __syncthreads();
 }
 
-// Lane groups of G = 16 or 4: the group's bits of a wave mask, and sums over
-// a group in every lane of it.
+// Lane groups of G = 16, 8, 4 or 1: the group's bits of a wave mask, and sums
+// over a group in every lane of it.
 template <int G>
 __device__ __forceinline__ unsigned group_bits(unsigned long long m) {
   return (unsigned)(m >> (threadIdx.x & 63 & ~(G - 1))) & ((1u << G) - 1);
 }
 template <int G>
 __device__ __forceinline__ double group_total(double v) {
-  v += dpp64<0xB1>(v);  // quad_perm [1,0,3,2]
-  v += dpp64<0x4E>(v);  // quad_perm [2,3,0,1]
+  if (G >= 4) v += dpp64<0xB1>(v);    // quad_perm [1,0,3,2]
+  if (G >= 4) v += dpp64<0x4E>(v);    // quad_perm [2,3,0,1]
   if (G >= 8) v += dpp64<0x141>(v);   // row_half_mirror
   if (G == 16) v += dpp64<0x140>(v);  // row_mirror
   return v;
+}
+
+// A row's lengths and its atom's build position, by the row's 16 lanes.
+__device__ __forceinline__ void row_end(const BatchArgs &B, bool on, int i, int m0, int m1,
+                                        const double4 &pi) {
+  const int sub = threadIdx.x & 15, cap = B.cap;
+  if (!on) return;
+  if (sub == 0) {
+    if (m0 + m1 > cap) {
+      B.flags[0] = 1;
+      atomicMax(&B.flags[1], m0 + m1);
+    }
+    const int f = min(m0, cap);
+    B.nn[i] = (unsigned)f | ((unsigned)min(m1, cap - f) << 16);
+  }
+  if (sub < 3) B.xold[sub * B.ld + i] = sub == 0 ? pi.x : sub == 1 ? pi.y : pi.z;
 }
 
 // The row of atom k of a system (verlet_self, Neighbour.F90:676-759: all
@@ -201,16 +220,7 @@ __device__ __forceinline__ void batch_row(const BatchArgs &B, bool on, int a0, i
       m1 += __popc(b1);
     }
   }
-  if (!on) return;
-  if (sub == 0) {
-    if (m0 + m1 > cap) {
-      B.flags[0] = 1;
-      atomicMax(&B.flags[1], m0 + m1);
-    }
-    const int f = min(m0, cap);
-    B.nn[i] = (unsigned)f | ((unsigned)min(m1, cap - f) << 16);
-  }
-  if (sub < 3) B.xold[sub * B.ld + i] = sub == 0 ? pi.x : sub == 1 ? pi.y : pi.z;
+  row_end(B, on, i, m0, m1, pi);
 }
 
 // The row of atom i: its ends and, for 16 and 8 lanes, the first 16 pairs of
@@ -219,7 +229,7 @@ __device__ __forceinline__ void batch_row(const BatchArgs &B, bool on, int a0, i
 // together with the atom's own data.
 template <int G>
 struct RowHead {
-  static constexpr int NF = 16 / G, NB = 48 / G;  // entries of a lane
+  static constexpr int NF = G >= 8 ? 16 / G : 0, NB = G >= 8 ? 48 / G : 0;  // entries of a lane
   const unsigned short *row;
   int m0, m1, s[G >= 8 ? NF + NB : 1];
 };
@@ -241,9 +251,9 @@ __device__ __forceinline__ RowHead<G> row_head(const BatchArgs &B, int i, bool o
 }
 // Runs f(u) for every pair of a row after load(u, s), s the neighbour's index
 // in the system, four payloads in flight.  16 and 8 lanes: lane sub takes
-// entries sub, sub + G, ... of the front, then of the back.  4 lanes: lane sub
-// takes the quads sub, sub + 4, ... (one 8-byte load each, the next one in
-// flight while one is used).
+// entries sub, sub + G, ... of the front, then of the back.  4 lanes and one:
+// lane sub takes the quads sub, sub + G, ... (one 8-byte load each, the next one
+// in flight while one is used).
 template <int G, class LOAD, class F>
 __device__ __forceinline__ void batch_each(const BatchArgs &B, const RowHead<G> &r, LOAD &&load,
                                            F &&f) {
@@ -277,15 +287,16 @@ __device__ __forceinline__ void batch_each(const BatchArgs &B, const RowHead<G> 
     run(sub + 16, r.m0, r.row, 1);
     run(sub + 48, r.m1, r.row + (B.cap - 1), -1);
   } else {
-    static_assert(G == 4, "16, 8 or 4 lanes per atom");
-    // virtual quads: the front's, padded to whole rounds of the four lanes,
-    // then the back's
+    static_assert(G == 4 || G == 1, "16, 8, 4 lanes per atom or one");
+    // virtual quads: the front's, padded to whole rounds of the lanes, then the
+    // back's
     const unsigned long long *qf = reinterpret_cast<const unsigned long long *>(r.row);
-    const int nf = ((r.m0 + 15) >> 4) << 2, nq = nf + ((r.m1 + 3) >> 2), last = (B.cap >> 2) - 1;
+    const int nf = (r.m0 + 4 * G - 1) / (4 * G) * G, nq = nf + ((r.m1 + 3) >> 2),
+              last = (B.cap >> 2) - 1;
     auto quad = [&](int v) { return v < nf ? qf[min(v, last)] : qf[max(last - (v - nf), 0)]; };
     unsigned long long w = nq > 0 ? quad(sub) : 0ull;
-    for (int v = sub; v < nq; v += 4) {
-      const unsigned long long nw = quad(min(v + 4, nq));
+    for (int v = sub; v < nq; v += G) {
+      const unsigned long long nw = quad(min(v + G, nq));
       const bool front = v < nf;
       const int k0 = 4 * (front ? v : v - nf), m = front ? r.m0 : r.m1;
 #pragma unroll
@@ -636,13 +647,6 @@ struct FireState {  // between the launches, per system
   int npos, it, done, conv;
 };
 
-// The rows of the system's atoms; ends with a barrier.
-__device__ void sys_build(const BatchArgs &B, int a0, int n) {
-  const int per = (int)blockDim.x >> 4, g = (int)threadIdx.x >> 4;
-  for (int k0 = 0; k0 < n; k0 += per) batch_row(B, k0 + g < n, a0, n, min(k0 + g, n - 1));
-  __syncthreads();
-}
-
 #define GH_FG 4  // lanes per atom
 // LDS staging of a mixed system: positions in steps of 2^-GH_BFXK A about its
 // first atom with eband32 as the fourth word, and types; `far`: an atom lies
@@ -660,26 +664,82 @@ __device__ __forceinline__ void stage_atom(const Stage &S, int k, const double (
   S.q[k] = make_int4(__double2int_rn(dx), __double2int_rn(dy), __double2int_rn(dz), 0);
 }
 
-template <bool MIXED, bool QUANT, bool SINGLE>
+// The row of atom k as batch_row builds it, entry for entry, from the staged
+// positions: FP32 decides all pairs but those near a bound, which the FP64 rd
+// decides (150 systems of 2,000 atoms, 50 Langevin steps: 8.6 -> 8.3 ms).
+__device__ __forceinline__ void batch_row_staged(const BatchArgs &B, const Stage &S, bool on,
+                                                 int a0, int n, int k) {
+  const int sub = threadIdx.x & 15, i = a0 + k, cap = B.cap;
+  const unsigned below = (1u << sub) - 1;
+  const double4 pi = B.pos[i];
+  const int4 qi = S.q[k];
+  unsigned short *row = B.list + (size_t)i * cap;
+  int m0 = 0, m1 = 0;
+  for (int j0 = 0; __any(on && j0 < n); j0 += 64) {
+    int4 q[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) q[u] = S.q[min(j0 + 16 * u + sub, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int j = j0 + 16 * u + sub;
+      const float ux = (float)(int)((unsigned)q[u].x - (unsigned)qi.x),
+                  uy = (float)(int)((unsigned)q[u].y - (unsigned)qi.y),
+                  uz = (float)(int)((unsigned)q[u].z - (unsigned)qi.z);
+      const float r2 = fmaf(ux, ux, fmaf(uy, uy, uz * uz));
+      bool keep = on && j < n && j != k && r2 <= B.hi2q, near = r2 < B.near2q;
+      if (keep && (r2 >= B.lo2q || fabsf(r2 - B.near2q) <= B.band2q)) {
+        const double4 p = B.pos[a0 + j];
+        const double rd = dist2_rn(p.x - pi.x, p.y - pi.y, p.z - pi.z);
+        keep = rd <= B.rl2;
+        near = rd < B.near2;
+      }
+      const unsigned long long kept = __ballot(keep);
+      if (kept == 0ull) continue;
+      const unsigned b0 = group_bits<16>(kept & __ballot(near));
+      const unsigned b1 = group_bits<16>(kept & ~__ballot(near));
+      const int d = near ? m0 + __popc(b0 & below) : cap - 1 - (m1 + __popc(b1 & below));
+      if (keep && d >= 0 && d < cap) row[d] = (unsigned short)j;
+      m0 += __popc(b0);
+      m1 += __popc(b1);
+    }
+  }
+  row_end(B, on, i, m0, m1, pi);
+}
+
+// The rows of the system's atoms; ends with a barrier.
+template <bool QUANT>
+__device__ void sys_build(const BatchArgs &B, const Stage &S, int a0, int n) {
+  const int per = (int)blockDim.x >> 4, g = (int)threadIdx.x >> 4;
+  const bool lds = QUANT && !*S.far;
+  for (int k0 = 0; k0 < n; k0 += per) {
+    const bool on = k0 + g < n;
+    const int k = min(k0 + g, n - 1);
+    if (lds) batch_row_staged(B, S, on, a0, n, k);
+    else batch_row(B, on, a0, n, k);
+  }
+  __syncthreads();
+}
+
+template <bool MIXED, bool QUANT, bool SINGLE, int G>
 __device__ __forceinline__ void fire_rho(const BatchArgs &B, const Stage &S,
                                          const BTable<MIXED, SINGLE> &T, const BForm<MIXED> &p1,
                                          int a0, int n) {
-  const int sub = threadIdx.x & (GH_FG - 1), g = (int)threadIdx.x / GH_FG;
-  const int per = (int)blockDim.x / GH_FG;
+  const int sub = threadIdx.x & (G - 1), g = (int)threadIdx.x / G;
+  const int per = (int)blockDim.x / G;
   const bool lds = QUANT && !*S.far;
   for (int k0 = 0; k0 < n; k0 += per) {
     const bool on = k0 + g < n;
     const int k = min(k0 + g, n - 1), i = a0 + k;
-    const RowHead<GH_FG> row = row_head<GH_FG>(B, i, on);
+    const RowHead<G> row = row_head<G>(B, i, on);
     if (!lds) {
-      batch_rho<MIXED, QUANT, SINGLE, GH_FG>(B, T, p1, a0, i, on, row);
+      batch_rho<MIXED, QUANT, SINGLE, G>(B, T, p1, a0, i, on, row);
     } else if constexpr (QUANT) {
       const int4 qi = S.q[k];
       const int ti = SINGLE ? 0 : S.ty[k];
       double acc = 0.0;
       int4 q[4];
       int t[4];
-      batch_each<GH_FG>(
+      batch_each<G>(
           B, row,
           [&](int u, int s) {
             q[u] = S.q[s];
@@ -692,7 +752,7 @@ __device__ __forceinline__ void fire_rho(const BatchArgs &B, const Stage &S,
                           fma(dx, dx, fma(dy, dy, dz * dz)), band))
               acc += (double)band;
           });
-      acc = group_total<GH_FG>(acc);
+      acc = group_total<G>(acc);
       if (on && sub == 0) {
         B.rho[i] = acc;
         S.q[k].w = __float_as_int((float)(1.0 / sqrt(acc) - B.e0));
@@ -708,30 +768,30 @@ __device__ __forceinline__ void fire_rho(const BatchArgs &B, const Stage &S,
 // part of the force anyway, a pass of its own for them costs registers: 12.1 ms
 // against 13.9).  hdt > 0: then the second half kick (v += hdt F / m) and the sums pv = {F.v, |v|^2, |F|^2} of
 // the thread's atoms.  fm2: the largest |F|^2 of its atoms.
-template <bool MIXED, bool QUANT, bool SINGLE, int WHAT>
+template <bool MIXED, bool QUANT, bool SINGLE, int WHAT, int G>
 __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
                                            const BTable<MIXED, SINGLE> &T, const BForm<MIXED> &p1,
                                            int a0, int n, double hdt, double (&pv)[3],
                                            double &fm2) {
-  const int sub = threadIdx.x & (GH_FG - 1), g = (int)threadIdx.x / GH_FG;
-  const int per = (int)blockDim.x / GH_FG;
+  const int sub = threadIdx.x & (G - 1), g = (int)threadIdx.x / G;
+  const int per = (int)blockDim.x / G;
   const bool lds = QUANT && !*S.far;
   for (int k0 = 0; k0 < n; k0 += per) {
     const bool on = k0 + g < n;
     const int k = min(k0 + g, n - 1), i = a0 + k;
-    const RowHead<GH_FG> row = row_head<GH_FG>(B, i, on);
+    const RowHead<G> row = row_head<G>(B, i, on);
     const int ax = min(sub, 2);
-    const double v0 = WHAT != 1 && hdt > 0.0 ? B.vel[ax * B.ld + i] : 0.0;
+    const double v0 = G == 4 && WHAT != 1 && hdt > 0.0 ? B.vel[ax * B.ld + i] : 0.0;
     double f[4] = {0.0, 0.0, 0.0, 0.0};
     if (!lds) {
-      batch_force<MIXED, SINGLE, GH_FG, (WHAT > 0)>(B, T, p1, a0, i, row, f);
+      batch_force<MIXED, SINGLE, G, (WHAT > 0)>(B, T, p1, a0, i, row, f);
     } else if constexpr (QUANT) {
       const int4 qi = S.q[k];
       const int ti = SINGLE ? 0 : S.ty[k];
       const float di = __int_as_float(qi.w);
       int4 q[4];
       int t[4];
-      batch_each<GH_FG>(
+      batch_each<G>(
           B, row,
           [&](int u, int s) {
             q[u] = S.q[s];
@@ -751,10 +811,29 @@ __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
             }
           });
 #pragma unroll
-      for (int d = WHAT == 1 ? 3 : 0; d < (WHAT > 0 ? 4 : 3); ++d) f[d] = group_total<GH_FG>(f[d]);
+      for (int d = WHAT == 1 ? 3 : 0; d < (WHAT > 0 ? 4 : 3); ++d) f[d] = group_total<G>(f[d]);
     }
-    if (WHAT > 0 && on && sub == 3) B.e[i] = (f[3] - sqrt(B.rho[i])) * B.ev_ui;
+    if (WHAT > 0 && on && sub == G - 1) B.e[i] = (f[3] - sqrt(B.rho[i])) * B.ev_ui;
     if (WHAT == 1) continue;
+    if constexpr (G == 1) {
+      if (!on) continue;
+      double F2 = 0.0;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const double F = f[d] * B.ev_ui;
+        B.frc[d * B.ld + i] = F;
+        F2 += F * F;
+        if (hdt > 0.0) {
+          const double v = B.vel[d * B.ld + i] + hdt * F * B.om[SINGLE ? 0 : B.type[i]];
+          B.vel[d * B.ld + i] = v;
+          pv[0] += F * v;
+          pv[1] += v * v;
+        }
+      }
+      pv[2] += F2;
+      fm2 = fmax(fm2, F2);
+      continue;
+    }
     const double F = (ax == 0 ? f[0] : ax == 1 ? f[1] : f[2]) * B.ev_ui;
     if (on && sub < 3) {
       B.frc[sub * B.ld + i] = F;
@@ -810,7 +889,6 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
     st.dt = fc.dt_max * 0.1;
     st.alpha = fc.alpha0;
     st.npos = st.it = st.done = st.conv = 0;
-    sys_build(B, a0, n);
   }
   if (QUANT) {
     const double4 o4 = B.pos[a0];
@@ -823,10 +901,11 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
     }
     __syncthreads();
   }
+  if (!fc.resume) sys_build<QUANT>(B, S, a0, n);
   constexpr int kForce = MIXED ? 0 : 2;
   double pv[3] = {0.0, 0.0, 0.0}, fm2 = 0.0;
-  fire_rho<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n);
-  fire_force<MIXED, QUANT, SINGLE, kForce>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+  fire_rho<MIXED, QUANT, SINGLE, GH_FG>(B, S, T, p1, a0, n);
+  fire_force<MIXED, QUANT, SINGLE, kForce, GH_FG>(B, S, T, p1, a0, n, 0.0, pv, fm2);
   // the mixing of the last iteration, still to be applied to v: v <- cm v + mixv F
   double cm = 1.0, mixv = 0.0;
   bool pend = false;
@@ -878,10 +957,10 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
     }
     double none[3] = {0.0, 0.0, 0.0};
     bred<BS, 0>(R, none, d2);
-    if (2.0 * sqrt(d2) > skin) sys_build(B, a0, n);
+    if (2.0 * sqrt(d2) > skin) sys_build<QUANT>(B, S, a0, n);
     pv[0] = pv[1] = pv[2] = fm2 = 0.0;
-    fire_rho<MIXED, QUANT, SINGLE>(B, S, T, p1, a0, n);
-    fire_force<MIXED, QUANT, SINGLE, kForce>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
+    fire_rho<MIXED, QUANT, SINGLE, GH_FG>(B, S, T, p1, a0, n);
+    fire_force<MIXED, QUANT, SINGLE, kForce, GH_FG>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
     bred<BS, 3>(R, pv, fm2);
     fnow = sqrt(fm2) * fc.ui_ev;
     pend = true;
@@ -911,7 +990,7 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   double ep = 0.0, ek = 0.0;
   if (done) {
     if (MIXED) {
-      fire_force<MIXED, QUANT, SINGLE, 1>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+      fire_force<MIXED, QUANT, SINGLE, 1, GH_FG>(B, S, T, p1, a0, n, 0.0, pv, fm2);
       __syncthreads();
     }
     sys_energies(B, R, a0, a1, ep, ek);
@@ -935,20 +1014,24 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
 
 // Langevin steps of mixed systems staged in LDS, a workgroup per system (largest
 // first) and all steps in one launch: no random gathers from the L2, which bound
-// the passes over all atoms, but the largest system takes its own time on one
-// CU (2,000 atoms 150 us a step).  Chosen by batch_staged.  The first step's
-// ermak_a has run.
-template <bool SINGLE, int BS>
-__global__ __launch_bounds__(BS, 4) void k_batch_langevin(BatchArgs B, ErmakC k_arg, double skin,
-                                                          TbF p_arg, unsigned long long seed,
-                                                          long long step0, int nsteps) {
+// the passes over all atoms, and no launches per step.  Chosen by batch_staged,
+// its threads by staged_threads; the first step's ermak_a has run.
+//
+// G lanes per atom: four, or one in large systems (split_systems).  The update
+// takes a thread per atom and axis and draws each normal once: the next step's
+// pair waits in pos_next, which the passes over all atoms rewrite (150 systems of
+// 2,000 Ag-Cu atoms, 50 steps: 8.3 -> 7.9 ms).
+template <bool SINGLE, int G>
+__global__ __launch_bounds__(1024, 4) void k_batch_langevin(BatchArgs B, ErmakC k_arg, double skin,
+                                                            TbF p_arg, unsigned long long seed,
+                                                            long long step0, int nsteps) {
   __shared__ ErmakC k;
   __shared__ TbF p1;
   extern __shared__ int4 dyn_q[];
   __shared__ BTable<true, SINGLE> T;
-  __shared__ BlockRed<BS> R;
+  __shared__ double top[16];
   __shared__ int sfar;
-  const int s = B.order[blockIdx.x], a0 = B.off[s], n = B.off[s + 1] - a0;
+  const int s = B.order[B.first + blockIdx.x], a0 = B.off[s], n = B.off[s + 1] - a0;
   if (threadIdx.x == 0) {
     k = k_arg;
     p1 = p_arg;
@@ -956,14 +1039,19 @@ __global__ __launch_bounds__(BS, 4) void k_batch_langevin(BatchArgs B, ErmakC k_
   load_table<true, true, SINGLE>(T, B);
   Stage S{dyn_q, reinterpret_cast<unsigned char *>(dyn_q + B.nst), &sfar};
   const double skt = sqrt(k_arg.kB_ui * B.T[s]);
-  const int sub = threadIdx.x & (GH_FG - 1), g = (int)threadIdx.x / GH_FG;
+  auto normals = [&](int q) { return reinterpret_cast<float2 *>(B.pos_next + a0 + q / 3) + q % 3; };
+  for (int q = threadIdx.x; q < 3 * n; q += blockDim.x) {
+    float2 g;
+    axis_normals(seed, step0, a0 + q / 3, q % 3, g.x, g.y);
+    *normals(q) = g;
+  }
   for (int st = 0; st < nsteps; ++st) {
     if (threadIdx.x == 0) sfar = 0;
     __syncthreads();
     const double4 o4 = B.pos[a0];
     const double o[3] = {o4.x, o4.y, o4.z};
-    double d2 = 0.0, none[3] = {0.0, 0.0, 0.0};
-    for (int q = threadIdx.x; q < n; q += BS) {
+    double d2 = 0.0, none[3] = {0.0, 0.0, 0.0}, fm2 = 0.0;
+    for (int q = threadIdx.x; q < n; q += blockDim.x) {
       const double4 p = B.pos[a0 + q];
       const double x[3] = {p.x, p.y, p.z};
       double e2 = 0.0;
@@ -976,35 +1064,36 @@ __global__ __launch_bounds__(BS, 4) void k_batch_langevin(BatchArgs B, ErmakC k_
       stage_atom(S, q, x, o);
       if (!SINGLE) S.ty[q] = (unsigned char)(int)p.w;
     }
-    bred<BS, 0>(R, none, d2);
+    d2 = wave_top(d2);
+    if ((threadIdx.x & 63) == 0) top[threadIdx.x >> 6] = d2;
+    __syncthreads();
+    for (int w = 0; w < (int)(blockDim.x >> 6); ++w) d2 = fmax(d2, top[w]);
     if (2.0 * sqrt(d2) > skin) {
-      sys_build(B, a0, n);
+      sys_build<true>(B, S, a0, n);
       if (threadIdx.x == 0) B.out[s * OUTW + 2] += 1.0;
     }
-    fire_rho<true, true, SINGLE>(B, S, T, p1, a0, n);
     const bool last = st + 1 == nsteps;
-    double fm2 = 0.0;
-    if (last) fire_force<true, true, SINGLE, 2>(B, S, T, p1, a0, n, 0.0, none, fm2);
-    else fire_force<true, true, SINGLE, 0>(B, S, T, p1, a0, n, 0.0, none, fm2);
-    // ermak_b, and ermak_a of the next step: the lane that stored an axis'
-    // force moves it (the passes read positions from LDS)
+    fire_rho<true, true, SINGLE, G>(B, S, T, p1, a0, n);
+    if (last) fire_force<true, true, SINGLE, 2, G>(B, S, T, p1, a0, n, 0.0, none, fm2);
+    else fire_force<true, true, SINGLE, 0, G>(B, S, T, p1, a0, n, 0.0, none, fm2);
+    __syncthreads();
+    // ermak_b, and ermak_a of the next step (the passes read positions from LDS)
     const long long step = step0 + st;
-    for (int k0 = 0; k0 < n; k0 += BS / GH_FG) {
-      if (sub == 3 || k0 + g >= n) continue;
-      const int i = a0 + k0 + g, t = SINGLE ? 0 : B.type[i];
-      float ga, gb, gn, un;
-      axis_normals(seed, step, i, sub, ga, gb);
-      const double F = B.frc[sub * B.ld + i], om = B.om[t], f_lan = skt * B.osm[t];
-      const double vel_v = f_lan * k.sdv * (k.crv1 * (double)ga + k.crv2 * (double)gb);
-      const double v = k.c0 * B.vel[sub * B.ld + i] + (k.c1 - k.c2) * B.acc[sub * B.ld + i] +
+    for (int q = threadIdx.x; q < 3 * n; q += blockDim.x) {
+      const int i = a0 + q / 3, ax = q % 3, t = SINGLE ? 0 : S.ty[q / 3];
+      float2 g = *normals(q);
+      const double F = B.frc[ax * B.ld + i], om = B.om[t], f_lan = skt * B.osm[t];
+      const double vel_v = f_lan * k.sdv * (k.crv1 * (double)g.x + k.crv2 * (double)g.y);
+      const double v = k.c0 * B.vel[ax * B.ld + i] + (k.c1 - k.c2) * B.acc[ax * B.ld + i] +
                        k.c2 * F * om + vel_v;
       const double a = F * om;
-      B.vel[sub * B.ld + i] = v;
-      B.acc[sub * B.ld + i] = a;
+      B.vel[ax * B.ld + i] = v;
+      B.acc[ax * B.ld + i] = a;
       if (!last) {
-        axis_normals(seed, step + 1, i, sub, gn, un);
-        double *x = reinterpret_cast<double *>(B.pos + i) + sub;
-        *x = *x + k.c1 * v + k.c2 * k.dt * a + f_lan * k.sdr * (double)gn;
+        axis_normals(seed, step + 1, i, ax, g.x, g.y);
+        *normals(q) = g;
+        double *x = reinterpret_cast<double *>(B.pos + i) + ax;
+        *x = *x + k.c1 * v + k.c2 * k.dt * a + f_lan * k.sdr * (double)g.x;
       }
     }
     __syncthreads();
@@ -1096,6 +1185,13 @@ static BatchArgs bargs(const gh_batch *b) {
   for (int i = 0; i < b->nt; ++i)
     for (int j = 0; j < b->nt; ++j) rci = std::min(rci, b->tb[i * GH_MAXT + j].rci);
   A.near2 = rci * rci;
+  // FP32 on the staged positions: its error on r^2 stays below 1e-4 A^2 for
+  // pairs near the bounds; the margins are thirty times that
+  const double q2 = GH_BFXS * GH_BFXS, margin = std::max(3e-3, 1e-4 * A.rl2);
+  A.hi2q = (float)((A.rl2 + margin) * q2);
+  A.lo2q = (float)((A.rl2 - margin) * q2);
+  A.near2q = (float)(A.near2 * q2);
+  A.band2q = (float)(std::max(3e-3, 1e-4 * A.near2) * q2);
   A.ev_ui = ghc::ev_ui();
   A.T = b->T;
   A.out = b->out;
@@ -1165,6 +1261,70 @@ static int batch_ready(gh_batch *b) {
   return 0;
 }
 
+static int largest_system(const gh_batch *b) {
+  const int big = b->order_h[0];
+  return b->off_h[big + 1] - b->off_h[big];
+}
+
+// Threads of the workgroups of k_batch_langevin.  A CU runs 16 of its wavefronts:
+// as one workgroup while the atoms' sum is at most one system of the largest size
+// per CU, as two, four, ... of half, a quarter, ... the wavefronts where it is
+// two, four, ..., so that all systems are in flight; no fewer than the largest
+// power of two in the largest system's atoms (more systems in flight then only
+// outgrow the L2), and no more than four lanes for each of them.  50 steps of Ag-Cu
+// systems, ms, 64 / 128 / 256 / 512 / 1024 threads, with the largest systems per CU:
+// 10,000 of 13 atoms (40) 1.7 / 2.5 / 4.3 / 7.9 / 15; 6000 of 147 (23) 12.5 / 10.9 / 12.2 /
+// 16 / 18; 2000 of 147 (7.8) 6.7 / 3.8 / 4.3 / 5.4 / 6.1; 4000 of 309 (16) 27 / 16.1 / 15.5 /
+// 17.0 / 21; 1000 of 309 (3.9) 13 / 7.0 / 4.2 / 4.5 / 5.5; 600 of 147 (2.3) 5.8 / 3.4 / 2.0 /
+// 2.4 / 2.3; 400 of 1000 (1.6) - / 20 / 10 / 6.5 / 6.7; 1024 of 13 to 309, log-uniform
+// (1.2) 11 / 5.8 / 3.1 / 1.9 / 2.9; 512 of 38 to 1000, log-uniform (0.57) 38 / 20 / 10 /
+// 5.7 / 3.8.
+static int staged_threads(const gh_batch *b) {
+  const int nmax = largest_system(b);
+  const double r = b->ntot / (256.0 * nmax);
+  int bs = 1024;
+  while (bs > 64 && r > 1024.0 / bs && bs > nmax) bs /= 2;
+  while (bs > 64 && bs / 2 >= GH_FG * nmax) bs /= 2;
+  return bs;
+}
+
+// How many of the systems, largest first, take one lane per atom: those of one
+// and a half times the workgroup's threads and more.  Their wavefronts are full
+// either way, and four lanes pay a row's padding and the sums four times (50
+// Langevin steps, Ag-Cu, ms, four lanes and one: 150 systems of 2,000 atoms 9.2 and
+// 7.9, 1000 of 400 5.6 and 5.1, 1000 of 309 4.2 and 4.3, 600 of 147 2.0 and 2.5).
+static int split_systems(const gh_batch *b, int bs) {
+  int k = 0;
+  while (k < b->nsys) {
+    const int s = b->order_h[k];
+    if (2 * (b->off_h[s + 1] - b->off_h[s]) < 3 * bs) break;
+    ++k;
+  }
+  return k;
+}
+
+// Runs launch(lanes, first, count, stream) for the systems of one lane per atom
+// and of four, on two streams where there are both.
+template <class LAUNCH>
+static int launch_split(gh_batch *b, int bs, LAUNCH &&launch) {
+  const int one = split_systems(b, bs);
+  const bool both = one > 0 && one < b->nsys;
+  if (both) {
+    BH(b, hipEventRecord(b->ev_fork, b->stream));
+    BH(b, hipStreamWaitEvent(b->stream2, b->ev_fork, 0));
+  }
+  // (the large ones first)
+  if (one > 0) launch(1, 0, one, b->stream);
+  BH(b, hipGetLastError());
+  if (one < b->nsys) launch(GH_FG, one, b->nsys - one, both ? b->stream2 : b->stream);
+  BH(b, hipGetLastError());
+  if (both) {
+    BH(b, hipEventRecord(b->ev_join, b->stream2));
+    BH(b, hipStreamWaitEvent(b->stream, b->ev_join, 0));
+  }
+  return 0;
+}
+
 // The FIRE kernel over all systems, a workgroup each.  Threads: 256 where four
 // systems share a compute unit and hide each other's barriers (1024 Au clusters,
 // mixed, a quench of 100 iterations: 128 threads 9.9 ms, 256 6.7, 512 7.2;
@@ -1179,7 +1339,7 @@ static int batch_ready(gh_batch *b) {
 template <bool MIXED, bool QUANT>
 static int launch_fire(gh_batch *b, const BatchArgs &A, const FireC &fc, const BForm<MIXED> &p) {
   const size_t lds = QUANT ? 17 * (size_t)b->nst : 0;
-  const int big = b->order_h[0], nmax = b->off_h[big + 1] - b->off_h[big];
+  const int nmax = largest_system(b);
   int bs = b->nsys <= 256 ? 1024 : b->nsys <= 768 ? 512 : GH_FBS;
   while (bs > GH_FBS && bs / 2 >= GH_FG * nmax) bs /= 2;
   const int nbig = b->nt > 1 && bs < 1024 ? b->nbig : 0;
@@ -1492,18 +1652,18 @@ int gh_batch_compute(gh_batch *b, double *F, double *epot) {
 }
 
 // Mixed Langevin steps by a workgroup per system (k_batch_langevin) or over all
-// atoms: the former takes the largest system's time, the latter the sum's, so by
-// their ratio.  50 steps and an exchange, Ag-Cu clusters from 38 atoms, over all atoms and
-// per system, ms: 512 systems to 150 atoms 2.0 and 1.8, to 600 4.5 and 3.6, to 1000
-// 6.3 and 5.9, to 2000 10.1 and 13.3 (0.50 of the largest system per CU);
-// 256 to 150 1.28 and 1.00, to 600 2.5 and 3.1 (0.34); in long runs 304 to 500
-// (0.48) 43 and 33 us a step, 512 of 642 atoms on average, 2000 at most (0.64), 183
-// and 170.
+// atoms.  The former takes the largest system's time, the latter the sum's, so
+// by their ratio: 50 steps, Ag-Cu, ms, over all atoms and per system: 512 systems of
+// 38 to 2000 atoms, log-uniform, 6.8 and 7.8 (129 of the largest in all), 150 of 2000
+// 9.5 and 8.0, 304 of 38 to 500 2.1 and 1.8 (124), 120 of 13 0.67 and 0.43; 64 of 309
+// 1.2 and 1.4, 16 of 2000 1.9 and 7.6.  And where the largest system's step takes
+// less than two launches, whatever their number: one of 13 0.61 and 0.41, ten of 38
+// 0.68 and 0.68, ten of 55 0.67 and 0.71.
 static bool batch_staged(const gh_batch *b) {
-  const int big = b->order_h[0], nmax = b->off_h[big + 1] - b->off_h[big];
-  return b->precision == GH_MIXED && b->nst > 0 && b->ntot >= (nmax <= 512 ? 115ll : 144ll) * nmax;
+  const int nmax = largest_system(b);
+  return b->precision == GH_MIXED && b->nst > 0 &&
+         (nmax <= 32 || b->ntot >= (nmax <= 512 ? 115ll : 144ll) * nmax);
 }
-
 int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t seed,
                       double *epot, double *ekin) {
   if (!b || nsteps < 0 || !(dt > 0) || !(gamma > 0))
@@ -1528,8 +1688,18 @@ int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t
     k_batch_ermak_a<<<batch_blocks(b, 16), GH_BWG, 0, b->stream>>>(A, k, seed, step0);
     if (batch_staged(b)) {
       const size_t lds = 17 * (size_t)b->nst;
-      if (b->nt == 1) k_batch_langevin<true, 1024><<<b->nsys, 1024, lds, b->stream>>>(A, k, b->skin, b->tbf0, seed, step0, nsteps);
-      else k_batch_langevin<false, 1024><<<b->nsys, 1024, lds, b->stream>>>(A, k, b->skin, b->tbf0, seed, step0, nsteps);
+      const int bs = staged_threads(b);
+      auto launch = [&](int lanes, int first, int count, hipStream_t stream) {
+        A.first = first;
+#define LAUNCH_LANGEVIN(SG, G) \
+  k_batch_langevin<SG, G><<<count, bs, lds, stream>>>(A, k, b->skin, b->tbf0, seed, step0, nsteps)
+        if (b->nt == 1 && lanes == 1) LAUNCH_LANGEVIN(true, 1);
+        else if (b->nt == 1) LAUNCH_LANGEVIN(true, GH_FG);
+        else if (lanes == 1) LAUNCH_LANGEVIN(false, 1);
+        else LAUNCH_LANGEVIN(false, GH_FG);
+#undef LAUNCH_LANGEVIN
+      };
+      BT(launch_split(b, bs, launch));
     }
     for (int st = 0; st < nsteps && !batch_staged(b); ++st) {
       const long long step = step0 + st;
