@@ -30,8 +30,7 @@
 
 #include "gh_device.h"
 
-#define GH_FBS 256  // workgroup of the FIRE kernel
-#define GH_BIGSYS 1024  // systems above this many atoms get 1024-thread workgroups
+#define GH_FBS 256  // smallest workgroup of the FIRE kernel
 
 namespace {
 struct FireState;
@@ -72,9 +71,7 @@ struct gh_batch {
   TbF tbf0;
   double tb_e0 = 0.0;
   int nst = 0;   // LDS staging slots per workgroup (largest system + sentinel)
-  // FIRE: systems above GH_BIGSYS atoms (the first nbig of the largest-first
-  // order) run on a second stream beside the rest
-  int nbig = 0;
+  // systems of one lane per atom and of four run beside one another (launch_split)
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_fork = nullptr, ev_join = nullptr;
 };
@@ -111,14 +108,13 @@ struct BatchArgs {
 
 #define OUTW 6
 
-template <int BS>
-struct BlockRed {
-  double v[BS / 64][8];  // up to 8 values per reduction
+struct BlockRed {  // workgroups of 256, 512 or 1024 threads
+  double v[16][8];  // up to 8 values per reduction
 };
 
 // Block-wide sums of NV values; the result is returned to every thread.
-template <int BS, int NV>
-__device__ __forceinline__ void bsum(BlockRed<BS> &R, double (&v)[NV]) {
+template <int NV>
+__device__ __forceinline__ void bsum(BlockRed &R, double (&v)[NV]) {
   static_assert(NV <= 8, "BlockRed holds 8 values per wave");
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
@@ -130,8 +126,10 @@ __device__ __forceinline__ void bsum(BlockRed<BS> &R, double (&v)[NV]) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     double s = 0.0;
-#pragma unroll 4  // fully unrolled, 16 wavefronts x 8 values would all sit in registers
-    for (int w = 0; w < BS / 64; ++w) s += R.v[w][k];
+    for (int w = 0; w < (int)(blockDim.x >> 6); w += 4) {  // (whole groups of four)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s += R.v[w + u][k];
+    }
     v[k] = s;
   }
   __syncthreads();
@@ -139,8 +137,8 @@ __device__ __forceinline__ void bsum(BlockRed<BS> &R, double (&v)[NV]) {
 
 // Block-wide sums of the first NV values of v and the maximum of m, returned
 // to every thread; two barriers, the second before the next use of R.
-template <int BS, int NV>
-__device__ __forceinline__ void bred(BlockRed<BS> &R, double (&v)[3], double &m) {
+template <int NV>
+__device__ __forceinline__ void bred(BlockRed &R, double (&v)[3], double &m) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = wave_total(v[k]);
   m = wave_top(m);
@@ -152,11 +150,13 @@ __device__ __forceinline__ void bred(BlockRed<BS> &R, double (&v)[3], double &m)
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = 0.0;
-#pragma unroll 4
-  for (int w = 0; w < BS / 64; ++w) {
+  for (int w = 0; w < (int)(blockDim.x >> 6); w += 4) {
 #pragma unroll
-    for (int k = 0; k < NV; ++k) v[k] += R.v[w][k];
-    m = fmax(m, R.v[w][3]);
+    for (int u = 0; u < 4; ++u) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) v[k] += R.v[w + u][k];
+      m = fmax(m, R.v[w + u][3]);
+    }
   }
   __syncthreads();
 }
@@ -582,8 +582,7 @@ __global__ __launch_bounds__(GH_BWG) void k_batch_force(BatchArgs B, BForm<MIXED
 }
 
 // epot (ui) and ekin about the centre of mass (ui) of one system.
-template <int BS>
-__device__ void sys_energies(const BatchArgs &B, BlockRed<BS> &R, int a0, int a1, double &epot,
+__device__ void sys_energies(const BatchArgs &B, BlockRed &R, int a0, int a1, double &epot,
                              double &ekin) {
   double s[5] = {0, 0, 0, 0, 0};
   for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
@@ -594,7 +593,7 @@ __device__ void sys_energies(const BatchArgs &B, BlockRed<BS> &R, int a0, int a1
     s[3] += m * B.vel[B.ld + i];
     s[4] += m * B.vel[2 * B.ld + i];
   }
-  bsum<BS, 5>(R, s);
+  bsum<5>(R, s);
   const double cx = s[2] / s[1], cy = s[3] / s[1], cz = s[4] / s[1];
   double k[1] = {0.0};
   for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
@@ -602,13 +601,13 @@ __device__ void sys_energies(const BatchArgs &B, BlockRed<BS> &R, int a0, int a1
     const double wx = B.vel[i] - cx, wy = B.vel[B.ld + i] - cy, wz = B.vel[2 * B.ld + i] - cz;
     k[0] += (wx * wx + wy * wy + wz * wz) * m;
   }
-  bsum<BS, 1>(R, k);
+  bsum<1>(R, k);
   epot = s[0];
   ekin = 0.5 * k[0];
 }
 // The energies of every system, a workgroup each.
 __global__ __launch_bounds__(GH_BWG) void k_batch_energies(BatchArgs B) {
-  __shared__ BlockRed<GH_BWG> R;
+  __shared__ BlockRed R;
   const int s = blockIdx.x;
   double ep, ek;
   sys_energies(B, R, B.off[s], B.off[s + 1], ep, ek);
@@ -852,9 +851,9 @@ __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
   }
 }
 
-template <bool MIXED, bool QUANT, bool SINGLE, int BS>
-__global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg, double skin_arg,
-                                                   FireState *fst, BForm<MIXED> p_arg) {
+template <bool MIXED, bool QUANT, bool SINGLE, int G>
+__global__ __launch_bounds__(1024, 4) void k_batch_fire(BatchArgs B, FireC fc_arg, double skin_arg,
+                                                       FireState *fst, BForm<MIXED> p_arg) {
   // The constants live in LDS and are read where they are used: held in
   // scalar registers for a whole kernel of this kind they were spilled, and
   // the ROCm 7.2 compiler has mis-allocated such spills (a later
@@ -864,7 +863,7 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   __shared__ BForm<MIXED> p1;
   extern __shared__ int4 dyn_q[];
   __shared__ BTable<MIXED, SINGLE> T;
-  __shared__ BlockRed<BS> R;
+  __shared__ BlockRed R;
   __shared__ int sfar;
   // Systems come largest first and 256 workgroups fill one slot on each CU:
   // every other 256 run in reverse, so that a CU's systems add up alike (1024
@@ -904,12 +903,12 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   if (!fc.resume) sys_build<QUANT>(B, S, a0, n);
   constexpr int kForce = MIXED ? 0 : 2;
   double pv[3] = {0.0, 0.0, 0.0}, fm2 = 0.0;
-  fire_rho<MIXED, QUANT, SINGLE, GH_FG>(B, S, T, p1, a0, n);
-  fire_force<MIXED, QUANT, SINGLE, kForce, GH_FG>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+  fire_rho<MIXED, QUANT, SINGLE, G>(B, S, T, p1, a0, n);
+  fire_force<MIXED, QUANT, SINGLE, kForce, G>(B, S, T, p1, a0, n, 0.0, pv, fm2);
   // the mixing of the last iteration, still to be applied to v: v <- cm v + mixv F
   double cm = 1.0, mixv = 0.0;
   bool pend = false;
-  bred<BS, 0>(R, pv, fm2);
+  bred<0>(R, pv, fm2);
   double dt = st.dt, alpha = st.alpha, fnow = sqrt(fm2) * fc.ui_ev;  // eV/A
   int it = st.it, npos = st.npos;
   bool stop = false;
@@ -956,12 +955,12 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
       if (QUANT) stage_atom(S, k, x, o);
     }
     double none[3] = {0.0, 0.0, 0.0};
-    bred<BS, 0>(R, none, d2);
+    bred<0>(R, none, d2);
     if (2.0 * sqrt(d2) > skin) sys_build<QUANT>(B, S, a0, n);
     pv[0] = pv[1] = pv[2] = fm2 = 0.0;
-    fire_rho<MIXED, QUANT, SINGLE, GH_FG>(B, S, T, p1, a0, n);
-    fire_force<MIXED, QUANT, SINGLE, kForce, GH_FG>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
-    bred<BS, 3>(R, pv, fm2);
+    fire_rho<MIXED, QUANT, SINGLE, G>(B, S, T, p1, a0, n);
+    fire_force<MIXED, QUANT, SINGLE, kForce, G>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
+    bred<3>(R, pv, fm2);
     fnow = sqrt(fm2) * fc.ui_ev;
     pend = true;
     if (pv[0] > 0.0) {
@@ -990,7 +989,7 @@ __global__ __launch_bounds__(BS, 4) void k_batch_fire(BatchArgs B, FireC fc_arg,
   double ep = 0.0, ek = 0.0;
   if (done) {
     if (MIXED) {
-      fire_force<MIXED, QUANT, SINGLE, 1, GH_FG>(B, S, T, p1, a0, n, 0.0, pv, fm2);
+      fire_force<MIXED, QUANT, SINGLE, 1, G>(B, S, T, p1, a0, n, 0.0, pv, fm2);
       __syncthreads();
     }
     sys_energies(B, R, a0, a1, ep, ek);
@@ -1325,53 +1324,49 @@ static int launch_split(gh_batch *b, int bs, LAUNCH &&launch) {
   return 0;
 }
 
-// The FIRE kernel over all systems, a workgroup each.  Threads: 256 where four
-// systems share a compute unit and hide each other's barriers (1024 Au clusters,
-// mixed, a quench of 100 iterations: 128 threads 9.9 ms, 256 6.7, 512 7.2;
-// registers for five wavefronts per SIMD instead of four spill: 9.0); fewer
-// systems leave units idle, and a system's rounds of atoms, one memory round
-// trip after another, bound its iteration: 512 up to 768 systems, 1024 up to 256,
-// no more than the largest system has lanes for.  80 iterations, clusters to 309
+// Threads of the FIRE kernel's workgroups: 256 where four systems share a compute
+// unit and hide each other's barriers (1024 Au clusters, mixed, a quench of 100
+// iterations: 128 threads 9.9 ms, 256 6.7, 512 7.2; registers for five wavefronts
+// per SIMD instead of four spill: 9.0); fewer systems leave units idle, and a
+// system's rounds of atoms, one memory round trip after another, bound its
+// iteration: 512 up to 768 systems, 1024 up to 256.  80 iterations, clusters to 309
 // atoms, 256 / 512 / 1024 threads, ms, mixed (FP64): 200 systems 3.4 / 2.4 / 2.2
 // (5.3 / 4.2 / 4.2), 500 4.4 / 3.2 / 4.0 (7.0 / 5.6 / 7.3), 700 5.0 / 4.2 / 5.4
-// (8.2 / 7.4 / 9.4).  Beside them multi-type systems above GH_BIGSYS atoms,
-// which bound a run (largest first), get 1024 threads on a second stream.
+// (8.2 / 7.4 / 9.4).  But by the atoms' sum per CU in systems of the largest size:
+// where it is more than two, 256 instead of 512 (40 iterations, Ag-Cu, ms, mixed and
+// FP64, 256 / 512: 600 systems of 147 atoms 1.65 / 2.08 and 2.87 / 3.47), and where it
+// is below three quarters and the largest needs more than three rounds of 512
+// threads, 1024 (512 of 38 to 1000, log-uniform, 512 / 1024: 4.5 / 3.2 and 7.5 / 5.6);
+// 512 also for more systems where the largest needs that many (2000 of 13 to 2000,
+// log-uniform, 256 / 512: 16 / 11 and 26 / 20).
+// No more than the largest system has lanes for.
+static int fire_threads(const gh_batch *b) {
+  const int nmax = largest_system(b);
+  const double r = b->ntot / (256.0 * nmax);
+  int bs = GH_FBS;
+  if (b->nsys <= 256 || (nmax > 384 && r <= 0.75)) bs = 1024;
+  else if (r <= 2.1 && (b->nsys <= 768 || nmax > 384)) bs = 512;
+  while (bs > GH_FBS && bs / 2 >= GH_FG * nmax) bs /= 2;
+  return bs;
+}
+
+// The FIRE kernel over all systems, a workgroup each.
 template <bool MIXED, bool QUANT>
 static int launch_fire(gh_batch *b, const BatchArgs &A, const FireC &fc, const BForm<MIXED> &p) {
   const size_t lds = QUANT ? 17 * (size_t)b->nst : 0;
-  const int nmax = largest_system(b);
-  int bs = b->nsys <= 256 ? 1024 : b->nsys <= 768 ? 512 : GH_FBS;
-  while (bs > GH_FBS && bs / 2 >= GH_FG * nmax) bs /= 2;
-  const int nbig = b->nt > 1 && bs < 1024 ? b->nbig : 0;
+  const int bs = fire_threads(b);
   BatchArgs A1 = A;
-#define LAUNCH_FIRE(SG, BS, COUNT, STREAM) \
-  k_batch_fire<MIXED, QUANT, SG, BS><<<COUNT, BS, lds, STREAM>>>(A1, fc, b->skin, b->fst, p)
-  if (nbig > 0) {
-    BH(b, hipEventRecord(b->ev_fork, b->stream));
-    BH(b, hipStreamWaitEvent(b->stream2, b->ev_fork, 0));
-    LAUNCH_FIRE(false, 1024, nbig, b->stream2);
-    BH(b, hipGetLastError());
-  }
-  if (b->nsys > nbig) {
-    A1.first = nbig;
-    const int count = b->nsys - nbig;
-    if (b->nt == 1) {
-      if (bs == 1024) LAUNCH_FIRE(true, 1024, count, b->stream);
-      else if (bs == 512) LAUNCH_FIRE(true, 512, count, b->stream);
-      else LAUNCH_FIRE(true, GH_FBS, count, b->stream);
-    } else {
-      if (bs == 1024) LAUNCH_FIRE(false, 1024, count, b->stream);
-      else if (bs == 512) LAUNCH_FIRE(false, 512, count, b->stream);
-      else LAUNCH_FIRE(false, GH_FBS, count, b->stream);
-    }
-    BH(b, hipGetLastError());
-  }
+  auto launch = [&](int lanes, int first, int count, hipStream_t stream) {
+    A1.first = first;
+#define LAUNCH_FIRE(SG, G) \
+  k_batch_fire<MIXED, QUANT, SG, G><<<count, bs, lds, stream>>>(A1, fc, b->skin, b->fst, p)
+    if (b->nt == 1 && lanes == 1) LAUNCH_FIRE(true, 1);
+    else if (b->nt == 1) LAUNCH_FIRE(true, GH_FG);
+    else if (lanes == 1) LAUNCH_FIRE(false, 1);
+    else LAUNCH_FIRE(false, GH_FG);
 #undef LAUNCH_FIRE
-  if (nbig > 0) {
-    BH(b, hipEventRecord(b->ev_join, b->stream2));
-    BH(b, hipStreamWaitEvent(b->stream, b->ev_join, 0));
-  }
-  return 0;
+  };
+  return launch_split(b, bs, launch);
 }
 
 static int batch_blocks(const gh_batch *b, int lanes) {
@@ -1491,9 +1486,6 @@ int gh_batch_set_systems(gh_batch *b, int nsys, const int *off, const double *x,
   std::stable_sort(b->order_h.begin(), b->order_h.end(), [&](int a, int c) {
     return off[a + 1] - off[a] > off[c + 1] - off[c];
   });
-  b->nbig = 0;
-  while (b->nbig < nsys && off[b->order_h[b->nbig] + 1] - off[b->order_h[b->nbig]] > GH_BIGSYS)
-    ++b->nbig;
   b->T_h.assign(nsys, 0.0);
   BT(balloc(b, &b->off, nsys + 1));
   BT(balloc(b, &b->order, nsys));

@@ -80,3 +80,26 @@ def test_largest_staged_system_quenches(n):
             assert np.all(r["iters"] == 3)
     assert np.max(np.abs(out[0] - out[1])) < 1e-7
     assert np.max(np.abs(out[1] - x)) > 1e-5
+
+
+@pytest.mark.parametrize("prec,bar", [(hip.GH_FP64, 1e-11), (hip.GH_MIXED, 1e-6)],
+                         ids=["fp64", "mixed"])
+@pytest.mark.parametrize("nt", [1, 2])
+@pytest.mark.parametrize("edge,others", [((383, 384, 385), [384] * 557), ((767, 768, 769), [768] * 297),
+                                         ((1535, 1536, 1537), [1000] * 300)],
+                         ids=["384-of-256", "768-of-512", "1536-of-1024"])
+def test_quench_with_one_lane_and_four(edge, others, nt, prec, bar):
+    # the same quench alone (1,024 threads) and among many: FP64 forces sum the same
+    # pairs in another order, 2^-53 of a few eV/A over 30 steps as in
+    # test_gpu_fire_threads.py; mixed as above
+    off, x, t = _systems(list(edge))
+    off2, x2, t2 = _systems(others, seed=2)
+    out = []
+    for o, y, ty in ((off, x, t), (np.concatenate([off, off[-1] + off2[1:]]).astype(np.int32),
+                                   np.concatenate([x, x2]), np.concatenate([t, t2]))):
+        with _batch(o, y, ty, nt, prec) as b:
+            r = b.fire(max_iter=30)
+            out.append((b.state()[0][:len(x)], r["epot"][:3], r["fmax"][:3]))
+    assert np.max(np.abs(out[0][0] - x)) > 0.01
+    assert np.max(np.abs(out[0][0] - out[1][0])) <= bar
+    assert np.allclose(out[0][1], out[1][1], rtol=bar, atol=0)
