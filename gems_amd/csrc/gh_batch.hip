@@ -108,13 +108,28 @@ struct BatchArgs {
 
 #define OUTW 6
 
-struct BlockRed {  // workgroups of 256, 512 or 1024 threads
-  double v[16][8];  // up to 8 values per reduction
+// BS threads; 0: as launched (256, 512 or 1024).
+template <int BS>
+struct BlockRed {
+  double v[BS ? BS / 64 : 16][8];  // up to 8 values per reduction
 };
+// Runs f(w) for every wavefront of the workgroup, four at a time (fully
+// unrolled, 16 wavefronts x 8 values would all sit in registers).
+template <int BS, class F>
+__device__ __forceinline__ void each_wave(F &&f) {
+  if constexpr (BS > 0) {
+#pragma unroll 4
+    for (int w = 0; w < BS / 64; ++w) f(w);
+  } else {
+    for (int w0 = 0; w0 < (int)(blockDim.x >> 6); w0 += 4)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) f(w0 + u);
+  }
+}
 
 // Block-wide sums of NV values; the result is returned to every thread.
-template <int NV>
-__device__ __forceinline__ void bsum(BlockRed &R, double (&v)[NV]) {
+template <int BS, int NV>
+__device__ __forceinline__ void bsum(BlockRed<BS> &R, double (&v)[NV]) {
   static_assert(NV <= 8, "BlockRed holds 8 values per wave");
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = wave_sum(v[k]);
@@ -126,10 +141,7 @@ __device__ __forceinline__ void bsum(BlockRed &R, double (&v)[NV]) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
     double s = 0.0;
-    for (int w = 0; w < (int)(blockDim.x >> 6); w += 4) {  // (whole groups of four)
-#pragma unroll
-      for (int u = 0; u < 4; ++u) s += R.v[w + u][k];
-    }
+    each_wave<BS>([&](int w) { s += R.v[w][k]; });
     v[k] = s;
   }
   __syncthreads();
@@ -137,8 +149,8 @@ __device__ __forceinline__ void bsum(BlockRed &R, double (&v)[NV]) {
 
 // Block-wide sums of the first NV values of v and the maximum of m, returned
 // to every thread; two barriers, the second before the next use of R.
-template <int NV>
-__device__ __forceinline__ void bred(BlockRed &R, double (&v)[3], double &m) {
+template <int BS, int NV>
+__device__ __forceinline__ void bred(BlockRed<BS> &R, double (&v)[3], double &m) {
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = wave_total(v[k]);
   m = wave_top(m);
@@ -150,14 +162,11 @@ __device__ __forceinline__ void bred(BlockRed &R, double (&v)[3], double &m) {
   __syncthreads();
 #pragma unroll
   for (int k = 0; k < NV; ++k) v[k] = 0.0;
-  for (int w = 0; w < (int)(blockDim.x >> 6); w += 4) {
+  each_wave<BS>([&](int w) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-#pragma unroll
-      for (int k = 0; k < NV; ++k) v[k] += R.v[w + u][k];
-      m = fmax(m, R.v[w + u][3]);
-    }
-  }
+    for (int k = 0; k < NV; ++k) v[k] += R.v[w][k];
+    m = fmax(m, R.v[w][3]);
+  });
   __syncthreads();
 }
 
@@ -582,7 +591,8 @@ __global__ __launch_bounds__(GH_BWG) void k_batch_force(BatchArgs B, BForm<MIXED
 }
 
 // epot (ui) and ekin about the centre of mass (ui) of one system.
-__device__ void sys_energies(const BatchArgs &B, BlockRed &R, int a0, int a1, double &epot,
+template <int BS>
+__device__ void sys_energies(const BatchArgs &B, BlockRed<BS> &R, int a0, int a1, double &epot,
                              double &ekin) {
   double s[5] = {0, 0, 0, 0, 0};
   for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
@@ -593,7 +603,7 @@ __device__ void sys_energies(const BatchArgs &B, BlockRed &R, int a0, int a1, do
     s[3] += m * B.vel[B.ld + i];
     s[4] += m * B.vel[2 * B.ld + i];
   }
-  bsum<5>(R, s);
+  bsum<BS, 5>(R, s);
   const double cx = s[2] / s[1], cy = s[3] / s[1], cz = s[4] / s[1];
   double k[1] = {0.0};
   for (int i = a0 + threadIdx.x; i < a1; i += blockDim.x) {
@@ -601,13 +611,13 @@ __device__ void sys_energies(const BatchArgs &B, BlockRed &R, int a0, int a1, do
     const double wx = B.vel[i] - cx, wy = B.vel[B.ld + i] - cy, wz = B.vel[2 * B.ld + i] - cz;
     k[0] += (wx * wx + wy * wy + wz * wz) * m;
   }
-  bsum<1>(R, k);
+  bsum<BS, 1>(R, k);
   epot = s[0];
   ekin = 0.5 * k[0];
 }
 // The energies of every system, a workgroup each.
 __global__ __launch_bounds__(GH_BWG) void k_batch_energies(BatchArgs B) {
-  __shared__ BlockRed R;
+  __shared__ BlockRed<GH_BWG> R;
   const int s = blockIdx.x;
   double ep, ek;
   sys_energies(B, R, B.off[s], B.off[s + 1], ep, ek);
@@ -851,8 +861,9 @@ __device__ __forceinline__ void fire_force(const BatchArgs &B, const Stage &S,
   }
 }
 
-template <bool MIXED, bool QUANT, bool SINGLE, int G>
-__global__ __launch_bounds__(1024, 4) void k_batch_fire(BatchArgs B, FireC fc_arg, double skin_arg,
+// (G lanes per atom; BS threads, 0: as launched)
+template <bool MIXED, bool QUANT, bool SINGLE, int G, int BS>
+__global__ __launch_bounds__(BS ? BS : 1024, 4) void k_batch_fire(BatchArgs B, FireC fc_arg, double skin_arg,
                                                        FireState *fst, BForm<MIXED> p_arg) {
   // The constants live in LDS and are read where they are used: held in
   // scalar registers for a whole kernel of this kind they were spilled, and
@@ -863,7 +874,7 @@ __global__ __launch_bounds__(1024, 4) void k_batch_fire(BatchArgs B, FireC fc_ar
   __shared__ BForm<MIXED> p1;
   extern __shared__ int4 dyn_q[];
   __shared__ BTable<MIXED, SINGLE> T;
-  __shared__ BlockRed R;
+  __shared__ BlockRed<BS> R;
   __shared__ int sfar;
   // Systems come largest first and 256 workgroups fill one slot on each CU:
   // every other 256 run in reverse, so that a CU's systems add up alike (1024
@@ -908,7 +919,7 @@ __global__ __launch_bounds__(1024, 4) void k_batch_fire(BatchArgs B, FireC fc_ar
   // the mixing of the last iteration, still to be applied to v: v <- cm v + mixv F
   double cm = 1.0, mixv = 0.0;
   bool pend = false;
-  bred<0>(R, pv, fm2);
+  bred<BS, 0>(R, pv, fm2);
   double dt = st.dt, alpha = st.alpha, fnow = sqrt(fm2) * fc.ui_ev;  // eV/A
   int it = st.it, npos = st.npos;
   bool stop = false;
@@ -955,12 +966,12 @@ __global__ __launch_bounds__(1024, 4) void k_batch_fire(BatchArgs B, FireC fc_ar
       if (QUANT) stage_atom(S, k, x, o);
     }
     double none[3] = {0.0, 0.0, 0.0};
-    bred<0>(R, none, d2);
+    bred<BS, 0>(R, none, d2);
     if (2.0 * sqrt(d2) > skin) sys_build<QUANT>(B, S, a0, n);
     pv[0] = pv[1] = pv[2] = fm2 = 0.0;
     fire_rho<MIXED, QUANT, SINGLE, G>(B, S, T, p1, a0, n);
     fire_force<MIXED, QUANT, SINGLE, kForce, G>(B, S, T, p1, a0, n, 0.5 * dt, pv, fm2);
-    bred<3>(R, pv, fm2);
+    bred<BS, 3>(R, pv, fm2);
     fnow = sqrt(fm2) * fc.ui_ev;
     pend = true;
     if (pv[0] > 0.0) {
@@ -1287,26 +1298,20 @@ static int staged_threads(const gh_batch *b) {
   return bs;
 }
 
-// How many of the systems, largest first, take one lane per atom: those of one
-// and a half times the workgroup's threads and more.  Their wavefronts are full
-// either way, and four lanes pay a row's padding and the sums four times (50
-// Langevin steps, Ag-Cu, ms, four lanes and one: 150 systems of 2,000 atoms 9.2 and
-// 7.9, 1000 of 400 5.6 and 5.1, 1000 of 309 4.2 and 4.3, 600 of 147 2.0 and 2.5).
-static int split_systems(const gh_batch *b, int bs) {
-  int k = 0;
-  while (k < b->nsys) {
-    const int s = b->order_h[k];
-    if (2 * (b->off_h[s + 1] - b->off_h[s]) < 3 * bs) break;
-    ++k;
-  }
-  return k;
-}
-
-// Runs launch(lanes, first, count, stream) for the systems of one lane per atom
-// and of four, on two streams where there are both.
+// Runs launch(lanes, first, count, stream) for the systems of one lane per atom,
+// those of `least` atoms and more (systems come largest first), and of four, on
+// two streams where there are both.  One and a half times the workgroup's threads:
+// its wavefronts are full either way, and four lanes pay a row's padding and the
+// sums four times (50 Langevin steps, Ag-Cu, ms, four lanes and one: 150 systems of
+// 2,000 atoms 9.2 and 7.9, 1000 of 400 5.6 and 5.1, 1000 of 309 4.2 and 4.3, 600 of 147
+// 2.0 and 2.5).
 template <class LAUNCH>
-static int launch_split(gh_batch *b, int bs, LAUNCH &&launch) {
-  const int one = split_systems(b, bs);
+static int launch_split(gh_batch *b, int least, LAUNCH &&launch) {
+  int one = 0;
+  for (; one < b->nsys; ++one) {
+    const int s = b->order_h[one];
+    if (b->off_h[s + 1] - b->off_h[s] < least) break;
+  }
   const bool both = one > 0 && one < b->nsys;
   if (both) {
     BH(b, hipEventRecord(b->ev_fork, b->stream));
@@ -1358,15 +1363,24 @@ static int launch_fire(gh_batch *b, const BatchArgs &A, const FireC &fc, const B
   BatchArgs A1 = A;
   auto launch = [&](int lanes, int first, int count, hipStream_t stream) {
     A1.first = first;
-#define LAUNCH_FIRE(SG, G) \
-  k_batch_fire<MIXED, QUANT, SG, G><<<count, bs, lds, stream>>>(A1, fc, b->skin, b->fst, p)
-    if (b->nt == 1 && lanes == 1) LAUNCH_FIRE(true, 1);
-    else if (b->nt == 1) LAUNCH_FIRE(true, GH_FG);
-    else if (lanes == 1) LAUNCH_FIRE(false, 1);
-    else LAUNCH_FIRE(false, GH_FG);
+#define LAUNCH_FIRE(SG, G, BS) \
+  k_batch_fire<MIXED, QUANT, SG, G, BS><<<count, bs, lds, stream>>>(A1, fc, b->skin, b->fst, p)
+    if (b->nt == 1) {
+      if (lanes == 1) LAUNCH_FIRE(true, 1, 0);
+      else if (bs == 1024) LAUNCH_FIRE(true, GH_FG, 1024);
+      else if (bs == 512) LAUNCH_FIRE(true, GH_FG, 512);
+      else LAUNCH_FIRE(true, GH_FG, GH_FBS);
+    } else {
+      if (lanes == 1) LAUNCH_FIRE(false, 1, 0);
+      else if (bs == 1024) LAUNCH_FIRE(false, GH_FG, 1024);
+      else if (bs == 512) LAUNCH_FIRE(false, GH_FG, 512);
+      else LAUNCH_FIRE(false, GH_FG, GH_FBS);
+    }
 #undef LAUNCH_FIRE
   };
-  return launch_split(b, bs, launch);
+  // (FP64 of one type is short of registers either way: 40 iterations, four lanes and
+  // one, 1000 systems of 400 atoms 8.3 and 8.9 ms, 300 of 2000 27.3 and 26.4)
+  return launch_split(b, !MIXED && b->nt == 1 ? 3 * bs : bs + bs / 2, launch);
 }
 
 static int batch_blocks(const gh_batch *b, int lanes) {
@@ -1691,7 +1705,7 @@ int gh_batch_langevin(gh_batch *b, int nsteps, double dt, double gamma, uint64_t
         else LAUNCH_LANGEVIN(false, GH_FG);
 #undef LAUNCH_LANGEVIN
       };
-      BT(launch_split(b, bs, launch));
+      BT(launch_split(b, bs + bs / 2, launch));
     }
     for (int st = 0; st < nsteps && !batch_staged(b); ++st) {
       const long long step = step0 + st;
