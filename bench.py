@@ -410,7 +410,7 @@ def au_32k(hip, steps=2000, warmup=20):
 def batch_re(hip, rounds, swap_every=500):
     """Replica-exchange Langevin of 512 Ag-Cu clusters (64 geometries x 8
     temperatures, 300..900 K geometric), friction 1/ps, dt 2 fs, swaps every
-    `swap_every` steps; two launches per step over all clusters."""
+    `swap_every` steps; each interval a workgroup per cluster, staged in LDS."""
     from gems_amd import clusters as CL
     off, x, t, T, lad = CL.agcu_re_batch()
     b = hip.Batch(0, hip.GH_MIXED)

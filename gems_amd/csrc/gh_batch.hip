@@ -7,14 +7,16 @@
 // (Integration.F90:963-1031).  A system's atoms are contiguous; all state is
 // FP64 in HBM (SoA with stride ld).
 //
-// Forces and Langevin dynamics run over the atoms of all systems at once, 16
+// Forces and most Langevin dynamics run over the atoms of all systems at once, 16
 // or 8 lanes per atom, two launches per step (density; forces with the update to
 // the next step): a step then costs the chip's throughput, not the time one
 // compute unit needs for the largest cluster (a workgroup per system took 170
 // us per step for 2,000 atoms while the compute units of the smaller systems
 // idled; 128 Ag-Cu clusters of 38..2000 atoms, mixed: 206 -> 68 us per step;
-// 16 clusters of 38..600 96 -> 18).  FIRE, whose every iteration needs sums over each system, keeps a
-// workgroup per system (largest first) and all iterations in one launch.
+// 16 clusters of 38..600 96 -> 18).  Mixed batches that fill the chip with a
+// workgroup per system all the same, or whose systems are tiny, take all Langevin
+// steps in one launch (k_batch_langevin, by batch_staged), and FIRE, whose every
+// iteration needs sums over each system, all iterations (largest system first).
 //
 // Neighbour rows: cap 16-bit indices local to the system, contiguous per
 // atom; the pairs inside the inner bound at build time fill a row from its
@@ -488,7 +490,7 @@ struct ErmakC {
 // The workgroup's displacements folded into their systems' maxima: one atomic
 // where its atoms share a system, one per atom otherwise.  Each maximum has a
 // cache line of its own (128 of them on eight lines, one atomic per
-// wavefront: 66 us per step more at 82,000 atoms).  d2: the same in a group's
+// wavefront: 66 us per step more at 67,896 atoms).  d2: the same in a group's
 // lanes; all threads call it.
 template <int G>
 __device__ __forceinline__ void fold_sys_disp2(const BatchArgs &B, double d2, int s, bool live,
@@ -1027,7 +1029,7 @@ __global__ __launch_bounds__(BS ? BS : 1024, 4) void k_batch_fire(BatchArgs B, F
 // the passes over all atoms, and no launches per step.  Chosen by batch_staged,
 // its threads by staged_threads; the first step's ermak_a has run.
 //
-// G lanes per atom: four, or one in large systems (split_systems).  The update
+// G lanes per atom: four, or one in large systems (launch_split).  The update
 // takes a thread per atom and axis and draws each normal once: the next step's
 // pair waits in pos_next, which the passes over all atoms rewrite (150 systems of
 // 2,000 Ag-Cu atoms, 50 steps: 8.3 -> 7.9 ms).
@@ -1259,10 +1261,12 @@ static int batch_ready(gh_batch *b) {
     b->cap = (b->cap + 7) / 8 * 8;
     BT(balloc(b, &b->list, (size_t)b->cap * b->ld));
     // LDS staging of the largest system (int4 + type byte per atom, and the
-    // sentinel) beside tables of 344 B per type pair, within 64 KB; larger
+    // sentinel) beside tables of 344 B per type pair and the sums of eight
+    // wavefronts, within 64 KB: 3,799 atoms of one type, 2,525 of several; larger
     // systems use global memory.  The rule also says which FP32 form a mixed
-    // batch computes (quantised positions where it holds), so it does not
-    // follow the size of the tables' structures.
+    // batch computes (quantised positions where it holds), so it follows neither
+    // the size of the tables' structures nor the kernels' threads (with 1024 they
+    // hold up to 65.8 KB in all, of the 160 KB of a compute unit).
     const size_t stat = (b->nt > 1 ? GH_MAXT * GH_MAXT : 1) * 344 +
                         sizeof(double) * 8 * 8 + 64;
     const size_t need = 17 * (size_t)(nmax + 1);

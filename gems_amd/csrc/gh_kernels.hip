@@ -528,7 +528,8 @@ __device__ __forceinline__ void block_sum_dd(double (&s)[NV], double (&c)[NV]) {
 
 // True in every thread of the grid's last workgroup to arrive, whose reads then
 // see the others' writes; the ticket is left at zero.  (256 workgroups at
-// most: each arrival is a fence.)
+// most in the reductions, 512 in k_row_force's sum of the calls without
+// allocation: each arrival is a fence.)
 __device__ __forceinline__ bool last_block(unsigned *ticket) {
   __shared__ bool last;
   __syncthreads();

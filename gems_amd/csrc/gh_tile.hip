@@ -2141,9 +2141,9 @@ static BuildArgs build_args(const gh_ctx *c, int cap, size_t *lds_out) {
 // sizing count (cap 0, any halo), slot numbers beyond the 14 bits a tagged
 // row entry leaves, or LDS too small for one cell's candidate lists beside
 // the staged halo.  The per-thread build is left for those (us a rebuild,
-// per thread and cooperative: 1M-atom SMA-TB, mixed, 558 and 428, 500,000 atoms
-// FP64 386 and 280, 442,000 Ag-Cu 393 and 246, the 1M-atom LJ liquid 1271 and 630,
-// 4,000 atoms 235 and 37).
+// per thread and cooperative: 1M-atom SMA-TB, mixed, 501 and 385, 500,000 atoms
+// FP64 386 and 280, 442,000 Ag-Cu 393 and 246, the 1M-atom LJ liquid 1028 and 570,
+// 4,000 atoms 231 and 23).
 static bool coop_args(const gh_ctx *c, BuildArgs &A, size_t *lds_out) {
   const int slot_cap = c->tg.slot_cap;
   if (c->list_rows == 1 || A.cap <= 0 || slot_cap >= 16000) return false;

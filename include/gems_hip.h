@@ -274,10 +274,13 @@ int gh_get_timing(gh_ctx *ctx, double ms[4], int64_t count[4]);
  * (src/Program_Types.F90:89-102) and replica exchange as one replica per MPI
  * rank (src/ReplicaExchange.f90:27-151); a batch holds many independent
  * unboxed systems on one device and advances all of them together (Langevin:
- * two launches per step over all atoms; FIRE: one launch, a workgroup per
- * system, largest first).  Neighbour lists are the O(N^2)
- * verlet_self lists of each system (Neighbour.F90:676-759); forces are the
- * SMA-TB passes of TB.F90:367-586; Langevin is ermak_a/ermak_b
+ * two launches per step over all atoms, or, in mixed batches whose atoms
+ * outnumber the largest system's 115 to 144 times or whose systems hold 32 atoms
+ * at most, all steps in one launch with a workgroup per system; FIRE: a
+ * workgroup per system and all iterations in one launch, largest first).  Large
+ * and small systems of such a launch run as two, beside one another.  Neighbour
+ * lists are the O(N^2) verlet_self lists of each system (Neighbour.F90:676-759);
+ * forces are the SMA-TB passes of TB.F90:367-586; Langevin is ermak_a/ermak_b
  * (Integration.F90:963-1031) with the Philox stream.
  * ------------------------------------------------------------------------ */
 typedef struct gh_batch gh_batch;
